@@ -87,7 +87,8 @@ inline long cdiv(long a, long b) { return (a + b - 1) / b; }
 // weight-streaming kernel is not built.
 constexpr int64_t kStreamMaxP = 2048;
 constexpr size_t kWeightSlack = 32768;  // bytes of mapped memory kept behind weight planes (the streaming kernel walks 96 blocks per tile whatever K is)
-constexpr int kStreamWgPerCu = 2;  // resident workgroups of the streaming kernel per compute unit
+constexpr int kStreamWgPerCu = 2;  // resident workgroups of the streaming kernel per compute unit ...
+constexpr size_t kStreamLdsHalf = 80 * 1024 - 512;  // ... if each takes no more LDS than this (and its few static words)
 
 // ---- workspace shared by every layer (single stream, one call at a time) --
 struct Workspace {
@@ -425,17 +426,48 @@ int launch_mx3(const float* x, uint16_t* x3, int64_t rows, int64_t H, const int*
   return check_launch("mx3_rows_kernel");
 }
 
-// Small batches stream the weights once (HBM-bound, activations quantised in the kernel); larger
+// Tokens of an expert contracted per pass over its weights by the streaming kernel.  An
+// expert with more tokens than that is streamed once per group, so larger batches take
+// as many as two workgroups per compute unit can hold in LDS at the longer of the two row
+// lengths (seven at K = 2880, measured against six: 20b T = 64 162 -> 151 us, 120b T = 64
+// 245 -> 239 us); up to 16 tokens few experts see more than four, the second pass of those
+// that do is served by the memory-side cache, and the four-token form is marginally the
+// faster one (measured at T = 8, 16, 32).
+inline int stream_group_tokens(int64_t T, int64_t H, int64_t F) {
+  if (T == 1) return 1;
+  if (T <= 16) return kStreamG;
+  const int ns = std::max(stream_steps((int)(H / 32)), stream_steps((int)(F / 32)));
+  return ns <= 3 ? 12 : ns <= 5 ? 8 : ns == 6 ? 7 : ns == 8 ? 5 : kStreamG;
+}
+
+// Small batches stream the weights (HBM-bound, activations quantised in the kernel); larger
 // ones run the grouped GEMM on the block-scaled matrix instruction (three-term FP6
 // activations).  One decision per forward: it fixes the activation format of both GEMMs.
-// What counts is tokens per expert: a 64-token M tile of the GEMM that holds a handful of
-// tokens costs as much as a full one, while the streaming kernel passes over an expert once
-// per seven of its tokens.  Measured crossover: about twelve assignments per expert (20b
-// shape: T = 96 a tie, T = 128 the GEMM 16 % faster; 120b shape: T = 128 streaming 17 %
-// faster, T = 256 8 %, T = 512 the GEMM 33 % faster).
+// The GEMM passes over an expert once per 64 of its tokens but has about 25 us more of
+// latency in front and behind; the streaming kernel passes over it once per token group, so
+// what counts is how many bytes are streamed again by second and further passes.  Both move
+// about 5 TB/s, hence the line at 120 MB of repeated weights.  Measured (layer, us, streaming
+// / GEMM), m assignments per expert: 128 x 2880 x 2880 (1.7 GB) m = 2 308 / 350, 4 400 / 396,
+// 8 505 / 409; 32 experts of it m = 6 124 / 124, 8 141 / 125; 8 experts m = 4 50 / 66, 12 70 / 69,
+// 16 75 / 70; 16 x 4096 x 6144 (0.6 GB, groups of four) m = 4 164 / 164, 6 207 / 165.  Tokens per
+// expert are taken as Poisson distributed about m.
 bool stream_path(int64_t T, int64_t H, int64_t F, int64_t E, int64_t k) {
-  if (H / 32 > 96 || F / 32 > 96) return false;
-  return T <= 64 || (T * k <= 10 * E && T * k <= kStreamMaxP);
+  if (H / 32 > kStreamMaxBlocks || F / 32 > kStreamMaxBlocks || T * k > kStreamMaxP) return false;
+  const int g = stream_group_tokens(T, H, F);
+  const double m = std::min((double)(T * k) / (double)E, (double)T);
+  if (T > 64 && m > g) return false;  // two passes and more, however small the matrices
+  double again = 0.0;  // expected passes per expert beyond the first
+  if (m > 64.0) {
+    again = m / g - 1.0;
+  } else {
+    double p = std::exp(-m), above = 1.0 - p;  // P(n), P(more than n)
+    for (int n = 1; above > 1e-4; ++n) {
+      p *= m / n;
+      above -= p;
+      if (n % g == 0) again += std::max(above, 0.0);
+    }
+  }
+  return again * (double)(E * 3 * H * F) * (17.0 / 32.0) <= 120e6;
 }
 
 // mx3_out: also rewrite the rows x as FP6 terms (the grouped GEMM's operand), riding on the
@@ -479,56 +511,93 @@ int launch_router(const float* x, const float* gate_w, const float* gate_b, int6
   return check_launch("router_topk_kernel");
 }
 
-// Tokens of an expert contracted per pass over its weights by the streaming kernel.  An
-// expert with more tokens than that is streamed once per group, so larger batches take
-// groups of seven (what two workgroups per compute unit can hold in LDS; measured against
-// six: 20b T = 64 162 -> 151 us, 120b T = 64 245 -> 239 us); up to 16 tokens few experts see
-// more than four, the second pass of those that do is served by the memory-side cache, and
-// the four-token form is marginally the faster one (measured at T = 8, 16, 32).
-inline int stream_group_tokens(int64_t T) { return T <= 16 ? kStreamG : kStreamGWide; }
-
 int launch_dispatch(const int* ids, const float* pairs, int64_t P, int64_t k, int64_t E,
-                    const ExpertW* ew, Workspace& ws) {
+                    const ExpertW* ew, Workspace& ws, int group_tokens) {
   dispatch_scatter_kernel<<<dim3((unsigned)cdiv(std::max<int64_t>(P, 1), kDispatchThreads)), kDispatchThreads, 0, g_stream>>>(
       ids, pairs, (int)P, (int)k, (int)E, ws.counts, ew, ws.offsets, ws.desc,
       P <= kStreamMaxP ? ws.groups : nullptr, ws.nv, ws.tiles, ws.n_tiles, ws.list_tok, ws.list_w,
-      ws.pos, stream_group_tokens(P / std::max<int64_t>(k, 1)));
+      ws.pos, group_tokens);
   return check_launch("dispatch_scatter_kernel");
 }
 
 // Weight-streaming kernel for small batches (every expert sees few tokens, the
 // layer is HBM-bound); grouped GEMM otherwise.
-template <int NMAT, int G, bool ROUTE1 = false>
+template <int MODE, int LG, int NS, bool ROUTE1>
+int launch_stream_form(ExpertStreamArgs a, int64_t P) {
+  // kStreamWgPerCu workgroups per compute unit in steady state (one where the rows of a
+  // group take more than half of the LDS); a batch so small that every work unit can have a
+  // resident workgroup of its own gets that
+  constexpr int TU = MODE == 0 ? stream_tiles(NS) / 2 : stream_tiles(NS);
+  size_t lds = stream_lds_bytes(NS, LG, a.group_tokens);
+  if (ROUTE1) lds = std::max(lds, sizeof(CloseCallLds));  // a close call is recomputed where the rows go afterwards
+  const int64_t units = cdiv(a.ntile, TU);
+  const int64_t places = (lds <= kStreamLdsHalf ? kStreamWgPerCu : 1) * (int64_t)std::max(g_cus, 1);
+  const int64_t nwg = LG == 1 ? std::min(P * units, places) : places;
+  static bool lds_attr_set = false;  // per instantiation: dynamic LDS beyond the default limit is asked for once
+  if (!lds_attr_set) {
+    HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(&expert_stream_kernel<MODE, LG, NS, ROUTE1>),
+                                hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)std::max(stream_lds_bytes(NS, LG, 4 * LG), sizeof(CloseCallLds))));
+    lds_attr_set = true;
+  }
+  launch_expert_kernel(MODE, expert_stream_kernel<MODE, LG, NS, ROUTE1>, dim3((unsigned)nwg), dim3(256), lds, a);
+  return check_launch("expert_stream_kernel");
+}
+template <int MODE, int LG, bool ROUTE1 = false>
+int launch_stream_steps(const ExpertStreamArgs& a, int64_t P) {
+  switch (stream_steps(a.nblk)) {
+    case 2: return launch_stream_form<MODE, LG, 2, ROUTE1>(a, P);
+    case 3: return launch_stream_form<MODE, LG, 3, ROUTE1>(a, P);
+    // the longer rows come in smaller groups (stream_group_tokens)
+    case 4: if constexpr (LG <= 2) return launch_stream_form<MODE, LG, 4, ROUTE1>(a, P); break;
+    case 5: if constexpr (LG <= 2) return launch_stream_form<MODE, LG, 5, ROUTE1>(a, P); break;
+    case 6: if constexpr (LG <= 2) return launch_stream_form<MODE, LG, 6, ROUTE1>(a, P); break;
+    case 8: if constexpr (LG <= 2) return launch_stream_form<MODE, LG, 8, ROUTE1>(a, P); break;
+    case 12: if constexpr (LG <= 1) return launch_stream_form<MODE, LG, 12, ROUTE1>(a, P); break;
+    case 16: if constexpr (LG <= 1) return launch_stream_form<MODE, LG, 16, ROUTE1>(a, P); break;
+  }
+  return fail(CSK_ERR_STATE, "expert_stream_kernel: token groups too large for these rows");
+}
+template <int MODE>
 int launch_stream(ExpertStreamArgs a, int64_t P, Workspace& ws) {
   a.groups = ws.groups;
   a.nv = ws.nv;
-  // kStreamWgPerCu workgroups per compute unit in steady state; a batch so small that
-  // every work unit can have a resident workgroup of its own gets that
-  const int64_t npair = NMAT == 2 ? a.ntile : (a.ntile + 1) / 2;
-  const int64_t cus = std::max(g_cus, 1);
-  const int64_t nwg = (G == kStreamG && P * npair <= kStreamWgPerCu * cus) ? P * npair : kStreamWgPerCu * cus;  // (small P implies G == kStreamG)
-  // activation rows as three FP6 terms (96 B per block, 96 blocks per row: zeros past K) + the reduction buffers
-  size_t lds = (size_t)G * 96 * (kMx3ChunksPerBlock * 16) + (size_t)2 * 4 * ((G + 3) / 4) * 8 * 16 * sizeof(float);
-  if (ROUTE1) lds = std::max(lds, sizeof(CloseCallLds));  // a close call is recomputed where the rows go afterwards
-  static bool lds_attr_set = false;  // per instantiation: dynamic LDS beyond the default limit is asked for once
+  if constexpr (MODE == 0)
+    if (a.rin.logits) return launch_stream_steps<MODE, 1, true>(a, P);  // one token, routed by the kernel itself
+  return a.group_tokens <= 4 ? launch_stream_steps<MODE, 1>(a, P)
+         : a.group_tokens <= 8 ? launch_stream_steps<MODE, 2>(a, P)
+                               : launch_stream_steps<MODE, 3>(a, P);
+}
+
+// Weight rows per work unit of the grouped GEMM: 512, or 256 where that many leave the chip
+// short of units or where an M tile holds few tokens -- the matrix work per activation byte,
+// which the tall tile is for, does not matter while the weights are what is waited for.
+// Measured (layer, us, 512 / 256 rows): 32 experts of 2880 x 2880 m = 8 135 / 125, 16 141 / 131, 32
+// 157 / 155, 64 222 / 221, 256 440 / 478; 8 experts m = 4 80 / 66; 128 experts m = 8 412 / 409, 32 488 / 505.
+bool gemm_wide_tiles(int64_t E, int64_t P, int64_t ntile) {
+  const int64_t mtiles = P / kGemmBM + std::min<int64_t>(E, P);
+  return P > 16 * E && mtiles * cdiv(ntile, 4 * kMxNG) > 2 * std::max(g_cus, 1);
+}
+template <int MODE, int NG>
+int launch_gemm_mx(ExpertGemmMxArgs& ga, int64_t E, int64_t P) {
+  using Geom = MxGeom<NG, 2>;
+  ga.n_ntiles = (int)cdiv(ga.ntile, Geom::tiles_per_wg(MODE));
+  static bool lds_attr_set = false;
   if (!lds_attr_set) {
-    HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(&expert_stream_kernel<NMAT == 2 ? 0 : 1, G, ROUTE1>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(&expert_gemm_mx_kernel<MODE, NG>),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)Geom::kLdsBytes));
     lds_attr_set = true;
   }
-  launch_expert_kernel(NMAT == 2 ? 0 : 1, expert_stream_kernel<NMAT == 2 ? 0 : 1, G, ROUTE1>, dim3((unsigned)nwg), dim3(256), lds, a);
-  return check_launch("expert_stream_kernel");
+  const int64_t max_mtiles = P / kGemmBM + std::min<int64_t>(E, P);
+  const dim3 grid((unsigned)(cdiv(max_mtiles * ga.n_ntiles, kDies) * kDies));
+  launch_expert_kernel(MODE, expert_gemm_mx_kernel<MODE, NG>, grid, dim3(64 * kMxWaves), Geom::kLdsBytes, ga);
+  return check_launch("expert_gemm_mx_kernel");
 }
 
 template <int NMAT>
 int launch_experts(ExpertStreamArgs a, const uint16_t* a_mx3, uint16_t* act_mx3, int64_t E, int64_t T, int64_t P,
                    Workspace& ws, bool stream) {
-  if (stream) {
-    if constexpr (NMAT == 2)
-      if (a.rin.logits) return launch_stream<NMAT, kStreamG, true>(a, P, ws);  // one token, routed by the kernel itself
-    return stream_group_tokens(T) == kStreamG ? launch_stream<NMAT, kStreamG>(a, P, ws)
-                                              : launch_stream<NMAT, kStreamGWide>(a, P, ws);
-  }
+  if (stream) return launch_stream<NMAT == 2 ? 0 : 1>(a, P, ws);
   ExpertGemmMxArgs ga{};
   ga.desc = a.desc;
   ga.mtiles = ws.tiles;
@@ -541,24 +610,13 @@ int launch_experts(ExpertStreamArgs a, const uint16_t* a_mx3, uint16_t* act_mx3,
   ga.act_type = a.act_type;
   ga.act_out = reinterpret_cast<u32x4*>(act_mx3);
   ga.y_out = a.y_out;
-  using Geom = MxGeom<kMxNG, 2>;
-  constexpr int kMode = NMAT == 2 ? 0 : 1;
   if (a.ntile % 2) return fail(CSK_ERR_ARG, "grouped GEMM: the number of output features must be a multiple of 32");
-  ga.n_ntiles = (int)cdiv(a.ntile, Geom::tiles_per_wg(kMode));
   // per-lane offsets into the activation rows are 32-bit (the weight offsets are tile-relative)
   const int64_t a_rows = a.list_row ? T : P;
   if (a_rows * mx3_row_blocks(a.nblk) * 96 >= ((int64_t)1 << 32))
     return fail(CSK_ERR_ARG, "batch too large for the grouped GEMM (activation rows exceed 4 GiB)");
-  static bool lds_attr_set[2] = {false, false};
-  if (!lds_attr_set[kMode]) {
-    HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(&expert_gemm_mx_kernel<kMode, kMxNG>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)Geom::kLdsBytes));
-    lds_attr_set[kMode] = true;
-  }
-  const int64_t max_mtiles = P / kGemmBM + std::min<int64_t>(E, P);
-  const dim3 grid((unsigned)(cdiv(max_mtiles * ga.n_ntiles, kDies) * kDies));
-  launch_expert_kernel(kMode, expert_gemm_mx_kernel<kMode, kMxNG>, grid, dim3(64 * kMxWaves), Geom::kLdsBytes, ga);
-  return check_launch("expert_gemm_mx_kernel");
+  constexpr int kMode = NMAT == 2 ? 0 : 1;
+  return gemm_wide_tiles(E, P, a.ntile) ? launch_gemm_mx<kMode, kMxNG>(ga, E, P) : launch_gemm_mx<kMode, kMxNG / 2>(ga, E, P);
 }
 
 // Activation rows of the expert MLPs.  The streaming path reads them as fp32 (`x`, row of a
@@ -578,12 +636,12 @@ struct ExpertInput {
 
 // Experts' MLPs over the dispatched tokens: ws.y[P,H] <- down(act(gate, up)).
 int run_experts(int64_t E, int64_t T, int64_t k, int64_t H, int64_t F,
-                int act_type, const ExpertInput& in, Workspace& ws, bool timed = false) {
+                int act_type, const ExpertInput& in, Workspace& ws, bool stream, bool timed = false) {
   const int64_t P = T * k;
-  const bool stream = stream_path(T, H, F, E, k);
   ExpertStreamArgs a{};
   a.desc = ws.desc;
   a.act_type = act_type;
+  a.group_tokens = stream_group_tokens(T, H, F);
   // a single token of a routed layer names k different experts: k token groups, known here
   a.nv_known = (stream && T == 1 && E > 1) ? (int)k : 0;
   // gate/up + activation
@@ -1678,6 +1736,7 @@ int forward_pass(csk_layer* L, const float* hidden, int64_t T, float* out, int f
   }
   const int64_t P = T * L->k;
   const bool norm = (flags & CSK_FWD_RMSNORM) != 0;
+  const bool stream = !L->f16 && stream_path(T, L->H, L->F, L->E, L->k);
   const float* xr = norm ? ws.xn : hidden;
   bool route_in_kernel = false, rows_mx3_ready = false;
   RouteIn rin_kept{};
@@ -1688,9 +1747,10 @@ int forward_pass(csk_layer* L, const float* hidden, int64_t T, float* out, int f
     // small batch: prologue + logits in one launch, top-k + dispatch in another
     mark(CSK_STAGE_PREP);
     mark(CSK_STAGE_ROUTER);
-    // the streaming kernels copy their token rows as FP6 terms, written once per token by the
-    // prologue workgroups of this launch (not when the routing weight multiplies the rows first)
-    u32x4* rows_mx3 = (!L->f16 && !L->wbf && stream_path(T, L->H, L->F, L->E, L->k)) ? reinterpret_cast<u32x4*>(ws.xs) : nullptr;
+    // the expert kernels of either kind read their token rows as FP6 terms, written once per
+    // token by the prologue workgroups of this launch (not when the routing weight multiplies
+    // the rows first)
+    u32x4* rows_mx3 = (!L->f16 && !L->wbf) ? reinterpret_cast<u32x4*>(ws.xs) : nullptr;
     rows_mx3_ready = rows_mx3 != nullptr;
     // a workgroup takes one expert (latency) as long as all of them are resident at once, four beyond
     if (cdiv(T, 4) * (L->E + 4) <= 4 * std::max(g_cus, 1) + 64)  // four of these workgroups fit a compute unit
@@ -1704,15 +1764,15 @@ int forward_pass(csk_layer* L, const float* hidden, int64_t T, float* out, int f
     if ((rc = check_launch("router_prep_logits_kernel")) != CSK_OK) return rc;
     mark(CSK_STAGE_DISPATCH);
     RouteIn rin{ws.logits, xr, L->gate_w, L->has_gate_b ? L->gate_b : nullptr, L->ew_dev,
-                (int)T, (int)L->E, (int)L->k, (int)L->H, L->sigmoid, stream_group_tokens(T)};
+                (int)T, (int)L->E, (int)L->k, (int)L->H, L->sigmoid, stream_group_tokens(T, L->H, L->F)};
     RouteOut rout{ws.pairs, ws.ids, ws.pos, ws.counts, ws.offsets, ws.desc, ws.groups, ws.nv,
                   ws.tiles, ws.n_tiles, ws.list_tok, ws.list_w};
-    if (T == 1 && phase == 0 && L->E > 1 && !L->f16 && stream_path(T, L->H, L->F, L->E, L->k)) {
+    if (T == 1 && phase == 0 && L->E > 1 && stream) {
       // one token: the gate/up kernel routes it itself (no launch here); phases keep the
       // routing kernel, whose output they hand out before the experts run
       route_in_kernel = true;
       rin_kept = rin, rout_kept = rout;
-    } else if (T <= kRouteTinyTokens && P <= kRouteTinyMaxP && !L->f16 && stream_path(T, L->H, L->F, L->E, L->k)) {
+    } else if (T <= kRouteTinyTokens && P <= kRouteTinyMaxP && stream) {
       // a handful of tokens on the streaming kernels: each active expert is one token group
       route_tiny_kernel<<<dim3(1), 256, 0, g_stream>>>(rin, rout);
       if ((rc = check_launch("route_tiny_kernel")) != CSK_OK) return rc;
@@ -1723,18 +1783,13 @@ int forward_pass(csk_layer* L, const float* hidden, int64_t T, float* out, int f
           ws.logits, ws.pairs, ws.ids, (int)T, (int)L->E, (int)L->k, L->sigmoid, xr, L->gate_w,
           L->has_gate_b ? L->gate_b : nullptr, (int)L->H, ws.logits + T * L->E, 0, Mx3Rider{});
       if ((rc = check_launch("router_topk_kernel")) != CSK_OK) return rc;
-      if ((rc = launch_dispatch(ws.ids, ws.pairs, P, L->k, L->E, L->ew_dev, ws)) != CSK_OK) return rc;
+      if ((rc = launch_dispatch(ws.ids, ws.pairs, P, L->k, L->E, L->ew_dev, ws, stream_group_tokens(T, L->H, L->F))) != CSK_OK) return rc;
     } else {
       route_small_kernel<<<dim3(1), kRouteSmallThreads, 0, g_stream>>>(rin, rout);
       if ((rc = check_launch("route_small_kernel")) != CSK_OK) return rc;
     }
-    if (!L->f16 && !stream_path(T, L->H, L->F, L->E, L->k) && !L->wbf) {
-      // few tokens but rows too long for the streaming kernel: the GEMM wants the FP6 form
-      if ((rc = launch_mx3(xr, ws.xs, T, L->H, nullptr, nullptr)) != CSK_OK) return rc;
-    }
   } else {
     mark(CSK_STAGE_PREP);
-    const bool stream = !L->f16 && stream_path(T, L->H, L->F, L->E, L->k);
     if (norm) {
       rc = launch_prep(hidden, L->norm_w, L->eps, ws.xn, T, L->H);
       if (rc != CSK_OK) return rc;
@@ -1747,7 +1802,7 @@ int forward_pass(csk_layer* L, const float* hidden, int64_t T, float* out, int f
                        L->sigmoid, ws.logits, ws.pairs, ws.ids, ride ? ws.xs : nullptr);
     if (rc != CSK_OK) return rc;
     mark(CSK_STAGE_DISPATCH);
-    rc = launch_dispatch(ws.ids, ws.pairs, P, L->k, L->E, L->ew_dev, ws);
+    rc = launch_dispatch(ws.ids, ws.pairs, P, L->k, L->E, L->ew_dev, ws, stream_group_tokens(T, L->H, L->F));
     if (rc != CSK_OK) return rc;
   }
   if (phase == 1) return CSK_OK;
@@ -1767,12 +1822,12 @@ int forward_pass(csk_layer* L, const float* hidden, int64_t T, float* out, int f
   ExpertInput in{xr, ws.list_tok, L->wbf ? ws.list_w : nullptr, ws.xs, ws.list_tok};
   if (route_in_kernel) in.rin = &rin_kept, in.rout = &rout_kept;
   if (rows_mx3_ready) in.x_mx3_tokens = ws.xs;
-  if (L->wbf && !stream_path(T, L->H, L->F, L->E, L->k)) {
+  if (L->wbf && !stream) {
     if ((rc = launch_mx3(xr, ws.xg, P, L->H, ws.list_tok, ws.list_w)) != CSK_OK) return rc;
     in.x_mx3 = ws.xg;
     in.mx3_list_row = nullptr;
   }
-  rc = run_experts(L->E, T, L->k, L->H, L->F, L->act, in, ws, true);
+  rc = run_experts(L->E, T, L->k, L->H, L->F, L->act, in, ws, stream, true);
   if (rc != CSK_OK) return rc;
   mark(CSK_STAGE_COMBINE);
   rc = launch_combine(ws.y, ws.pairs, ws.pos, (flags & CSK_FWD_RESIDUAL) ? hidden : nullptr, out, T,
@@ -2171,9 +2226,10 @@ extern "C" int csk_expert_mlp_mxfp4(int expert_id, const float* hidden, int64_t 
     select_expert_ids_kernel<<<dim3((unsigned)cdiv(P, 256)), 256, 0, g_stream>>>(
         up.pairs, ws.ids, (int)P, expert_id, ws.list_tok, ws.list_w);
     if ((rc = check_launch("select_expert_ids_kernel")) != CSK_OK) return rc;
-    if ((rc = launch_dispatch(ws.ids, up.pairs, P, k, 1, up.ew, ws)) != CSK_OK) return rc;
+    if ((rc = launch_dispatch(ws.ids, up.pairs, P, k, 1, up.ew, ws, stream_group_tokens(tn, H, F))) != CSK_OK) return rc;
     ExpertInput in{up.x, ws.list_tok, weight_before_ffn ? ws.list_w : nullptr, ws.xs, ws.list_tok};
-    if (!stream_path(tn, H, F, 1, k)) {
+    const bool stream = stream_path(tn, H, F, 1, k);
+    if (!stream) {
       if (weight_before_ffn) {
         // The expert's token count is only known on the device, and at most tn
         // tokens can select it: gather tn rows.  Positions past the count read the
@@ -2186,7 +2242,7 @@ extern "C" int csk_expert_mlp_mxfp4(int expert_id, const float* hidden, int64_t 
       }
       if (rc != CSK_OK) return rc;
     }
-    rc = run_experts(1, tn, k, H, F, activation, in, ws);
+    rc = run_experts(1, tn, k, H, F, activation, in, ws, stream);
     if (rc != CSK_OK) return rc;
     expand_expert_rows_kernel<<<dim3((unsigned)cdiv(H, 256), (unsigned)tn), 256, 0, g_stream>>>(
         ws.y, ws.ids, ws.pos, dout.as<float>(), (int)k, (int)H, 0);
@@ -2241,7 +2297,7 @@ extern "C" int csk_expert_mlp_f16(int expert_id, const float* hidden, int64_t T,
     select_expert_ids_kernel<<<dim3((unsigned)cdiv(P, 256)), 256, 0, g_stream>>>(
         up.pairs, ws.ids, (int)P, expert_id, ws.list_tok, ws.list_w);
     if ((rc = check_launch("select_expert_ids_kernel")) != CSK_OK) return rc;
-    if ((rc = launch_dispatch(ws.ids, up.pairs, P, k, 1, up.ew, ws)) != CSK_OK) return rc;
+    if ((rc = launch_dispatch(ws.ids, up.pairs, P, k, 1, up.ew, ws, stream_group_tokens(tn, H, F))) != CSK_OK) return rc;
     // with weight_before_ffn at most tn tokens can select the expert: tn rows are gathered; the
     // ones past its count read the zeroed tail of the lists and are never consumed
     rc = run_experts_f16(1, tn, k, H, F, activation, up.x, weight_before_ffn != 0, tn, ws);

@@ -1,7 +1,7 @@
 // Expert MLP for the weight-streaming (decode) regime.
 //
 // Every active expert's matrices are streamed from HBM once per group of up to
-// four (or six) of its tokens: 64 lanes x 16 bytes = 1 KiB of contiguous nibbles per
+// twelve of its tokens: 64 lanes x 16 bytes = 1 KiB of contiguous nibbles per
 // 16-row tile per K step, the four waves of a workgroup taking interleaved K
 // steps (128 elements each).  The MXFP4 entries are the B operand of the block-scaled
 // matrix instruction as they are stored, their E8M0 bytes its scale operand; the group's
@@ -33,6 +33,7 @@ struct ExpertStreamArgs {
   const float* X;        // [rows][32 nblk] fp32 activation rows
   const u32x4* X3;       // the same rows already as three FP6 terms, [rows][mx3_row_blocks(nblk)][6] (mx3.h), or null
   const float* zeros;    // at least 16 bytes of zeros (with X3)
+  int group_tokens;      // tokens per group: what the groups were formed with
   int nblk;              // K / 32
   int ntile;             // ceil(N / 16)
   int N;                 // output features (F for gate/up, H for down)
@@ -62,16 +63,19 @@ __device__ __forceinline__ float moe_activation(float gate_v, float up_v, int ac
 }
 
 // ---------------------------------------------------------------------------
-// Persistent, software-pipelined kernel (K <= 3072) on the block-scaled matrix
+// Persistent, software-pipelined kernel (K <= 8192) on the block-scaled matrix
 // instruction v_mfma_scale_f32_16x16x128_f8f6f4: A = the group's activation rows as
 // three FP6 terms (mx3.h), B = the MXFP4 weights exactly as they are stored -- lane
 // (g = lane / 16, n = lane % 16) holds K block g of the step of weight row n, which is the
 // 16-byte entry the repacked plane keeps for it, and passes that block's E8M0 byte as the
 // instruction's scale operand.  No conversion instruction touches a weight.
 //
-// MODE 0: a work unit is the pair (gate tile R, up tile R), SwiGLU epilogue.
-// MODE 1: a work unit is the pair of down tiles (2R, 2R+1).
-// G = tokens contracted per pass (rows 0..G-1 of the instruction's 16 token rows).
+// NS = K steps per wave (4 waves x NS x 128 elements cover K), NT = weight tiles per work
+// unit (stream_tiles: together they set the loads in flight).
+// MODE 0: a work unit is NT/2 gate tiles and the up tiles of the same features, SwiGLU epilogue.
+// MODE 1: a work unit is NT consecutive down tiles.
+// LG = lane groups that hold tokens: up to 4 LG tokens are contracted per pass (rows
+// 0..4 LG - 1 of the instruction's 16 token rows; the launch says how many, a.group_tokens).
 //
 // The work is (token group of an expert) x (tile pair): every group costs the
 // same, so teams of gridDim.x / groups workgroups take one group each and
@@ -106,22 +110,47 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t stream_plane_rsrc(const void* 
 // positions, lists, counts, token groups) for the down kernel, the combine and
 // csk_layer_last_dispatch.  A 5.4 us launch with its dependent reads is replaced by 3 us in
 // front of this kernel's first weight loads (120b shape: 32.6 -> 30.0 us per layer).
-template <int MODE, int G, bool ROUTE1 = false>
+//
+// Shape of a work unit.  Twelve or more 1 KiB weight loads in flight per wave keep the memory
+// system busy; a K of 2880 gives that from two tiles of six steps, a shorter one walks fewer
+// steps (a K of 768 used to walk six, four of them past the end of K) and takes four tiles,
+// a longer one more steps.  Measured: 64 experts of 2048 x 768, 50 tokens x top-8, down kernel
+// 40.5 -> 22.0 us, gate/up 34.0 -> 29.1; 16 experts of 4096 x 6144, 6 tokens, which the grouped GEMM
+// used to take (62 + 65 us): 52 + 29.  Tiles per unit: with two everywhere the first case's down kernel
+// takes 23.8 us, with six at two steps 23 us and more; at twelve and sixteen steps two down tiles
+// beat one by 2 to 3 % of the layer, and at six steps one tile loses 6 %.
+constexpr int kStreamMaxBlocks = 256;  // K / 32
+constexpr int stream_steps(int nblk) {  // K steps per wave, of the forms that are instantiated
+  const int ns = (nblk + 15) / 16;
+  return ns <= 2 ? 2 : ns <= 6 ? ns : ns <= 8 ? 8 : ns <= 12 ? 12 : 16;
+}
+constexpr int stream_tiles(int ns) {
+  return ns <= 3 ? 4 : 2;
+}
+constexpr int stream_depth(int ns) { return ns <= 8 ? ns : ns / 2; }  // divides ns: a step's registers are known at compile time
+constexpr size_t stream_lds_bytes(int ns, int lg, int group_tokens) {
+  // activation rows as three FP6 terms (96 B per block, 16 ns blocks per row: zeros past K) + the reduction buffers
+  return (size_t)group_tokens * ns * 16 * 96 + (size_t)2 * 4 * lg * (4 * stream_tiles(ns)) * 16 * sizeof(float);
+}
+
+template <int MODE, int LG, int NS, bool ROUTE1 = false>
 __global__ __launch_bounds__(256, 2) void expert_stream_kernel(ExpertStreamArgs a) {
   static_assert(!ROUTE1 || MODE == 0, "the gate/up kernel is the one that routes");
-  constexpr int NS = 6;  // K steps per wave: 4 waves x 6 x 128 = 3072 elements
-  constexpr int NV = 8;  // accumulator floats per lane per unit
+  constexpr int NT = stream_tiles(NS);  // weight tiles per unit
+  constexpr int TU = MODE == 0 ? NT / 2 : NT; // tiles of one plane per unit
+  constexpr int ND = stream_depth(NS);        // K steps whose weights are held or in flight
+  constexpr int NV = 4 * NT;                  // accumulator floats per lane per unit
+  constexpr int G = 4 * LG;                   // tokens per pass, at most
   extern __shared__ __align__(16) unsigned char smem[];
   const int nblk = a.nblk;
   // blocks per activation row in LDS: all the blocks the steps touch, those past K zero, so
   // that nothing in the main loop is clamped or masked (weight blocks past K are then the
   // next tile's, or the slack behind the plane, times exact zeros)
   constexpr int lrb = NS * 16;
-  u32x4* As = reinterpret_cast<u32x4*>(smem);  // [G][lrb][3 terms][2] x 16 B
-  constexpr int LG = (G + 3) / 4;  // lane groups g whose accumulator rows 4g..4g+3 hold tokens
-  float* red = reinterpret_cast<float*>(smem + (size_t)G * lrb * (kMx3ChunksPerBlock * 16));  // [2][4][LG][NV][16]: live lanes only
+  u32x4* As = reinterpret_cast<u32x4*>(smem);  // [group_tokens][lrb][3 terms][2] x 16 B
+  float* red = reinterpret_cast<float*>(smem + (size_t)a.group_tokens * lrb * (kMx3ChunksPerBlock * 16));  // [2][4][LG][NV][16]: live lanes only
 
-  const int npair = MODE == 0 ? a.ntile : (a.ntile + 1) >> 1;
+  const int npair = (a.ntile + TU - 1) / TU;  // units per token group
   // Teams of W workgroups share one token group and interleave its units
   // (workgroup j takes units j, j + W, ...), so that at any moment a team reads one
   // contiguous window of the expert's planes.
@@ -203,10 +232,13 @@ __global__ __launch_bounds__(256, 2) void expert_stream_kernel(ExpertStreamArgs 
     }
   }
 
+  // a lane's scale bytes of one tile: 8 (up to 8 steps per wave) or 16 (scale_slots)
+  constexpr int kScWords = NS <= 8 ? 2 : 4;
+  typedef uint32_t ScaleCell __attribute__((ext_vector_type(kScWords)));
   struct WSet {
-    u32x4 q[NS][2];
-    u32x2 sc[2];  // this wave's scale bytes of the two tiles, one byte per K step
-    float b0, b1;
+    u32x4 q[ND][NT];
+    ScaleCell sc[NT];  // this wave's scale bytes of the tiles, one byte per K step
+    float b[NT];
   };
 
   int par = 0;
@@ -225,7 +257,7 @@ __global__ __launch_bounds__(256, 2) void expert_stream_kernel(ExpertStreamArgs 
       r_gw = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(r_wt), sl));
     }
     const ExpertW* gw_ptr = ROUTE1 ? reinterpret_cast<const ExpertW*>(s_ew) + r_e : &gr->w;
-    const int gcount = ROUTE1 ? 1 : min(G, gr->left);
+    const int gcount = ROUTE1 ? 1 : min(a.group_tokens, gr->left);
     const int base = ROUTE1 ? v : gr->base;
     // One buffer descriptor per weight plane: the unit's tile and the K step go into the
     // scalar offset of a load, the lane's place within the step (block g, row n) into its
@@ -233,35 +265,37 @@ __global__ __launch_bounds__(256, 2) void expert_stream_kernel(ExpertStreamArgs 
     const auto q_rsrc0 = stream_plane_rsrc(MODE == 0 ? gw_ptr->q_gate : gw_ptr->q_down);
     const auto q_rsrc1 = stream_plane_rsrc(MODE == 0 ? gw_ptr->q_up : gw_ptr->q_down);
     const uint32_t qoff = (uint32_t)((g * 16 + n) * 16);
-    const CSK_GLOBAL u32x2* s0 = as_global(reinterpret_cast<const u32x2*>(MODE == 0 ? gw_ptr->s_gate : gw_ptr->s_down)) + wv * 64 + lane;
-    const CSK_GLOBAL u32x2* s1 = as_global(reinterpret_cast<const u32x2*>(MODE == 0 ? gw_ptr->s_up : gw_ptr->s_down)) + wv * 64 + lane;
+    const CSK_GLOBAL ScaleCell* s0 = as_global(reinterpret_cast<const ScaleCell*>(MODE == 0 ? gw_ptr->s_gate : gw_ptr->s_down)) + wv * 64 + lane;
+    const CSK_GLOBAL ScaleCell* s1 = as_global(reinterpret_cast<const ScaleCell*>(MODE == 0 ? gw_ptr->s_up : gw_ptr->s_down)) + wv * 64 + lane;
     const CSK_GLOBAL float* bp0 = as_global(MODE == 0 ? gw_ptr->b_gate : gw_ptr->b_down);
     const CSK_GLOBAL float* bp1 = as_global(MODE == 0 ? gw_ptr->b_up : gw_ptr->b_down);
 
-    // tiles of a unit: (R, R) for gate/up, (2R, 2R+1) for down.
+    // Tile m of a unit: gate tiles TU unit .. then the up tiles of the same features, or down
+    // tiles NT unit ..; past the last tile the last one again (its results are dropped).
+    auto tile_of = [&](int unit, int m) { return min(unit * TU + m % TU, a.ntile - 1); };
     // `idle`: a refill whose data nobody will use (past the workgroup's last unit).  It is
     // still issued, so that the count of loads in flight is the same on every path, but
     // every step aims at the same 1 KiB of the unit, which the caches hold: the tail of a
     // workgroup must not cost HBM traffic.
     auto load_step = [&](WSet& ws, int unit, int s, bool idle) {
-      const int ta = MODE == 0 ? unit : 2 * unit;
-      const int tb = MODE == 0 ? unit : min(2 * unit + 1, a.ntile - 1);
       // four blocks of 16 rows x 16 B per step; a step that lies wholly past K (its activations
       // are zeros) re-reads the cached start of the tile instead of fetching the next tile's blocks
       const uint32_t step = (idle || 4 * (wv + 4 * s) >= nblk) ? 0u : (uint32_t)(wv + 4 * s) * 1024u;
-      ws.q[s][0] = __builtin_amdgcn_raw_buffer_load_b128(q_rsrc0, qoff, (uint32_t)ta * (uint32_t)nblk * 256u + step, 0);
-      ws.q[s][1] = __builtin_amdgcn_raw_buffer_load_b128(q_rsrc1, qoff, (uint32_t)tb * (uint32_t)nblk * 256u + step, 0);
+#pragma unroll
+      for (int m = 0; m < NT; ++m)
+        ws.q[s % ND][m] = __builtin_amdgcn_raw_buffer_load_b128(m < TU ? q_rsrc0 : q_rsrc1, qoff,
+                                                           (uint32_t)tile_of(unit, m) * (uint32_t)nblk * 256u + step, 0);
     };
-    // per-unit scalars: the wave's scale bytes (scale plane: [tile][wave][lane][8]) and biases
-    auto load_unit_scalars = [&](u32x2& sc0, u32x2& sc1, float& b0, float& b1, int unit) {
-      const int ta = MODE == 0 ? unit : 2 * unit;
-      const int tb = MODE == 0 ? unit : min(2 * unit + 1, a.ntile - 1);
-      sc0 = s0[(size_t)ta * 256];
-      sc1 = s1[(size_t)tb * 256];
-      b0 = bp0[min(ta * 16 + n, a.N - 1)];  // bias pointers are never null (absent bias = zero vector)
-      b1 = bp1[min(tb * 16 + n, a.N - 1)];
+    // per-unit scalars: the wave's scale bytes (scale plane: [tile][wave][lane][slots]) and biases
+    auto load_unit_scalars = [&](WSet& ws, int unit) {
+#pragma unroll
+      for (int m = 0; m < NT; ++m) {
+        const int t = tile_of(unit, m);
+        ws.sc[m] = (m < TU ? s0 : s1)[(size_t)t * 256];
+        ws.b[m] = (m < TU ? bp0 : bp1)[min(t * 16 + n, a.N - 1)];  // bias pointers are never null (absent bias = zero vector)
+      }
     };
-    static_assert(G <= 8, "the reduction buffer holds two lane groups");
+    static_assert(LG <= 4, "the instruction has sixteen token rows");
     const bool live = g < LG;  // token t is accumulator row t % 4 of lanes 16 (t / 4) .. 16 (t / 4) + 15
 
     // A thread's first block of activations is requested first (loads return in order: asked
@@ -290,8 +324,8 @@ __global__ __launch_bounds__(256, 2) void expert_stream_kernel(ExpertStreamArgs 
     }
     WSet ws;
 #pragma unroll
-    for (int s = 0; s < NS; ++s) load_step(ws, p_begin, s, false);
-    load_unit_scalars(ws.sc[0], ws.sc[1], ws.b0, ws.b1, p_begin);
+    for (int s = 0; s < ND; ++s) load_step(ws, p_begin, s, false);
+    load_unit_scalars(ws, p_begin);
 
     // ... and while those are under way the group's activation rows are
     // quantised into LDS, one thread per 32-value block (every wave is past its last read
@@ -306,11 +340,10 @@ __global__ __launch_bounds__(256, 2) void expert_stream_kernel(ExpertStreamArgs 
       // not count these loads, so none of them may be in flight past the wait below.
       const int rowblk = mx3_row_blocks(nblk);
       constexpr int kRowChunks = lrb * kMx3ChunksPerBlock;
-      constexpr int kCopyInstr = (G * kRowChunks + 255) / 256;
       const int total = gcount * kRowChunks;
       const uint32_t lds_as = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem;
 #pragma unroll 1
-      for (int i = 0; i < kCopyInstr; ++i) {
+      for (int i = 0; i * 256 < total; ++i) {
         const int ch0 = (4 * i + wv) * 64;
         const int ch = ch0 + lane;
         if (ch < total) {
@@ -365,11 +398,13 @@ __global__ __launch_bounds__(256, 2) void expert_stream_kernel(ExpertStreamArgs 
     // Contracts unit `unit` out of ws and, step by step, refills ws with unit `next`.
     auto compute_unit = [&](WSet& ws, int unit, int next) {
       const bool idle = next == unit;
-      const float bias0 = ws.b0, bias1 = ws.b1;
-      const u32x2 scb0 = ws.sc[0], scb1 = ws.sc[1];
-      floatx4 acc[2];  // one 16 x 16 tile each
+      float bias[NT];
+      ScaleCell scb[NT];
 #pragma unroll
-      for (int m = 0; m < 2; ++m) acc[m] = floatx4{0.f, 0.f, 0.f, 0.f};
+      for (int m = 0; m < NT; ++m) bias[m] = ws.b[m], scb[m] = ws.sc[m];
+      floatx4 acc[NT];  // one 16 x 16 tile each
+#pragma unroll
+      for (int m = 0; m < NT; ++m) acc[m] = floatx4{0.f, 0.f, 0.f, 0.f};
       u32x4 flo[2], fhi[2];  // activation fragments run one term ahead of the matrix cores
       auto read_frag = [&](int i) {  // fragment i = (step, term)
         const int s = i / kMx3Terms, t = i - s * kMx3Terms;
@@ -380,37 +415,39 @@ __global__ __launch_bounds__(256, 2) void expert_stream_kernel(ExpertStreamArgs 
       read_frag(0);
 #pragma unroll
       for (int s = 0; s < NS; ++s) {
-        const int byte0 = (int)(((s < 4 ? scb0.x : scb0.y) >> (8 * (s & 3))) & 0xFFu);
-        const int byte1 = (int)(((s < 4 ? scb1.x : scb1.y) >> (8 * (s & 3))) & 0xFFu);
-        const i32x8 bw0 = (i32x8)__builtin_shufflevector(ws.q[s][0], ws.q[s][0], 0, 1, 2, 3, -1, -1, -1, -1);
-        const i32x8 bw1 = (i32x8)__builtin_shufflevector(ws.q[s][1], ws.q[s][1], 0, 1, 2, 3, -1, -1, -1, -1);
 #pragma unroll
         for (int t = 0; t < kMx3Terms; ++t) {
           const int i = s * kMx3Terms + t;
           if (i + 1 < NS * kMx3Terms) read_frag(i + 1);
           // FP6 reads the first six registers; register 6 holds the term's scale byte
           const i32x8 aw = (i32x8)__builtin_shufflevector(flo[i & 1], fhi[i & 1], 0, 1, 2, 3, 4, 5, 6, 7);
-          acc[0] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(aw, bw0, acc[0], 2, 4, 0, aw[6], 0, byte0);
-          acc[1] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(aw, bw1, acc[1], 2, 4, 0, aw[6], 0, byte1);
+#pragma unroll
+          for (int m = 0; m < NT; ++m) {
+            const int byte = (int)((scb[m][s >> 2] >> (8 * (s & 3))) & 0xFFu);
+            const i32x8 bw = (i32x8)__builtin_shufflevector(ws.q[s % ND][m], ws.q[s % ND][m], 0, 1, 2, 3, -1, -1, -1, -1);
+            acc[m] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(aw, bw, acc[m], 2, 4, 0, aw[6], 0, byte);
+          }
           // fragments are read one ahead, not all at once: the scheduler may not hoist the LDS reads over this point
           __builtin_amdgcn_sched_barrier(0);
         }
-        load_step(ws, next, s, idle);  // this step's registers are free: start the next unit's loads
+        // this step's registers are free: start the loads of the step ND further on, in this unit or the next
+        if (s + ND < NS) load_step(ws, unit, s + ND, false);
+        else load_step(ws, next, s + ND - NS, idle);
       }
-      load_unit_scalars(ws.sc[0], ws.sc[1], ws.b0, ws.b1, next);
+      load_unit_scalars(ws, next);
       float* rbuf = red + (size_t)par * 4 * LG * NV * 16;
       par ^= 1;
       if (live) {
 #pragma unroll
-        for (int m = 0; m < 2; ++m)
+        for (int m = 0; m < NT; ++m)
 #pragma unroll
           for (int i = 0; i < 4; ++i) rbuf[((wv * LG + g) * NV + m * 4 + i) * 16 + n] = acc[m][i];
       }
       __syncthreads();
       if (wv == (unit & 3) && live) {
-        float v2[2][4];
+        float v2[NT][4];
 #pragma unroll
-        for (int m = 0; m < 2; ++m)
+        for (int m = 0; m < NT; ++m)
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
             const int o = m * 4 + i;
@@ -422,13 +459,14 @@ __global__ __launch_bounds__(256, 2) void expert_stream_kernel(ExpertStreamArgs 
           const int t = g * 4 + i;  // token slot within the group
           if (t < gcount) {
             const size_t p = (size_t)(base + t);
-            if (MODE == 0) {
-              const int r = unit * 16 + n;  // output feature
-              if (r < a.N) a.act_out[p * (size_t)a.N + r] = moe_activation(v2[0][i] + bias0, v2[1][i] + bias1, a.act_type);
-            } else {
-              const int ra = 2 * unit * 16 + n, rb = ra + 16;
-              if (ra < a.N) a.y_out[p * (size_t)a.N + ra] = v2[0][i] + bias0;
-              if (rb < a.N) a.y_out[p * (size_t)a.N + rb] = v2[1][i] + bias1;
+#pragma unroll
+            for (int m = 0; m < TU; ++m) {
+              const int r = (unit * TU + m) * 16 + n;  // output feature
+              if (r >= a.N) continue;
+              if (MODE == 0)
+                a.act_out[p * (size_t)a.N + r] = moe_activation(v2[m][i] + bias[m], v2[TU + m < NT ? TU + m : m][i] + bias[TU + m < NT ? TU + m : m], a.act_type);
+              else
+                a.y_out[p * (size_t)a.N + r] = v2[m][i] + bias[m];
             }
           }
         }

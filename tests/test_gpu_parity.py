@@ -567,6 +567,28 @@ def test_layer_streaming_row_length_limits(lib, oracle, H, F, T):
     _check_layer(lib, oracle, L, T, norm=True, residual=True)
 
 
+@pytest.mark.parametrize("D", [1024, 1056, 1568, 2080, 2592, 3104, 4096, 4128, 6176, 8192])
+@pytest.mark.parametrize("long_rows", ["gate/up", "down"])
+def test_layer_streaming_step_counts(lib, oracle, D, long_rows):
+    """The streaming kernels' forms for row lengths up to 8192 -- two to sixteen K steps per
+    wave, four or two tiles per unit -- at the last length of a form and one block past it;
+    one token (routed by the gate/up kernel), one group per expert, several groups."""
+    H, F = (D, 96) if long_rows == "gate/up" else (96, D)
+    L = synth.LayerInputs(3, 2, H, F, seed=D + len(long_rows))
+    for T in (1, 6, 29):
+        _check_layer(lib, oracle, L, T)
+
+
+@pytest.mark.parametrize("H,F", [(96, 1056), (1056, 96), (1024, 1024)])
+def test_layer_grouped_gemm_wide_and_narrow_tiles(lib, oracle, H, F):
+    """Both heights of the grouped GEMM's tile -- 512 weight rows where there are many work
+    units of many tokens, 256 otherwise -- over feature counts that end inside a tile (66
+    tiles of 16) and on its edge."""
+    L = synth.LayerInputs(64, 8, H, F, seed=H)
+    _check_layer(lib, oracle, L, 512, oracle_tokens=64)
+    _check_layer(lib, oracle, L, 250, oracle_tokens=40)
+
+
 def test_layer_many_tokens_per_expert(lib, oracle):
     """More than 64 tokens on one expert: several passes of the M tiles."""
     L = synth.LayerInputs(4, 2, 128, 96, seed=3)

@@ -21,6 +21,7 @@
 #include "mxfp4_kernels.h"
 #include "router_kernels.h"
 #include "node_extra_kernels.h"
+#include "host_link.h"
 
 using namespace csk;
 
@@ -342,17 +343,117 @@ struct csk_layer {
 
 namespace {
 
+#define CSK_TRY(expr)                  \
+  do {                                 \
+    const int _rc = (expr);            \
+    if (_rc != CSK_OK) return _rc;     \
+  } while (0)
+
+// Small transfers share one pinned area: space is handed out in order and taken back all at
+// once when the stream is idle (finish_fetches, or the last DevBuf of a call going out of
+// scope), so that a call's pieces queue one behind the other and the call waits once, at its
+// end.  Larger ones go through the ring of HostLink (host_link.h).
+struct PinnedArena {
+  static constexpr size_t kBytes = (size_t)8 << 20;
+  static constexpr size_t kMaxTransfer = (size_t)256 << 10;  // as long as one thread takes 8 us to copy
+  char* base = nullptr;
+  size_t used = 0;
+  bool failed = false;
+  void* take(size_t bytes) {
+    if (bytes == 0 || bytes > kMaxTransfer || failed) return nullptr;
+    if (!base) {
+      if (hipHostMalloc(reinterpret_cast<void**>(&base), kBytes, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        base = nullptr, failed = true;
+        return nullptr;
+      }
+    }
+    const size_t at = (used + 255) & ~(size_t)255;
+    if (at + bytes > kBytes) return nullptr;
+    used = at + bytes;
+    return base + at;
+  }
+  void reset() { used = 0; }
+};
+PinnedArena g_pinned;
+HostLink g_link;
+int g_live_devbufs = 0;
+
+int link_copy(void* dst, const void* src, size_t bytes) {  // either side may be pinned host memory
+  const size_t per_block = (size_t)kLinkThreads * kLinkUnroll * 16;
+  const unsigned blocks = (unsigned)std::min<size_t>(kLinkBlocks, (bytes + per_block - 1) / per_block);
+  link_copy_kernel<<<dim3(blocks), kLinkThreads, 0, g_stream>>>(static_cast<const unsigned char*>(src),
+                                                               static_cast<unsigned char*>(dst), bytes);
+  return check_launch("link_copy_kernel");
+}
+
+// dst (device) <- the caller's memory, queued on the stream; the caller's memory is free again on return
+int upload(void* dst, const void* host, size_t bytes) {
+  if (bytes == 0) return CSK_OK;
+  if (void* stage = g_pinned.take(bytes)) {
+    std::memcpy(stage, host, bytes);
+    return link_copy(dst, stage, bytes);
+  }
+  HIP_TRY(g_link.to_device(dst, host, bytes, g_stream));
+  return CSK_OK;
+}
+
+// Results on their way to the caller's memory: copied out of the arena once the stream is
+// idle, or (pinned == null) brought down through the link.
+struct PendingFetch {
+  void* host;
+  const void* pinned;
+  const void* dev;
+  size_t bytes;
+};
+std::vector<PendingFetch> g_fetches;
+
+int fetch(void* host, const void* dev, size_t bytes, bool now = false) {
+  if (bytes == 0) return CSK_OK;
+  if (now) {
+    HIP_TRY(g_link.to_host(host, dev, bytes, g_stream));
+    return CSK_OK;
+  }
+  void* stage = g_pinned.take(bytes);
+  if (stage) {
+    const int rc = link_copy(stage, dev, bytes);
+    if (rc != CSK_OK) return rc;
+  }
+  g_fetches.push_back(PendingFetch{host, stage, dev, bytes});
+  return CSK_OK;
+}
+
+// Completes the fetches and waits for the stream.  Every transfer staged in the arena has
+// been consumed by then, so its space is free again.
+int finish_fetches() {
+  hipError_t e = hipSuccess;
+  bool waited = false;
+  for (const PendingFetch& f : g_fetches)
+    if (!f.pinned && e == hipSuccess) e = g_link.to_host(f.host, f.dev, f.bytes, g_stream), waited = true;
+  if (!waited || e != hipSuccess) {  // (a transfer down has waited for everything queued before it)
+    const hipError_t es = hipStreamSynchronize(g_stream);
+    if (e == hipSuccess) e = es;
+  }
+  g_link.idle();
+  if (e == hipSuccess)
+    for (const PendingFetch& f : g_fetches)
+      if (f.pinned) std::memcpy(f.host, f.pinned, f.bytes);
+  g_fetches.clear();
+  g_pinned.reset();
+  if (e != hipSuccess) return fail(CSK_ERR_HIP, std::string("stream synchronize: ") + hipGetErrorString(e));
+  return CSK_OK;
+}
+
 // Upload `rows x K` reference blocks and repack into (q, s).  The staging buffer is kept
-// between calls (a checkpoint is hundreds of matrices of one size); the scale bytes are
-// checked by the pack kernel as it reads them, so the host touches the blocks only to hand
-// them to the copy.  After a refused block the planes of m hold partial data.
+// between calls (a checkpoint is hundreds of matrices of one size; the stream orders one
+// matrix behind the other); the scale bytes are checked by the pack kernel as it reads
+// them, so the host touches the blocks only to hand them to the link.  After a refused block
+// the planes of m hold partial data.
 uint8_t* g_stage = nullptr;
 size_t g_stage_cap = 0;
-unsigned long long* g_bad = nullptr;
+unsigned long long* g_bad = nullptr;  // first refused block of up to three matrices
 
-int pack_into(const uint8_t* host, csk_mxfp4& m) {
-  const int64_t nblocks = m.rows * m.nblk;
-  const size_t bytes = (size_t)nblocks * 17;
+int stage_bytes(size_t bytes) {
   if (bytes > g_stage_cap) {
     HIP_TRY(hipStreamSynchronize(g_stream));
     if (g_stage) (void)hipFree(g_stage);
@@ -360,21 +461,36 @@ int pack_into(const uint8_t* host, csk_mxfp4& m) {
     HIP_TRY(counted_malloc((void**)&g_stage, bytes));
     g_stage_cap = bytes;
   }
-  if (!g_bad) HIP_TRY(counted_malloc((void**)&g_bad, sizeof(unsigned long long)));
-  HIP_TRY(hipMemsetAsync(g_bad, 0xFF, sizeof(unsigned long long), g_stream));
-  HIP_TRY(hipMemcpyAsync(g_stage, host, bytes, hipMemcpyHostToDevice, g_stream));
-  const long ent = m.entries();
-  pack_mxfp4_kernel<<<dim3((unsigned)cdiv(ent, 256)), 256, 0, g_stream>>>(
-      g_stage, m.q, m.s, (int)m.rows, (int)m.nblk, ent, g_bad);
-  int rc = check_launch("pack_mxfp4_kernel");
-  if (rc != CSK_OK) return rc;
-  unsigned long long bad = 0;
-  HIP_TRY(hipMemcpyAsync(&bad, g_bad, sizeof bad, hipMemcpyDeviceToHost, g_stream));
-  HIP_TRY(hipStreamSynchronize(g_stream));
-  if (bad != ~0ull)
-    return fail(CSK_ERR_SCALE, "MXFP4 scale byte 255 on block " + std::to_string(bad) +
-                                   ", which holds a code of magnitude 1 or more: that value (code x 2^128) "
-                                   "overflows fp32 in the reference's decoding as well");
+  if (!g_bad) HIP_TRY(counted_malloc((void**)&g_bad, 3 * sizeof(unsigned long long)));
+  return CSK_OK;
+}
+
+// n <= 3 matrices, queued one behind the other; finish_pack waits for them
+int queue_pack(const uint8_t* const* host, csk_mxfp4* const* ms, int n) {
+  size_t most = 0;
+  for (int i = 0; i < n; ++i) most = std::max(most, (size_t)(ms[i]->rows * ms[i]->nblk) * 17);
+  CSK_TRY(stage_bytes(most));
+  fill_cells_kernel<<<1, 64, 0, g_stream>>>(g_bad, n, ~0ull);
+  CSK_TRY(check_launch("fill_cells_kernel"));
+  for (int i = 0; i < n; ++i) {
+    csk_mxfp4& m = *ms[i];
+    CSK_TRY(upload(g_stage, host[i], (size_t)(m.rows * m.nblk) * 17));
+    const long ent = m.entries();
+    pack_mxfp4_kernel<<<dim3((unsigned)cdiv(ent, 256)), 256, 0, g_stream>>>(
+        g_stage, m.q, m.s, (int)m.rows, (int)m.nblk, ent, g_bad + i);
+    CSK_TRY(check_launch("pack_mxfp4_kernel"));
+  }
+  return CSK_OK;
+}
+int finish_pack(int n) {
+  unsigned long long bad[3] = {~0ull, ~0ull, ~0ull};
+  CSK_TRY(fetch(bad, g_bad, n * sizeof bad[0]));
+  CSK_TRY(finish_fetches());
+  for (int i = 0; i < n; ++i)
+    if (bad[i] != ~0ull)
+      return fail(CSK_ERR_SCALE, "MXFP4 scale byte 255 on block " + std::to_string(bad[i]) +
+                                     ", which holds a code of magnitude 1 or more: that value (code x 2^128) "
+                                     "overflows fp32 in the reference's decoding as well");
   return CSK_OK;
 }
 
@@ -385,13 +501,11 @@ int dequant_to_host(const csk_mxfp4& m, float* host_out) {
   const long ent = m.entries();
   dequant_mxfp4_kernel<<<dim3((unsigned)cdiv(ent, 256)), 256, 0, g_stream>>>(
       m.q, m.s, d, (int)m.rows, (int)m.nblk, ent);
-  hipError_t e = hipGetLastError();
-  if (e == hipSuccess) e = hipMemcpyAsync(host_out, d, n * sizeof(float), hipMemcpyDeviceToHost, g_stream);
-  hipError_t e2 = hipStreamSynchronize(g_stream);
+  int rc = check_launch("dequant_mxfp4_kernel");
+  if (rc == CSK_OK) rc = fetch(host_out, d, n * sizeof(float));
+  const int rs = finish_fetches();
   (void)hipFree(d);
-  if (e != hipSuccess) return fail(CSK_ERR_HIP, std::string("dequant: ") + hipGetErrorString(e));
-  if (e2 != hipSuccess) return fail(CSK_ERR_HIP, std::string("dequant sync: ") + hipGetErrorString(e2));
-  return CSK_OK;
+  return rc == CSK_OK ? rs : rc;
 }
 
 int export_to_host(const csk_mxfp4& m, uint8_t* host_out) {
@@ -401,13 +515,11 @@ int export_to_host(const csk_mxfp4& m, uint8_t* host_out) {
   const long ent = m.entries();
   export_mxfp4_kernel<<<dim3((unsigned)cdiv(ent, 256)), 256, 0, g_stream>>>(
       m.q, m.s, d, (int)m.rows, (int)m.nblk, ent);
-  hipError_t e = hipGetLastError();
-  if (e == hipSuccess) e = hipMemcpyAsync(host_out, d, n, hipMemcpyDeviceToHost, g_stream);
-  hipError_t e2 = hipStreamSynchronize(g_stream);
+  int rc = check_launch("export_mxfp4_kernel");
+  if (rc == CSK_OK) rc = fetch(host_out, d, n);
+  const int rs = finish_fetches();
   (void)hipFree(d);
-  if (e != hipSuccess) return fail(CSK_ERR_HIP, std::string("export: ") + hipGetErrorString(e));
-  if (e2 != hipSuccess) return fail(CSK_ERR_HIP, std::string("export sync: ") + hipGetErrorString(e2));
-  return CSK_OK;
+  return rc == CSK_OK ? rs : rc;
 }
 
 int launch_prep(const float* src, const float* norm_w, float eps, float* xn, int64_t rows, int64_t H) {
@@ -1003,7 +1115,9 @@ extern "C" int csk_mxfp4_upload(const uint8_t* blocks, int64_t rows, int64_t K, 
   int rc = dev_alloc(&m->q, (size_t)m->entries() + kWeightSlack / sizeof(uint4));
   if (rc == CSK_OK) rc = dev_alloc(&m->s, (size_t)m->scale_bytes() + kWeightSlack);
   if (rc == CSK_OK && hipMemset(m->s, 127, (size_t)m->scale_bytes()) != hipSuccess) rc = fail(CSK_ERR_HIP, "hipMemset failed");
-  if (rc == CSK_OK) rc = pack_into(blocks, *m);
+  csk_mxfp4* const ms[1] = {m};
+  if (rc == CSK_OK) rc = queue_pack(&blocks, ms, 1);
+  if (rc == CSK_OK) rc = finish_pack(1);
   if (rc != CSK_OK) {
     csk_mxfp4_free(m);
     return rc;
@@ -1131,31 +1245,44 @@ extern "C" int csk_layer_set_options(csk_layer* L, int sigmoid_gating, int activ
 extern "C" int csk_layer_set_router(csk_layer* L, const float* gate_w, const float* gate_b) {
   REQUIRE_INIT();
   if (!L || !gate_w) return fail(CSK_ERR_ARG, "csk_layer_set_router: null argument");
-  HIP_TRY(hipMemcpyAsync(L->gate_w, gate_w, (size_t)L->E * L->H * sizeof(float), hipMemcpyHostToDevice, g_stream));
-  if (gate_b)
-    HIP_TRY(hipMemcpyAsync(L->gate_b, gate_b, (size_t)L->E * sizeof(float), hipMemcpyHostToDevice, g_stream));
-  HIP_TRY(hipStreamSynchronize(g_stream));
+  CSK_TRY(upload(L->gate_w, gate_w, (size_t)L->E * L->H * sizeof(float)));
+  if (gate_b) CSK_TRY(upload(L->gate_b, gate_b, (size_t)L->E * sizeof(float)));
+  CSK_TRY(finish_fetches());
   L->has_gate = true;
   L->has_gate_b = gate_b != nullptr;
   return CSK_OK;
 }
 
+static int check_biases(const float* b_up, const float* b_gate, const float* b_down) {
+  const int nb = (b_up != nullptr) + (b_gate != nullptr) + (b_down != nullptr);
+  return nb == 0 || nb == 3 ? CSK_OK : fail(CSK_ERR_ARG, "biases must be all present or all absent");
+}
+
+// Queued on the stream: the caller waits (finish_fetches).
 static int upload_biases(csk_layer* L, int64_t e, const float* b_up, const float* b_gate,
                          const float* b_down) {
-  const int nb = (b_up != nullptr) + (b_gate != nullptr) + (b_down != nullptr);
-  if (nb != 0 && nb != 3) return fail(CSK_ERR_ARG, "biases must be all present or all absent");
+  CSK_TRY(check_biases(b_up, b_gate, b_down));
+  const int nb = b_up ? 3 : 0;
   ExpertW& w = L->ew_host[(size_t)e];
   if (nb == 3) {
     float* base = L->bias_all + (size_t)e * (2 * L->F + L->H);
-    HIP_TRY(hipMemcpyAsync(base, b_gate, (size_t)L->F * sizeof(float), hipMemcpyHostToDevice, g_stream));
-    HIP_TRY(hipMemcpyAsync(base + L->F, b_up, (size_t)L->F * sizeof(float), hipMemcpyHostToDevice, g_stream));
-    HIP_TRY(hipMemcpyAsync(base + 2 * L->F, b_down, (size_t)L->H * sizeof(float), hipMemcpyHostToDevice, g_stream));
+    // the three vectors lie side by side: one transfer where they fit the pinned area
+    const size_t nF = (size_t)L->F * sizeof(float), nH = (size_t)L->H * sizeof(float);
+    if (char* stage = static_cast<char*>(g_pinned.take(2 * nF + nH))) {
+      std::memcpy(stage, b_gate, nF);
+      std::memcpy(stage + nF, b_up, nF);
+      std::memcpy(stage + 2 * nF, b_down, nH);
+      CSK_TRY(link_copy(base, stage, 2 * nF + nH));
+    } else {
+      CSK_TRY(upload(base, b_gate, nF));
+      CSK_TRY(upload(base + L->F, b_up, nF));
+      CSK_TRY(upload(base + 2 * L->F, b_down, nH));
+    }
     w.b_gate = base, w.b_up = base + L->F, w.b_down = base + 2 * L->F;
   } else {
     w.b_gate = w.b_up = w.b_down = g_zero;
   }
-  HIP_TRY(hipMemcpyAsync(L->ew_dev + e, &w, sizeof(ExpertW), hipMemcpyHostToDevice, g_stream));
-  HIP_TRY(hipStreamSynchronize(g_stream));
+  CSK_TRY(upload(L->ew_dev + e, &w, sizeof(ExpertW)));
   L->expert_bias[(size_t)e] = nb == 3;
   return CSK_OK;
 }
@@ -1168,25 +1295,28 @@ extern "C" int csk_layer_set_expert(csk_layer* L, int64_t e, const uint8_t* w_up
   if (L->f16 && w_up) return fail(CSK_ERR_STATE, "csk_layer_set_expert: this layer holds fp16 experts (csk_layer_set_expert_f16)");
   if ((w_up == nullptr) != (w_gate == nullptr) || (w_up == nullptr) != (w_down == nullptr))
     return fail(CSK_ERR_ARG, "weights must be all present or all absent");
+  CSK_TRY(check_biases(b_up, b_gate, b_down));
   if (w_up) {
     const uint8_t* src[3] = {w_up, w_gate, w_down};
     const int which[3] = {CSK_W_UP, CSK_W_GATE, CSK_W_DOWN};
     L->expert_set[(size_t)e] = 0;  // a refused matrix (scale byte out of range) leaves the expert unset
-    for (int i = 0; i < 3; ++i) {
-      csk_mxfp4 m = L->view(e, which[i]);
-      int rc = pack_into(src[i], m);
-      if (rc != CSK_OK) return rc;
-    }
+    csk_mxfp4 m[3] = {L->view(e, which[0]), L->view(e, which[1]), L->view(e, which[2])};
+    csk_mxfp4* const ms[3] = {&m[0], &m[1], &m[2]};
+    CSK_TRY(queue_pack(src, ms, 3));
+    CSK_TRY(upload_biases(L, e, b_up, b_gate, b_down));
+    CSK_TRY(finish_pack(3));
     L->expert_set[(size_t)e] = 1;
+    return CSK_OK;
   }
-  return upload_biases(L, e, b_up, b_gate, b_down);
+  CSK_TRY(upload_biases(L, e, b_up, b_gate, b_down));
+  return finish_fetches();
 }
 
 extern "C" int csk_layer_set_norm(csk_layer* L, const float* weight, float eps) {
   REQUIRE_INIT();
   if (!L || !weight) return fail(CSK_ERR_ARG, "csk_layer_set_norm: null argument");
-  HIP_TRY(hipMemcpyAsync(L->norm_w, weight, (size_t)L->H * sizeof(float), hipMemcpyHostToDevice, g_stream));
-  HIP_TRY(hipStreamSynchronize(g_stream));
+  CSK_TRY(upload(L->norm_w, weight, (size_t)L->H * sizeof(float)));
+  CSK_TRY(finish_fetches());
   L->eps = eps;
   L->has_norm = true;
   return CSK_OK;
@@ -1273,30 +1403,26 @@ size_t ggml_matrix_bytes(int type, int64_t rows, int64_t K) {
   if (type == kGgmlQ6K) return n % 256 ? 0 : n / 256 * 210;
   return 0;
 }
-// row-major matrix on the host (halves, or a Q4_K / Q6_K stream) -> fp16 tiles at dst
-int f16_pack_into(const void* data, int type, int64_t rows, int64_t K, u32x4* dst) {
+// row-major matrix on the host (halves, or a Q4_K / Q6_K stream) -> fp16 tiles at dst, queued on the stream
+int queue_f16_pack(const void* data, int type, int64_t rows, int64_t K, u32x4* dst) {
   const size_t bytes = ggml_matrix_bytes(type, rows, K);
   if (!bytes)
     return fail(CSK_ERR_ARG, "fp16 experts take ggml types F16 (1), Q4_K (12) and Q6_K (14), K-quants with rows * K a multiple of 256");
-  uint8_t* stage = nullptr;
-  HIP_TRY(counted_malloc((void**)&stage, bytes));
-  hipError_t e = hipMemcpyAsync(stage, data, bytes, hipMemcpyHostToDevice, g_stream);
-  int rc = CSK_OK;
-  if (e != hipSuccess) rc = fail(CSK_ERR_HIP, std::string("hipMemcpy: ") + hipGetErrorString(e));
-  if (rc == CSK_OK) {
-    const long ent = f16_entries(rows, K);
-    const dim3 grid((unsigned)cdiv(ent, 256));
-    if (type == kGgmlF16Type)
-      f16_pack_kernel<<<grid, 256, 0, g_stream>>>(reinterpret_cast<const uint16_t*>(stage), dst, rows, K, ent);
-    else if (type == kGgmlQ4K)
-      kquant_pack_kernel<kGgmlQ4K><<<grid, 256, 0, g_stream>>>(stage, dst, rows, K, ent);
-    else
-      kquant_pack_kernel<kGgmlQ6K><<<grid, 256, 0, g_stream>>>(stage, dst, rows, K, ent);
-    rc = check_launch("f16_pack_kernel");
-  }
-  (void)hipStreamSynchronize(g_stream);
-  (void)hipFree(stage);
-  return rc;
+  CSK_TRY(stage_bytes(bytes));
+  CSK_TRY(upload(g_stage, data, bytes));
+  const long ent = f16_entries(rows, K);
+  const dim3 grid((unsigned)cdiv(ent, 256));
+  if (type == kGgmlF16Type)
+    f16_pack_kernel<<<grid, 256, 0, g_stream>>>(reinterpret_cast<const uint16_t*>(g_stage), dst, rows, K, ent);
+  else if (type == kGgmlQ4K)
+    kquant_pack_kernel<kGgmlQ4K><<<grid, 256, 0, g_stream>>>(g_stage, dst, rows, K, ent);
+  else
+    kquant_pack_kernel<kGgmlQ6K><<<grid, 256, 0, g_stream>>>(g_stage, dst, rows, K, ent);
+  return check_launch("f16_pack_kernel");
+}
+int f16_pack_into(const void* data, int type, int64_t rows, int64_t K, u32x4* dst) {
+  CSK_TRY(queue_f16_pack(data, type, rows, K, dst));
+  return finish_fetches();
 }
 int f16_export_from(const u32x4* src, int64_t rows, int64_t K, uint16_t* halves) {
   uint16_t* stage = nullptr;
@@ -1305,13 +1431,10 @@ int f16_export_from(const u32x4* src, int64_t rows, int64_t K, uint16_t* halves)
   const long ent = f16_entries(rows, K);
   f16_unpack_kernel<<<dim3((unsigned)cdiv(ent, 256)), 256, 0, g_stream>>>(src, stage, rows, K, ent);
   int rc = check_launch("f16_unpack_kernel");
-  if (rc == CSK_OK) {
-    hipError_t e = hipMemcpyAsync(halves, stage, n * sizeof(uint16_t), hipMemcpyDeviceToHost, g_stream);
-    if (e != hipSuccess) rc = fail(CSK_ERR_HIP, std::string("hipMemcpy: ") + hipGetErrorString(e));
-  }
-  (void)hipStreamSynchronize(g_stream);
+  if (rc == CSK_OK) rc = fetch(halves, stage, n * sizeof(uint16_t));
+  const int rs = finish_fetches();
   (void)hipFree(stage);
-  return rc;
+  return rc == CSK_OK ? rs : rc;
 }
 }  // namespace
 
@@ -1361,75 +1484,6 @@ struct StagingPool {
 };
 StagingPool g_staging;
 
-// Pinned host memory between the caller's pageable buffers and the device.  A copy between
-// pageable memory and the device is staged by the runtime anyway and returns only when it is
-// done, one round trip per call; a node-level call makes five or six small ones.  Through
-// this arena they become plain host copies plus asynchronous transfers that overlap one
-// another and the kernels, and the call waits once, at its end.  Space is handed out in
-// order and taken back all at once when the stream is idle (finish_fetches, or the last
-// DevBuf of a call going out of scope); a transfer that does not fit takes the direct path.
-struct PinnedArena {
-  static constexpr size_t kBytes = (size_t)32 << 20;
-  static constexpr size_t kMaxTransfer = (size_t)4 << 20;
-  char* base = nullptr;
-  size_t used = 0;
-  bool failed = false;
-  void* take(size_t bytes) {
-    if (bytes == 0 || bytes > kMaxTransfer || failed) return nullptr;
-    if (!base) {
-      if (hipHostMalloc(reinterpret_cast<void**>(&base), kBytes, hipHostMallocDefault) != hipSuccess) {
-        (void)hipGetLastError();
-        base = nullptr, failed = true;
-        return nullptr;
-      }
-    }
-    const size_t at = (used + 255) & ~(size_t)255;
-    if (at + bytes > kBytes) return nullptr;
-    used = at + bytes;
-    return base + at;
-  }
-  void reset() { used = 0; }
-};
-PinnedArena g_pinned;
-int g_live_devbufs = 0;
-
-// Results on their way to the caller's memory: copied out of the arena once the stream is idle.
-struct PendingFetch {
-  void* host;
-  const void* pinned;
-  size_t bytes;
-};
-std::vector<PendingFetch> g_fetches;
-
-int fetch(void* host, const void* dev, size_t bytes) {
-  if (bytes == 0) return CSK_OK;
-  if (void* stage = g_pinned.take(bytes)) {
-    HIP_TRY(hipMemcpyAsync(stage, dev, bytes, hipMemcpyDeviceToHost, g_stream));
-    g_fetches.push_back(PendingFetch{host, stage, bytes});
-    return CSK_OK;
-  }
-  HIP_TRY(hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, g_stream));
-  return CSK_OK;
-}
-
-// Waits for the stream, then completes the fetches.  Every transfer staged in the arena has
-// been consumed by then, so its space is free again.
-int finish_fetches() {
-  const hipError_t e = hipStreamSynchronize(g_stream);
-  if (e == hipSuccess)
-    for (const PendingFetch& f : g_fetches) std::memcpy(f.host, f.pinned, f.bytes);
-  g_fetches.clear();
-  g_pinned.reset();
-  if (e != hipSuccess) return fail(CSK_ERR_HIP, std::string("stream synchronize: ") + hipGetErrorString(e));
-  return CSK_OK;
-}
-
-#define CSK_TRY(expr)                  \
-  do {                                 \
-    const int _rc = (expr);            \
-    if (_rc != CSK_OK) return _rc;     \
-  } while (0)
-
 // Scoped device buffer for the host-pointer entry points.
 struct DevBuf {
   void* p = nullptr;
@@ -1453,14 +1507,8 @@ struct DevBuf {
     return g_staging.take(bytes ? bytes : 1, &p, &cap);
   }
   int upload(const void* host, size_t bytes) {
-    int rc = alloc(bytes);
-    if (rc != CSK_OK) return rc;
-    if (void* stage = g_pinned.take(bytes)) {
-      std::memcpy(stage, host, bytes);
-      host = stage;
-    }
-    HIP_TRY(hipMemcpyAsync(p, host, bytes, hipMemcpyHostToDevice, g_stream));
-    return CSK_OK;
+    const int rc = alloc(bytes);
+    return rc == CSK_OK ? ::upload(p, host, bytes) : rc;
   }
   template <class T>
   T* as() {
@@ -1468,20 +1516,19 @@ struct DevBuf {
   }
 };
 
-// Several host arrays in one transfer: the pieces are laid out back to back (256-byte
-// aligned) in one device block and, when they fit, copied into the pinned arena and sent
-// together; otherwise each piece goes up by itself.  A reserved piece is filled by the caller
-// once the block's device address is known (a table of pointers into the same block).
+// Several host arrays in one device block, laid out back to back (256-byte aligned).  Runs
+// of small pieces are collected in the pinned area and sent as one transfer each.  A
+// reserved piece is filled by the caller once the block's device address is known (a table of
+// pointers into the same block).
 struct PackedUpload {
   struct Piece {
-    const void* host;  // null: reserved, filled through fill()
+    const void* host;  // null: reserved, contents in `own`
     size_t bytes, off;
-    std::vector<char> own;  // a reserved piece's contents when there is no stage: alive as long as the object
+    std::vector<char> own;
   };
   DevBuf dev;
   std::vector<Piece> pieces;
   size_t total = 0;
-  char* stage = nullptr;
   size_t add(const void* host, size_t bytes) {
     const size_t off = (total + 255) & ~(size_t)255;
     pieces.push_back(Piece{host, bytes, off, {}});
@@ -1489,16 +1536,8 @@ struct PackedUpload {
     return off;
   }
   size_t reserve(size_t bytes) { return add(nullptr, bytes); }
-  int begin() {  // after the last add: the device block exists from here on
-    CSK_TRY(dev.alloc(total));
-    stage = static_cast<char*>(g_pinned.take(total));
-    return CSK_OK;
-  }
+  int begin() { return dev.alloc(total); }  // after the last add: the device block exists from here on
   void fill(size_t off, const void* src, size_t bytes) {
-    if (stage) {
-      std::memcpy(stage + off, src, bytes);
-      return;
-    }
     for (Piece& pc : pieces)
       if (pc.off == off) pc.own.assign(static_cast<const char*>(src), static_cast<const char*>(src) + bytes);
   }
@@ -1507,16 +1546,21 @@ struct PackedUpload {
     return reinterpret_cast<T*>(static_cast<char*>(dev.p) + off);
   }
   int commit() {
-    if (stage) {
-      for (const Piece& pc : pieces)
-        if (pc.host) std::memcpy(stage + pc.off, pc.host, pc.bytes);
-      HIP_TRY(hipMemcpyAsync(dev.p, stage, total, hipMemcpyHostToDevice, g_stream));
-      return CSK_OK;
-    }
-    for (const Piece& pc : pieces) {
-      const void* src = pc.host ? pc.host : static_cast<const void*>(pc.own.data());
-      if (pc.bytes && src)
-        HIP_TRY(hipMemcpyAsync(static_cast<char*>(dev.p) + pc.off, src, pc.bytes, hipMemcpyHostToDevice, g_stream));
+    auto data = [](const Piece& pc) { return pc.host ? pc.host : static_cast<const void*>(pc.own.data()); };
+    for (size_t i = 0; i < pieces.size();) {
+      const size_t first = pieces[i].off;
+      size_t j = i + 1;  // pieces [i, j) make one transfer
+      while (j < pieces.size() && pieces[j].off + pieces[j].bytes - first <= PinnedArena::kMaxTransfer) ++j;
+      const size_t span = pieces[j - 1].off + pieces[j - 1].bytes - first;
+      char* stage = j > i + 1 ? static_cast<char*>(g_pinned.take(span)) : nullptr;
+      if (stage) {
+        for (size_t q = i; q < j; ++q)
+          if (pieces[q].bytes) std::memcpy(stage + (pieces[q].off - first), data(pieces[q]), pieces[q].bytes);
+        CSK_TRY(link_copy(at<char>(first), stage, span));
+      } else {
+        for (size_t q = i; q < j; ++q) CSK_TRY(::upload(at<char>(pieces[q].off), data(pieces[q]), pieces[q].bytes));
+      }
+      i = j;
     }
     return CSK_OK;
   }
@@ -1613,20 +1657,20 @@ extern "C" int csk_f16_upload_f32(const float* w_host, int64_t rows, int64_t K, 
   DevBuf stage;
   int rc = dev_alloc(&m->w, (size_t)ent);
   if (rc == CSK_OK) rc = stage.upload(w_host, (size_t)rows * K * 4);
-  if (rc == CSK_OK && !g_bad && counted_malloc((void**)&g_bad, sizeof(unsigned long long)) != hipSuccess)
-    rc = fail(CSK_ERR_HIP, "hipMalloc failed");
+  if (rc == CSK_OK) rc = stage_bytes(0);
   if (rc == CSK_OK) {
     // largest magnitude first (g_bad's eight bytes serve as the 32-bit cell), then the split of w / wscale
     const long n = (long)rows * K;
     unsigned int top = 0u;
-    hipError_t e = hipMemsetAsync(g_bad, 0, sizeof(unsigned long long), g_stream);
+    fill_cells_kernel<<<1, 64, 0, g_stream>>>(g_bad, 1, 0ull);
     f32_absmax_bits_kernel<<<dim3((unsigned)std::min<long>(cdiv(n, 256), 8L * std::max(g_cus, 1))), 256, 0, g_stream>>>(
         stage.as<float>(), n, reinterpret_cast<unsigned int*>(g_bad));
-    if (e == hipSuccess) e = hipGetLastError();
-    if (e == hipSuccess) e = hipMemcpyAsync(&top, g_bad, sizeof top, hipMemcpyDeviceToHost, g_stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(g_stream);
-    if (e != hipSuccess) {
-      rc = fail(CSK_ERR_HIP, std::string("csk_f16_upload_f32: ") + hipGetErrorString(e));
+    rc = check_launch("f32_absmax_bits_kernel");
+    if (rc == CSK_OK) rc = fetch(&top, g_bad, sizeof top);
+    const int rs = finish_fetches();
+    if (rc == CSK_OK) rc = rs;
+    if (rc != CSK_OK) {
+      // the message is set
     } else if (top >= 0x7f800000u) {
       rc = fail(CSK_ERR_ARG, "csk_f16_upload_f32: the matrix holds a NaN or an infinity");
     } else {
@@ -1637,10 +1681,7 @@ extern "C" int csk_f16_upload_f32(const float* w_host, int64_t rows, int64_t K, 
       f32_split_pack_kernel<<<dim3((unsigned)cdiv(ent, 256)), 256, 0, g_stream>>>(stage.as<float>(), m->w, rows, K, ent,
                                                                                 std::ldexp(1.0f, -sexp));
       rc = check_launch("f32_split_pack_kernel");
-      if (rc == CSK_OK) {
-        e = hipStreamSynchronize(g_stream);  // the staging buffer is released on return
-        if (e != hipSuccess) rc = fail(CSK_ERR_HIP, std::string("csk_f16_upload_f32: ") + hipGetErrorString(e));
-      }
+      if (rc == CSK_OK) rc = finish_fetches();  // the staging buffer is released on return
     }
   }
   if (rc != CSK_OK) {
@@ -1671,15 +1712,16 @@ extern "C" int csk_layer_set_expert_f16(csk_layer* L, int64_t e, const uint16_t*
   if (!L->f16) return fail(CSK_ERR_STATE, "csk_layer_set_expert_f16: this layer holds MXFP4 experts (csk_layer_create_f16 makes an fp16 one)");
   if ((w_up == nullptr) != (w_gate == nullptr) || (w_up == nullptr) != (w_down == nullptr))
     return fail(CSK_ERR_ARG, "weights must be all present or all absent");
+  CSK_TRY(check_biases(b_up, b_gate, b_down));
   if (w_up) {
-    int rc = f16_pack_into(w_up, kGgmlF16Type, L->F, L->H, L->view16(e, CSK_W_UP));
-    if (rc == CSK_OK) rc = f16_pack_into(w_gate, kGgmlF16Type, L->F, L->H, L->view16(e, CSK_W_GATE));
-    if (rc == CSK_OK) rc = f16_pack_into(w_down, kGgmlF16Type, L->H, L->F, L->view16(e, CSK_W_DOWN));
-    if (rc != CSK_OK) return rc;
+    CSK_TRY(queue_f16_pack(w_up, kGgmlF16Type, L->F, L->H, L->view16(e, CSK_W_UP)));
+    CSK_TRY(queue_f16_pack(w_gate, kGgmlF16Type, L->F, L->H, L->view16(e, CSK_W_GATE)));
+    CSK_TRY(queue_f16_pack(w_down, kGgmlF16Type, L->H, L->F, L->view16(e, CSK_W_DOWN)));
     L->matrix_set[(size_t)e] = 7;
     L->expert_set[(size_t)e] = 1;
   }
-  return upload_biases(L, e, b_up, b_gate, b_down);
+  CSK_TRY(upload_biases(L, e, b_up, b_gate, b_down));
+  return finish_fetches();
 }
 extern "C" int csk_layer_set_expert_matrix(csk_layer* L, int64_t e, int which, int ggml_type,
                                            const void* data) {
@@ -1897,23 +1939,14 @@ extern "C" int csk_moe_forward_host(csk_layer* L, const float* hidden, int64_t T
   // kernels and the copies out are queued on the stream and awaited once
   const size_t n = (size_t)T * L->H;
   DevBuf dbh, dbo;
-  {
-    int rc0 = dbh.alloc(n * sizeof(float));
-    if (rc0 == CSK_OK) rc0 = dbo.alloc(n * sizeof(float));
-    if (rc0 != CSK_OK) return rc0;
-  }
+  CSK_TRY(dbh.upload(hidden, n * sizeof(float)));
   float* const dh = dbh.as<float>();
-  float* const dout = dbo.as<float>();
+  // a small result is written by the last kernel straight into pinned memory, a larger one
+  // into device memory first
+  float* const pinned_out = static_cast<float*>(g_pinned.take(n * sizeof(float)));
+  if (!pinned_out) CSK_TRY(dbo.alloc(n * sizeof(float)));
+  float* const dout = pinned_out ? pinned_out : dbo.as<float>();
   int rc = CSK_OK;
-  {
-    const void* src = hidden;
-    if (void* stage = g_pinned.take(n * sizeof(float))) {
-      std::memcpy(stage, hidden, n * sizeof(float));
-      src = stage;
-    }
-    const hipError_t e = hipMemcpyAsync(dh, src, n * sizeof(float), hipMemcpyHostToDevice, g_stream);
-    if (e != hipSuccess) rc = fail(CSK_ERR_HIP, std::string("copy in: ") + hipGetErrorString(e));
-  }
   if (rc == CSK_OK && !pairs_out) rc = csk_moe_forward(L, dh, T, dout, flags);
   if (rc == CSK_OK && pairs_out) {
     // pass by pass, as csk_moe_forward does: the router output lives in the workspace of a pass
@@ -1925,10 +1958,12 @@ extern "C" int csk_moe_forward_host(csk_layer* L, const float* hidden, int64_t T
       const int64_t tn = std::min(each, T - t0);
       rc = forward_pass(L, dh + t0 * L->H, tn, dout + t0 * L->H, flags);
       if (rc == CSK_OK)
-        rc = csk_copy_d2h(pairs_out + t0 * L->k * 2, g_ws.pairs, (size_t)tn * L->k * 2 * sizeof(float));
+        // (before the next pass overwrites them)
+        rc = fetch(pairs_out + t0 * L->k * 2, g_ws.pairs, (size_t)tn * L->k * 2 * sizeof(float), /*now=*/np > 1);
     }
   }
-  if (rc == CSK_OK) rc = fetch(out, dout, n * sizeof(float));
+  if (rc == CSK_OK && pinned_out) g_fetches.push_back(PendingFetch{out, pinned_out, nullptr, n * sizeof(float)});
+  if (rc == CSK_OK && !pinned_out) rc = fetch(out, dout, n * sizeof(float));
   const int rs = finish_fetches();  // also when an earlier step failed: the stream is left idle
   return rc == CSK_OK ? rs : rc;
 }
@@ -1968,6 +2003,7 @@ extern "C" int csk_layer_attach_expert(csk_layer* L, int64_t e, const csk_mxfp4*
   ExpertW& w = L->ew_host[(size_t)e];
   w.q_gate = gate->q, w.s_gate = gate->s, w.q_up = up->q, w.s_up = up->s, w.q_down = down->q, w.s_down = down->s;
   int rc = upload_biases(L, e, b_up, b_gate, b_down);  // also publishes the entry
+  if (rc == CSK_OK) rc = finish_fetches();
   if (rc != CSK_OK) return rc;
   L->attached[(size_t)e] = 1;
   L->expert_set[(size_t)e] = 1;
@@ -2008,14 +2044,7 @@ extern "C" int csk_moe_frame_begin(csk_layer* L, const float* hidden, int64_t T,
     f.cap = n;
   }
   Workspace& ws = *static_cast<Workspace*>(L->own_ws);
-  {
-    const void* src = hidden;
-    if (void* stage = g_pinned.take(n * sizeof(float))) {
-      std::memcpy(stage, hidden, n * sizeof(float));
-      src = stage;
-    }
-    HIP_TRY(hipMemcpyAsync(f.d_hidden, src, n * sizeof(float), hipMemcpyHostToDevice, g_stream));
-  }
+  CSK_TRY(upload(f.d_hidden, hidden, n * sizeof(float)));
   int rc = forward_pass(L, f.d_hidden, T, f.d_out, flags, ws, 1);
   const size_t np = (size_t)T * L->k;
   f.pairs.resize(np * 2);
@@ -2053,9 +2082,9 @@ extern "C" int csk_moe_frame_expert_rows(csk_layer* L, int64_t e, float* out) {
     Workspace& ws = *static_cast<Workspace*>(L->own_ws);
     f.y.resize(np * H);
     f.pos.resize(np);
-    HIP_TRY(hipMemcpyAsync(f.y.data(), ws.y, np * H * sizeof(float), hipMemcpyDeviceToHost, g_stream));
-    HIP_TRY(hipMemcpyAsync(f.pos.data(), ws.pos, np * sizeof(int), hipMemcpyDeviceToHost, g_stream));
-    HIP_TRY(hipStreamSynchronize(g_stream));
+    CSK_TRY(fetch(f.y.data(), ws.y, np * H * sizeof(float)));
+    CSK_TRY(fetch(f.pos.data(), ws.pos, np * sizeof(int)));
+    CSK_TRY(finish_fetches());
     f.rows_fetched = true;
   }
   // row t = the expert's output for token t if t selected it (first matching slot, as

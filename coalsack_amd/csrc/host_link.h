@@ -1,0 +1,310 @@
+// Transfers between the caller's pageable memory and the device.
+//
+// The caller's memory is not pinned, so every byte crosses one pinned buffer on its way.
+// Left to the runtime (hipMemcpyAsync on pageable memory) that costs 155 us for 4 MiB up and
+// 265 us down (27 and 16 GB/s) where the PCIe link itself takes 76, and 12 to 30 us for a
+// few kilobytes.  Here the pinned side is a ring of slots that the host fills or empties
+// while the device moves the slots before and after: a transfer is as long as the slower
+// of the two, and both sides reach the link's rate --
+//  * the device side is a copy kernel that reads or writes the pinned memory directly:
+//    sixteen workgroups reach 55 GB/s either way (the most measured with any number), a small
+//    copy is 3 us of the stream's time, and nothing waits for another engine;
+//  * the host side is memcpy, 28 GB/s on one core for memory that no cache holds, so a large
+//    transfer is copied by the calling thread and a few helpers together.
+// Measured: experts of 13.2 MB from host memory into HBM 20 -> 42 GB/s (3 matrices each, a wait per
+// expert); 3.3 MB of results down 255 -> 95 us; a two-token frame through host buffers 79 -> 59 us.
+#pragma once
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <atomic>
+#include <condition_variable>
+#include <cstddef>
+#include <cstdint>
+#include <cstring>
+#include <mutex>
+#include <thread>
+#include <vector>
+
+#include "common.h"
+
+namespace csk {
+
+// Any alignment and size; 16 bytes per lane and access where both sides are aligned.
+constexpr int kLinkThreads = 256, kLinkUnroll = 4, kLinkBlocks = 16;
+__global__ __launch_bounds__(kLinkThreads) void link_copy_kernel(const unsigned char* __restrict__ src,
+                                                                 unsigned char* __restrict__ dst, size_t bytes) {
+  const size_t tid = (size_t)blockIdx.x * (kLinkThreads * kLinkUnroll) + threadIdx.x;
+  const size_t stride = (size_t)gridDim.x * (kLinkThreads * kLinkUnroll);
+  const size_t tid1 = (size_t)blockIdx.x * kLinkThreads + threadIdx.x, stride1 = (size_t)gridDim.x * kLinkThreads;
+  size_t done = 0;
+  if (((reinterpret_cast<uintptr_t>(src) | reinterpret_cast<uintptr_t>(dst)) & 15) == 0) {
+    const u32x4* s = reinterpret_cast<const u32x4*>(src);
+    u32x4* d = reinterpret_cast<u32x4*>(dst);
+    const size_t n = bytes / 16;
+    for (size_t i = tid; i < n; i += stride) {
+      u32x4 v[kLinkUnroll];
+#pragma unroll
+      for (int j = 0; j < kLinkUnroll; ++j)
+        if (i + (size_t)j * kLinkThreads < n) v[j] = s[i + (size_t)j * kLinkThreads];
+#pragma unroll
+      for (int j = 0; j < kLinkUnroll; ++j)
+        if (i + (size_t)j * kLinkThreads < n) d[i + (size_t)j * kLinkThreads] = v[j];
+    }
+    done = n * 16;
+  } else if (((reinterpret_cast<uintptr_t>(src) | reinterpret_cast<uintptr_t>(dst)) & 3) == 0) {
+    const uint32_t* s = reinterpret_cast<const uint32_t*>(src);
+    uint32_t* d = reinterpret_cast<uint32_t*>(dst);
+    const size_t n = bytes / 4;
+    for (size_t i = tid1; i < n; i += stride1) d[i] = s[i];
+    done = n * 4;
+  }
+  for (size_t i = done + tid1; i < bytes; i += stride1) dst[i] = src[i];
+}
+
+constexpr size_t kLinkPiece = (size_t)64 << 10;  // what one thread copies at a time
+constexpr size_t kLinkRing = (size_t)16 << 20;
+
+// The calling thread and its helpers copy the pieces of one transfer between the caller's
+// memory and the ring, in ascending order; piece i may be taken once `open` is past it.
+// Helpers sleep between transfers (after a short spin, so that the calls of a loop find them
+// awake) and end with the process.
+class CopyCrew {
+ public:
+  static constexpr int kHelpers = 3;
+
+  ~CopyCrew() {
+    {
+      std::lock_guard<std::mutex> g(m_);
+      stop_.store(true);
+    }
+    cv_.notify_all();
+    for (std::thread& t : threads_) t.join();
+  }
+
+  // byte o of the transfer lies at ring[(at + o) % ring_bytes]; `at` is a multiple of a piece
+  struct Job {
+    char* host;
+    char* ring;
+    size_t bytes, at, ring_bytes;
+    bool up;
+    long pieces() const { return (long)((bytes + kLinkPiece - 1) / kLinkPiece); }
+  };
+
+  void begin(const Job& j) {
+    job_ = j;
+    n_ = j.pieces();
+    next_.store(0), open_.store(0);
+    if (done_.size() < (size_t)n_) done_ = std::vector<std::atomic<bool>>((size_t)n_);
+    for (long i = 0; i < n_; ++i) done_[(size_t)i].store(false, std::memory_order_relaxed);
+    if (threads_.empty()) {
+      const int n = std::min<int>(kHelpers, (int)std::thread::hardware_concurrency() / 4);
+      for (int i = 0; i < n; ++i) threads_.emplace_back([this] { help(); });
+    }
+    {
+      std::lock_guard<std::mutex> g(m_);
+      running_.store(true);
+      epoch_.fetch_add(1);
+    }
+    cv_.notify_all();
+  }
+  void open_to(long piece) { open_.store(std::min(piece, n_), std::memory_order_release); }
+  bool done(long i) const { return done_[(size_t)i].load(std::memory_order_acquire); }
+  // takes one open piece, if there is one
+  bool work_one() {
+    long i = next_.load(std::memory_order_relaxed);
+    do {
+      if (i >= open_.load(std::memory_order_acquire)) return false;
+    } while (!next_.compare_exchange_weak(i, i + 1, std::memory_order_acq_rel));
+    const size_t off = (size_t)i * kLinkPiece, len = std::min(kLinkPiece, job_.bytes - off);
+    char* const r = job_.ring + (job_.at + off) % job_.ring_bytes;
+    if (job_.up)
+      std::memcpy(r, job_.host + off, len);
+    else
+      std::memcpy(job_.host + off, r, len);
+    done_[(size_t)i].store(true, std::memory_order_release);
+    return true;
+  }
+  // no helper touches the transfer after this; pieces that were never opened stay uncopied
+  void end() {
+    {
+      std::lock_guard<std::mutex> g(m_);
+      running_.store(false);
+    }
+    while (inside_.load(std::memory_order_acquire) != 0) relax();
+  }
+
+  static void relax() { __builtin_ia32_pause(); }
+
+ private:
+  void help() {
+    uint64_t seen = 0;
+    for (;;) {
+      for (int spin = 0; spin < 20000 && epoch_.load(std::memory_order_acquire) == seen && !stop_.load(); ++spin) relax();
+      {
+        std::unique_lock<std::mutex> g(m_);
+        cv_.wait(g, [&] { return stop_.load() || epoch_.load() != seen; });
+        if (stop_.load()) return;
+        seen = epoch_.load();
+        if (!running_.load()) continue;
+        inside_.fetch_add(1);
+      }
+      while (running_.load(std::memory_order_acquire) && next_.load(std::memory_order_relaxed) < n_)
+        if (!work_one()) relax();
+      inside_.fetch_sub(1, std::memory_order_release);
+    }
+  }
+
+  std::vector<std::thread> threads_;
+  std::mutex m_;
+  std::condition_variable cv_;
+  std::atomic<bool> stop_{false}, running_{false};
+  std::atomic<uint64_t> epoch_{0};
+  std::atomic<int> inside_{0};
+  Job job_{};
+  long n_ = 0;
+  std::atomic<long> next_{0}, open_{0};
+  std::vector<std::atomic<bool>> done_;
+};
+
+// The pinned ring.  One transfer at a time (the library's lock).
+class HostLink {
+ public:
+  // dst (device) <- host memory, queued on the stream.  The host memory may be reused on return.
+  hipError_t to_device(void* dst, const void* host, size_t bytes, hipStream_t st) {
+    if (bytes == 0) return hipSuccess;
+    hipError_t err = ready();
+    if (err != hipSuccess) return err;
+    CopyCrew::Job job{static_cast<char*>(const_cast<void*>(host)), ring_, bytes, at_, kLinkRing, true};
+    const long n = job.pieces();
+    // A copy kernel costs about 3.5 us of its own.  Onto an idle stream the first ones are
+    // short, so that the device starts early; they grow as the host gets ahead.
+    const long first = (long)(at_ / kLinkPiece);
+    long ready_to = 0, sent = 0, opened = 0, want = first == 0 ? 3 : 16;
+    crew_.begin(job);
+    while (sent < n && err == hipSuccess) {
+      while (opened < n) {  // pieces whose place in the ring is free, up to the end of their quarter
+        const long end = quarter_end(first + opened);
+        // what lay there a round before has been sent, and the device has read it
+        if (first + sent < end - kPieces || !free_quarter((int)((end - 1) % kPieces / kPerQuarter), err)) break;
+        opened = std::min(n, end - first);
+        crew_.open_to(opened);
+      }
+      if (err != hipSuccess) break;
+      const bool worked = crew_.work_one();
+      while (ready_to < n && ready_to < opened && crew_.done(ready_to)) ++ready_to;
+      // up to the end of a quarter of the ring: its event says when it may be filled again
+      const long q_end = quarter_end(first + sent) - first;
+      const long to = std::min(ready_to, q_end);
+      if (to > sent && (to - sent >= want || to == n || to == q_end)) {
+        const size_t a = (size_t)sent * kLinkPiece, len = std::min(bytes, (size_t)to * kLinkPiece) - a;
+        err = launch(static_cast<char*>(dst) + a, ring_ + (at_ + a) % kLinkRing, len, st);
+        if (err == hipSuccess && to == q_end) {
+          const int q = (int)((first + sent) % kPieces / kPerQuarter);
+          err = hipEventRecord(quarter_[q], st);
+          in_use_[q] = true;
+        }
+        sent = to;
+        want = std::min(2 * want, 16L);  // (longer ones would leave the device waiting for the host)
+      } else if (!worked) {
+        CopyCrew::relax();
+      }
+    }
+    crew_.end();
+    at_ = (at_ + (size_t)n * kLinkPiece) % kLinkRing;
+    return err;
+  }
+
+  // host memory <- src (device), after the work queued on the stream.  Waits for all of it.
+  hipError_t to_host(void* host, const void* src, size_t bytes, hipStream_t st) {
+    if (bytes == 0) return hipSuccess;
+    hipError_t err = ready();
+    if (err != hipSuccess) return err;
+    // (places in the ring that an earlier transfer up still reads are written after it, in stream order)
+    CopyCrew::Job job{static_cast<char*>(host), ring_, bytes, 0, kLinkRing, false};
+    const long n = job.pieces();
+    long queued = 0, landed = 0, freed = 0;  // pieces requested, in pinned memory, copied out
+    long ends[kDown];
+    int put = 0, got = 0;  // chunks requested and landed
+    crew_.begin(job);
+    while (freed < n && err == hipSuccess) {
+      // Half of what is left per chunk, at most 1 MiB: few chunks (each costs about 6 us for
+      // its kernel and event), and little left to copy once the last has landed.
+      while (queued < n && put - got < kDown && err == hipSuccess) {
+        long len = std::max(4L, std::min(16L, (n - queued + 1) / 2));
+        len = std::min(len, n - queued);
+        const long to_wrap = kPieces - queued % kPieces;
+        len = std::min(len, to_wrap);
+        if (queued + len > freed + kPieces) break;
+        const size_t a = (size_t)queued * kLinkPiece, cb = std::min(bytes, (size_t)(queued + len) * kLinkPiece) - a;
+        err = launch(ring_ + a % kLinkRing, static_cast<const char*>(src) + a, cb, st);
+        if (err == hipSuccess) err = hipEventRecord(down_[put % kDown], st);
+        queued += len;
+        ends[put++ % kDown] = queued;
+      }
+      while (got < put && err == hipSuccess) {
+        const hipError_t rc = hipEventQuery(down_[got % kDown]);
+        if (rc == hipErrorNotReady) {
+          (void)hipGetLastError();
+          break;
+        }
+        err = rc;
+        landed = ends[got++ % kDown];
+        crew_.open_to(landed);
+      }
+      if (!crew_.work_one()) CopyCrew::relax();
+      while (freed < landed && crew_.done(freed)) ++freed;
+    }
+    crew_.end();
+    idle();
+    return err;
+  }
+
+  // the stream is known to be idle: the whole ring is free
+  void idle() {
+    at_ = 0;
+    for (bool& b : in_use_) b = false;
+  }
+
+ private:
+  static constexpr long kPieces = (long)(kLinkRing / kLinkPiece);
+  static constexpr int kQuarters = 4;
+  static constexpr long kPerQuarter = kPieces / kQuarters;
+  static constexpr int kDown = 8;  // chunks on their way down at once
+  char* ring_ = nullptr;
+  size_t at_ = 0;  // where the next transfer up starts
+  hipEvent_t quarter_[kQuarters] = {}, down_[kDown] = {};
+  bool in_use_[kQuarters] = {};  // the device may still be reading that quarter
+  CopyCrew crew_;
+
+  hipError_t ready() {
+    if (ring_) return hipSuccess;
+    for (hipEvent_t& e : quarter_)
+      if (!e)
+        if (const hipError_t rc = hipEventCreateWithFlags(&e, hipEventDisableTiming); rc != hipSuccess) return rc;
+    for (hipEvent_t& e : down_)
+      if (!e)
+        if (const hipError_t rc = hipEventCreateWithFlags(&e, hipEventDisableTiming); rc != hipSuccess) return rc;
+    return hipHostMalloc(reinterpret_cast<void**>(&ring_), kLinkRing, hipHostMallocDefault);
+  }
+  static long quarter_end(long piece) { return (piece / kPerQuarter + 1) * kPerQuarter; }
+  static hipError_t launch(void* dst, const void* src, size_t bytes, hipStream_t st) {
+    const size_t per_block = (size_t)kLinkThreads * kLinkUnroll * 16;
+    const unsigned blocks = (unsigned)std::min<size_t>(kLinkBlocks, std::max<size_t>(1, (bytes + per_block - 1) / per_block));
+    link_copy_kernel<<<dim3(blocks), kLinkThreads, 0, st>>>(static_cast<const unsigned char*>(src), static_cast<unsigned char*>(dst), bytes);
+    return hipGetLastError();
+  }
+  bool free_quarter(int q, hipError_t& err) {
+    if (!in_use_[q]) return true;
+    const hipError_t rc = hipEventQuery(quarter_[q]);
+    if (rc == hipErrorNotReady) {
+      (void)hipGetLastError();
+      return false;
+    }
+    in_use_[q] = false;
+    err = rc;
+    return rc == hipSuccess;
+  }
+};
+
+}  // namespace csk

@@ -161,6 +161,10 @@ __global__ void dequant_mxfp4_kernel(const uint4* __restrict__ q, const uint8_t*
   }
 }
 
+__global__ void fill_cells_kernel(unsigned long long* __restrict__ p, int n, unsigned long long v) {
+  if ((int)threadIdx.x < n) p[threadIdx.x] = v;
+}
+
 // Synthetic weights, generated straight into the packed layout.  Block b =
 // row * nblk + kb of the stream with key `key` is, in the reference's format,
 //   scale byte = scale_lo + (h0 >> 33) % scale_span,

@@ -30,6 +30,24 @@ def test_dequant_bit_exact_and_roundtrip(lib, oracle):
             lib.mxfp4_free(h)
 
 
+def test_transfers_around_the_pinned_ring(lib):
+    """Uploads and results from a few bytes to several times the pinned ring between host and
+    device (16 MiB, quarters of 4, pieces of 64 KiB), odd lengths among them, one behind the
+    other so that the ring is entered at every offset: nothing is lost or moved."""
+    rng = np.random.default_rng(5)
+    for rows, K in ((3, 32), (17, 4096), (1000, 2080), (2880, 2880), (33, 65504), (9001, 8192), (1, 64), (16384, 6144)):
+        b = rng.integers(0, 256, (rows * (K // 32), 17), dtype=np.uint8)
+        b[:, 0] = 100 + b[:, 0] % 50
+        b = b.reshape(-1)
+        h = lib.mxfp4_upload(b, rows, K)
+        assert np.array_equal(lib.mxfp4_export(h, rows, K), b), (rows, K)
+        lib.mxfp4_free(h)
+        w = rng.standard_normal((rows, K - 3), np.float32).astype(np.float16)
+        h = lib.f16_upload(w)
+        assert np.array_equal(lib.f16_export(h, rows, K - 3).view(np.uint16), w.view(np.uint16)), (rows, K)
+        lib.f16_free(h)
+
+
 def test_dequant_every_scale_and_code(lib, oracle):
     """Every scale byte the reference decodes to finite values, 0 and 1 (fp32 denormals)
     included, with all 16 codes in both nibble positions: bit-exact against the fixture

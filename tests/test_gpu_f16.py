@@ -43,6 +43,21 @@ def test_kquant_upload_equals_weight_provider_halves(lib, oracle, kind, ty, rows
     assert np.array_equal(got.view(np.uint16), want)
 
 
+@pytest.mark.parametrize("kind,ty", [("q4_k", 12), ("q6_k", 14)])
+@pytest.mark.parametrize("rows,K", [(64, 100), (128, 2), (32, 8), (96, 264)])
+def test_kquant_rows_on_and_off_multiples_of_eight(lib, oracle, kind, ty, rows, K):
+    """The two forms of the K-quant pack kernel: eight values of a row at once where rows are
+    multiples of eight, value by value otherwise; rows that end inside a tile's 32 columns."""
+    from tests.golden.make_kquant_golden import random_blocks
+    blocks = random_blocks(np.random.default_rng([rows, K, ty]), kind, rows * K // 256).reshape(-1)
+    h = lib.f16_upload_ggml(ty, blocks, rows, K)
+    try:
+        got = lib.f16_export(h, rows, K)
+    finally:
+        lib.f16_free(h)
+    assert np.array_equal(got.view(np.uint16), oracle.kquant_to_fp16(kind, blocks, rows * K).reshape(rows, K))
+
+
 def test_kquant_upload_fixture_and_errors(lib):
     import os
     gold = np.load(os.path.join(os.path.dirname(__file__), "golden", "kquant_codec.npz"))

@@ -346,6 +346,21 @@ def test_matmul_transpose_float32_weight_matches_oracle(lib, oracle, M, K, N):
         lib.matmul_transpose_f16(a[:, :K - 1] if K > 1 else a, w)
 
 
+@pytest.mark.parametrize("K", [12, 20, 4100, 8184, 8192, 8193, 8200, 16388])
+@pytest.mark.parametrize("dtype", [np.float16, np.float32])
+def test_row_split_chunk_edges(lib, K, dtype):
+    """Rows whose chunks of eight straddle the row's end (and, for two-term weights, the repeated
+    row's seam), and rows on both sides of what the splitting kernel keeps in registers.
+    Two fp16 terms leave 2^-22 of each value and fp32 sums of K terms about 2^-24 sqrt(K):
+    2e-5 of the largest output holds both."""
+    rng = np.random.default_rng([K, 8])
+    a = rng.standard_normal((3, K)).astype(np.float32)
+    w = (rng.standard_normal((32, K)) * 0.1).astype(dtype)
+    got = lib.matmul_transpose_f16(a, w)
+    ref = a.astype(np.float64) @ w.astype(np.float64).T
+    assert np.abs(got - ref).max() <= 2e-5 * np.abs(ref).max()
+
+
 @pytest.mark.parametrize("scale", [1e-6, 1e5, 3e-30, 1e30])
 def test_float32_weights_of_any_magnitude(lib, oracle, scale):
     """fp32 weights far outside the fp16 range (matmul_transpose_mixed_node.h:83-92 and

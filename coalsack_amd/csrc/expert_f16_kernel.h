@@ -557,11 +557,20 @@ __global__ __launch_bounds__(256) void expert_f16_kernel(ExpertF16Args a) {
 // and up, or 256 rows of down) on v_mfma_f32_32x32x16_f16: tokens are the A operand
 // (accumulator register <-> token), weight rows the B operand (lane % 32 <-> row), so a
 // wave's stores are 128 contiguous bytes per token.  Per K step of 64 the token panel
-// (64 tokens x [hi | lo] = 16 KB) goes through LDS, double buffered, 16-byte chunks
-// XOR-swizzled by token so that the 32 lanes of a fragment read hit distinct banks; the
-// weights go from memory straight to registers, one step ahead, each slice reloaded into
-// the registers it has just been consumed from.  Work units (M tile, N
-// tile) are numbered expert by expert and dealt to the eight dies in contiguous eighths.
+// (64 tokens x [hi | lo] = 16 KB) goes to one of three LDS stages by global_load_lds, 16-byte
+// chunks XOR-swizzled by token on the source side so that the 32 lanes of a fragment read hit
+// distinct banks; the weights go from memory straight to one of two register sets, each slice
+// reloaded into the registers it has just been consumed from.  Everything is requested two steps
+// ahead: with one step of lead (and three workgroups per compute unit instead of two) a step took
+// as long as a load, 1 us on an idle memory system and 3 under load, for 0.5 us of matrix
+// instructions.  What bounds it now is what is fetched from behind the L2 (1.7 GB per gate/up launch
+// at 1000 tokens for 1.06 GB of weights, as the M tiles of an expert drift apart).  Layer of 32
+// experts, 2880 x 2880, top-4, us, before / now: 100 tokens 357 / 334, 300 390 / 382, 1000 681 / 648,
+// 2048 1106 / 1060; 8 experts, 300 tokens, top-2 200 / 180; 200 x 2880 x 4096 projection (host
+// buffers) 212 / 202.  Eight waves and 128 tokens per workgroup, which fetch the weights of a
+// full tile once, were slower (1000 tokens: 715), and so were 128 tokens per four waves (690).
+// Work units (M tile, N tile) are numbered expert by expert and dealt to the eight dies in
+// contiguous eighths.
 struct ExpertF16GemmArgs {
   const WorkDesc* desc;
   const int* mtiles;    // (slot, first token) per 64-token M tile
@@ -576,10 +585,200 @@ struct ExpertF16GemmArgs {
 
 constexpr int kF16Dies = 8;
 
+constexpr int kF16Stages = 3;
+struct F16GemmLds {
+  u32x4 panel[kF16Stages][64 * 16];  // [stage][token][16 chunks: block 0 hi 0-3, lo 0-3, block 1 ...]
+  float rs[64];
+};
+
+// One work unit: MS = 2 for M tiles of more than 32 tokens, MS = 1 for those of at most 32 (the
+// ragged end of an expert's list), which cost half the matrix instructions and half the panel.
+template <int MODE, int MS>
+__device__ __forceinline__ void expert_f16_gemm_unit(const ExpertF16GemmArgs& a, const WorkDesc* wd, int m0, int mcount,
+                                                     int nt, F16GemmLds& lds) {
+  auto& panel = lds.panel;
+  auto& rs_sh = lds.rs;
+  constexpr int NC = 2 * MS;  // panel copies per wave and step
+  const int base = wd->base + m0;
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n32 = lane & 31, kg = lane >> 5;
+  const int n16 = n32 & 15, th = n32 >> 4;
+  const int nkb = a.nkb, nsteps = (nkb + 1) >> 1, nfull = nkb >> 1;
+
+  // this lane's weight entries: row n32 of the wave's two 32-row groups
+  int rows[2];
+  const CSK_GLOBAL u32x4* W[2];
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    const int t = MODE == 0 ? nt * 8 + wv * 2 + th : nt * 16 + wv * 4 + 2 * s + th;
+    rows[s] = t * 16 + n16;
+    const uint4* q = MODE == 0 ? (s == 0 ? wd->w.q_gate : wd->w.q_up) : wd->w.q_down;
+    W[s] = as_global(reinterpret_cast<const u32x4*>(q)) + (long)min(t, a.ntile - 1) * nkb * 64 + n16 + 16 * kg;
+  }
+  // Panel copies: instruction i of the wave fills 64 consecutive chunks of the stage, those of
+  // four tokens; the swizzle is applied on the source side.  (The rows' numbers are requested
+  // together, and their scales behind them: one after the other they were eight dependent
+  // reads in front of every unit.)
+  const int cpos = lane & 15;
+  const CSK_GLOBAL u32x4* Arow[NC];
+  int arow[NC], sblk[NC];
+#pragma unroll
+  for (int i = 0; i < NC; ++i) {
+    arow[i] = base + min((NC * wv + i) * 4 + (lane >> 4), mcount - 1);  // tokens past the tile re-read its last
+    if (a.list_row) arow[i] = as_global(a.list_row)[arow[i]];
+  }
+  float rs_val[NC];
+#pragma unroll
+  for (int i = 0; i < NC; ++i) {
+    const int c = cpos ^ (((NC * wv + i) * 4 + (lane >> 4)) & 15);  // the chunk that belongs at this lane's place
+    sblk[i] = c >> 3;                                                // its block of the step
+    Arow[i] = as_global(a.B) + (long)arow[i] * nkb * 8 + (c & 7);
+    rs_val[i] = as_global(a.rscale)[arow[i]];
+  }
+  const uint32_t lds_wave = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)&panel[0][0] +
+                            (uint32_t)(NC * wv * 64 * 16);
+
+  floatx16 acc[MS][2];  // [32-token half][row group]
+#pragma unroll
+  for (int ms = 0; ms < MS; ++ms)
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[ms][s][r] = 0.0f;
+
+  u32x4 wq[2][2][4];  // [step parity][row group][16-wide K slice of the step]
+  // Every load of the loop is unconditional (addresses are clamped, never branched around):
+  // with a branch around a load the compiler's wait-count pass gives up at the join and
+  // drains the whole queue at the head of every step.
+  auto load_w = [&](int u, int s, int sl, int j) {
+    const int kb = min(2 * j + (sl >> 1), nkb - 1);
+    wq[u][s][sl] = W[s][(long)kb * 64 + 32 * (sl & 1)];
+  };
+  auto copy_panel = [&](int stage, int j) {
+#pragma unroll
+    for (int i = 0; i < NC; ++i)
+      asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
+                   :
+                   : "v"(Arow[i] + (long)min(2 * j + sblk[i], nkb - 1) * 8), "s"(lds_wave + (uint32_t)((stage * 64 * 16 + i * 64) * 16))
+                   : "memory");
+  };
+  // Steps 0 and 1 in the order of the steady state, then each step requests the one two
+  // further on: its panel rows at its head (into the stage that the step before has left), its
+  // weights slice by slice into the registers just consumed.  With a single step of lead every
+  // step took as long as a load does, 1 us on an idle memory system and 3 under load, twice to
+  // six times its matrix instructions.
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    copy_panel(u, min(u, nsteps - 1));
+#pragma unroll
+    for (int sl = 0; sl < 4; ++sl)
+#pragma unroll
+      for (int s = 0; s < 2; ++s) load_w(u, s, sl, min(u, nsteps - 1));
+  }
+#pragma unroll
+  for (int i = 0; i < NC; ++i)
+    if (cpos == 0) rs_sh[(NC * wv + i) * 4 + (lane >> 4)] = rs_val[i];
+  // One step = 64 of K: four 16-wide slices, each 2 row groups x 2 token halves x 2 terms of
+  // matrix instructions.  The panel fragments of a token half are read from LDS while the
+  // matrix instructions of the other half issue.  At a step's head its panel has to have landed: what
+  // may still be in flight is its own weights and what was requested a step later.  SL = 2: the last
+  // block of an odd number of them.
+  int stage = 0;
+  auto step = [&](auto u_t, int j, auto more_t, auto sl_t) {
+    constexpr int u = decltype(u_t)::value, SL = decltype(sl_t)::value;
+    constexpr bool more = decltype(more_t)::value;
+    constexpr int kInFlight = more ? 16 + NC : 8;
+    __builtin_amdgcn_s_waitcnt((kInFlight & 15) | (7 << 4) | (0 << 8) | ((kInFlight >> 4) << 14));
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    const int jn = min(j + 2, nsteps - 1);
+    if (more) copy_panel(stage == 0 ? 2 : stage - 1, jn);
+    half8 hi[2], lo[2];
+    auto read_frag = [&](int q) {  // fragment q = (slice q / MS, token half q % MS)
+      const int sl = q / MS, ms = q % MS;
+      // logical chunk of this lane's 8 halves: block sl / 2, [hi | lo], quarter 2 (sl % 2) + kg
+      const int c_hi = (sl >> 1) * 8 + 2 * (sl & 1) + kg, c_lo = c_hi + 4;
+      const int tok = ms * 32 + n32;
+      hi[q & 1] = __builtin_bit_cast(half8, panel[stage][tok * 16 + (c_hi ^ n16)]);
+      lo[q & 1] = __builtin_bit_cast(half8, panel[stage][tok * 16 + (c_lo ^ n16)]);
+    };
+    read_frag(0);
+#pragma unroll
+    for (int q = 0; q < SL * MS; ++q) {
+      const int sl = q / MS, ms = q % MS;
+      if (q + 1 < SL * MS) read_frag(q + 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        const half8 w = __builtin_bit_cast(half8, wq[u][s][sl]);
+        acc[ms][s] = __builtin_amdgcn_mfma_f32_32x32x16_f16(hi[q & 1], w, acc[ms][s], 0, 0, 0);
+        acc[ms][s] = __builtin_amdgcn_mfma_f32_32x32x16_f16(lo[q & 1], w, acc[ms][s], 0, 0, 0);
+      }
+#pragma unroll
+      for (int s = 0; s < 2; ++s) asm volatile("" : "+v"(acc[ms][s]));
+      if (more && ms == MS - 1) {
+        load_w(u, 0, sl, jn);
+        load_w(u, 1, sl, jn);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    stage = stage == 2 ? 0 : stage + 1;
+  };
+  {
+    using I0 = std::integral_constant<int, 0>;
+    using I1 = std::integral_constant<int, 1>;
+    using Full = std::integral_constant<int, 4>;
+    using Half = std::integral_constant<int, 2>;
+    int j = 0;
+    for (; j + 1 < nfull; j += 2) {
+      step(I0{}, j, std::true_type{}, Full{});
+      step(I1{}, j + 1, std::true_type{}, Full{});
+    }
+    if (j < nfull) {
+      step(I0{}, j, std::false_type{}, Full{});
+      if (nkb & 1) step(I1{}, j + 1, std::false_type{}, Half{});
+    } else if (nkb & 1) {
+      step(I0{}, j, std::false_type{}, Half{});
+    }
+  }
+  __builtin_amdgcn_s_waitcnt((0 << 4) | (7 << 4) | (15 << 8));  // copies requested past the last step are still in flight
+  __syncthreads();  // (the row scales below, where there was no step in between)
+
+  // accumulator register r is token (r % 4) + 8 (r / 4) + 4 kg of its 32-token half
+  const CSK_GLOBAL float* b0 = as_global(MODE == 0 ? wd->w.b_gate : wd->w.b_down);
+  const CSK_GLOBAL float* b1 = as_global(MODE == 0 ? wd->w.b_up : wd->w.b_down);
+  float bias[2];
+  bool rv[2];
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    rv[s] = rows[s] < a.N;
+    bias[s] = rv[s] ? (s == 0 ? b0 : b1)[rows[s]] : 0.0f;
+  }
+#pragma unroll
+  for (int ms = 0; ms < MS; ++ms) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int tl = ms * 32 + (r & 3) + 8 * (r >> 2) + 4 * kg;
+      if (tl >= mcount) continue;
+      const float sc_t = rs_sh[tl] * a.wscale[0];
+      float* o = a.out + (long)(base + tl) * a.N;
+      if (MODE == 0) {
+        const float sc_u = rs_sh[tl] * a.wscale[1];
+        if (rv[0])
+          o[rows[0]] = moe_activation(acc[ms][0][r] * sc_t + bias[0], acc[ms][1][r] * sc_u + bias[1], a.act_type);
+      } else {
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+          if (rv[s]) o[rows[s]] = acc[ms][s][r] * sc_t + bias[s];
+      }
+    }
+  }
+}
+
 template <int MODE>
-__global__ __launch_bounds__(256, 3) void expert_f16_gemm_kernel(ExpertF16GemmArgs a) {
-  __shared__ u32x4 panel[2][64 * 16];  // [buffer][token][16 chunks: block 0 hi 0-3, lo 0-3, block 1 ...]
-  __shared__ float rs_sh[64];
+__global__ __launch_bounds__(256, 2) void expert_f16_gemm_kernel(ExpertF16GemmArgs a) {
+  __shared__ F16GemmLds lds;
   const int n_units = *a.n_mtiles * a.n_ntiles;
   const int per_die = (n_units + kF16Dies - 1) / kF16Dies;
   const int slot_i = blockIdx.x / kF16Dies;
@@ -600,156 +799,11 @@ __global__ __launch_bounds__(256, 3) void expert_f16_gemm_kernel(ExpertF16GemmAr
     nt = r / tiles_e;
     m0 = (r - nt * tiles_e) * 64;
   }
-  const int base = wd->base + m0;
   const int mcount = min(64, wd->Te - m0);
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int n32 = lane & 31, kg = lane >> 5;
-  const int n16 = n32 & 15, th = n32 >> 4;
-  const int nkb = a.nkb, nsteps = (nkb + 1) >> 1;
-
-  // this lane's weight entries: row n32 of the wave's two 32-row groups
-  int rows[2];
-  const CSK_GLOBAL u32x4* W[2];
-#pragma unroll
-  for (int s = 0; s < 2; ++s) {
-    const int t = MODE == 0 ? nt * 8 + wv * 2 + th : nt * 16 + wv * 4 + 2 * s + th;
-    rows[s] = t * 16 + n16;
-    const uint4* q = MODE == 0 ? (s == 0 ? wd->w.q_gate : wd->w.q_up) : wd->w.q_down;
-    W[s] = as_global(reinterpret_cast<const u32x4*>(q)) + (long)min(t, a.ntile - 1) * nkb * 64 + n16 + 16 * kg;
-  }
-  // staging: thread copies chunk sc of tokens st + 16 i
-  const int sc = threadIdx.x & 15, st = threadIdx.x >> 4;
-  const CSK_GLOBAL u32x4* Arow[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int pos = base + min(st + 16 * i, mcount - 1);  // tokens past the tile re-read its last
-    const long row = a.list_row ? a.list_row[pos] : pos;
-    Arow[i] = as_global(a.B) + row * nkb * 8 + (sc & 7);
-    if (sc == 0) rs_sh[st + 16 * i] = a.rscale[row];
-  }
-  const int sblk = sc >> 3;  // block of the step this thread's chunk belongs to
-
-  floatx16 acc[2][2];  // [32-token half][row group]
-#pragma unroll
-  for (int ms = 0; ms < 2; ++ms)
-#pragma unroll
-    for (int s = 0; s < 2; ++s)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[ms][s][r] = 0.0f;
-
-  u32x4 wq[2][4];  // [row group][16-wide K slice of the step]
-  u32x4 aq[4];
-  // Every load of the loop is unconditional (addresses are clamped, never branched around):
-  // with a branch around a load the compiler's wait-count pass gives up at the join and
-  // drains the whole queue at the head of every step.  A block past K (odd block count: the
-  // second half of the last step) re-reads the last block of the weights and meets a panel
-  // chunk of zeros.
-  auto load_w = [&](int s, int sl, int j) {
-    const int kb = min(2 * j + (sl >> 1), nkb - 1);
-    wq[s][sl] = W[s][(long)kb * 64 + 32 * (sl & 1)];
-  };
-  auto load_a = [&](int j) {
-    const int kbs = min(2 * j + sblk, nkb - 1);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) aq[i] = Arow[i][(long)kbs * 8];
-  };
-  auto stash = [&](int buf, int j) {
-    const bool past = 2 * j + sblk >= nkb;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int tok = st + 16 * i;
-      panel[buf][tok * 16 + (sc ^ (tok & 15))] = past ? u32x4{0u, 0u, 0u, 0u} : aq[i];
-    }
-  };
-#pragma unroll
-  for (int s = 0; s < 2; ++s)
-#pragma unroll
-    for (int sl = 0; sl < 4; ++sl) load_w(s, sl, 0);
-  load_a(0);
-  stash(0, 0);
-  __syncthreads();
-  // One step = 64 of K: four 16-wide slices, each 2 row groups x 2 token halves x 2 terms of
-  // matrix instructions.  The panel fragments of a token half are read from LDS while the
-  // matrix instructions of the other half issue (the same four fragment registers in
-  // rotation); a slice's weight registers are reloaded for the next step as soon as its
-  // matrix instructions have issued; the next step's panel rows are requested at the head
-  // of the step and stored to the other LDS buffer at its end, behind a wait that leaves the
-  // weight loads in flight.
-  auto step = [&](int j, auto more_t) {
-    constexpr bool more = decltype(more_t)::value;
-    const int buf = j & 1;
-    if (more) load_a(j + 1);
-    half8 hi[2], lo[2];
-    auto read_half = [&](int sl, int ms) {
-      // logical chunk of this lane's 8 halves: block sl / 2, [hi | lo], quarter 2 (sl % 2) + kg
-      const int c_hi = (sl >> 1) * 8 + 2 * (sl & 1) + kg, c_lo = c_hi + 4;
-      const int tok = ms * 32 + n32;
-      hi[ms] = __builtin_bit_cast(half8, panel[buf][tok * 16 + (c_hi ^ n16)]);
-      lo[ms] = __builtin_bit_cast(half8, panel[buf][tok * 16 + (c_lo ^ n16)]);
-    };
-    read_half(0, 0);
-#pragma unroll
-    for (int sl = 0; sl < 4; ++sl) {
-      read_half(sl, 1);
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int s = 0; s < 2; ++s) {
-        const half8 w = __builtin_bit_cast(half8, wq[s][sl]);
-        acc[0][s] = __builtin_amdgcn_mfma_f32_32x32x16_f16(hi[0], w, acc[0][s], 0, 0, 0);
-        acc[0][s] = __builtin_amdgcn_mfma_f32_32x32x16_f16(lo[0], w, acc[0][s], 0, 0, 0);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-      if (sl + 1 < 4) read_half(sl + 1, 0);
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int s = 0; s < 2; ++s) {
-        const half8 w = __builtin_bit_cast(half8, wq[s][sl]);
-        acc[1][s] = __builtin_amdgcn_mfma_f32_32x32x16_f16(hi[1], w, acc[1][s], 0, 0, 0);
-        acc[1][s] = __builtin_amdgcn_mfma_f32_32x32x16_f16(lo[1], w, acc[1][s], 0, 0, 0);
-      }
-      // the slice's registers are free as soon as its matrix instructions have issued:
-      // the next step's weights go straight back into them (one register set in rotation)
-      if (more) {
-        load_w(0, sl, j + 1);
-        load_w(1, sl, j + 1);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    if (more) stash(buf ^ 1, j + 1);
-    __syncthreads();
-  };
-  for (int j = 0; j + 1 < nsteps; ++j) step(j, std::true_type{});
-  step(nsteps - 1, std::false_type{});
-
-  // accumulator register r is token (r % 4) + 8 (r / 4) + 4 kg of its 32-token half
-  const CSK_GLOBAL float* b0 = as_global(MODE == 0 ? wd->w.b_gate : wd->w.b_down);
-  const CSK_GLOBAL float* b1 = as_global(MODE == 0 ? wd->w.b_up : wd->w.b_down);
-  float bias[2];
-  bool rv[2];
-#pragma unroll
-  for (int s = 0; s < 2; ++s) {
-    rv[s] = rows[s] < a.N;
-    bias[s] = rv[s] ? (s == 0 ? b0 : b1)[rows[s]] : 0.0f;
-  }
-#pragma unroll
-  for (int ms = 0; ms < 2; ++ms) {
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int tl = ms * 32 + (r & 3) + 8 * (r >> 2) + 4 * kg;
-      if (tl >= mcount) continue;
-      const float sc_t = rs_sh[tl] * a.wscale[0];
-      float* o = a.out + (long)(base + tl) * a.N;
-      if (MODE == 0) {
-        const float sc_u = rs_sh[tl] * a.wscale[1];
-        if (rv[0])
-          o[rows[0]] = moe_activation(acc[ms][0][r] * sc_t + bias[0], acc[ms][1][r] * sc_u + bias[1], a.act_type);
-      } else {
-#pragma unroll
-        for (int s = 0; s < 2; ++s)
-          if (rv[s]) o[rows[s]] = acc[ms][s][r] * sc_t + bias[s];
-      }
-    }
-  }
+  if (mcount <= 32)
+    expert_f16_gemm_unit<MODE, 1>(a, wd, m0, mcount, nt, lds);
+  else
+    expert_f16_gemm_unit<MODE, 2>(a, wd, m0, mcount, nt, lds);
 }
 
 }  // namespace csk

@@ -361,6 +361,19 @@ def test_row_split_chunk_edges(lib, K, dtype):
     assert np.abs(got - ref).max() <= 2e-5 * np.abs(ref).max()
 
 
+@pytest.mark.parametrize("K", [20, 64, 96, 128, 150, 192, 224])
+@pytest.mark.parametrize("M", [65, 96, 97, 129])
+def test_gemm_step_and_tile_edges(lib, M, K):
+    """The grouped GEMM with one to seven blocks of 32 along K (even and odd numbers of them, fewer than
+    its pipeline is deep) and last M tiles of 1, 32 and 33 tokens; the same bound as above."""
+    rng = np.random.default_rng([M, K, 9])
+    a = rng.standard_normal((M, K)).astype(np.float32)
+    w = (rng.standard_normal((296, K)) * 0.1).astype(np.float16)
+    got = lib.matmul_transpose_f16(a, w)
+    ref = a.astype(np.float64) @ w.astype(np.float64).T
+    assert np.abs(got - ref).max() <= 2e-5 * np.abs(ref).max()
+
+
 @pytest.mark.parametrize("scale", [1e-6, 1e5, 3e-30, 1e30])
 def test_float32_weights_of_any_magnitude(lib, oracle, scale):
     """fp32 weights far outside the fp16 range (matmul_transpose_mixed_node.h:83-92 and

@@ -624,10 +624,10 @@ int launch_router(const float* x, const float* gate_w, const float* gate_b, int6
 }
 
 int launch_dispatch(const int* ids, const float* pairs, int64_t P, int64_t k, int64_t E,
-                    const ExpertW* ew, Workspace& ws, int group_tokens) {
+                    const ExpertW* ew, Workspace& ws, int group_tokens, bool stream) {
   dispatch_scatter_kernel<<<dim3((unsigned)cdiv(std::max<int64_t>(P, 1), kDispatchThreads)), kDispatchThreads, 0, g_stream>>>(
       ids, pairs, (int)P, (int)k, (int)E, ws.counts, ew, ws.offsets, ws.desc,
-      P <= kStreamMaxP ? ws.groups : nullptr, ws.nv, ws.tiles, ws.n_tiles, ws.list_tok, ws.list_w,
+      stream ? ws.groups : nullptr, ws.nv, ws.tiles, ws.n_tiles, ws.list_tok, ws.list_w,
       ws.pos, group_tokens);
   return check_launch("dispatch_scatter_kernel");
 }
@@ -1825,7 +1825,7 @@ int forward_pass(csk_layer* L, const float* hidden, int64_t T, float* out, int f
           ws.logits, ws.pairs, ws.ids, (int)T, (int)L->E, (int)L->k, L->sigmoid, xr, L->gate_w,
           L->has_gate_b ? L->gate_b : nullptr, (int)L->H, ws.logits + T * L->E, 0, Mx3Rider{});
       if ((rc = check_launch("router_topk_kernel")) != CSK_OK) return rc;
-      if ((rc = launch_dispatch(ws.ids, ws.pairs, P, L->k, L->E, L->ew_dev, ws, stream_group_tokens(T, L->H, L->F))) != CSK_OK) return rc;
+      if ((rc = launch_dispatch(ws.ids, ws.pairs, P, L->k, L->E, L->ew_dev, ws, stream_group_tokens(T, L->H, L->F), stream)) != CSK_OK) return rc;
     } else {
       route_small_kernel<<<dim3(1), kRouteSmallThreads, 0, g_stream>>>(rin, rout);
       if ((rc = check_launch("route_small_kernel")) != CSK_OK) return rc;
@@ -1844,7 +1844,7 @@ int forward_pass(csk_layer* L, const float* hidden, int64_t T, float* out, int f
                        L->sigmoid, ws.logits, ws.pairs, ws.ids, ride ? ws.xs : nullptr);
     if (rc != CSK_OK) return rc;
     mark(CSK_STAGE_DISPATCH);
-    rc = launch_dispatch(ws.ids, ws.pairs, P, L->k, L->E, L->ew_dev, ws, stream_group_tokens(T, L->H, L->F));
+    rc = launch_dispatch(ws.ids, ws.pairs, P, L->k, L->E, L->ew_dev, ws, stream_group_tokens(T, L->H, L->F), stream);
     if (rc != CSK_OK) return rc;
   }
   if (phase == 1) return CSK_OK;
@@ -2255,9 +2255,9 @@ extern "C" int csk_expert_mlp_mxfp4(int expert_id, const float* hidden, int64_t 
     select_expert_ids_kernel<<<dim3((unsigned)cdiv(P, 256)), 256, 0, g_stream>>>(
         up.pairs, ws.ids, (int)P, expert_id, ws.list_tok, ws.list_w);
     if ((rc = check_launch("select_expert_ids_kernel")) != CSK_OK) return rc;
-    if ((rc = launch_dispatch(ws.ids, up.pairs, P, k, 1, up.ew, ws, stream_group_tokens(tn, H, F))) != CSK_OK) return rc;
-    ExpertInput in{up.x, ws.list_tok, weight_before_ffn ? ws.list_w : nullptr, ws.xs, ws.list_tok};
     const bool stream = stream_path(tn, H, F, 1, k);
+    if ((rc = launch_dispatch(ws.ids, up.pairs, P, k, 1, up.ew, ws, stream_group_tokens(tn, H, F), stream)) != CSK_OK) return rc;
+    ExpertInput in{up.x, ws.list_tok, weight_before_ffn ? ws.list_w : nullptr, ws.xs, ws.list_tok};
     if (!stream) {
       if (weight_before_ffn) {
         // The expert's token count is only known on the device, and at most tn
@@ -2326,7 +2326,7 @@ extern "C" int csk_expert_mlp_f16(int expert_id, const float* hidden, int64_t T,
     select_expert_ids_kernel<<<dim3((unsigned)cdiv(P, 256)), 256, 0, g_stream>>>(
         up.pairs, ws.ids, (int)P, expert_id, ws.list_tok, ws.list_w);
     if ((rc = check_launch("select_expert_ids_kernel")) != CSK_OK) return rc;
-    if ((rc = launch_dispatch(ws.ids, up.pairs, P, k, 1, up.ew, ws, stream_group_tokens(tn, H, F))) != CSK_OK) return rc;
+    if ((rc = launch_dispatch(ws.ids, up.pairs, P, k, 1, up.ew, ws, stream_group_tokens(tn, H, F), false)) != CSK_OK) return rc;
     // with weight_before_ffn at most tn tokens can select the expert: tn rows are gathered; the
     // ones past its count read the zeroed tail of the lists and are never consumed
     rc = run_experts_f16(1, tn, k, H, F, activation, up.x, weight_before_ffn != 0, tn, ws);

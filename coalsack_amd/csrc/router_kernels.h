@@ -539,6 +539,7 @@ __global__ __launch_bounds__(kDispatchThreads) void dispatch_scatter_kernel(
   const bool pub = blockIdx.x == 0;
   const int chunk0 = blockIdx.x * kDispatchThreads;
   __shared__ int cnt[kMaxExperts], before[kMaxExperts], off_sh[kMaxExperts], act_e[kMaxExperts];
+  __shared__ int first_sh[kMaxExperts], slot_sh[kMaxExperts];
   __shared__ int wcnt[NW][kMaxExperts];
   __shared__ int na_sh;
   if (tid < kMaxExperts) cnt[tid] = 0, before[tid] = 0;
@@ -594,19 +595,11 @@ __global__ __launch_bounds__(kDispatchThreads) void dispatch_scatter_kernel(
         off_sh[ee] = run;
         if (pub) offsets[ee] = run;
         if (cc[j] > 0) {
-          if (pub) {
-            if (groups) {
-              for (int gb = 0; gb < cc[j]; gb += group_tokens) {
-                write_stream_group(groups + gi, ew + ee, ee, cc[j] - gb, run + gb);
-                ++gi;
-              }
-            }
-            for (int m0 = 0; m0 < cc[j]; m0 += 64) {
-              mtiles[2 * mi] = slot;
-              mtiles[2 * mi + 1] = m0;
-              ++mi;
-            }
-          }
+          // where the expert's list entries start; the workgroup writes them side by side below
+          first_sh[ee] = groups ? gi : mi;
+          slot_sh[ee] = slot;
+          gi += group_count(cc[j], group_tokens);
+          mi += (cc[j] + 63) / 64;
           act_e[slot++] = ee;
         }
         run += cc[j];
@@ -617,7 +610,7 @@ __global__ __launch_bounds__(kDispatchThreads) void dispatch_scatter_kernel(
       if (pub) {
         offsets[E] = s_tot;
         *nv = groups ? s_grp : 0;
-        *n_mtiles = s_mt;
+        *n_mtiles = groups ? 0 : s_mt;
       }
     }
   }
@@ -634,6 +627,26 @@ __global__ __launch_bounds__(kDispatchThreads) void dispatch_scatter_kernel(
   const int rank_in_wave = __popcll(same & ((1ull << lane) - 1ull));
   if (my_id >= 0 && rank_in_wave == 0) wcnt[wv][my_id] = __popcll(same);
   __syncthreads();
+  if (pub) {
+    // The list that the expert kernels walk (token groups or M tiles, not both): four threads per
+    // expert.  One lane per four experts, one entry after the other, each behind the nine loads of
+    // an expert's pointers, took half of this kernel's time (128 experts, 300 tokens: 17.0 us, now 10.1).
+    constexpr int kPer = kDispatchThreads / kMaxExperts;
+    const int e = tid / kPer;
+    if (e < E) {
+      const int c = cnt[e];
+      if (groups) {
+        for (int i = tid % kPer, gb = i * group_tokens; gb < c; i += kPer, gb += kPer * group_tokens)
+          write_stream_group(groups + first_sh[e] + i, ew + e, e, c - gb, off_sh[e] + gb);
+      } else {
+        for (int i = tid % kPer; 64 * i < c; i += kPer) {
+          const int mi = first_sh[e] + i;
+          mtiles[2 * mi] = slot_sh[e];
+          mtiles[2 * mi + 1] = 64 * i;
+        }
+      }
+    }
+  }
   if (pub && tid < E) {
     counts[tid] = cnt[tid];
     const bool on = tid < na_sh;

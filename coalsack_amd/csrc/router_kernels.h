@@ -435,7 +435,12 @@ __global__ __launch_bounds__(256) void router_topk_kernel(float* __restrict__ lo
                                                           const float* __restrict__ b, int H,
                                                           const float* __restrict__ partial,
                                                           int nsplit, Mx3Rider rider) {
-  __shared__ CloseCallLds cc;
+  union Lds {
+    CloseCallLds cc;
+    float rows[4 * kMx3LdsWave];
+  };
+  __shared__ __align__(16) Lds lds;
+  CloseCallLds& cc = lds.cc;
   __shared__ float cc_thr[4];
   __shared__ int cc_flag[4];
   // Riders: workgroups past the tokens' rewrite the activation rows as FP6 terms for the
@@ -443,8 +448,9 @@ __global__ __launch_bounds__(256) void router_topk_kernel(float* __restrict__ lo
   // one workgroup of this kernel busy for a chain of H dependent additions, during which
   // the rest of the chip would have nothing to do.
   if (rider.x3 && (int)blockIdx.x >= rider.first_wg) {
-    mx3_rows_block((long)(blockIdx.x - rider.first_wg) * 256 + threadIdx.x, rider.x, rider.x3, rider.rows, rider.nblk,
-                   nullptr, nullptr);
+    const int w = threadIdx.x >> 6;
+    mx3_rows_wave((long)(blockIdx.x - rider.first_wg) * 256 + w * 64, rider.x, rider.x3, rider.rows, rider.nblk,
+                  nullptr, nullptr, lds.rows + w * kMx3LdsWave);
     return;
   }
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;

@@ -604,7 +604,10 @@ int launch_router(const float* x, const float* gate_w, const float* gate_b, int6
     splits = std::min<int64_t>(std::min<int64_t>(splits, kRouterMaxSplits), nchunk);
     const int64_t cps = cdiv(nchunk, splits);
     nsplit = (int)cdiv(nchunk, cps);
-    router_logits_mfma_kernel<<<dim3((unsigned)cdiv(T, 32), (unsigned)nsplit), 256, 0, g_stream>>>(
+    // experts are spread over workgroups, too, while there are places left on the chip (two
+    // workgroups fit a compute unit): 128 experts, 300 tokens 23.4 -> 12.8 us
+    const int64_t esplit = std::max<int64_t>(1, std::min(cdiv(E, 32), 2 * std::max(g_cus, 1) / (cdiv(T, 32) * nsplit)));
+    router_logits_mfma_kernel<<<dim3((unsigned)cdiv(T, 32), (unsigned)nsplit, (unsigned)esplit), 256, 0, g_stream>>>(
         x, gate_w, logits + T * E, (int)T, (int)E, (int)H, (int)cps);
   } else {
     router_logits_kernel<4><<<dim3(gx, (unsigned)cdiv(T, 4)), 256, 0, g_stream>>>(

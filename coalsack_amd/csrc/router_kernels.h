@@ -105,7 +105,7 @@ __global__ __launch_bounds__(256) void router_logits_mfma_kernel(const float* __
   // the last chunk this lane may load from the expert rows (clamped loads meet zeros above)
   const int c_last = max(0, (H - k_lane - 8) / 64);
   float* out = partial + (size_t)blockIdx.y * T * E;
-  for (int e0 = 0; e0 < E; e0 += 32) {
+  for (int e0 = blockIdx.z * 32; e0 < E; e0 += 32 * gridDim.z) {
     const float* gr = g + (size_t)min(e0 + r32, E - 1) * H + k_lane;
     floatx16 acc;
 #pragma unroll

@@ -607,6 +607,21 @@ def test_layer_grouped_gemm_wide_and_narrow_tiles(lib, oracle, H, F):
     _check_layer(lib, oracle, L, 250, oracle_tokens=40)
 
 
+@pytest.mark.parametrize("E,k,H,F,T", [(2, 2, 64, 96, 64), (2, 1, 32, 64, 700), (3, 2, 32, 96, 70), (5, 3, 160, 64, 131)])
+def test_layer_long_expert_lists_and_short_rows(lib, oracle, E, k, H, F, T):
+    """More token groups and more M tiles per expert than the dispatch has threads for one, and rows of
+    one, two and five blocks, which the rewriting of 64 blocks per wave crosses many of."""
+    L = synth.LayerInputs(E, k, H, F, seed=T)
+    _check_layer(lib, oracle, L, T)
+
+
+@pytest.mark.parametrize("E,T", [(33, 65), (100, 65), (128, 300), (256, 97)])
+def test_layer_router_experts_over_workgroups(lib, oracle, E, T):
+    """The matrix-core router with its experts spread over workgroups, the last tile of experts ragged."""
+    L = synth.LayerInputs(E, 4, 96, 64, seed=E)
+    _check_layer(lib, oracle, L, T)
+
+
 def test_layer_many_tokens_per_expert(lib, oracle):
     """More than 64 tokens on one expert: several passes of the M tiles."""
     L = synth.LayerInputs(4, 2, 128, 96, seed=3)

@@ -336,21 +336,24 @@ __device__ __forceinline__ void expert_gemm_mx_unit(const ExpertGemmMxArgs& a, c
   // that every wave is done reading the stage about to be overwritten.
   constexpr int kInFlight = 2 * NG;
   constexpr int kWaitStep = (kInFlight & 15) | (7 << 4) | (15 << 8) | ((kInFlight >> 4) << 14);
-  // First step: the activation tile and the weights in the order of the steady state, then
-  // the biases.
+  // First step: the biases (unconditional, the row clamped: what belongs to rows past N is
+  // dropped), then the activation tile and the weights in the order of the steady state.  Behind
+  // the operands, each under its own branch, the biases were four full waits in a row (20b shape, 2048
+  // tokens: 462 -> 458 us per layer; 64 experts of 2048 x 768, 1000 tokens: 169.3 -> 166.9).
+  float bias0[NG];
+#pragma unroll
+  for (int g = 0; g < NG; ++g) {
+    const float* bias = MODE == 1 ? w.b_down : (g < NG / 2 ? w.b_gate : w.b_up);
+    bias0[g] = as_global(bias)[min(group_tile(g) * 16 + n32, a.N - 1)];
+  }
   BSet bs[kStages];
 #pragma unroll
   for (int x = 0; x < kPart0Items; ++x) issue_part(0, x, 0, bs[0], 0);
 #pragma unroll
   for (int x = 0; x < NG; ++x) issue_part(1, x, 0, bs[0], 0);
-  float bias0[NG];
 #pragma unroll
-  for (int g = 0; g < NG; ++g) {
-    const int row = group_tile(g) * 16 + n32;
-    const float* bias = MODE == 1 ? wd->w.b_down : (g < NG / 2 ? wd->w.b_gate : wd->w.b_up);
-    bias0[g] = row < a.N ? bias[row] : 0.0f;
-  }
-  // The accumulators start from the bias of the lane's weight row (features past N: zero),
+  for (int g = 0; g < NG; ++g) asm volatile("" : "+v"(bias0[g]));  // (not loaded into the accumulators themselves: that spills)
+  // The accumulators start from the bias of the lane's weight row,
   // so that the epilogue has neither a load nor an addition left to do for it.
 #pragma unroll
   for (int g = 0; g < NG; ++g)

@@ -88,7 +88,11 @@ struct MxGeom {
   static constexpr int kStageChunks = kBM * kMxRowChunks;            // 16-byte chunks per LDS stage
   static constexpr int kCopies = kStageChunks / 64 / kMxWaves;       // copy instructions per wave per step
   static constexpr int kFrags = 6 * MS;                              // activation fragments per step
-  static constexpr int kStages = 2;
+  // LDS stages and register sets, one more than the steps of lead.  Units of few tokens (and the
+  // low tile, whose accumulators leave the registers) wait for memory, not for the matrix cores: they ask
+  // two steps ahead (32 experts of 2880 x 2880, 70 tokens: 125.5 -> 119.5 us per layer; 128 of them, 150
+  // tokens 365 -> 350, 300 tokens 420 -> 416).
+  static constexpr int kStages = NG == 2 && MS == 1 ? 3 : 2;
   static constexpr int kEpiRow = 16 * NG + 1;  // floats per token in a wave's epilogue tile (+1: bank spread)
   static constexpr size_t kLdsBytes =
       (size_t)kStages * kStageChunks * 16 > (size_t)kMxWaves * kBM * kEpiRow * 4
@@ -121,7 +125,8 @@ template <int MODE, int NG, int MS>
 __device__ __forceinline__ void expert_gemm_mx_unit(const ExpertGemmMxArgs& a, const WorkDesc* wd, int m0, int mcount,
                                                     int nt, unsigned char* smem) {
   using G = MxGeom<NG, MS>;
-  constexpr int kCopies = G::kCopies, kStages = G::kStages;
+  constexpr int kCopies = G::kCopies, kStages = G::kStages, kLead = kStages - 1;
+  static_assert(kStages * G::kStageChunks * 16 <= MxGeom<NG, 2>::kLdsBytes, "the launch asks for the LDS of full tiles");
   constexpr int kStageChunks = G::kStageChunks, kFrags = G::kFrags, kBM = G::kBM;
   const int base = wd->base + m0;
   const int lane = threadIdx.x & 63;
@@ -256,12 +261,17 @@ __device__ __forceinline__ void expert_gemm_mx_unit(const ExpertGemmMxArgs& a, c
     // the same sequence of copies, waits and barriers as below without the weights and the
     // arithmetic; what this wave owes the output is the zero padding of the rows
 #pragma unroll
-    for (int c = 0; c < kCopies; ++c) issue_copy(c, 0, 0);
+    for (int u = 0; u < kLead; ++u)
+#pragma unroll
+      for (int c = 0; c < kCopies; ++c) issue_copy(c, u, min(u, nsteps - 1));
+    int stage = kLead;  // of step j + kLead
     for (int j = 0; j < nsteps; ++j) {
-      __builtin_amdgcn_s_waitcnt(kWaitAll);
+      constexpr int kAhead = (kLead - 1) * kCopies;
+      __builtin_amdgcn_s_waitcnt(kAhead | (7 << 4) | (15 << 8));
       __builtin_amdgcn_s_barrier();
 #pragma unroll
-      for (int c = 0; c < kCopies; ++c) issue_copy(c, (j + 1) & 1, min(j + 1, nsteps - 1));
+      for (int c = 0; c < kCopies; ++c) issue_copy(c, stage, min(j + kLead, nsteps - 1));
+      stage = stage + 1 == kStages ? 0 : stage + 1;
     }
     __builtin_amdgcn_s_waitcnt(kWaitAll);
     if (MODE == 0) {
@@ -329,13 +339,15 @@ __device__ __forceinline__ void expert_gemm_mx_unit(const ExpertGemmMxArgs& a, c
     }
   };
 
-  // Two LDS stages and register sets, loads one step ahead.  The step boundary is an explicit
+  // Loads one (or two) steps ahead.  The step boundary is an explicit
   // wait + bare barrier: the first part of what this wave requested for step j (during step
-  // j - 1) has landed once at most the 2 NG loads of the second part are still in flight,
+  // j - kLead) has landed once at most the 2 NG loads of the second part and what was
+  // requested for later steps are still in flight,
   // and the barrier extends that to the other waves' parts of the activation tile and tells
   // that every wave is done reading the stage about to be overwritten.
-  constexpr int kInFlight = 2 * NG;
+  constexpr int kInFlight = 2 * NG + (kLead - 1) * (kCopies + 4 * NG);
   constexpr int kWaitStep = (kInFlight & 15) | (7 << 4) | (15 << 8) | ((kInFlight >> 4) << 14);
+  constexpr int kWaitLast = 2 * NG | (7 << 4) | (15 << 8);  // nothing was requested for a step after the last one
   // First step: the biases (unconditional, the row clamped: what belongs to rows past N is
   // dropped), then the activation tile and the weights in the order of the steady state.  Behind
   // the operands, each under its own branch, the biases were four full waits in a row (20b shape, 2048
@@ -348,9 +360,12 @@ __device__ __forceinline__ void expert_gemm_mx_unit(const ExpertGemmMxArgs& a, c
   }
   BSet bs[kStages];
 #pragma unroll
-  for (int x = 0; x < kPart0Items; ++x) issue_part(0, x, 0, bs[0], 0);
+  for (int u = 0; u < kLead; ++u) {
 #pragma unroll
-  for (int x = 0; x < NG; ++x) issue_part(1, x, 0, bs[0], 0);
+    for (int x = 0; x < kPart0Items; ++x) issue_part(0, x, u, bs[u], min(u, nsteps - 1));
+#pragma unroll
+    for (int x = 0; x < NG; ++x) issue_part(1, x, u, bs[u], min(u, nsteps - 1));
+  }
 #pragma unroll
   for (int g = 0; g < NG; ++g) asm volatile("" : "+v"(bias0[g]));  // (not loaded into the accumulators themselves: that spills)
   // The accumulators start from the bias of the lane's weight row,
@@ -372,11 +387,12 @@ __device__ __forceinline__ void expert_gemm_mx_unit(const ExpertGemmMxArgs& a, c
     for (int g = 0; g < NG; ++g) asm volatile("" : "+a"(acc[ms][g]));
 
   {
-    auto step = [&](int u, int jj, auto prefetch) {
-      __builtin_amdgcn_s_waitcnt(kWaitStep);
+    auto step = [&](int u, int jj, auto prefetch, auto last) {
+      __builtin_amdgcn_s_waitcnt(decltype(last)::value ? kWaitLast : kWaitStep);
       __builtin_amdgcn_s_barrier();
       __builtin_amdgcn_sched_barrier(0);
-      compute(bs[u], u, bs[u ^ 1], u ^ 1, min(jj + 1, nsteps - 1), prefetch);
+      const int un = (u + kLead) % kStages;
+      compute(bs[u], u, bs[un], un, min(jj + kLead, nsteps - 1), prefetch);
       __builtin_amdgcn_sched_barrier(0);
     };
     // Steps in pairs (the two register sets and LDS stages alternate), the last step of an
@@ -384,12 +400,25 @@ __device__ __forceinline__ void expert_gemm_mx_unit(const ExpertGemmMxArgs& a, c
     // back edge: with an exit in the middle of the body the compiler's wait-count pass
     // loses track across the two exits and drains the load queue before the first fragment
     // reads of every step.
+    // (With three stages: in threes, and one or two last steps.)
     int j = 0;
-    for (; j + 1 < nsteps; j += 2) {
-      step(0, j, std::true_type{});
-      step(1, j + 1, std::true_type{});
+    for (; j + kStages - 1 < nsteps; j += kStages) {
+      step(0, j, std::true_type{}, std::false_type{});
+      step(1, j + 1, std::true_type{}, std::false_type{});
+      if constexpr (kStages == 3) step(2, j + 2, std::true_type{}, std::false_type{});
     }
-    if (j < nsteps) step(0, j, std::false_type{});
+    // (none of the steps left over requests anything: weights that nobody reads would be dropped
+    // by the compiler, and the waits count them)
+    if constexpr (kStages == 3) {
+      if (j + 1 < nsteps) {
+        step(0, j, std::false_type{}, std::false_type{});
+        step(1, j + 1, std::false_type{}, std::true_type{});
+      } else if (j < nsteps) {
+        step(0, j, std::false_type{}, std::true_type{});
+      }
+    } else {
+      if (j < nsteps) step(0, j, std::false_type{}, std::true_type{});
+    }
   }
   // the copies requested past the last step are still in flight: nothing may reuse their LDS before they land
   __builtin_amdgcn_s_waitcnt(kWaitAll);
@@ -464,7 +493,7 @@ __device__ __forceinline__ void expert_gemm_mx_unit(const ExpertGemmMxArgs& a, c
 // so that the workgroups resident on one die at one time share a few activation panels and
 // a few experts' weights, which then come from that L2 instead of from memory.
 template <int MODE, int NG>
-__global__ __launch_bounds__(64 * kMxWaves, 2) void expert_gemm_mx_kernel(ExpertGemmMxArgs a) {
+__global__ __launch_bounds__(64 * kMxWaves, NG == 2 ? 3 : 2) void expert_gemm_mx_kernel(ExpertGemmMxArgs a) {
   extern __shared__ __align__(16) unsigned char smem[];
   const int n_units = *a.n_mtiles * a.n_ntiles;
   const int per_die = (n_units + kDies - 1) / kDies;

@@ -22,6 +22,7 @@
 #include <cstddef>
 #include <cstdint>
 #include <cstring>
+#include <exception>
 #include <mutex>
 #include <thread>
 #include <vector>
@@ -91,15 +92,24 @@ class CopyCrew {
     long pieces() const { return (long)((bytes + kLinkPiece - 1) / kLinkPiece); }
   };
 
-  void begin(const Job& j) {
+  // false: no memory for the list of pieces.  Helpers that cannot be started are done
+  // without: the calling thread takes every piece that nobody else takes.
+  bool begin(const Job& j) {
+    try {
+      if (done_.size() < (size_t)j.pieces()) done_ = std::vector<std::atomic<bool>>((size_t)j.pieces());
+    } catch (const std::exception&) {
+      return false;
+    }
     job_ = j;
     n_ = j.pieces();
     next_.store(0), open_.store(0);
-    if (done_.size() < (size_t)n_) done_ = std::vector<std::atomic<bool>>((size_t)n_);
     for (long i = 0; i < n_; ++i) done_[(size_t)i].store(false, std::memory_order_relaxed);
     if (threads_.empty()) {
       const int n = std::min<int>(kHelpers, (int)std::thread::hardware_concurrency() / 4);
-      for (int i = 0; i < n; ++i) threads_.emplace_back([this] { help(); });
+      try {
+        for (int i = 0; i < n; ++i) threads_.emplace_back([this] { help(); });
+      } catch (const std::exception&) {
+      }
     }
     {
       std::lock_guard<std::mutex> g(m_);
@@ -107,6 +117,7 @@ class CopyCrew {
       epoch_.fetch_add(1);
     }
     cv_.notify_all();
+    return true;
   }
   void open_to(long piece) { open_.store(std::min(piece, n_), std::memory_order_release); }
   bool done(long i) const { return done_[(size_t)i].load(std::memory_order_acquire); }
@@ -181,7 +192,7 @@ class HostLink {
     // short, so that the device starts early; they grow as the host gets ahead.
     const long first = (long)(at_ / kLinkPiece);
     long ready_to = 0, sent = 0, opened = 0, want = first == 0 ? 3 : 16;
-    crew_.begin(job);
+    if (!crew_.begin(job)) return hipErrorOutOfMemory;
     while (sent < n && err == hipSuccess) {
       while (opened < n) {  // pieces whose place in the ring is free, up to the end of their quarter
         const long end = quarter_end(first + opened);
@@ -226,7 +237,7 @@ class HostLink {
     long queued = 0, landed = 0, freed = 0;  // pieces requested, in pinned memory, copied out
     long ends[kDown];
     int put = 0, got = 0;  // chunks requested and landed
-    crew_.begin(job);
+    if (!crew_.begin(job)) return hipErrorOutOfMemory;
     while (freed < n && err == hipSuccess) {
       // Half of what is left per chunk, at most 1 MiB: few chunks (each costs about 6 us for
       // its kernel and event), and little left to copy once the last has landed.

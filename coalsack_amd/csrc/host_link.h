@@ -24,8 +24,11 @@
 #include <cstring>
 #include <exception>
 #include <mutex>
+#include <new>
 #include <thread>
 #include <vector>
+
+#include <unistd.h>
 
 #include "common.h"
 
@@ -178,6 +181,27 @@ class CopyCrew {
   std::vector<std::atomic<bool>> done_;
 };
 
+// The crew of this process.  A forked child has the object but not its threads: joining them, or
+// destroying what they sleep on, would wait for ever at its exit, so the child leaves both alone.
+class CrewOwner {
+ public:
+  CrewOwner() = default;
+  CrewOwner(const CrewOwner&) = delete;
+  CrewOwner& operator=(const CrewOwner&) = delete;
+  ~CrewOwner() {
+    if (crew_ && pid_ == getpid()) delete crew_;
+  }
+  bool ready() {
+    if (!crew_) crew_ = new (std::nothrow) CopyCrew, pid_ = getpid();
+    return crew_ != nullptr;
+  }
+  CopyCrew* operator->() { return crew_; }
+
+ private:
+  CopyCrew* crew_ = nullptr;
+  pid_t pid_ = 0;
+};
+
 // The pinned ring.  One transfer at a time (the library's lock).
 class HostLink {
  public:
@@ -192,18 +216,18 @@ class HostLink {
     // short, so that the device starts early; they grow as the host gets ahead.
     const long first = (long)(at_ / kLinkPiece);
     long ready_to = 0, sent = 0, opened = 0, want = first == 0 ? 3 : 16;
-    if (!crew_.begin(job)) return hipErrorOutOfMemory;
+    if (!crew_.ready() || !crew_->begin(job)) return hipErrorOutOfMemory;
     while (sent < n && err == hipSuccess) {
       while (opened < n) {  // pieces whose place in the ring is free, up to the end of their quarter
         const long end = quarter_end(first + opened);
         // what lay there a round before has been sent, and the device has read it
         if (first + sent < end - kPieces || !free_quarter((int)((end - 1) % kPieces / kPerQuarter), err)) break;
         opened = std::min(n, end - first);
-        crew_.open_to(opened);
+        crew_->open_to(opened);
       }
       if (err != hipSuccess) break;
-      const bool worked = crew_.work_one();
-      while (ready_to < n && ready_to < opened && crew_.done(ready_to)) ++ready_to;
+      const bool worked = crew_->work_one();
+      while (ready_to < n && ready_to < opened && crew_->done(ready_to)) ++ready_to;
       // up to the end of a quarter of the ring: its event says when it may be filled again
       const long q_end = quarter_end(first + sent) - first;
       const long to = std::min(ready_to, q_end);
@@ -221,7 +245,7 @@ class HostLink {
         CopyCrew::relax();
       }
     }
-    crew_.end();
+    crew_->end();
     at_ = (at_ + (size_t)n * kLinkPiece) % kLinkRing;
     return err;
   }
@@ -237,7 +261,7 @@ class HostLink {
     long queued = 0, landed = 0, freed = 0;  // pieces requested, in pinned memory, copied out
     long ends[kDown];
     int put = 0, got = 0;  // chunks requested and landed
-    if (!crew_.begin(job)) return hipErrorOutOfMemory;
+    if (!crew_.ready() || !crew_->begin(job)) return hipErrorOutOfMemory;
     while (freed < n && err == hipSuccess) {
       // Half of what is left per chunk, at most 1 MiB: few chunks (each costs about 6 us for
       // its kernel and event), and little left to copy once the last has landed.
@@ -261,12 +285,12 @@ class HostLink {
         }
         err = rc;
         landed = ends[got++ % kDown];
-        crew_.open_to(landed);
+        crew_->open_to(landed);
       }
-      if (!crew_.work_one()) CopyCrew::relax();
-      while (freed < landed && crew_.done(freed)) ++freed;
+      if (!crew_->work_one()) CopyCrew::relax();
+      while (freed < landed && crew_->done(freed)) ++freed;
     }
-    crew_.end();
+    crew_->end();
     idle();
     return err;
   }
@@ -286,7 +310,7 @@ class HostLink {
   size_t at_ = 0;  // where the next transfer up starts
   hipEvent_t quarter_[kQuarters] = {}, down_[kDown] = {};
   bool in_use_[kQuarters] = {};  // the device may still be reading that quarter
-  CopyCrew crew_;
+  CrewOwner crew_;
 
   hipError_t ready() {
     if (ring_) return hipSuccess;

@@ -38,7 +38,27 @@ int g_cus = 0;
 // of the reference's scheduler (layer_scheduler_node), without locking of their own.
 std::recursive_mutex g_api;
 thread_local bool t_device_bound = false;  // the current device is a per-thread setting
-#define API_LOCK() std::lock_guard<std::recursive_mutex> csk_api_guard_(g_api)
+void drop_transfers();
+// Also the place where a call that failed halfway is cleaned up after.
+struct ApiGuard {
+  ApiGuard() {
+    g_api.lock();
+    ++depth();
+  }
+  ApiGuard(const ApiGuard&) = delete;
+  ApiGuard& operator=(const ApiGuard&) = delete;
+  ~ApiGuard() {
+    if (--depth() == 0) drop_transfers();
+    g_api.unlock();
+  }
+
+ private:
+  static int& depth() {  // entry points inside one another (under the lock)
+    static int d = 0;
+    return d;
+  }
+};
+#define API_LOCK() ApiGuard csk_api_guard_
 
 int fail(int code, const std::string& msg) {
   g_err = msg;
@@ -350,8 +370,8 @@ namespace {
   } while (0)
 
 // Small transfers share one pinned area: space is handed out in order and taken back all at
-// once when the stream is idle (finish_fetches, or the last DevBuf of a call going out of
-// scope), so that a call's pieces queue one behind the other and the call waits once, at its
+// once when the stream is idle (finish_fetches, or drop_transfers for a call that failed before
+// that), so that a call's pieces queue one behind the other and the call waits once, at its
 // end.  Larger ones go through the ring of HostLink (host_link.h).
 struct PinnedArena {
   static constexpr size_t kBytes = (size_t)8 << 20;
@@ -377,7 +397,6 @@ struct PinnedArena {
 };
 PinnedArena g_pinned;
 HostLink g_link;
-int g_live_devbufs = 0;
 
 int link_copy(void* dst, const void* src, size_t bytes) {  // either side may be pinned host memory
   const size_t per_block = (size_t)kLinkThreads * kLinkUnroll * 16;
@@ -442,6 +461,16 @@ int finish_fetches() {
   g_pinned.reset();
   if (e != hipSuccess) return fail(CSK_ERR_HIP, std::string("stream synchronize: ") + hipGetErrorString(e));
   return CSK_OK;
+}
+
+// The end of an entry point: a call that came to its end has finished its transfers, so only one that
+// failed in between leaves any.  Its results go nowhere -- the caller's memory may be gone after
+// the return -- and nothing queued may still touch the pinned area when the next call fills it.
+void drop_transfers() {
+  if (g_fetches.empty() && g_pinned.used == 0) return;
+  (void)hipStreamSynchronize(g_stream);
+  g_fetches.clear();
+  g_pinned.reset();
 }
 
 // Upload `rows x K` reference blocks and repack into (q, s).  The staging buffer is kept
@@ -1446,7 +1475,8 @@ namespace {
 // buffers whose sizes repeat from frame to frame (one call per expert node per frame), so
 // blocks are kept in a small pool instead of going back to hipFree -- which synchronises the
 // device -- and to hipMalloc on the next call.  The entry points hold the library's lock and
-// end with the stream idle, so a block returned at scope exit is free for the next call.
+// end with the stream idle (drop_transfers for one that fails), so a block returned at scope exit
+// is free for the next call.
 struct StagingPool {
   struct Block {
     void* p;
@@ -1491,15 +1521,11 @@ StagingPool g_staging;
 struct DevBuf {
   void* p = nullptr;
   size_t cap = 0;
-  DevBuf() { ++g_live_devbufs; }
+  DevBuf() = default;
   DevBuf(const DevBuf&) = delete;
   DevBuf& operator=(const DevBuf&) = delete;
   ~DevBuf() {
     if (p) g_staging.give(p, cap);
-    if (--g_live_devbufs == 0) {  // the call is over: the stream is idle, or the call failed and its fetches are void
-      g_fetches.clear();
-      g_pinned.reset();
-    }
   }
   int alloc(size_t bytes) {
     if (p) {

@@ -1,0 +1,285 @@
+// The host side of the library without a GPU: this program defines the runtime functions that the
+// library calls (an executable's definitions come before a shared library's), so that what
+// the stream does can be put off as long as a real one may put it off, and can be made to fail.
+//
+// The stream executes what is queued on it when somebody waits for it, or piece by piece while
+// an event is polled.  Kernels are known by name; those that a check does not look at do nothing.
+#include <hip/hip_runtime_api.h>
+#include <malloc.h>
+
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <deque>
+#include <functional>
+#include <map>
+#include <mutex>
+#include <string>
+#include <vector>
+
+#include "coalsack_moe.h"
+
+namespace fake {
+std::recursive_mutex m;
+// (used by the library's own initialisation, before this program's)
+std::map<const void*, std::string>& kernels() {  // host stub -> device name
+  static std::map<const void*, std::string> k;
+  return k;
+}
+std::map<const void*, std::vector<char>>& vars() {
+  static std::map<const void*, std::vector<char>> v;
+  return v;
+}
+std::map<void*, size_t> device;              // live allocations
+size_t device_bytes = 0;
+std::deque<std::function<void()>> queue;     // the library's stream
+std::deque<std::function<void()>> null_queue;  // the null stream, which nothing orders against it
+long executed = 0, queued = 0;               // of the library's stream
+int fail_launch_in = -1;                     // launches until one fails
+hipError_t last = hipSuccess;
+long launches = 0;
+dim3 grid, block;
+size_t shmem;
+hipStream_t st;
+
+void run(std::deque<std::function<void()>>& q, size_t n) {
+  for (; n && !q.empty(); --n) {
+    auto f = q.front();
+    q.pop_front();
+    f();
+    if (&q == &queue) ++executed;
+  }
+}
+void run_all() { run(queue, (size_t)-1); }
+void put(std::function<void()> f) {
+  queue.push_back(std::move(f));
+  ++queued;
+}
+struct Event {
+  long at = 0;
+};
+
+hipError_t launch(const void* f, void** args) {
+  std::lock_guard<std::recursive_mutex> g(m);
+  ++launches;
+  if (fail_launch_in >= 0 && fail_launch_in-- == 0) return last = hipErrorLaunchFailure;
+  const std::string& name = kernels()[f];
+  auto is = [&](const char* s) { return name.find(s) != std::string::npos; };
+  if (is("link_copy_kernel")) {
+    auto src = *(const char**)args[0];
+    auto dst = *(char**)args[1];
+    auto n = *(size_t*)args[2];
+    put([=] { std::memmove(dst, src, n); });
+  } else if (is("fill_cells_kernel")) {
+    auto p = *(unsigned long long**)args[0];
+    auto n = *(int*)args[1];
+    auto v = *(unsigned long long*)args[2];
+    put([=] {
+      for (int i = 0; i < n; ++i) p[i] = v;
+    });
+  } else if (is("10add_kernel")) {
+    auto a = *(const float**)args[0];
+    auto b = *(const float**)args[1];
+    auto o = *(float**)args[2];
+    auto n = *(long*)args[3];
+    put([=] {
+      for (long i = 0; i < n; ++i) o[i] = a[i] + b[i];
+    });
+  } else {
+    put([] {});
+  }
+  return hipSuccess;
+}
+}  // namespace fake
+
+extern "C" {
+void** __hipRegisterFatBinary(const void*) {
+  static void* h;
+  return &h;
+}
+void __hipUnregisterFatBinary(void**) {}
+void __hipRegisterFunction(void**, const void* f, char*, const char* name, unsigned, void*, void*, dim3*, dim3*, int*) {
+  fake::kernels()[f] = name;
+}
+void __hipRegisterVar(void**, void* var, char*, char*, int, size_t size, int, int) { fake::vars()[var].resize(size); }
+hipError_t __hipPushCallConfiguration(dim3 g, dim3 b, size_t s, hipStream_t t) {
+  fake::grid = g, fake::block = b, fake::shmem = s, fake::st = t;
+  return hipSuccess;
+}
+hipError_t __hipPopCallConfiguration(dim3* g, dim3* b, size_t* s, hipStream_t* t) {
+  *g = fake::grid, *b = fake::block, *s = fake::shmem, *t = fake::st;
+  return hipSuccess;
+}
+hipError_t hipLaunchKernel(const void* f, dim3, dim3, void** args, size_t, hipStream_t) { return fake::launch(f, args); }
+hipError_t hipExtLaunchKernel(const void* f, dim3, dim3, void** args, size_t, hipStream_t, hipEvent_t, hipEvent_t, int) {
+  return fake::launch(f, args);
+}
+hipError_t hipFuncSetAttribute(const void*, hipFuncAttribute, int) { return hipSuccess; }
+hipError_t hipGetLastError() {
+  std::lock_guard<std::recursive_mutex> g(fake::m);
+  const hipError_t e = fake::last;
+  fake::last = hipSuccess;
+  return e;
+}
+const char* hipGetErrorString(hipError_t) { return "(stated by the test)"; }
+hipError_t hipGetDeviceCount(int* n) {
+  *n = 1;
+  return hipSuccess;
+}
+hipError_t hipSetDevice(int) { return hipSuccess; }
+hipError_t hipGetDeviceProperties(hipDeviceProp_t* p, int) {
+  std::memset(p, 0, sizeof *p);
+  std::strcpy(p->gcnArchName, "gfx950");
+  p->multiProcessorCount = 256;
+  return hipSuccess;
+}
+hipError_t hipMemGetInfo(size_t* f, size_t* t) {
+  *t = (size_t)288 << 30;
+  *f = *t - fake::device_bytes;
+  return hipSuccess;
+}
+hipError_t hipGetSymbolAddress(void** p, const void* s) {
+  *p = fake::vars()[s].data();
+  return hipSuccess;
+}
+hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) {
+  *s = (hipStream_t)8;
+  return hipSuccess;
+}
+hipError_t hipStreamSynchronize(hipStream_t) {
+  std::lock_guard<std::recursive_mutex> g(fake::m);
+  fake::run_all();
+  return hipSuccess;
+}
+hipError_t hipMalloc(void** p, size_t n) {
+  std::lock_guard<std::recursive_mutex> g(fake::m);
+  *p = std::calloc(n, 1);
+  fake::device[*p] = n;
+  fake::device_bytes += n;
+  return *p ? hipSuccess : hipErrorOutOfMemory;
+}
+hipError_t hipFree(void* p) {  // waits for the device, as the real one does
+  std::lock_guard<std::recursive_mutex> g(fake::m);
+  fake::run_all();
+  fake::run(fake::null_queue, (size_t)-1);
+  fake::device_bytes -= fake::device[p];
+  fake::device.erase(p);
+  std::free(p);
+  return hipSuccess;
+}
+hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
+  *p = std::malloc(n);
+  return *p ? hipSuccess : hipErrorOutOfMemory;
+}
+hipError_t hipMemset(void* p, int v, size_t n) {  // on the null stream; device memory: not awaited
+  std::lock_guard<std::recursive_mutex> g(fake::m);
+  fake::null_queue.push_back([=] { std::memset(p, v, n); });
+  return hipSuccess;
+}
+hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) {
+  std::lock_guard<std::recursive_mutex> g(fake::m);
+  fake::run(fake::null_queue, (size_t)-1);
+  std::memcpy(d, s, n);
+  return hipSuccess;
+}
+hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) {
+  std::lock_guard<std::recursive_mutex> g(fake::m);
+  fake::put([=] { std::memcpy(d, s, n); });
+  return hipSuccess;
+}
+hipError_t hipEventCreate(hipEvent_t* e) {
+  *e = (hipEvent_t) new fake::Event;
+  return hipSuccess;
+}
+hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { return hipEventCreate(e); }
+hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t) {
+  std::lock_guard<std::recursive_mutex> g(fake::m);
+  ((fake::Event*)e)->at = fake::queued;
+  return hipSuccess;
+}
+hipError_t hipEventQuery(hipEvent_t e) {
+  std::lock_guard<std::recursive_mutex> g(fake::m);
+  const long at = ((fake::Event*)e)->at;
+  if (fake::executed < at && std::rand() % 4 == 0) fake::run(fake::queue, 1);
+  return fake::executed >= at ? hipSuccess : (fake::last = hipErrorNotReady);
+}
+hipError_t hipEventSynchronize(hipEvent_t e) {
+  std::lock_guard<std::recursive_mutex> g(fake::m);
+  const long at = ((fake::Event*)e)->at;
+  while (fake::executed < at) fake::run(fake::queue, 1);
+  return hipSuccess;
+}
+hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) {
+  *ms = 0.f;
+  return hipSuccess;
+}
+}  // extern "C"
+
+#define CHECK(cond)                                                                        \
+  do {                                                                                     \
+    if (!(cond)) {                                                                         \
+      std::printf("line %d: %s (last error: %s)\n", __LINE__, #cond, csk_last_error());    \
+      return 1;                                                                            \
+    }                                                                                      \
+  } while (0)
+#define OK(call) CHECK((call) == CSK_OK)
+
+// A call fails between two results on their way down; the layer they were meant for goes away
+// and the next call ends.  (Vectors above 64 KiB are mappings of their own here: one that is
+// gone cannot be written without notice.)
+static int results_of_a_failed_call() {
+  mallopt(M_MMAP_THRESHOLD, 64 << 10);
+  const int64_t E = 2, k = 2, H = 2880, F = 32, T = 8;
+  std::vector<float> gate(E * H), hidden(T * H, 1.f), out(T * H), pairs(T * k * 2), norm(H);
+  std::vector<uint8_t> bytes(F * H / 32 * 17, 1);
+  csk_mxfp4 *u, *g, *d;
+  OK(csk_mxfp4_upload(bytes.data(), F, H, &u));
+  OK(csk_mxfp4_upload(bytes.data(), F, H, &g));
+  OK(csk_mxfp4_upload(bytes.data(), H, F, &d));
+  csk_layer *L, *other;
+  OK(csk_layer_create_view(E, k, H, F, &L));
+  OK(csk_layer_create_view(E, k, H, F, &other));
+  OK(csk_layer_set_router(L, gate.data(), nullptr));
+  for (int e = 0; e < E; ++e) OK(csk_layer_attach_expert(L, e, u, g, d, nullptr, nullptr, nullptr));
+  int running = 0;
+  OK(csk_moe_frame_begin(L, hidden.data(), T, pairs.data(), 0, &running));
+  CHECK(running);
+  fake::fail_launch_in = 1;  // the rows' copy is queued, that of their positions is refused
+  CHECK(csk_moe_frame_expert_rows(L, 0, out.data()) == CSK_ERR_HIP);
+  fake::fail_launch_in = -1;
+  csk_layer_destroy(L);
+  OK(csk_layer_set_norm(other, norm.data(), 1e-5f));
+  return 0;
+}
+
+// A call fails with a copy into the pinned area still queued; the next call's values pass
+// through the same place.
+static int pinned_area_after_a_failed_call() {
+  const int64_t T = 8, H = 256, E = 16, k = 4, n = 60000;
+  std::vector<double> hidden(T * H, 1.0), gate(E * H, 1.0), logits(T * E);
+  std::vector<float> pairs(T * k * 2), a(n), b(n), out(n);
+  fake::fail_launch_in = 5;  // gate, hidden, logits, selection, pairs down, logits down
+  CHECK(csk_moe_router_f64(hidden.data(), T, H, gate.data(), E, nullptr, k, 0, pairs.data(), logits.data()) == CSK_ERR_HIP);
+  CHECK(fake::fail_launch_in == -1);
+  for (int64_t i = 0; i < n; ++i) a[i] = (float)i, b[i] = 0.5f;
+  OK(csk_add(a.data(), b.data(), out.data(), n));
+  for (int64_t i = 0; i < n; ++i) CHECK(out[i] == a[i] + b[i]);
+  return 0;
+}
+
+int main(int argc, char** argv) {
+  const std::map<std::string, int (*)()> checks = {
+      {"results_of_a_failed_call", results_of_a_failed_call},
+      {"pinned_area_after_a_failed_call", pinned_area_after_a_failed_call},
+  };
+  if (argc != 2 || !checks.count(argv[1])) return 2;
+  if (csk_init(0) != CSK_OK) {
+    std::printf("csk_init: %s\n", csk_last_error());
+    return 3;
+  }
+  const int rc = checks.at(argv[1])();
+  std::printf("%s: %s\n", argv[1], rc ? "failed" : "ok");
+  std::fflush(stdout);
+  std::_Exit(rc);
+}

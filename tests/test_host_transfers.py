@@ -1,0 +1,29 @@
+"""The host side of the library on the CPU: tests/cpp/host_transfers.cpp stands in for the HIP
+runtime under libcoalsack_moe.so and says when the stream gets on and which call fails."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
+
+
+@pytest.fixture(scope="module")
+def driver(tmp_path_factory):
+    if not shutil.which("g++") or not os.path.isdir(os.path.join(ROCM, "include", "hip")):
+        pytest.skip("no g++ or no HIP headers")
+    lib = os.path.join(ROOT, "coalsack_amd")
+    exe = tmp_path_factory.mktemp("host_transfers") / "host_transfers"
+    subprocess.run(["g++", "-std=c++17", "-O1", "-g", "-rdynamic", "-pthread", "-D__HIP_PLATFORM_AMD__", "-I" + os.path.join(ROCM, "include"),
+                    "-I" + os.path.join(ROOT, "include"), os.path.join(ROOT, "tests", "cpp", "host_transfers.cpp"),
+                    "-o", str(exe), "-L" + lib, "-lcoalsack_moe", "-Wl,-rpath," + lib, "-Wl,-rpath-link," + os.path.join(ROCM, "lib")],
+                   check=True, timeout=300)
+    return str(exe)
+
+
+@pytest.mark.parametrize("check", ["results_of_a_failed_call", "pinned_area_after_a_failed_call"])
+def test_host_side(driver, check):
+    p = subprocess.run([driver, check], capture_output=True, text=True, timeout=120)
+    assert p.returncode == 0, (p.returncode, p.stdout[-2000:], p.stderr[-2000:])

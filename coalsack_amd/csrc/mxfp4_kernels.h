@@ -165,6 +165,11 @@ __global__ void fill_cells_kernel(unsigned long long* __restrict__ p, int n, uns
   if ((int)threadIdx.x < n) p[threadIdx.x] = v;
 }
 
+__global__ __launch_bounds__(256) void fill_words_kernel(uint32_t* __restrict__ p, long n, uint32_t v) {
+  const long stride = (long)gridDim.x * 256;
+  for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < n; i += stride) p[i] = v;
+}
+
 // Synthetic weights, generated straight into the packed layout.  Block b =
 // row * nblk + kb of the stream with key `key` is, in the reference's format,
 //   scale byte = scale_lo + (h0 >> 33) % scale_span,

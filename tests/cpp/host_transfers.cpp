@@ -38,6 +38,7 @@ long executed = 0, queued = 0;               // of the library's stream
 int fail_launch_in = -1;                     // launches until one fails
 hipError_t last = hipSuccess;
 long launches = 0;
+unsigned char* packed_scales = nullptr;      // scale plane that the last pack kernel wrote
 dim3 grid, block;
 size_t shmem;
 hipStream_t st;
@@ -77,6 +78,17 @@ hipError_t launch(const void* f, void** args) {
     put([=] {
       for (int i = 0; i < n; ++i) p[i] = v;
     });
+  } else if (is("fill_words_kernel")) {
+    auto p = *(uint32_t**)args[0];
+    auto n = *(long*)args[1];
+    auto v = *(uint32_t*)args[2];
+    put([=] {
+      for (long i = 0; i < n; ++i) p[i] = v;
+    });
+  } else if (is("pack_mxfp4_kernel")) {
+    auto s = *(unsigned char**)args[2];
+    packed_scales = s;
+    put([=] { std::memset(s, 0x55, 256); });
   } else if (is("10add_kernel")) {
     auto a = *(const float**)args[0];
     auto b = *(const float**)args[1];
@@ -268,10 +280,23 @@ static int pinned_area_after_a_failed_call() {
   return 0;
 }
 
+// Nothing orders the null stream against the library's: what is written there may land late.
+static int scales_of_an_uploaded_matrix() {
+  std::vector<uint8_t> bytes(16 * 17, 1);
+  csk_mxfp4* m;
+  OK(csk_mxfp4_upload(bytes.data(), 16, 32, &m));
+  fake::run(fake::null_queue, (size_t)-1);
+  for (int i = 0; i < 256; ++i) CHECK(fake::packed_scales[i] == 0x55);
+  // padding (this plane has 2 KiB) holds the scale of 1
+  for (int i = 256; i < 2048; ++i) CHECK(fake::packed_scales[i] == 127);
+  return 0;
+}
+
 int main(int argc, char** argv) {
   const std::map<std::string, int (*)()> checks = {
       {"results_of_a_failed_call", results_of_a_failed_call},
       {"pinned_area_after_a_failed_call", pinned_area_after_a_failed_call},
+      {"scales_of_an_uploaded_matrix", scales_of_an_uploaded_matrix},
   };
   if (argc != 2 || !checks.count(argv[1])) return 2;
   if (csk_init(0) != CSK_OK) {

@@ -23,7 +23,10 @@ def driver(tmp_path_factory):
     return str(exe)
 
 
-@pytest.mark.parametrize("check", ["results_of_a_failed_call", "pinned_area_after_a_failed_call"])
+CHECKS = ["results_of_a_failed_call", "pinned_area_after_a_failed_call", "scales_of_an_uploaded_matrix"]
+
+
+@pytest.mark.parametrize("check", CHECKS)
 def test_host_side(driver, check):
     p = subprocess.run([driver, check], capture_output=True, text=True, timeout=120)
     assert p.returncode == 0, (p.returncode, p.stdout[-2000:], p.stderr[-2000:])

@@ -208,15 +208,15 @@ class HostLink {
   // dst (device) <- host memory, queued on the stream.  The host memory may be reused on return.
   hipError_t to_device(void* dst, const void* host, size_t bytes, hipStream_t st) {
     if (bytes == 0) return hipSuccess;
-    hipError_t err = ready();
-    if (err != hipSuccess) return err;
+    if (!ready()) return by_runtime(dst, host, bytes, hipMemcpyHostToDevice, st);
+    hipError_t err = hipSuccess;
     CopyCrew::Job job{static_cast<char*>(const_cast<void*>(host)), ring_, bytes, at_, kLinkRing, true};
     const long n = job.pieces();
     // A copy kernel costs about 3.5 us of its own.  Onto an idle stream the first ones are
     // short, so that the device starts early; they grow as the host gets ahead.
     const long first = (long)(at_ / kLinkPiece);
     long ready_to = 0, sent = 0, opened = 0, want = first == 0 ? 3 : 16;
-    if (!crew_.ready() || !crew_->begin(job)) return hipErrorOutOfMemory;
+    if (!crew_->begin(job)) return by_runtime(dst, host, bytes, hipMemcpyHostToDevice, st);
     while (sent < n && err == hipSuccess) {
       while (opened < n) {  // pieces whose place in the ring is free, up to the end of their quarter
         const long end = quarter_end(first + opened);
@@ -253,15 +253,15 @@ class HostLink {
   // host memory <- src (device), after the work queued on the stream.  Waits for all of it.
   hipError_t to_host(void* host, const void* src, size_t bytes, hipStream_t st) {
     if (bytes == 0) return hipSuccess;
-    hipError_t err = ready();
-    if (err != hipSuccess) return err;
+    if (!ready()) return by_runtime(host, src, bytes, hipMemcpyDeviceToHost, st);
+    hipError_t err = hipSuccess;
     // (places in the ring that an earlier transfer up still reads are written after it, in stream order)
     CopyCrew::Job job{static_cast<char*>(host), ring_, bytes, 0, kLinkRing, false};
     const long n = job.pieces();
     long queued = 0, landed = 0, freed = 0;  // pieces requested, in pinned memory, copied out
     long ends[kDown];
     int put = 0, got = 0;  // chunks requested and landed
-    if (!crew_.ready() || !crew_->begin(job)) return hipErrorOutOfMemory;
+    if (!crew_->begin(job)) return by_runtime(host, src, bytes, hipMemcpyDeviceToHost, st);
     while (freed < n && err == hipSuccess) {
       // Half of what is left per chunk, at most 1 MiB: few chunks (each costs about 6 us for
       // its kernel and event), and little left to copy once the last has landed.
@@ -311,16 +311,29 @@ class HostLink {
   hipEvent_t quarter_[kQuarters] = {}, down_[kDown] = {};
   bool in_use_[kQuarters] = {};  // the device may still be reading that quarter
   CrewOwner crew_;
+  bool refused_ = false;
 
-  hipError_t ready() {
-    if (ring_) return hipSuccess;
-    for (hipEvent_t& e : quarter_)
-      if (!e)
-        if (const hipError_t rc = hipEventCreateWithFlags(&e, hipEventDisableTiming); rc != hipSuccess) return rc;
-    for (hipEvent_t& e : down_)
-      if (!e)
-        if (const hipError_t rc = hipEventCreateWithFlags(&e, hipEventDisableTiming); rc != hipSuccess) return rc;
-    return hipHostMalloc(reinterpret_cast<void**>(&ring_), kLinkRing, hipHostMallocDefault);
+  // false: the machine gives no pinned memory (asked for once), or no memory for the crew
+  bool ready() {
+    if (ring_) return true;
+    if (refused_ || !crew_.ready()) return false;
+    hipError_t rc = hipSuccess;
+    for (hipEvent_t* e = quarter_; e < quarter_ + kQuarters && rc == hipSuccess; ++e)
+      if (!*e) rc = hipEventCreateWithFlags(e, hipEventDisableTiming);
+    for (hipEvent_t* e = down_; e < down_ + kDown && rc == hipSuccess; ++e)
+      if (!*e) rc = hipEventCreateWithFlags(e, hipEventDisableTiming);
+    if (rc == hipSuccess) rc = hipHostMalloc(reinterpret_cast<void**>(&ring_), kLinkRing, hipHostMallocDefault);
+    if (rc == hipSuccess) return true;
+    (void)hipGetLastError();
+    ring_ = nullptr, refused_ = true;
+    return false;
+  }
+  // The runtime's own copy of pageable memory, with the same promise: the host's side is done on return.
+  hipError_t by_runtime(void* dst, const void* src, size_t bytes, hipMemcpyKind kind, hipStream_t st) {
+    const hipError_t rc = hipMemcpyAsync(dst, src, bytes, kind, st);
+    const hipError_t rs = hipStreamSynchronize(st);
+    if (rc == hipSuccess && rs == hipSuccess) idle();
+    return rc != hipSuccess ? rc : rs;
   }
   static long quarter_end(long piece) { return (piece / kPerQuarter + 1) * kPerQuarter; }
   static hipError_t launch(void* dst, const void* src, size_t bytes, hipStream_t st) {

@@ -38,6 +38,7 @@ long executed = 0, queued = 0;               // of the library's stream
 int fail_launch_in = -1;                     // launches until one fails
 hipError_t last = hipSuccess;
 long launches = 0;
+bool refuse_pinned = false;
 unsigned char* packed_scales = nullptr;      // scale plane that the last pack kernel wrote
 dim3 grid, block;
 size_t shmem;
@@ -180,6 +181,7 @@ hipError_t hipFree(void* p) {  // waits for the device, as the real one does
   return hipSuccess;
 }
 hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
+  if (fake::refuse_pinned) return fake::last = hipErrorOutOfMemory;
   *p = std::malloc(n);
   return *p ? hipSuccess : hipErrorOutOfMemory;
 }
@@ -280,6 +282,18 @@ static int pinned_area_after_a_failed_call() {
   return 0;
 }
 
+// Pageable memory is enough for every call where the machine gives no pinned memory.
+static int no_pinned_memory() {
+  fake::refuse_pinned = true;
+  for (int64_t n : {100, 300000}) {
+    std::vector<float> a(n), b(n), out(n);
+    for (int64_t i = 0; i < n; ++i) a[i] = (float)i, b[i] = 0.5f;
+    OK(csk_add(a.data(), b.data(), out.data(), n));
+    for (int64_t i = 0; i < n; ++i) CHECK(out[i] == a[i] + b[i]);
+  }
+  return 0;
+}
+
 // Nothing orders the null stream against the library's: what is written there may land late.
 static int scales_of_an_uploaded_matrix() {
   std::vector<uint8_t> bytes(16 * 17, 1);
@@ -296,6 +310,7 @@ int main(int argc, char** argv) {
   const std::map<std::string, int (*)()> checks = {
       {"results_of_a_failed_call", results_of_a_failed_call},
       {"pinned_area_after_a_failed_call", pinned_area_after_a_failed_call},
+      {"no_pinned_memory", no_pinned_memory},
       {"scales_of_an_uploaded_matrix", scales_of_an_uploaded_matrix},
   };
   if (argc != 2 || !checks.count(argv[1])) return 2;

@@ -23,7 +23,8 @@ def driver(tmp_path_factory):
     return str(exe)
 
 
-CHECKS = ["results_of_a_failed_call", "pinned_area_after_a_failed_call", "scales_of_an_uploaded_matrix"]
+CHECKS = ["results_of_a_failed_call", "pinned_area_after_a_failed_call", "scales_of_an_uploaded_matrix",
+          "no_pinned_memory"]
 
 
 @pytest.mark.parametrize("check", CHECKS)

@@ -18,6 +18,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <chrono>
 #include <condition_variable>
 #include <cstddef>
 #include <cstdint>
@@ -71,11 +72,13 @@ constexpr size_t kLinkRing = (size_t)16 << 20;
 
 // The calling thread and its helpers copy the pieces of one transfer between the caller's
 // memory and the ring, in ascending order; piece i may be taken once `open` is past it.
-// Helpers sleep between transfers (after a short spin, so that the calls of a loop find them
-// awake) and end with the process.
+// Helpers sleep between transfers and while no piece is open -- a result may be behind a long forward --
+// after a short spin each time, so that the calls of a loop and the chunks of a running transfer find
+// them awake.  They end with the process.
 class CopyCrew {
  public:
   static constexpr int kHelpers = 3;
+  static constexpr int kSpins = 20000;  // some hundred microseconds
 
   ~CopyCrew() {
     {
@@ -122,7 +125,10 @@ class CopyCrew {
     cv_.notify_all();
     return true;
   }
-  void open_to(long piece) { open_.store(std::min(piece, n_), std::memory_order_release); }
+  void open_to(long piece) {
+    open_.store(std::min(piece, n_));
+    wake();
+  }
   bool done(long i) const { return done_[(size_t)i].load(std::memory_order_acquire); }
   // takes one open piece, if there is one
   bool work_one() {
@@ -145,6 +151,7 @@ class CopyCrew {
       std::lock_guard<std::mutex> g(m_);
       running_.store(false);
     }
+    wake();
     while (inside_.load(std::memory_order_acquire) != 0) relax();
   }
 
@@ -154,7 +161,7 @@ class CopyCrew {
   void help() {
     uint64_t seen = 0;
     for (;;) {
-      for (int spin = 0; spin < 20000 && epoch_.load(std::memory_order_acquire) == seen && !stop_.load(); ++spin) relax();
+      for (int spin = 0; spin < kSpins && epoch_.load(std::memory_order_acquire) == seen && !stop_.load(); ++spin) relax();
       {
         std::unique_lock<std::mutex> g(m_);
         cv_.wait(g, [&] { return stop_.load() || epoch_.load() != seen; });
@@ -163,10 +170,28 @@ class CopyCrew {
         if (!running_.load()) continue;
         inside_.fetch_add(1);
       }
-      while (running_.load(std::memory_order_acquire) && next_.load(std::memory_order_relaxed) < n_)
-        if (!work_one()) relax();
+      int spin = 0;
+      while (running_.load(std::memory_order_acquire) && next_.load(std::memory_order_relaxed) < n_) {
+        if (work_one()) {
+          spin = 0;
+        } else if (++spin < kSpins) {
+          relax();
+        } else {
+          std::unique_lock<std::mutex> g(m_);
+          asleep_.fetch_add(1);  // before the look at open_, as wake() looks after open_ has changed
+          cv_.wait(g, [&] { return !running_.load() || next_.load() < open_.load(); });
+          asleep_.fetch_sub(1);
+          spin = 0;
+        }
+      }
       inside_.fetch_sub(1, std::memory_order_release);
     }
+  }
+
+  void wake() {
+    if (asleep_.load() == 0) return;
+    { std::lock_guard<std::mutex> g(m_); }  // whoever counts as asleep holds the lock until it waits
+    cv_.notify_all();
   }
 
   std::vector<std::thread> threads_;
@@ -174,11 +199,30 @@ class CopyCrew {
   std::condition_variable cv_;
   std::atomic<bool> stop_{false}, running_{false};
   std::atomic<uint64_t> epoch_{0};
-  std::atomic<int> inside_{0};
+  std::atomic<int> inside_{0}, asleep_{0};
   Job job_{};
   long n_ = 0;
   std::atomic<long> next_{0}, open_{0};
   std::vector<std::atomic<bool>> done_;
+};
+
+// What the calling thread does while only the device can get a transfer on: it polls for a while -- a
+// chunk takes 20 us -- and leaves longer waits, for the work in front of the transfer, to the runtime.
+class DeviceWait {
+ public:
+  void progress() { since_ = std::chrono::steady_clock::now(); }
+  hipError_t once(hipEvent_t e) {
+    if (std::chrono::steady_clock::now() - since_ < std::chrono::microseconds(200)) {
+      CopyCrew::relax();
+      return hipSuccess;
+    }
+    const hipError_t rc = hipEventSynchronize(e);
+    progress();
+    return rc;
+  }
+
+ private:
+  std::chrono::steady_clock::time_point since_ = std::chrono::steady_clock::now();
 };
 
 // The crew of this process.  A forked child has the object but not its threads: joining them, or
@@ -217,6 +261,7 @@ class HostLink {
     const long first = (long)(at_ / kLinkPiece);
     long ready_to = 0, sent = 0, opened = 0, want = first == 0 ? 3 : 16;
     if (!crew_->begin(job)) return by_runtime(dst, host, bytes, hipMemcpyHostToDevice, st);
+    DeviceWait wait;
     while (sent < n && err == hipSuccess) {
       while (opened < n) {  // pieces whose place in the ring is free, up to the end of their quarter
         const long end = quarter_end(first + opened);
@@ -241,7 +286,12 @@ class HostLink {
         }
         sent = to;
         want = std::min(2 * want, 16L);  // (longer ones would leave the device waiting for the host)
-      } else if (!worked) {
+        wait.progress();
+      } else if (worked) {
+        wait.progress();
+      } else if (sent == opened && opened < n) {  // everything that fits the ring has been sent
+        err = wait.once(quarter_[(quarter_end(first + opened) - 1) % kPieces / kPerQuarter]);
+      } else {
         CopyCrew::relax();
       }
     }
@@ -262,6 +312,7 @@ class HostLink {
     long ends[kDown];
     int put = 0, got = 0;  // chunks requested and landed
     if (!crew_->begin(job)) return by_runtime(host, src, bytes, hipMemcpyDeviceToHost, st);
+    DeviceWait wait;
     while (freed < n && err == hipSuccess) {
       // Half of what is left per chunk, at most 1 MiB: few chunks (each costs about 6 us for
       // its kernel and event), and little left to copy once the last has landed.
@@ -287,7 +338,12 @@ class HostLink {
         landed = ends[got++ % kDown];
         crew_->open_to(landed);
       }
-      if (!crew_->work_one()) CopyCrew::relax();
+      if (crew_->work_one())
+        wait.progress();
+      else if (freed == landed && got < put && err == hipSuccess)
+        err = wait.once(down_[got % kDown]);
+      else
+        CopyCrew::relax();
       while (freed < landed && crew_->done(freed)) ++freed;
     }
     crew_->end();

@@ -7,14 +7,17 @@
 #include <hip/hip_runtime_api.h>
 #include <malloc.h>
 
+#include <chrono>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <ctime>
 #include <deque>
 #include <functional>
 #include <map>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "coalsack_moe.h"
@@ -39,11 +42,14 @@ int fail_launch_in = -1;                     // launches until one fails
 hipError_t last = hipSuccess;
 long launches = 0;
 bool refuse_pinned = false;
+double stream_busy_until = 0.0;              // by the process's wall clock: the stream does nothing before
 unsigned char* packed_scales = nullptr;      // scale plane that the last pack kernel wrote
 dim3 grid, block;
 size_t shmem;
 hipStream_t st;
 
+std::function<void()> before_kernel;         // called once, when the next add_kernel is queued
+double now() { return std::chrono::duration<double>(std::chrono::steady_clock::now().time_since_epoch()).count(); }
 void run(std::deque<std::function<void()>>& q, size_t n) {
   for (; n && !q.empty(); --n) {
     auto f = q.front();
@@ -52,7 +58,13 @@ void run(std::deque<std::function<void()>>& q, size_t n) {
     if (&q == &queue) ++executed;
   }
 }
-void run_all() { run(queue, (size_t)-1); }
+void wait_for_stream() {
+  while (now() < stream_busy_until) std::this_thread::sleep_for(std::chrono::milliseconds(1));
+}
+void run_all() {
+  wait_for_stream();
+  run(queue, (size_t)-1);
+}
 void put(std::function<void()> f) {
   queue.push_back(std::move(f));
   ++queued;
@@ -95,6 +107,7 @@ hipError_t launch(const void* f, void** args) {
     auto b = *(const float**)args[1];
     auto o = *(float**)args[2];
     auto n = *(long*)args[3];
+    if (before_kernel) run_all(), before_kernel(), before_kernel = nullptr;
     put([=] {
       for (long i = 0; i < n; ++i) o[i] = a[i] + b[i];
     });
@@ -215,12 +228,13 @@ hipError_t hipEventRecord(hipEvent_t e, hipStream_t) {
 hipError_t hipEventQuery(hipEvent_t e) {
   std::lock_guard<std::recursive_mutex> g(fake::m);
   const long at = ((fake::Event*)e)->at;
-  if (fake::executed < at && std::rand() % 4 == 0) fake::run(fake::queue, 1);
+  if (fake::executed < at && fake::now() >= fake::stream_busy_until && std::rand() % 4 == 0) fake::run(fake::queue, 1);
   return fake::executed >= at ? hipSuccess : (fake::last = hipErrorNotReady);
 }
 hipError_t hipEventSynchronize(hipEvent_t e) {
   std::lock_guard<std::recursive_mutex> g(fake::m);
   const long at = ((fake::Event*)e)->at;
+  if (fake::executed < at) fake::wait_for_stream();
   while (fake::executed < at) fake::run(fake::queue, 1);
   return hipSuccess;
 }
@@ -294,6 +308,32 @@ static int no_pinned_memory() {
   return 0;
 }
 
+// Processor time of the whole process while the stream is at work for half a second in front of a
+// result, and in front of the room that an upload waits for: the threads sleep, the caller too.
+static int threads_sleep_while_the_stream_works() {
+  const int64_t n = 6000000;  // 24 MB: larger than the ring
+  std::vector<float> a(n, 1.f), b(n, 2.f), out(n);
+  OK(csk_add(a.data(), b.data(), out.data(), n));
+  for (int part = 0; part < 2; ++part) {
+    std::this_thread::sleep_for(std::chrono::milliseconds(50));
+    const double t0 = fake::now();
+    const std::clock_t c0 = std::clock();
+    if (part == 0) {
+      fake::stream_busy_until = t0 + 0.5;  // the uploads find the ring full
+      OK(csk_add(a.data(), b.data(), out.data(), n));
+    } else {
+      fake::before_kernel = [] { fake::stream_busy_until = fake::now() + 0.5; };  // the result comes late
+      OK(csk_add(a.data(), b.data(), out.data(), n));
+    }
+    const double wall = fake::now() - t0, cpu = double(std::clock() - c0) / CLOCKS_PER_SEC;
+    std::printf("part %d: %.3f s wall, %.3f s of processor time\n", part, wall, cpu);
+    CHECK(wall >= 0.5);
+    CHECK(cpu < 0.25);
+    CHECK(out[0] == 3.f && out[n - 1] == 3.f);
+  }
+  return 0;
+}
+
 // Nothing orders the null stream against the library's: what is written there may land late.
 static int scales_of_an_uploaded_matrix() {
   std::vector<uint8_t> bytes(16 * 17, 1);
@@ -311,6 +351,7 @@ int main(int argc, char** argv) {
       {"results_of_a_failed_call", results_of_a_failed_call},
       {"pinned_area_after_a_failed_call", pinned_area_after_a_failed_call},
       {"no_pinned_memory", no_pinned_memory},
+      {"threads_sleep_while_the_stream_works", threads_sleep_while_the_stream_works},
       {"scales_of_an_uploaded_matrix", scales_of_an_uploaded_matrix},
   };
   if (argc != 2 || !checks.count(argv[1])) return 2;

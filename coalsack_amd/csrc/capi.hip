@@ -38,7 +38,7 @@ int g_cus = 0;
 // of the reference's scheduler (layer_scheduler_node), without locking of their own.
 std::recursive_mutex g_api;
 thread_local bool t_device_bound = false;  // the current device is a per-thread setting
-void drop_transfers();
+void end_call();
 // Also the place where a call that failed halfway is cleaned up after.
 struct ApiGuard {
   ApiGuard() {
@@ -48,7 +48,7 @@ struct ApiGuard {
   ApiGuard(const ApiGuard&) = delete;
   ApiGuard& operator=(const ApiGuard&) = delete;
   ~ApiGuard() {
-    if (--depth() == 0) drop_transfers();
+    if (--depth() == 0) end_call();
     g_api.unlock();
   }
 
@@ -380,7 +380,7 @@ namespace {
   } while (0)
 
 // Small transfers share one pinned area: space is handed out in order and taken back all at
-// once when the stream is idle (finish_fetches, or drop_transfers for a call that failed before
+// once when the stream is idle (finish_fetches, or end_call for a call that failed before
 // that), so that a call's pieces queue one behind the other and the call waits once, at its
 // end.  Larger ones go through the ring of HostLink (host_link.h).
 struct PinnedArena {
@@ -473,24 +473,31 @@ int finish_fetches() {
   return CSK_OK;
 }
 
-// The end of an entry point: a call that came to its end has finished its transfers, so only one that
-// failed in between leaves any.  Its results go nowhere -- the caller's memory may be gone after
-// the return -- and nothing queued may still touch the pinned area when the next call fills it.
-void drop_transfers() {
-  if (g_fetches.empty() && g_pinned.used == 0) return;
-  (void)hipStreamSynchronize(g_stream);
-  g_fetches.clear();
-  g_pinned.reset();
-}
-
 // Upload `rows x K` reference blocks and repack into (q, s).  The staging buffer is kept
 // between calls (a checkpoint is hundreds of matrices of one size; the stream orders one
-// matrix behind the other); the scale bytes are checked by the pack kernel as it reads
-// them, so the host touches the blocks only to hand them to the link.  After a refused block
-// the planes of m hold partial data.
+// matrix behind the other) up to the size of a large expert matrix; the scale bytes are
+// checked by the pack kernel as it reads them, so the host touches the blocks only to hand
+// them to the link.  After a refused block the planes of m hold partial data.
 uint8_t* g_stage = nullptr;
 size_t g_stage_cap = 0;
+constexpr size_t kStageKept = (size_t)256 << 20;  // (8192 x 8192 halves are 128 MiB)
 unsigned long long* g_bad = nullptr;  // first refused block of up to three matrices
+
+// The end of an entry point.  A call that came to its end has finished its transfers, so only one
+// that failed in between leaves any: its results go nowhere -- the caller's memory may be gone
+// after the return -- and nothing queued may still touch the pinned area when the next call fills it.
+void end_call() {
+  if (!g_fetches.empty() || g_pinned.used != 0) {
+    (void)hipStreamSynchronize(g_stream);
+    g_fetches.clear();
+    g_pinned.reset();
+  }
+  if (g_stage_cap > kStageKept) {  // an output head's size: not for the rest of the process
+    (void)hipStreamSynchronize(g_stream);
+    (void)hipFree(g_stage);
+    g_stage = nullptr, g_stage_cap = 0;
+  }
+}
 
 int stage_bytes(size_t bytes) {
   if (bytes > g_stage_cap) {
@@ -1486,7 +1493,7 @@ namespace {
 // buffers whose sizes repeat from frame to frame (one call per expert node per frame), so
 // blocks are kept in a small pool instead of going back to hipFree -- which synchronises the
 // device -- and to hipMalloc on the next call.  The entry points hold the library's lock and
-// end with the stream idle (drop_transfers for one that fails), so a block returned at scope exit
+// end with the stream idle (end_call for one that fails), so a block returned at scope exit
 // is free for the next call.
 struct StagingPool {
   struct Block {

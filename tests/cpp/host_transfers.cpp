@@ -334,6 +334,30 @@ static int threads_sleep_while_the_stream_works() {
   return 0;
 }
 
+// What an upload stages on the device is given back if it is large: an output head of 300 MB
+// must not cost that much memory for good.
+static int staging_memory_after_a_large_upload() {
+  const int64_t rows = 65536, K = 2304;
+  const size_t before = fake::device_bytes;
+  std::vector<uint16_t> w((size_t)rows * K);
+  csk_f16* m;
+  OK(csk_f16_upload(w.data(), rows, K, &m));
+  CHECK(fake::device_bytes >= before + w.size() * 2);
+  csk_f16_free(m);
+  CHECK(fake::device_bytes <= before + ((size_t)256 << 20));
+  // an expert's matrices, on the other hand, find it there the second time
+  std::vector<uint8_t> bytes(2880 * 90 * 17, 1);
+  csk_mxfp4* q;
+  OK(csk_mxfp4_upload(bytes.data(), 2880, 2880, &q));
+  csk_mxfp4_free(q);
+  uint64_t count0 = 0, count1 = 0;
+  OK(csk_alloc_count(&count0));
+  OK(csk_mxfp4_upload(bytes.data(), 2880, 2880, &q));
+  OK(csk_alloc_count(&count1));
+  CHECK(count1 - count0 == 2);  // the two planes
+  return 0;
+}
+
 // Nothing orders the null stream against the library's: what is written there may land late.
 static int scales_of_an_uploaded_matrix() {
   std::vector<uint8_t> bytes(16 * 17, 1);
@@ -352,6 +376,7 @@ int main(int argc, char** argv) {
       {"pinned_area_after_a_failed_call", pinned_area_after_a_failed_call},
       {"no_pinned_memory", no_pinned_memory},
       {"threads_sleep_while_the_stream_works", threads_sleep_while_the_stream_works},
+      {"staging_memory_after_a_large_upload", staging_memory_after_a_large_upload},
       {"scales_of_an_uploaded_matrix", scales_of_an_uploaded_matrix},
   };
   if (argc != 2 || !checks.count(argv[1])) return 2;

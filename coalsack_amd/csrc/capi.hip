@@ -608,22 +608,23 @@ inline int stream_group_tokens(int64_t T, int64_t H, int64_t F) {
 // / GEMM), m assignments per expert: 128 x 2880 x 2880 (1.7 GB) m = 2 308 / 350, 4 400 / 396,
 // 8 505 / 409; 32 experts of it m = 6 124 / 124, 8 141 / 125; 8 experts m = 4 50 / 66, 12 70 / 69,
 // 16 75 / 70; 16 x 4096 x 6144 (0.6 GB, groups of four) m = 4 164 / 164, 6 207 / 165.  Tokens per
-// expert are taken as Poisson distributed about m.
+// expert are taken as Poisson distributed about m, except that none can have more than T: up to one
+// pass of tokens the weights are streamed once whatever their size (8 x 4096 x 8192, top-8, one token 90 / 121;
+// 8 x 6144 x 8192, top-8, four tokens 149 / 184).  (The exact distribution beyond that, binomial, moves calls
+// across the line both ways: 64 x 5120 x 6144, top-4, 30 tokens 485 / 656 to the streaming side, but
+// 16 x 2048 x 5120, top-2, 34 tokens 103 / 92 as well.)
 bool stream_path(int64_t T, int64_t H, int64_t F, int64_t E, int64_t k) {
   if (H / 32 > kStreamMaxBlocks || F / 32 > kStreamMaxBlocks || T * k > kStreamMaxP) return false;
   const int g = stream_group_tokens(T, H, F);
+  if (T <= g) return true;  // no expert holds more than T tokens: one pass each
   const double m = std::min((double)(T * k) / (double)E, (double)T);
   if (T > 64 && m > g) return false;  // two passes and more, however small the matrices
   double again = 0.0;  // expected passes per expert beyond the first
-  if (m > 64.0) {
-    again = m / g - 1.0;
-  } else {
-    double p = std::exp(-m), above = 1.0 - p;  // P(n), P(more than n)
-    for (int n = 1; above > 1e-4; ++n) {
-      p *= m / n;
-      above -= p;
-      if (n % g == 0) again += std::max(above, 0.0);
-    }
+  double p = std::exp(-m), above = 1.0 - p;  // P(n), P(more than n); m is at most 64 here
+  for (int n = 1; above > 1e-4; ++n) {
+    p *= m / n;
+    above -= p;
+    if (n % g == 0) again += std::max(above, 0.0);
   }
   return again * (double)(E * 3 * H * F) * (17.0 / 32.0) <= 120e6;
 }

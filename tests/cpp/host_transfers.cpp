@@ -41,6 +41,7 @@ long executed = 0, queued = 0;               // of the library's stream
 int fail_launch_in = -1;                     // launches until one fails
 hipError_t last = hipSuccess;
 long launches = 0;
+std::vector<std::string> launched;           // names since the last clear()
 bool refuse_pinned = false;
 double stream_busy_until = 0.0;              // by the process's wall clock: the stream does nothing before
 unsigned char* packed_scales = nullptr;      // scale plane that the last pack kernel wrote
@@ -78,6 +79,7 @@ hipError_t launch(const void* f, void** args) {
   ++launches;
   if (fail_launch_in >= 0 && fail_launch_in-- == 0) return last = hipErrorLaunchFailure;
   const std::string& name = kernels()[f];
+  launched.push_back(name);
   auto is = [&](const char* s) { return name.find(s) != std::string::npos; };
   if (is("link_copy_kernel")) {
     auto src = *(const char**)args[0];
@@ -358,6 +360,43 @@ static int staging_memory_after_a_large_upload() {
   return 0;
 }
 
+// The kernels that a batch takes.  Where an expert cannot hold more tokens than one pass of the streaming
+// kernel contracts, no weight is streamed twice, however large the matrices.
+static int kernels_of_a_batch() {
+  struct Call {
+    int64_t E, k, H, F, T;
+    bool stream;
+  };
+  const Call calls[] = {
+      {8, 8, 4096, 8192, 1, true},    {16, 8, 6144, 8192, 1, true},  {8, 8, 4096, 6144, 4, true},
+      {1, 1, 8192, 8192, 4, true},    {8, 8, 4096, 6144, 5, false},  {8, 4, 4096, 6144, 8, false},
+      {4, 4, 2880, 1536, 33, true},   {4, 4, 2880, 1536, 37, false}, {32, 4, 2880, 2880, 16, true},
+      {128, 4, 2880, 2880, 64, true}, {32, 4, 2880, 2880, 64, false}, {8, 2, 8224, 64, 1, false},
+  };
+  for (const Call& c : calls) {
+    csk_layer* L;
+    OK(csk_layer_create(c.E, c.k, c.H, c.F, &L));
+    std::vector<float> gate(c.E * c.H), hidden(c.T * c.H), out(c.T * c.H);
+    OK(csk_layer_set_router(L, gate.data(), nullptr));
+    OK(csk_layer_fill_synthetic(L, 1, 0, 117, 5));
+    fake::launched.clear();
+    OK(csk_moe_forward(L, hidden.data(), c.T, out.data(), 0));
+    auto count = [](const char* s) {
+      int n = 0;
+      for (const std::string& name : fake::launched) n += name.find(s) != std::string::npos;
+      return n;
+    };
+    if (count("expert_stream_kernel") != (c.stream ? 2 : 0) || count("expert_gemm_mx_kernel") != (c.stream ? 0 : 2)) {
+      std::printf("E %ld k %ld H %ld F %ld T %ld: not the kernels expected\n", c.E, c.k, c.H, c.F, c.T);
+      return 1;
+    }
+    // a single token on the streaming kernels is routed by the first of them
+    if (c.T == 1) CHECK((count("route_") + count("dispatch_") == 0) == (c.stream && c.E > 1));
+    csk_layer_destroy(L);
+  }
+  return 0;
+}
+
 // Nothing orders the null stream against the library's: what is written there may land late.
 static int scales_of_an_uploaded_matrix() {
   std::vector<uint8_t> bytes(16 * 17, 1);
@@ -377,6 +416,7 @@ int main(int argc, char** argv) {
       {"no_pinned_memory", no_pinned_memory},
       {"threads_sleep_while_the_stream_works", threads_sleep_while_the_stream_works},
       {"staging_memory_after_a_large_upload", staging_memory_after_a_large_upload},
+      {"kernels_of_a_batch", kernels_of_a_batch},
       {"scales_of_an_uploaded_matrix", scales_of_an_uploaded_matrix},
   };
   if (argc != 2 || !checks.count(argv[1])) return 2;

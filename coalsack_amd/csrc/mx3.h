@@ -74,7 +74,8 @@ __device__ __forceinline__ void mx3_quantize_block(float (&r)[32], u32x4 (&out)[
     // operands alive past it keeps the registers apart.
     asm volatile("" : "+v"(q) : "v"(ev), "v"(od), "v"(sc));
     if (t + 1 < kMx3Terms) {
-      const f32x32 d = __builtin_amdgcn_cvt_scalef32_pk32_f32_fp6(q, sc);
+      f32x32 d = __builtin_amdgcn_cvt_scalef32_pk32_f32_fp6(q, sc);
+      asm volatile("" : "+v"(d) : "v"(q), "v"(sc));  // (this one, too, writes 32 registers over several passes)
 #pragma unroll
       for (int j = 0; j < 32; ++j) r[j] = r[j] - d[j];  // exact: d is r rounded to 4 bits
     }

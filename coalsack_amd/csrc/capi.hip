@@ -104,12 +104,13 @@ int dev_alloc(T** p, size_t count) {
 
 inline long cdiv(long a, long b) { return (a + b - 1) / b; }
 
-// n words of device memory, on the library's stream: that stream does not wait for the null
-// stream, on which hipMemset runs and from which it may return early.
-int fill_words(void* p, long n, uint32_t v) {
-  if (n == 0) return CSK_OK;
+// Device memory filled with a word (bytes: a multiple of 16), on the library's stream: that stream
+// does not wait for the null stream, on which hipMemset runs and from which it may return early.
+int fill_words(void* p, size_t bytes, uint32_t v) {
+  if (bytes == 0) return CSK_OK;
+  const long n = (long)(bytes / 16);
   fill_words_kernel<<<dim3((unsigned)std::min<long>(cdiv(n, 256), 8L * std::max(g_cus, 1))), 256, 0, g_stream>>>(
-      static_cast<uint32_t*>(p), n, v);
+      static_cast<u32x4*>(p), n, v);
   return check_launch("fill_words_kernel");
 }
 constexpr uint32_t kScalesOfOne = 0x7f7f7f7f;  // four E8M0 bytes
@@ -993,7 +994,7 @@ extern "C" int csk_init(int device) {
   if (!g_stream) HIP_TRY(hipStreamCreateWithFlags(&g_stream, hipStreamNonBlocking));
   if (!g_zero) {
     HIP_TRY(counted_malloc((void**)&g_zero, kZeroLen * sizeof(float)));
-    const int rc = fill_words(g_zero, (long)kZeroLen, 0u);
+    const int rc = fill_words(g_zero, kZeroLen * sizeof(float), 0u);
     if (rc != CSK_OK) return rc;
   }
   if (device >= kMaxDevices) return fail(CSK_ERR_HIP, "device index beyond the library's table");
@@ -1165,7 +1166,7 @@ extern "C" int csk_mxfp4_upload(const uint8_t* blocks, int64_t rows, int64_t K, 
   m->ntile = cdiv(rows, 16);
   int rc = dev_alloc(&m->q, (size_t)m->entries() + kWeightSlack / sizeof(uint4));
   if (rc == CSK_OK) rc = dev_alloc(&m->s, (size_t)m->scale_bytes() + kWeightSlack);
-  if (rc == CSK_OK) rc = fill_words(m->s, m->scale_bytes() / 4, kScalesOfOne);
+  if (rc == CSK_OK) rc = fill_words(m->s, (size_t)m->scale_bytes(), kScalesOfOne);
   csk_mxfp4* const ms[1] = {m};
   if (rc == CSK_OK) rc = queue_pack(&blocks, ms, 1);
   if (rc == CSK_OK) rc = finish_pack(1);
@@ -1227,7 +1228,7 @@ static int layer_create(int64_t E, int64_t k, int64_t H, int64_t F, bool f16, cs
   } else {
     if (rc == CSK_OK) rc = dev_alloc(&L->q_all, (size_t)E * L->ent_expert() + kWeightSlack / sizeof(uint4));
     if (rc == CSK_OK) rc = dev_alloc(&L->s_all, (size_t)E * L->sc_expert() + kWeightSlack);
-    if (rc == CSK_OK) rc = fill_words(L->s_all, E * L->sc_expert() / 4, kScalesOfOne);
+    if (rc == CSK_OK) rc = fill_words(L->s_all, (size_t)E * L->sc_expert(), kScalesOfOne);
   }
   if (rc == CSK_OK) rc = dev_alloc(&L->bias_all, (size_t)E * (2 * F + H));
   if (rc == CSK_OK) rc = dev_alloc(&L->ew_dev, (size_t)E);

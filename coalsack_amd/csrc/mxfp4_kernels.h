@@ -165,9 +165,9 @@ __global__ void fill_cells_kernel(unsigned long long* __restrict__ p, int n, uns
   if ((int)threadIdx.x < n) p[threadIdx.x] = v;
 }
 
-__global__ __launch_bounds__(256) void fill_words_kernel(uint32_t* __restrict__ p, long n, uint32_t v) {
+__global__ __launch_bounds__(256) void fill_words_kernel(u32x4* __restrict__ p, long n, uint32_t v) {  // n x 4 words
   const long stride = (long)gridDim.x * 256;
-  for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < n; i += stride) p[i] = v;
+  for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < n; i += stride) p[i] = u32x4{v, v, v, v};
 }
 
 // Synthetic weights, generated straight into the packed layout.  Block b =

@@ -98,7 +98,7 @@ hipError_t launch(const void* f, void** args) {
     auto n = *(long*)args[1];
     auto v = *(uint32_t*)args[2];
     put([=] {
-      for (long i = 0; i < n; ++i) p[i] = v;
+      for (long i = 0; i < 4 * n; ++i) p[i] = v;
     });
   } else if (is("pack_mxfp4_kernel")) {
     auto s = *(unsigned char**)args[2];

@@ -45,6 +45,7 @@ std::vector<std::string> launched;           // names since the last clear()
 bool refuse_pinned = false;
 double stream_busy_until = 0.0;              // by the process's wall clock: the stream does nothing before
 unsigned char* packed_scales = nullptr;      // scale plane that the last pack kernel wrote
+std::map<const void*, std::vector<char>> packed;  // by plane: the blocks that were staged when its pack kernel ran
 dim3 grid, block;
 size_t shmem;
 hipStream_t st;
@@ -101,9 +102,19 @@ hipError_t launch(const void* f, void** args) {
       for (long i = 0; i < 4 * n; ++i) p[i] = v;
     });
   } else if (is("pack_mxfp4_kernel")) {
+    auto src = *(const char**)args[0];
+    auto q = *(const void**)args[1];
     auto s = *(unsigned char**)args[2];
+    const size_t n = (size_t)*(int*)args[3] * *(int*)args[4] * 17;
     packed_scales = s;
-    put([=] { std::memset(s, 0x55, 256); });
+    put([=] {
+      packed[q].assign(src, src + n);
+      std::memset(s, 0x55, 256);
+    });
+  } else if (is("export_mxfp4_kernel")) {
+    auto q = *(const void**)args[0];
+    auto dst = *(char**)args[2];
+    put([=] { std::memcpy(dst, packed[q].data(), packed[q].size()); });
   } else if (is("10add_kernel")) {
     auto a = *(const float**)args[0];
     auto b = *(const float**)args[1];
@@ -372,6 +383,10 @@ static int kernels_of_a_batch() {
       {1, 1, 8192, 8192, 4, true},    {8, 8, 4096, 6144, 5, false},  {8, 4, 4096, 6144, 8, false},
       {4, 4, 2880, 1536, 33, true},   {4, 4, 2880, 1536, 37, false}, {32, 4, 2880, 2880, 16, true},
       {128, 4, 2880, 2880, 64, true}, {32, 4, 2880, 2880, 64, false}, {8, 2, 8224, 64, 1, false},
+      // (what the GPU tests of these shapes say they run)
+      {4, 2, 8224, 64, 3, false},     {4, 2, 64, 8224, 64, false},    {4, 2, 3200, 64, 6, true},
+      {32, 4, 2880, 2880, 32, true},  {32, 4, 2880, 2880, 48, true},  {128, 4, 2880, 2880, 128, true},
+      {128, 4, 2880, 2880, 160, false},
   };
   for (const Call& c : calls) {
     csk_layer* L;
@@ -397,6 +412,33 @@ static int kernels_of_a_batch() {
   return 0;
 }
 
+// The pinned ring (16 MiB, quarters of 4, pieces of 64 KiB) entered at many offsets and gone round
+// several times within a call, on a stream that reads and writes it as late as it may.
+static int ring_entered_anywhere() {
+  uint32_t x = 1;
+  auto random = [&x] { return (x = x * 1664525u + 1013904223u) >> 8; };
+  for (int round = 0; round < 6; ++round) {
+    const int64_t H = 32 * (8 + random() % 120), F = 32 * (8 + random() % 200);
+    csk_layer* L;
+    OK(csk_layer_create(1, 1, H, F, &L));
+    std::vector<uint8_t> w[3];
+    for (auto& m : w) {
+      m.resize(H * F / 32 * 17);
+      for (auto& b : m) b = (uint8_t)random();
+    }
+    fake::packed.clear();
+    OK(csk_layer_set_expert(L, 0, w[0].data(), w[1].data(), w[2].data(), nullptr, nullptr, nullptr));
+    const int which[3] = {CSK_W_UP, CSK_W_GATE, CSK_W_DOWN};
+    for (int i = 0; i < 3; ++i) {
+      std::vector<uint8_t> back(w[i].size());
+      OK(csk_layer_export(L, 0, which[i], back.data()));
+      CHECK(back == w[i]);
+    }
+    csk_layer_destroy(L);
+  }
+  return 0;
+}
+
 // Nothing orders the null stream against the library's: what is written there may land late.
 static int scales_of_an_uploaded_matrix() {
   std::vector<uint8_t> bytes(16 * 17, 1);
@@ -417,6 +459,7 @@ int main(int argc, char** argv) {
       {"threads_sleep_while_the_stream_works", threads_sleep_while_the_stream_works},
       {"staging_memory_after_a_large_upload", staging_memory_after_a_large_upload},
       {"kernels_of_a_batch", kernels_of_a_batch},
+      {"ring_entered_anywhere", ring_entered_anywhere},
       {"scales_of_an_uploaded_matrix", scales_of_an_uploaded_matrix},
   };
   if (argc != 2 || !checks.count(argv[1])) return 2;

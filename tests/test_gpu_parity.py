@@ -32,8 +32,9 @@ def test_dequant_bit_exact_and_roundtrip(lib, oracle):
 
 def test_transfers_around_the_pinned_ring(lib):
     """Uploads and results from a few bytes to several times the pinned ring between host and
-    device (16 MiB, quarters of 4, pieces of 64 KiB), odd lengths among them, one behind the
-    other so that the ring is entered at every offset: nothing is lost or moved."""
+    device (16 MiB, quarters of 4, pieces of 64 KiB), odd lengths among them: nothing is lost or
+    moved.  Each of these calls finds the ring empty; an expert's three matrices go up in one
+    call, the second and the third from where the one before has ended, around the ring's end."""
     rng = np.random.default_rng(5)
     for rows, K in ((3, 32), (17, 4096), (1000, 2080), (2880, 2880), (33, 65504), (9001, 8192), (1, 64), (16384, 6144)):
         b = rng.integers(0, 256, (rows * (K // 32), 17), dtype=np.uint8)
@@ -46,6 +47,14 @@ def test_transfers_around_the_pinned_ring(lib):
         h = lib.f16_upload(w)
         assert np.array_equal(lib.f16_export(h, rows, K - 3).view(np.uint16), w.view(np.uint16)), (rows, K)
         lib.f16_free(h)
+    for H, F in ((4096, 8192), (2880, 4000 // 32 * 32), (1056, 2080)):
+        b = rng.integers(0, 256, (3, H * F // 32, 17), dtype=np.uint8)
+        b[..., 0] = 100 + b[..., 0] % 50
+        b = b.reshape(3, -1)
+        with lib.layer(1, 1, H, F) as layer:
+            layer.set_expert(0, b[0], b[1], b[2], None, None, None)
+            for i, which in enumerate((capi.W_UP, capi.W_GATE, capi.W_DOWN)):
+                assert np.array_equal(layer.export(0, which), b[i]), (H, F, i)
 
 
 def test_dequant_every_scale_and_code(lib, oracle):
@@ -564,7 +573,8 @@ def test_layer_variants_grouped_gemm(lib, oracle, opts):
 
 
 def test_layer_few_tokens_long_rows(lib, oracle):
-    """Rows longer than the streaming kernel's LDS budget: few tokens still take the GEMM."""
+    """A handful of tokens on rows past 3072 (one group of the streaming kernels, with one workgroup
+    per compute unit) and past 4096."""
     L = synth.LayerInputs(4, 2, 3200, 64, seed=23, with_norm=True)
     _check_layer(lib, oracle, L, 6, norm=True, residual=True)
     L = synth.LayerInputs(4, 2, 64, 3200, seed=24)
@@ -575,12 +585,26 @@ def test_layer_few_tokens_long_rows(lib, oracle):
     _check_layer(lib, oracle, L, 7)
 
 
+@pytest.mark.parametrize("opts", [dict(), dict(weight_before_ffn=True), dict(norm=True, residual=True)])
+@pytest.mark.parametrize("H,F", [(8224, 64), (64, 8224)])
+def test_layer_few_tokens_on_the_grouped_gemm(lib, oracle, H, F, opts):
+    """Rows one block longer than the streaming kernels take (8192): batches of one to 64 tokens on the
+    grouped GEMM, whose M tiles are listed by the single-workgroup routing kernel up to 32 tokens and by
+    the dispatch kernel beyond, and whose FP6 rows come from the routing prologue -- or, with the weight
+    in front of the FFN, from the gathered and scaled rows."""
+    opts = dict(opts)
+    norm, residual = opts.pop("norm", False), opts.pop("residual", False)
+    L = synth.LayerInputs(4, 2, H, F, seed=H + 5, with_norm=True)
+    for T in (1, 3, 7, 32, 33, 64):
+        _check_layer(lib, oracle, L, T, norm=norm, residual=residual, **opts)
+
+
 @pytest.mark.parametrize("H,F", [(3072, 3072), (32, 3072), (3072, 32), (32, 32), (3040, 2976)])
 @pytest.mark.parametrize("T", [3, 23])
 def test_layer_streaming_row_length_limits(lib, oracle, H, F, T):
-    """The streaming kernels at the ends of the row lengths they accept: 3072 (every block
-    of the activation rows in LDS holds data, none is a zero tail), one block of 32, and
-    lengths whose last 128-wide step is partly past the row."""
+    """The streaming kernels' form for 3072-long rows at its end (every block of the activation rows
+    in LDS holds data, none is a zero tail), rows of one block of 32, and lengths whose last
+    128-wide step is partly past the row."""
     L = synth.LayerInputs(5, 2, H, F, seed=11 + H // 32 + F // 64, with_norm=True)
     _check_layer(lib, oracle, L, T, norm=True, residual=True)
 
@@ -600,10 +624,11 @@ def test_layer_streaming_step_counts(lib, oracle, D, long_rows):
 @pytest.mark.parametrize("H,F", [(96, 1056), (1056, 96), (1024, 1024)])
 def test_layer_grouped_gemm_wide_and_narrow_tiles(lib, oracle, H, F):
     """Both heights of the grouped GEMM's tile -- 512 weight rows where there are many work
-    units of many tokens, 256 otherwise -- over feature counts that end inside a tile (66
-    tiles of 16) and on its edge."""
+    units of many tokens (520 tokens: 129 M tiles of four or five N tiles each, for more than two units
+    per compute unit), 256 otherwise -- over feature counts that end inside a tile (66 tiles of 16)
+    and on its edge."""
     L = synth.LayerInputs(64, 8, H, F, seed=H)
-    _check_layer(lib, oracle, L, 512, oracle_tokens=64)
+    _check_layer(lib, oracle, L, 520, oracle_tokens=64)
     _check_layer(lib, oracle, L, 250, oracle_tokens=40)
 
 
@@ -635,9 +660,10 @@ def test_layer_120b_shape_skewed_16_tokens(lib, oracle):
     _check_layer(lib, oracle, L, 16, device_weights=True)
 
 
-@pytest.mark.parametrize("T", [32, 64])
+@pytest.mark.parametrize("T", [32, 48, 64])
 def test_layer_20b_shape_wide_token_groups(lib, oracle, T):
-    """BASELINE config 2 above 16 tokens: the wide-group streaming kernels at K = 2880."""
+    """32 experts of 2880 x 2880 above 16 tokens: 32 and 48 tokens stream in groups of seven, 64 (eight
+    assignments per expert) take the grouped GEMM with tiles of 256 weight rows."""
     L = synth.LayerInputs(32, 4, 2880, 2880, seed=52)
     _check_layer(lib, oracle, L, T, device_weights=True, subset=True)
 
@@ -649,10 +675,11 @@ def test_layer_120b_shape_skewed_1_and_64_tokens(lib, oracle, T):
     _check_layer(lib, oracle, L, T, device_weights=True, subset=True)
 
 
-@pytest.mark.parametrize("T", [160, 320])
+@pytest.mark.parametrize("T", [96, 128, 160, 320])
 def test_layer_120b_shape_many_experts_few_tokens_each(lib, oracle, T):
-    """More than 64 tokens, but at most ten assignments per expert on average: such a batch
-    still takes the streaming kernels (groups of seven tokens; the hot experts take many)."""
+    """More than 64 tokens, but at most ten assignments per expert on average: up to four such a batch
+    still streams (96 and 128 tokens, groups of seven; the hot experts take many), with more
+    it takes the grouped GEMM (160 and 320 tokens, most M tiles nearly empty)."""
     L = synth.LayerInputs(128, 4, 2880, 2880, seed=44, hot_experts=8)
     _check_layer(lib, oracle, L, T, device_weights=True, subset=True)
 

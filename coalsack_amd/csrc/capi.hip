@@ -118,7 +118,7 @@ constexpr uint32_t kScalesOfOne = 0x7f7f7f7f;  // four E8M0 bytes
 // Above this many token-expert assignments the token-group list of the
 // weight-streaming kernel is not built.
 constexpr int64_t kStreamMaxP = 2048;
-constexpr size_t kWeightSlack = 32768;  // bytes of mapped memory kept behind weight planes (the streaming kernel walks 96 blocks per tile whatever K is)
+constexpr size_t kWeightSlack = 32768;  // bytes of mapped memory kept behind weight planes (the expert kernels read whole K steps: up to three blocks, 768 bytes, past the last tile)
 constexpr int kStreamWgPerCu = 2;  // resident workgroups of the streaming kernel per compute unit ...
 constexpr size_t kStreamLdsHalf = 80 * 1024 - 512;  // ... if each takes no more LDS than this (and its few static words)
 
@@ -126,8 +126,8 @@ constexpr size_t kStreamLdsHalf = 80 * 1024 - 512;  // ... if each takes no more
 struct Workspace {
   int64_t T = 0, E = 0, k = 0, H = 0, F = 0;
   float* xn = nullptr;      // [T,H] normalised activations
-  uint16_t* xs = nullptr;   // [T][H/32][64] bf16 hi|lo
-  uint16_t* xg = nullptr;   // [P][H/32][64] gathered + pre-scaled (weight_before_ffn)
+  uint16_t* xs = nullptr;   // [T] rows of H as three FP6 terms (mx3.h) or two fp16 terms
+  uint16_t* xg = nullptr;   // [P] the same, gathered + pre-scaled (weight_before_ffn)
   float* logits = nullptr;  // [T,E]
   float* pairs = nullptr;   // [T,k,2]
   int* ids = nullptr;       // [P]
@@ -139,7 +139,7 @@ struct Workspace {
   int* list_tok = nullptr;  // [P]
   float* list_w = nullptr;  // [P]
   int* pos = nullptr;       // [P]
-  uint16_t* act = nullptr;  // [P][F/32][64] bf16 hi|lo
+  uint16_t* act = nullptr;  // [P] rows of F: fp32 (streaming kernels), three FP6 terms or two fp16 terms
   float* y = nullptr;       // [P,H]
   int* tiles = nullptr;     // prefill tile schedule
   int* n_tiles = nullptr;
@@ -168,12 +168,12 @@ struct Workspace {
 #define WS_ALLOC(ptr, cnt) \
   if ((rc = dev_alloc(&ptr, (cnt))) != CSK_OK) return rc
     WS_ALLOC(xn, (size_t)nT * nH);
-    // activation rows: two bf16 terms (128 B per block) or three FP6 terms padded to whole
-    // K steps (96 B per block), whichever is larger; counts are in uint16
+    // activation rows: fp32 or two fp16 terms (128 B per block of 32), or three FP6 terms padded to
+    // whole K steps (96 B per block), whichever is larger; counts are in uint16
     auto act_elems = [](size_t rows, int64_t dim) {
-      const size_t bf = rows * (size_t)dim * 2;
+      const size_t wide = rows * (size_t)dim * 2;
       const size_t mx = rows * (size_t)mx3_row_blocks((int)(dim / 32)) * 48;
-      return std::max(bf, mx);
+      return std::max(wide, mx);
     };
     WS_ALLOC(xs, act_elems((size_t)nT, nH));
     if (need_xg || had_xg) WS_ALLOC(xg, act_elems(P, nH));
@@ -209,7 +209,7 @@ constexpr int64_t kFixedMaxT = 64;      // tokens per call
 constexpr int64_t kFixedMaxP = 512;     // token-expert assignments per call (T * top_k)
 constexpr int64_t kFixedMaxDim = 3072;  // hidden_dim and expert_ffn_dim
 constexpr size_t fixed_align(size_t n) { return (n + 255) & ~(size_t)255; }
-constexpr size_t kFixedRowBytes = (size_t)kFixedMaxDim * 4;  // a row as f32, or as two bf16 terms
+constexpr size_t kFixedRowBytes = (size_t)kFixedMaxDim * 4;  // a row as f32; three FP6 terms take less (3072 is a whole number of K steps)
 constexpr size_t kFixedScratchBytes =
     fixed_align(kFixedMaxT * kFixedRowBytes) * 2 +                                     // xn, xs
     fixed_align(kFixedMaxP * kFixedRowBytes) * 3 +                                     // xg, act, y
@@ -737,6 +737,10 @@ int launch_stream(ExpertStreamArgs a, int64_t P, Workspace& ws) {
 // which the tall tile is for, does not matter while the weights are what is waited for.
 // Measured (layer, us, 512 / 256 rows): 32 experts of 2880 x 2880 m = 8 135 / 125, 16 141 / 131, 32
 // 157 / 155, 64 222 / 221, 256 440 / 478; 8 experts m = 4 80 / 66; 128 experts m = 8 412 / 409, 32 488 / 505.
+// Units are counted as those of the gate/up projection for both.  The down projection has half as many, so its
+// tall tiles begin at just over one unit per compute unit; counted by its own units they would begin at two, and
+// that is the worse line (layer, us, this / that): 32 experts of 2880 x 2880, top-4, 200 tokens 156 / 164, 300
+// 169 / 173, 450 163 / 170, 600 223 / 221; 8 of them, top-2, 600 tokens 110 / 107; 64 of 2048 x 768, 300 97.5 / 94.6.
 bool gemm_wide_tiles(int64_t E, int64_t P, int64_t ntile) {
   const int64_t mtiles = P / kGemmBM + std::min<int64_t>(E, P);
   return P > 16 * E && mtiles * cdiv(ntile, 4 * kMxNG) > 2 * std::max(g_cus, 1);

@@ -210,19 +210,21 @@ class CopyCrew {
 // chunk takes 20 us -- and leaves longer waits, for the work in front of the transfer, to the runtime.
 class DeviceWait {
  public:
-  void progress() { since_ = std::chrono::steady_clock::now(); }
+  void progress() { polling_ = false; }
   hipError_t once(hipEvent_t e) {
-    if (std::chrono::steady_clock::now() - since_ < std::chrono::microseconds(200)) {
+    const auto now = std::chrono::steady_clock::now();
+    if (!polling_) since_ = now, polling_ = true;
+    if (now - since_ < std::chrono::microseconds(200)) {
       CopyCrew::relax();
       return hipSuccess;
     }
-    const hipError_t rc = hipEventSynchronize(e);
-    progress();
-    return rc;
+    polling_ = false;
+    return hipEventSynchronize(e);
   }
 
  private:
-  std::chrono::steady_clock::time_point since_ = std::chrono::steady_clock::now();
+  bool polling_ = false;
+  std::chrono::steady_clock::time_point since_;
 };
 
 // The crew of this process.  A forked child has the object but not its threads: joining them, or

@@ -1767,14 +1767,15 @@ extern "C" int csk_layer_set_expert_f16(csk_layer* L, int64_t e, const uint16_t*
     return fail(CSK_ERR_ARG, "weights must be all present or all absent");
   CSK_TRY(check_biases(b_up, b_gate, b_down));
   if (w_up) {
+    L->matrix_set[(size_t)e] = L->expert_set[(size_t)e] = 0;  // until all of it has arrived
     CSK_TRY(queue_f16_pack(w_up, kGgmlF16Type, L->F, L->H, L->view16(e, CSK_W_UP)));
     CSK_TRY(queue_f16_pack(w_gate, kGgmlF16Type, L->F, L->H, L->view16(e, CSK_W_GATE)));
     CSK_TRY(queue_f16_pack(w_down, kGgmlF16Type, L->H, L->F, L->view16(e, CSK_W_DOWN)));
-    L->matrix_set[(size_t)e] = 7;
-    L->expert_set[(size_t)e] = 1;
   }
   CSK_TRY(upload_biases(L, e, b_up, b_gate, b_down));
-  return finish_fetches();
+  CSK_TRY(finish_fetches());
+  if (w_up) L->matrix_set[(size_t)e] = 7, L->expert_set[(size_t)e] = 1;
+  return CSK_OK;
 }
 extern "C" int csk_layer_set_expert_matrix(csk_layer* L, int64_t e, int which, int ggml_type,
                                            const void* data) {
@@ -1784,6 +1785,7 @@ extern "C" int csk_layer_set_expert_matrix(csk_layer* L, int64_t e, int which, i
   if (!L->f16) return fail(CSK_ERR_STATE, "csk_layer_set_expert_matrix: this layer holds MXFP4 experts (csk_layer_create_f16 makes an fp16 one)");
   const bool down = which == CSK_W_DOWN;
   int rc = f16_pack_into(data, ggml_type, down ? L->H : L->F, down ? L->F : L->H, L->view16(e, which));
+  if (rc == CSK_ERR_HIP) L->matrix_set[(size_t)e] &= (char)~(1 << which), L->expert_set[(size_t)e] = 0;  // it may hold a part
   if (rc != CSK_OK) return rc;
   L->matrix_set[(size_t)e] |= (char)(1 << which);
   if (L->matrix_set[(size_t)e] == 7) L->expert_set[(size_t)e] = 1;

@@ -43,6 +43,7 @@ hipError_t last = hipSuccess;
 long launches = 0;
 std::vector<std::string> launched;           // names since the last clear()
 bool refuse_pinned = false;
+bool fail_wait = false;                      // waiting for the stream reports an error
 double stream_busy_until = 0.0;              // by the process's wall clock: the stream does nothing before
 unsigned char* packed_scales = nullptr;      // scale plane that the last pack kernel wrote
 std::map<const void*, std::vector<char>> packed;  // by plane: the blocks that were staged when its pack kernel ran
@@ -188,7 +189,7 @@ hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) {
 hipError_t hipStreamSynchronize(hipStream_t) {
   std::lock_guard<std::recursive_mutex> g(fake::m);
   fake::run_all();
-  return hipSuccess;
+  return fake::fail_wait ? hipErrorLaunchFailure : hipSuccess;
 }
 hipError_t hipMalloc(void** p, size_t n) {
   std::lock_guard<std::recursive_mutex> g(fake::m);
@@ -439,6 +440,38 @@ static int ring_entered_anywhere() {
   return 0;
 }
 
+// An expert whose matrices did not arrive is not there, whichever format they have.
+static int expert_that_did_not_arrive() {
+  const int64_t H = 64, F = 64;
+  std::vector<uint16_t> halves(H * F);
+  std::vector<uint8_t> blocks(H * F / 32 * 17, 1);
+  std::vector<float> gate(H), x(H), y(H);
+  for (int f16 = 0; f16 < 3; ++f16) {
+    csk_layer* L;
+    OK(f16 ? csk_layer_create_f16(1, 1, H, F, &L) : csk_layer_create(1, 1, H, F, &L));
+    OK(csk_layer_set_router(L, gate.data(), nullptr));
+    auto set = [&] {
+      if (f16 == 2) {  // matrix by matrix
+        for (int which = 0; which < 3; ++which)
+          if (const int rc = csk_layer_set_expert_matrix(L, 0, which, 1, halves.data()); rc != CSK_OK) return rc;
+        return CSK_OK;
+      }
+      return f16 ? csk_layer_set_expert_f16(L, 0, halves.data(), halves.data(), halves.data(), nullptr, nullptr, nullptr)
+                 : csk_layer_set_expert(L, 0, blocks.data(), blocks.data(), blocks.data(), nullptr, nullptr, nullptr);
+    };
+    for (int first = 1; first >= 0; --first) {  // an expert that had none, and one that loses its old ones
+      fake::fail_wait = true;
+      CHECK(set() == CSK_ERR_HIP);
+      fake::fail_wait = false;
+      CHECK(csk_moe_forward(L, x.data(), 1, y.data(), 0) == CSK_ERR_STATE);
+      OK(set());
+      OK(csk_moe_forward(L, x.data(), 1, y.data(), 0));
+    }
+    csk_layer_destroy(L);
+  }
+  return 0;
+}
+
 // Nothing orders the null stream against the library's: what is written there may land late.
 static int scales_of_an_uploaded_matrix() {
   std::vector<uint8_t> bytes(16 * 17, 1);
@@ -460,6 +493,7 @@ int main(int argc, char** argv) {
       {"staging_memory_after_a_large_upload", staging_memory_after_a_large_upload},
       {"kernels_of_a_batch", kernels_of_a_batch},
       {"ring_entered_anywhere", ring_entered_anywhere},
+      {"expert_that_did_not_arrive", expert_that_did_not_arrive},
       {"scales_of_an_uploaded_matrix", scales_of_an_uploaded_matrix},
   };
   if (argc != 2 || !checks.count(argv[1])) return 2;

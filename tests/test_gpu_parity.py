@@ -57,6 +57,33 @@ def test_transfers_around_the_pinned_ring(lib):
                 assert np.array_equal(layer.export(0, which), b[i]), (H, F, i)
 
 
+def test_transfers_behind_a_busy_stream(lib):
+    """Transfers that wait for milliseconds of queued forwards: an upload larger than the pinned ring
+    (which fills it and has to wait for its first quarter) and a result that comes late."""
+    rng = np.random.default_rng(6)
+    b = rng.integers(0, 256, (8192 * 200, 17), dtype=np.uint8)  # 27.9 MB
+    b[:, 0] = 100 + b[:, 0] % 50
+    b = b.reshape(-1)
+    L = synth.LayerInputs(32, 4, 2880, 2880, seed=3)
+    x = synth.hidden_states(2048, 2880, seed=4)
+    with build_layer(lib, L, device_weights=True) as layer:
+        d_in, d_out = lib.to_device(x), lib.dev_alloc(x.nbytes)
+        want = layer.forward(x)
+        try:
+            for _ in range(2):
+                for _ in range(8):
+                    layer.forward_device(d_in, 2048, d_out)
+                h = lib.mxfp4_upload(b, 8192, 6400)
+                assert np.array_equal(lib.mxfp4_export(h, 8192, 6400), b)
+                lib.mxfp4_free(h)
+                for _ in range(8):
+                    layer.forward_device(d_in, 2048, d_out)
+                assert np.array_equal(layer.forward(x).view(np.uint32), want.view(np.uint32))
+        finally:
+            lib.dev_free(d_in)
+            lib.dev_free(d_out)
+
+
 def test_dequant_every_scale_and_code(lib, oracle):
     """Every scale byte the reference decodes to finite values, 0 and 1 (fp32 denormals)
     included, with all 16 codes in both nibble positions: bit-exact against the fixture

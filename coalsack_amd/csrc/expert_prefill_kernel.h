@@ -500,14 +500,21 @@ __device__ __forceinline__ void expert_gemm_mx_unit(const ExpertGemmMxArgs& a, c
 // and each die has its own L2: die x takes the x-th contiguous eighth of the unit sequence,
 // so that the workgroups resident on one die at one time share a few activation panels and
 // a few experts' weights, which then come from that L2 instead of from memory.
+// From three units per place on the chip on, a die takes two sixteenths, the x-th and the x-th from the end: an eighth in
+// one piece gives some dies more of the experts with many tokens than others, and the last die ended 10 % after the
+// first (layer, us, one part / two: 128 experts of 2880 x 2880, 4096 tokens 967 / 950, 1000 tokens 511 / 501; 16 of
+// 4096 x 6144, 2000 tokens 615 / 600).  With fewer units a part's ends, whose experts two dies share, weigh more (the same
+// 16 experts, 1000 tokens 366 / 374; units of 256 rows: 128 experts, 300 tokens 404 / 410).
+constexpr int kTwoPartUnits = 1536;
 template <int MODE, int NG>
 __global__ __launch_bounds__(64 * kMxWaves, NG == 2 ? 3 : 2) void expert_gemm_mx_kernel(ExpertGemmMxArgs a) {
   extern __shared__ __align__(16) unsigned char smem[];
   const int n_units = *a.n_mtiles * a.n_ntiles;
-  const int per_die = (n_units + kDies - 1) / kDies;
-  const int slot = blockIdx.x / kDies;
-  const int unit = (blockIdx.x % kDies) * per_die + slot;
-  if (slot >= per_die || unit >= n_units) return;
+  const int die = blockIdx.x % kDies, slot = blockIdx.x / kDies;
+  const bool two_parts = NG == kMxNG && n_units >= kTwoPartUnits;
+  const int part = two_parts ? (n_units + 2 * kDies - 1) / (2 * kDies) : (n_units + kDies - 1) / kDies;
+  const int unit = slot < part ? die * part + slot : (2 * kDies - 2 - die) * part + slot;  // (the part 2 kDies - 1 - die)
+  if (slot >= (two_parts ? 2 : 1) * part || unit >= n_units) return;
   const int mt = unit / a.n_ntiles;
   int nt = unit - mt * a.n_ntiles;
   const WorkDesc* wd = a.desc + a.mtiles[2 * mt];

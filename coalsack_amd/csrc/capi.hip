@@ -1850,14 +1850,13 @@ int forward_pass(csk_layer* L, const float* hidden, int64_t T, float* out, int f
     u32x4* rows_mx3 = (!L->f16 && !L->wbf) ? reinterpret_cast<u32x4*>(ws.xs) : nullptr;
     rows_mx3_ready = rows_mx3 != nullptr;
     // a workgroup takes one expert (latency) as long as all of them are resident at once, four beyond
-    if (cdiv(T, 4) * (L->E + 4) <= 4 * std::max(g_cus, 1) + 64)  // four of these workgroups fit a compute unit
-      router_prep_logits_kernel<1><<<dim3((unsigned)(L->E + 4), (unsigned)cdiv(T, 4)), 256, 0, g_stream>>>(
-          hidden, norm ? L->norm_w : nullptr, L->eps, ws.xn, L->gate_w,
-          L->has_gate_b ? L->gate_b : nullptr, ws.logits, (int)T, (int)L->E, (int)L->H, rows_mx3);
-    else
-      router_prep_logits_kernel<4><<<dim3((unsigned)(cdiv(L->E, 4) + 4), (unsigned)cdiv(T, 4)), 256, 0, g_stream>>>(
-          hidden, norm ? L->norm_w : nullptr, L->eps, ws.xn, L->gate_w,
-          L->has_gate_b ? L->gate_b : nullptr, ws.logits, (int)T, (int)L->E, (int)L->H, rows_mx3);
+    const bool one = cdiv(T, 4) * (L->E + 4) <= 4 * std::max(g_cus, 1) + 64;  // four of these workgroups fit a compute unit
+    const bool held = L->H <= 4096 || L->H > 8192;
+    const auto kernel = one ? (held ? router_prep_logits_kernel<1, 4> : router_prep_logits_kernel<1, 8>)
+                            : (held ? router_prep_logits_kernel<4, 4> : router_prep_logits_kernel<4, 8>);
+    kernel<<<dim3((unsigned)(cdiv(L->E, one ? 1 : 4) + 4), (unsigned)cdiv(T, 4)), 256, 0, g_stream>>>(
+        hidden, norm ? L->norm_w : nullptr, L->eps, ws.xn, L->gate_w,
+        L->has_gate_b ? L->gate_b : nullptr, ws.logits, (int)T, (int)L->E, (int)L->H, rows_mx3);
     if ((rc = check_launch("router_prep_logits_kernel")) != CSK_OK) return rc;
     mark(CSK_STAGE_DISPATCH);
     RouteIn rin{ws.logits, xr, L->gate_w, L->has_gate_b ? L->gate_b : nullptr, L->ew_dev,

@@ -158,8 +158,12 @@ __global__ __launch_bounds__(256) void router_logits_mfma_kernel(const float* __
 // over as many workgroups as there are experts (latency); EPW = 4 is for batches whose
 // one-expert workgroups would not all be resident at once (64 tokens, 128 experts: 2112 of
 // them, 18.6 us; a quarter as many read the token rows a quarter as often).
+// IT float4 per thread hold a row of up to 1024 IT values: rows up to 4096 take 4, up to 8192 8, and only longer ones
+// are read again in every pass (8 tokens of 5120 on 16 experts: read again 11.1 us, held 5.4; 16 of 4128 38.5 -> 35 us for a layer of 16
+// experts of 512, 64 of 8192 on 128 experts 170 -> 151; the registers leave two workgroups per compute unit instead of four, and
+// 60 tokens of 6144 on 64 experts are no faster).
 // Restates moe_router_node.h:161-167 and rmsnorm_node.h:62-83.
-template <int EPW>
+template <int EPW, int IT>
 __global__ __launch_bounds__(256) void router_prep_logits_kernel(
     const float* __restrict__ hidden, const float* __restrict__ norm_w, float eps,
     float* __restrict__ xn, const float* __restrict__ g,
@@ -173,11 +177,11 @@ __global__ __launch_bounds__(256) void router_prep_logits_kernel(
     const int t = (blockIdx.x - n_ewg) + 4 * blockIdx.y;
     if (blockIdx.x - n_ewg >= 4 || t >= T || (!norm_w && !x3)) return;  // without a norm the rows are used as they are
     // four columns per thread, the row's loads all in flight at once and kept in registers
-    // between the two passes (rows longer than 4096 take further rounds of the same)
+    // between the two passes (longer rows take further rounds of the same)
     const float4* x4 = reinterpret_cast<const float4*>(hidden + (size_t)t * H);
     const float4* nw4 = reinterpret_cast<const float4*>(norm_w);
     const int H4p = H >> 2;
-    constexpr int kIter = 4;
+    constexpr int kIter = IT;
     const bool one_round = H4p <= 256 * kIter;  // the row and the norm weights are then read once, up front
     float4 x0[kIter], w0[kIter];
     if (one_round) {
@@ -275,7 +279,7 @@ __global__ __launch_bounds__(256) void router_prep_logits_kernel(
   const int t0 = blockIdx.y * 4;
   const int nt = min(4, T - t0);  // tokens of this tile (the same in every thread)
   // this thread's part of the token rows stays in registers between the passes
-  constexpr int kMaxIter = 4;     // 256 threads x 4 float4 x 4 = H up to 4096; longer rows are read again
+  constexpr int kMaxIter = IT;
   float4 xr[4][kMaxIter];
   const bool held = H4 <= 256 * kMaxIter;
   if (held) {

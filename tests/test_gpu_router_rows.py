@@ -1,0 +1,25 @@
+"""Routing of small batches holds rows of up to 4096, and of up to 8192, values in registers and reads longer ones
+again: the rows at both lines, with and without RMSNorm, one expert and four per workgroup."""
+import numpy as np
+import pytest
+
+from coalsack_amd import capi, synth
+from tests.helpers import assert_layer_close, build_layer, classify_index_mismatches, oracle_layer
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("H", [4096, 4128, 8160, 8192, 8224])
+@pytest.mark.parametrize("E,k,T,norm", [(4, 2, 1, True), (5, 2, 6, False), (130, 2, 33, True)])
+def test_rows_at_the_lines(lib, oracle, H, E, k, T, norm):
+    L = synth.LayerInputs(E, k, H, 32, seed=3, with_norm=norm)
+    hidden = synth.hidden_states(T, H, seed=H + T)
+    with build_layer(lib, L, norm=norm) as layer:
+        got, pairs = layer.forward(hidden, capi.FWD_RMSNORM if norm else 0, want_pairs=True)
+    want, wpairs = oracle_layer(oracle, L, hidden, norm=norm)
+    x = oracle.rmsnorm(hidden, L.norm_w, 1e-5) if norm else hidden
+    real, near = classify_index_mismatches(oracle, x, L, pairs, wpairs)
+    assert real == 0, (real, near)
+    same = np.all(pairs[..., 0] == wpairs[..., 0], axis=1)
+    assert np.max(np.abs(pairs[same] - wpairs[same])) < 1.7e-5  # 1e-5 at 2880 values, growing with sqrt(H)
+    assert_layer_close(got[same], want[same])

@@ -669,7 +669,8 @@ int launch_router(const float* x, const float* gate_w, const float* gate_b, int6
     rider = Mx3Rider{x, reinterpret_cast<u32x4*>(mx3_out), (long)T, (int)(H / 32), (int)cdiv(T, 4)};
     riders = cdiv(T * mx3_row_blocks((int)(H / 32)), 256);
   }
-  router_topk_kernel<<<dim3((unsigned)(cdiv(T, 4) + riders)), 256, 0, g_stream>>>(
+  const auto topk = nsplit > 0 ? router_topk_kernel<true> : router_topk_kernel<false>;
+  topk<<<dim3((unsigned)(cdiv(T, 4) + riders)), 256, 0, g_stream>>>(
       logits, pairs, ids, (int)T, (int)E, (int)k, sigmoid, x, gate_w, gate_b, (int)H, logits + T * E, nsplit, rider);
   return check_launch("router_topk_kernel");
 }
@@ -1875,7 +1876,7 @@ int forward_pass(csk_layer* L, const float* hidden, int64_t T, float* out, int f
     } else if (T > kRouteSmallTokens) {
       // more tokens than the single workgroup has waves: selection spread over T / 4
       // workgroups, then the dispatch kernel -- a launch more, each much shorter
-      router_topk_kernel<<<dim3((unsigned)cdiv(T, 4)), 256, 0, g_stream>>>(
+      router_topk_kernel<false><<<dim3((unsigned)cdiv(T, 4)), 256, 0, g_stream>>>(
           ws.logits, ws.pairs, ws.ids, (int)T, (int)L->E, (int)L->k, L->sigmoid, xr, L->gate_w,
           L->has_gate_b ? L->gate_b : nullptr, (int)L->H, ws.logits + T * L->E, 0, Mx3Rider{});
       if ((rc = check_launch("router_topk_kernel")) != CSK_OK) return rc;

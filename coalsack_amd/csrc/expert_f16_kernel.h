@@ -569,6 +569,9 @@ __global__ __launch_bounds__(256) void expert_f16_kernel(ExpertF16Args a) {
 // 2048 1106 / 1060; 8 experts, 300 tokens, top-2 200 / 180; 200 x 2880 x 4096 projection (host
 // buffers) 212 / 202.  Eight waves and 128 tokens per workgroup, which fetch the weights of a
 // full tile once, were slower (1000 tokens: 715), and so were 128 tokens per four waves (690).
+// Where that leaves the chip short of units, the down projection takes units of 128 rows (NS = 1: one group of 32 rows per
+// wave, half the matrix instructions per fragment): the K loop of 45 steps is then the whole launch, and a step as long as its
+// products (200 x 2880 x 4096, host buffers, 64 units of 256 rows: 205 us, 128 of 128: 196).
 // Work units (M tile, N tile) are numbered expert by expert and dealt to the eight dies in
 // contiguous eighths.
 struct ExpertF16GemmArgs {
@@ -592,12 +595,14 @@ struct F16GemmLds {
 };
 
 // One work unit: MS = 2 for M tiles of more than 32 tokens, MS = 1 for those of at most 32 (the
-// ragged end of an expert's list), which cost half the matrix instructions and half the panel.
-template <int MODE, int MS>
+// ragged end of an expert's list), which cost half the matrix instructions and half the panel.  NS: groups of 32 weight
+// rows per wave (of gate and of up; one or two of down).
+template <int MODE, int MS, int NS>
 __device__ __forceinline__ void expert_f16_gemm_unit(const ExpertF16GemmArgs& a, const WorkDesc* wd, int m0, int mcount,
                                                      int nt, F16GemmLds& lds) {
   auto& panel = lds.panel;
   auto& rs_sh = lds.rs;
+  static_assert(NS == 2 || (NS == 1 && MODE == 1), "a wave pairs 32 gate rows with the 32 up rows of the same features");
   constexpr int NC = 2 * MS;  // panel copies per wave and step
   const int base = wd->base + m0;
   const int lane = threadIdx.x & 63;
@@ -607,11 +612,11 @@ __device__ __forceinline__ void expert_f16_gemm_unit(const ExpertF16GemmArgs& a,
   const int nkb = a.nkb, nsteps = (nkb + 1) >> 1, nfull = nkb >> 1;
 
   // this lane's weight entries: row n32 of the wave's two 32-row groups
-  int rows[2];
-  const CSK_GLOBAL u32x4* W[2];
+  int rows[NS];
+  const CSK_GLOBAL u32x4* W[NS];
 #pragma unroll
-  for (int s = 0; s < 2; ++s) {
-    const int t = MODE == 0 ? nt * 8 + wv * 2 + th : nt * 16 + wv * 4 + 2 * s + th;
+  for (int s = 0; s < NS; ++s) {
+    const int t = MODE == 0 ? nt * 8 + wv * 2 + th : nt * (8 * NS) + wv * (2 * NS) + 2 * s + th;
     rows[s] = t * 16 + n16;
     const uint4* q = MODE == 0 ? (s == 0 ? wd->w.q_gate : wd->w.q_up) : wd->w.q_down;
     W[s] = as_global(reinterpret_cast<const u32x4*>(q)) + (long)min(t, a.ntile - 1) * nkb * 64 + n16 + 16 * kg;
@@ -639,15 +644,15 @@ __device__ __forceinline__ void expert_f16_gemm_unit(const ExpertF16GemmArgs& a,
   const uint32_t lds_wave = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)&panel[0][0] +
                             (uint32_t)(NC * wv * 64 * 16);
 
-  floatx16 acc[MS][2];  // [32-token half][row group]
+  floatx16 acc[MS][NS];  // [32-token half][row group]
 #pragma unroll
   for (int ms = 0; ms < MS; ++ms)
 #pragma unroll
-    for (int s = 0; s < 2; ++s)
+    for (int s = 0; s < NS; ++s)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[ms][s][r] = 0.0f;
 
-  u32x4 wq[2][2][4];  // [step parity][row group][16-wide K slice of the step]
+  u32x4 wq[2][NS][4];  // [step parity][row group][16-wide K slice of the step]
   // Every load of the loop is unconditional (addresses are clamped, never branched around):
   // with a branch around a load the compiler's wait-count pass gives up at the join and
   // drains the whole queue at the head of every step.
@@ -674,7 +679,7 @@ __device__ __forceinline__ void expert_f16_gemm_unit(const ExpertF16GemmArgs& a,
 #pragma unroll
     for (int sl = 0; sl < 4; ++sl)
 #pragma unroll
-      for (int s = 0; s < 2; ++s) load_w(u, s, sl, min(u, nsteps - 1));
+      for (int s = 0; s < NS; ++s) load_w(u, s, sl, min(u, nsteps - 1));
   }
 #pragma unroll
   for (int i = 0; i < NC; ++i)
@@ -688,7 +693,7 @@ __device__ __forceinline__ void expert_f16_gemm_unit(const ExpertF16GemmArgs& a,
   auto step = [&](auto u_t, int j, auto more_t, auto sl_t) {
     constexpr int u = decltype(u_t)::value, SL = decltype(sl_t)::value;
     constexpr bool more = decltype(more_t)::value;
-    constexpr int kInFlight = more ? 16 + NC : 8;
+    constexpr int kInFlight = more ? 8 * NS + NC : 4 * NS;
     __builtin_amdgcn_s_waitcnt((kInFlight & 15) | (7 << 4) | (0 << 8) | ((kInFlight >> 4) << 14));
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
@@ -710,16 +715,16 @@ __device__ __forceinline__ void expert_f16_gemm_unit(const ExpertF16GemmArgs& a,
       if (q + 1 < SL * MS) read_frag(q + 1);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int s = 0; s < 2; ++s) {
+      for (int s = 0; s < NS; ++s) {
         const half8 w = __builtin_bit_cast(half8, wq[u][s][sl]);
         acc[ms][s] = __builtin_amdgcn_mfma_f32_32x32x16_f16(hi[q & 1], w, acc[ms][s], 0, 0, 0);
         acc[ms][s] = __builtin_amdgcn_mfma_f32_32x32x16_f16(lo[q & 1], w, acc[ms][s], 0, 0, 0);
       }
 #pragma unroll
-      for (int s = 0; s < 2; ++s) asm volatile("" : "+v"(acc[ms][s]));
+      for (int s = 0; s < NS; ++s) asm volatile("" : "+v"(acc[ms][s]));
       if (more && ms == MS - 1) {
-        load_w(u, 0, sl, jn);
-        load_w(u, 1, sl, jn);
+#pragma unroll
+        for (int s = 0; s < NS; ++s) load_w(u, s, sl, jn);
       }
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -748,10 +753,10 @@ __device__ __forceinline__ void expert_f16_gemm_unit(const ExpertF16GemmArgs& a,
   // accumulator register r is token (r % 4) + 8 (r / 4) + 4 kg of its 32-token half
   const CSK_GLOBAL float* b0 = as_global(MODE == 0 ? wd->w.b_gate : wd->w.b_down);
   const CSK_GLOBAL float* b1 = as_global(MODE == 0 ? wd->w.b_up : wd->w.b_down);
-  float bias[2];
-  bool rv[2];
+  float bias[NS];
+  bool rv[NS];
 #pragma unroll
-  for (int s = 0; s < 2; ++s) {
+  for (int s = 0; s < NS; ++s) {
     rv[s] = rows[s] < a.N;
     bias[s] = rv[s] ? (s == 0 ? b0 : b1)[rows[s]] : 0.0f;
   }
@@ -766,17 +771,17 @@ __device__ __forceinline__ void expert_f16_gemm_unit(const ExpertF16GemmArgs& a,
       if (MODE == 0) {
         const float sc_u = rs_sh[tl] * a.wscale[1];
         if (rv[0])
-          o[rows[0]] = moe_activation(acc[ms][0][r] * sc_t + bias[0], acc[ms][1][r] * sc_u + bias[1], a.act_type);
+          o[rows[0]] = moe_activation(acc[ms][0][r] * sc_t + bias[0], acc[ms][NS - 1][r] * sc_u + bias[NS - 1], a.act_type);
       } else {
 #pragma unroll
-        for (int s = 0; s < 2; ++s)
+        for (int s = 0; s < NS; ++s)
           if (rv[s]) o[rows[s]] = acc[ms][s][r] * sc_t + bias[s];
       }
     }
   }
 }
 
-template <int MODE>
+template <int MODE, int NS>
 __global__ __launch_bounds__(256, 2) void expert_f16_gemm_kernel(ExpertF16GemmArgs a) {
   __shared__ F16GemmLds lds;
   const int n_units = *a.n_mtiles * a.n_ntiles;
@@ -801,9 +806,9 @@ __global__ __launch_bounds__(256, 2) void expert_f16_gemm_kernel(ExpertF16GemmAr
   }
   const int mcount = min(64, wd->Te - m0);
   if (mcount <= 32)
-    expert_f16_gemm_unit<MODE, 1>(a, wd, m0, mcount, nt, lds);
+    expert_f16_gemm_unit<MODE, 1, NS>(a, wd, m0, mcount, nt, lds);
   else
-    expert_f16_gemm_unit<MODE, 2>(a, wd, m0, mcount, nt, lds);
+    expert_f16_gemm_unit<MODE, 2, NS>(a, wd, m0, mcount, nt, lds);
 }
 
 }  // namespace csk

@@ -161,7 +161,8 @@ __global__ __launch_bounds__(256) void router_logits_mfma_kernel(const float* __
 // IT float4 per thread hold a row of up to 1024 IT values: rows up to 4096 take 4, up to 8192 8, and only longer ones
 // are read again in every pass (8 tokens of 5120 on 16 experts: read again 11.1 us, held 5.4; 16 of 4128 38.5 -> 35 us for a layer of 16
 // experts of 512, 64 of 8192 on 128 experts 170 -> 151; the registers leave two workgroups per compute unit instead of four, and
-// 60 tokens of 6144 on 64 experts are no faster).
+// 60 tokens of 6144 on 64 experts are no faster).  The same products and partial sums either way; the compiler contracts
+// them differently, so a routing weight may differ in its last bits (fp16 layer of 16 x 5120 x 8192: 3e-7 of the output).
 // Restates moe_router_node.h:161-167 and rmsnorm_node.h:62-83.
 template <int EPW, int IT>
 __global__ __launch_bounds__(256) void router_prep_logits_kernel(

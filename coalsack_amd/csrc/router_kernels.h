@@ -149,6 +149,14 @@ __global__ __launch_bounds__(256) void router_logits_mfma_kernel(const float* __
 }
 
 // --------------------------------------------- small batches: prologue + logits
+// Four products summed, with the order and the contraction spelled out: left to the compiler they differ between forms of
+// the same loop, and a logit's last bits with them.
+template <bool Y_FIRST>
+__device__ __forceinline__ float quad_dot(const float4& a, const float4& b) {
+  const float two = Y_FIRST ? fmaf(a.x, b.x, a.y * b.y) : fmaf(a.y, b.y, a.x * b.x);
+  return fmaf(a.w, b.w, fmaf(a.z, b.z, two));
+}
+
 // One launch for small T: workgroups x in [0, ceil(E / EPW)) compute the logits of EPW experts
 // for the four tokens of tile y (the four waves split H, so all loads of a row are in flight
 // at once; the token rows stay in registers across the experts); the next four workgroups
@@ -161,8 +169,8 @@ __global__ __launch_bounds__(256) void router_logits_mfma_kernel(const float* __
 // IT float4 per thread hold a row of up to 1024 IT values: rows up to 4096 take 4, up to 8192 8, and only longer ones
 // are read again in every pass (8 tokens of 5120 on 16 experts: read again 11.1 us, held 5.4; 16 of 4128 38.5 -> 35 us for a layer of 16
 // experts of 512, 64 of 8192 on 128 experts 170 -> 151; the registers leave two workgroups per compute unit instead of four, and
-// 60 tokens of 6144 on 64 experts are no faster).  The same products and partial sums either way; the compiler contracts
-// them differently, so a routing weight may differ in its last bits (fp16 layer of 16 x 5120 x 8192: 3e-7 of the output).
+// 60 tokens of 6144 on 64 experts are no faster).  The same products and sums in the same order whether a row is held or read
+// again; only rows of up to 4096 begin a logit's quad with its second product, as they always have.
 // Restates moe_router_node.h:161-167 and rmsnorm_node.h:62-83.
 template <int EPW, int IT>
 __global__ __launch_bounds__(256) void router_prep_logits_kernel(
@@ -204,7 +212,7 @@ __global__ __launch_bounds__(256) void router_prep_logits_kernel(
           xv[j] = one_round ? x0[j] : (c < H4p ? x4[c] : make_float4(0.f, 0.f, 0.f, 0.f));
         }
 #pragma unroll
-        for (int j = 0; j < kIter; ++j) ss += xv[j].x * xv[j].x + xv[j].y * xv[j].y + xv[j].z * xv[j].z + xv[j].w * xv[j].w;
+        for (int j = 0; j < kIter; ++j) ss += quad_dot<true>(xv[j], xv[j]);
       }
       ss = wave_sum(ss);
       if (lane == 0) part[wv][0] = ss;
@@ -335,12 +343,12 @@ __global__ __launch_bounds__(256) void router_prep_logits_kernel(
 #pragma unroll
           for (int j = 0; j < kMaxIter; ++j) {
             const float4 xv = xr[i][j];  // chunks past H are zeros
-            ss[i] += xv.x * xv.x + xv.y * xv.y + xv.z * xv.z + xv.w * xv.w;
+            ss[i] += quad_dot<true>(xv, xv);
           }
         } else {
           for (int c = threadIdx.x; c < H4; c += 256) {
             const float4 xv = row(i, c);
-            ss[i] += xv.x * xv.x + xv.y * xv.y + xv.z * xv.z + xv.w * xv.w;
+            ss[i] += quad_dot<true>(xv, xv);
           }
         }
       }
@@ -387,7 +395,7 @@ __global__ __launch_bounds__(256) void router_prep_logits_kernel(
         for (int i = 0; i < 4; ++i) {
           if (i < nt) {
             const float4 xv = xr[i][j];
-            acc[i] += xv.x * gv.x + xv.y * gv.y + xv.z * gv.z + xv.w * gv.w;
+            acc[i] += quad_dot<IT == 4>(xv, gv);
           }
         }
       }
@@ -407,7 +415,7 @@ __global__ __launch_bounds__(256) void router_prep_logits_kernel(
               xv.z = (xv.z * inv[i]) * wv4.z;
               xv.w = (xv.w * inv[i]) * wv4.w;
             }
-            acc[i] += xv.x * gv.x + xv.y * gv.y + xv.z * gv.z + xv.w * gv.w;
+            acc[i] += quad_dot<false>(xv, gv);
           }
         }
       }

@@ -23,3 +23,24 @@ def test_rows_at_the_lines(lib, oracle, H, E, k, T, norm):
     same = np.all(pairs[..., 0] == wpairs[..., 0], axis=1)
     assert np.max(np.abs(pairs[same] - wpairs[same])) < 1.7e-5  # 1e-5 at 2880 values, growing with sqrt(H)
     assert_layer_close(got[same], want[same])
+
+
+@pytest.mark.parametrize("H,want", [(4096, 1.0), (4128, 0.0), (8192, 0.0), (8224, 0.0)])
+@pytest.mark.parametrize("E,T", [(4, 2), (130, 33)])
+@pytest.mark.parametrize("last", [False, True])
+def test_order_of_a_quads_sum(lib, H, want, E, T, last):
+    """A logit of one quad, 4097 * 4097 - (2^24 + 8192): 4097^2 = 2^24 + 8193 is a tie that fp32 rounds to 2^24 + 8192, so
+    the sum is 0 where the first product is rounded and 1 where the second is.  The latter is the order of rows of up to
+    4096 values; longer ones round the first, whether they are held in registers or read again."""
+    L = synth.LayerInputs(E, 1, H, 32, seed=3)
+    c = H - 4 if last else 0
+    hidden = np.zeros((T, H), np.float32)
+    hidden[:, c], hidden[:, c + 1] = 4097.0, 1.0
+    L.gate_w[:] = 0.0
+    L.gate_w[0, c], L.gate_w[0, c + 1] = 4097.0, -(2.0 ** 24 + 8192.0)
+    L.gate_b[:] = -1000.0  # no close call
+    L.gate_b[0] = 0.0
+    with build_layer(lib, L, device_weights=True, sigmoid=True) as layer:
+        _, pairs = layer.forward(hidden, want_pairs=True)
+    assert np.all(pairs[:, 0, 0] == 0)
+    assert np.all(np.abs(pairs[:, 0, 1] - 1.0 / (1.0 + np.exp(-want))) < 1e-6)

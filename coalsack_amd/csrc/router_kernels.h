@@ -389,14 +389,10 @@ __global__ __launch_bounds__(256) void router_prep_logits_kernel(
     if (held) {
       if (ee + 1 < EPW) load_gate(gq[(ee + 1) & 1], ee + 1);
 #pragma unroll
-      for (int j = 0; j < kMaxIter; ++j) {
-        const float4 gv = gq[ee & 1][j];  // chunks past H are zeros on both sides
+      for (int i = 0; i < 4; ++i) {  // (tokens outside, one branch each: inside, every quad has its own -- 64 tokens of
+        if (i < nt) {                // 5120 on 128 experts with RMSNorm 20.6 -> 25.3 us)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          if (i < nt) {
-            const float4 xv = xr[i][j];
-            acc[i] += quad_dot<IT == 4>(xv, gv);
-          }
+          for (int j = 0; j < kMaxIter; ++j) acc[i] += quad_dot<IT == 4>(xr[i][j], gq[ee & 1][j]);  // chunks past H are zeros
         }
       }
     } else {

@@ -1865,11 +1865,16 @@ int forward_pass(csk_layer* L, const float* hidden, int64_t T, float* out, int f
     // the rows first)
     u32x4* rows_mx3 = (!L->f16 && !L->wbf) ? reinterpret_cast<u32x4*>(ws.xs) : nullptr;
     rows_mx3_ready = rows_mx3 != nullptr;
-    // a workgroup takes one expert (latency) as long as all of them are resident at once, four beyond
-    const bool one = cdiv(T, 4) * (L->E + 4) <= 4 * std::max(g_cus, 1) + 64;  // four of these workgroups fit a compute unit
-    const bool held = L->H <= 4096 || L->H > 8192;
-    const auto kernel = one ? (held ? router_prep_logits_kernel<1, 4> : router_prep_logits_kernel<1, 8>)
-                            : (held ? router_prep_logits_kernel<4, 4> : router_prep_logits_kernel<4, 8>);
+    // A workgroup takes one expert (latency) as long as all of them are resident at once, four beyond.  Four workgroups fit
+    // a compute unit, but only two of those that hold rows of 4096 to 8192 values.  One expert / four, us for the launch on
+    // 256 compute units with RMSNorm (without): 468 workgroups (52 tokens of 6144, 32 experts) 10.8 / 12.8 (8.2 / 10.8), 528
+    // (16 of 5120, 128) 14.3 / 11.9 (9.9 / 10.0), 544 (32 of 6144, 64) 14.7 / 12.3 (10.3 / 10.3), 792 (24 of 5120,
+    // 128) 15.9 / 12.0 (10.8 / 10.1), 1056 (32 of 8192, 128) 23.6 / 15.1 (15.9 / 12.3).
+    const bool eight = L->H > 4096 && L->H <= 8192;  // float4 per thread and row
+    const int64_t cus = std::max(g_cus, 1), at_once = eight ? 2 * cus : 4 * cus + 64;
+    const bool one = cdiv(T, 4) * (L->E + 4) <= at_once;
+    const auto kernel = one ? (eight ? router_prep_logits_kernel<1, 8> : router_prep_logits_kernel<1, 4>)
+                            : (eight ? router_prep_logits_kernel<4, 8> : router_prep_logits_kernel<4, 4>);
     kernel<<<dim3((unsigned)(cdiv(L->E, one ? 1 : 4) + 4), (unsigned)cdiv(T, 4)), 256, 0, g_stream>>>(
         hidden, norm ? L->norm_w : nullptr, L->eps, ws.xn, L->gate_w,
         L->has_gate_b ? L->gate_b : nullptr, ws.logits, (int)T, (int)L->E, (int)L->H, rows_mx3);

@@ -168,8 +168,8 @@ __device__ __forceinline__ float quad_dot(const float4& a, const float4& b) {
 // them, 18.6 us; a quarter as many read the token rows a quarter as often).
 // IT float4 per thread hold a row of up to 1024 IT values: rows up to 4096 take 4, up to 8192 8, and only longer ones
 // are read again in every pass (8 tokens of 5120 on 16 experts: read again 11.1 us, held 5.4; 16 of 4128 38.5 -> 35 us for a layer of 16
-// experts of 512, 64 of 8192 on 128 experts 170 -> 151; the registers leave two workgroups per compute unit instead of four, and
-// 60 tokens of 6144 on 64 experts are no faster).  The same products and sums in the same order whether a row is held or read
+// experts of 512, 64 of 8192 on 128 experts 170 -> 151).  The registers of 8 leave two workgroups per compute unit instead
+// of four, which the choice of EPW goes by.  The same products and sums in the same order whether a row is held or read
 // again; only rows of up to 4096 begin a logit's quad with its second product, as they always have.
 // Restates moe_router_node.h:161-167 and rmsnorm_node.h:62-83.
 template <int EPW, int IT>

@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 
 from coalsack_amd import capi, synth
-from tests.helpers import assert_layer_close, build_layer, classify_index_mismatches, oracle_layer
+from tests.helpers import assert_layer_close, build_layer, classify_index_mismatches, nbits_differ, oracle_layer
 
 pytestmark = pytest.mark.gpu
 
@@ -44,3 +44,19 @@ def test_order_of_a_quads_sum(lib, H, want, E, T, last):
         _, pairs = layer.forward(hidden, want_pairs=True)
     assert np.all(pairs[:, 0, 0] == 0)
     assert np.all(np.abs(pairs[:, 0, 1] - 1.0 / (1.0 + np.exp(-want))) < 1e-6)
+
+
+@pytest.mark.parametrize("E,H,T,short,norm", [(128, 4096, 33, 12, True), (124, 8192, 17, 10, True), (128, 5120, 13, 8, False)])
+def test_four_experts_per_workgroup_give_the_bits_of_one(lib, E, H, T, short, norm):
+    """The shortest batches on 256 compute units that take four experts per workgroup, and the same tokens in passes that
+    take one: routing weights of the same bits."""
+    L = synth.LayerInputs(E, 4, H, 32, seed=6, with_norm=norm)
+    hidden = synth.hidden_states(T, H, seed=2)
+    with build_layer(lib, L, device_weights=True, norm=norm) as layer:
+        _, four = layer.forward(hidden, capi.FWD_RMSNORM if norm else 0, want_pairs=True)
+        try:
+            lib.set_pass_tokens(short)
+            _, one = layer.forward(hidden, capi.FWD_RMSNORM if norm else 0, want_pairs=True)
+        finally:
+            lib.set_pass_tokens(32768)
+    assert nbits_differ(four, one) == 0

@@ -571,7 +571,7 @@ __global__ __launch_bounds__(256) void expert_f16_kernel(ExpertF16Args a) {
 // full tile once, were slower (1000 tokens: 715), and so were 128 tokens per four waves (690).
 // Where that leaves the chip short of units, the down projection takes units of 128 rows (NS = 1: one group of 32 rows per
 // wave, half the matrix instructions per fragment): the K loop of 45 steps is then the whole launch, and a step as long as its
-// products (200 x 2880 x 4096, host buffers, 64 units of 256 rows: 205 us, 128 of 128: 196).
+// products (200 x 2880 x 4096, host buffers: 64 units of 256 rows 205 us, 128 of 128 196).
 // Work units (M tile, N tile) are numbered expert by expert and dealt to the eight dies in
 // contiguous eighths.
 struct ExpertF16GemmArgs {

@@ -95,7 +95,11 @@ struct MxGeom {
   // two steps ahead (32 experts of 2880 x 2880, 70 tokens: 125.5 -> 119.5 us per layer; 128 of them, 150
   // tokens 365 -> 350, 300 tokens 420 -> 416).
   static constexpr int kStages = NG == 2 && MS == 1 ? 3 : 2;
-  static constexpr int kEpiRow = 16 * NG + 1;  // floats per token in a wave's epilogue tile (+1: bank spread)
+  // Floats per token in a wave's epilogue tile: whole 16-byte chunks, four banks further with every token, so that a lane's
+  // blocks and the workgroup's stores are read 16 bytes at a time without conflicts (rows of 16 NG + 1 floats were read and
+  // written 4 at a time: us per layer, 16 experts of 4096 x 6144, top-2, 600 tokens 287 -> 284, 64 of 1504 x 3072, top-4, 2000
+  // tokens 296.5 -> 294.4, 8 of 1024 x 512, top-8, 1000 tokens 62.9 -> 62.0).
+  static constexpr int kEpiRow = 16 * NG + 4;
   static constexpr size_t kLdsBytes =
       (size_t)kStages * kStageChunks * 16 > (size_t)kMxWaves * kBM * kEpiRow * 4
           ? (size_t)kStages * kStageChunks * 16
@@ -277,14 +281,12 @@ __device__ __forceinline__ void expert_gemm_mx_unit(const ExpertGemmMxArgs& a, c
     for (int r = 0; r < 3; ++r) {
       const int i = threadIdx.x + r * 64 * kMxWaves;
       const int tl = i / kOutChunks, c = i - tl * kOutChunks, w = c / kWaveChunks, cw = c - w * kWaveChunks;
-      const float* t = reinterpret_cast<const float*>(smem) + (w * kBM + tl) * G::kEpiRow + 32 * (cw / kMx3ChunksPerBlock) +
-                       4 * (cw % kMx3ChunksPerBlock);
+      const u32x4* t = reinterpret_cast<const u32x4*>(smem) + ((w * kBM + tl) * G::kEpiRow) / 4 + 8 * (cw / kMx3ChunksPerBlock) +
+                       cw % kMx3ChunksPerBlock;
       const bool rows = w < waves, stored = kb0 + c / kMx3ChunksPerBlock < out_rowblk;
       u32x4 v[kGroups];
 #pragma unroll
-      for (int q = 0; q < kGroups; ++q)
-#pragma unroll
-        for (int d = 0; d < 4; ++d) v[q][d] = __float_as_uint(t[q * kTokens * G::kEpiRow + d]);
+      for (int q = 0; q < kGroups; ++q) v[q] = t[q * kTokens * G::kEpiRow / 4];
 #pragma unroll
       for (int q = 0; q < kGroups; ++q) {
         if (!rows) v[q] = u32x4{0u, 0u, c & 1 ? 127u : 0u, 0u};
@@ -451,7 +453,7 @@ __device__ __forceinline__ void expert_gemm_mx_unit(const ExpertGemmMxArgs& a, c
   // epilogue: lane holds weight row n32 of each group; accumulator register r is token
   // (r % 4) + 8 * (r / 4) + 4 * kg of the 32-token sub-tile
   if (MODE == 0) {
-    // bias + activation into this wave's LDS tile as fp32 [token][16 NG features + 1], then
+    // bias + activation into this wave's LDS tile as fp32 [token][16 NG features + 4], then
     // one lane per token re-quantises 32 features at a time to the three-term format
     __syncthreads();  // the copies issued for the steps after the last have landed; all waves are past their reads
     float* tile = reinterpret_cast<float*>(smem) + (size_t)wv * kBM * G::kEpiRow;
@@ -477,19 +479,22 @@ __device__ __forceinline__ void expert_gemm_mx_unit(const ExpertGemmMxArgs& a, c
     if (a.act_type == 0) activate(std::integral_constant<int, 0>{});
     else activate(std::integral_constant<int, 1>{});
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    // a lane re-quantises its token's blocks and puts them back where their 32 values were
-    float* mine = tile + (lane % kBM) * G::kEpiRow;
+    // a lane re-quantises blocks of its token, all of them or with 32 tokens every second one, and puts them back where
+    // their 32 values were
+    u32x4* mine = reinterpret_cast<u32x4*>(tile + (lane % kBM) * G::kEpiRow);
 #pragma unroll 1
-    for (int bi = 0; bi < NG / 2; ++bi) {
+    for (int bi = lane / kBM; bi < NG / 2; bi += 64 / kBM) {
       float v[32];
 #pragma unroll
-      for (int i = 0; i < 32; ++i) v[i] = mine[32 * bi + i];
+      for (int c = 0; c < 8; ++c) {
+        const u32x4 four = mine[8 * bi + c];
+#pragma unroll
+        for (int d = 0; d < 4; ++d) v[4 * c + d] = __uint_as_float(four[d]);
+      }
       u32x4 out[kMx3ChunksPerBlock];
       mx3_quantize_block(v, out);
 #pragma unroll
-      for (int c = 0; c < kMx3ChunksPerBlock; ++c)
-#pragma unroll
-        for (int d = 0; d < 4; ++d) mine[32 * bi + 4 * c + d] = __uint_as_float(out[c][d]);
+      for (int c = 0; c < kMx3ChunksPerBlock; ++c) mine[8 * bi + c] = out[c];
     }
     __syncthreads();
     store_rows();

@@ -750,6 +750,7 @@ template <int MODE, int NG>
 int launch_gemm_mx(ExpertGemmMxArgs& ga, int64_t E, int64_t P) {
   using Geom = MxGeom<NG, 2>;
   ga.n_ntiles = (int)cdiv(ga.ntile, Geom::tiles_per_wg(MODE));
+  ga.two_part_units = 3 * 2 * std::max(g_cus, 1);  // two workgroups of the tall tile per compute unit are the places
   static bool lds_attr_set = false;
   if (!lds_attr_set) {
     HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(&expert_gemm_mx_kernel<MODE, NG>),

@@ -69,6 +69,7 @@ struct ExpertGemmMxArgs {
   int n_ntiles;          // N tiles per M tile: ceil(ntile / (4 NG)) (MODE 0) or ceil(ntile / (8 NG))
   int N;
   int act_type;
+  int two_part_units;    // from this many work units on, a die takes two parts of their sequence
   u32x4* act_out;        // MODE 0: [P][mx3_row_blocks(N / 32)][6] x 16 B
   float* y_out;          // MODE 1: [P][N]
 };
@@ -295,8 +296,8 @@ __device__ __forceinline__ void expert_gemm_mx_unit(const ExpertGemmMxArgs& a, c
     }
   };
   if (idle_wave) {
-    // the same sequence of copies, waits and barriers as below without the weights and the
-    // arithmetic; what this wave owes the output is the zero padding of the rows
+    // the same sequence of copies, waits and barriers as below (two in front of the stores) without the weights and
+    // the arithmetic; the stores of the workgroup's rows are shared out over all its waves, this one among them
 #pragma unroll
     for (int u = 0; u < kLead; ++u)
 #pragma unroll
@@ -526,13 +527,12 @@ __device__ __forceinline__ void expert_gemm_mx_unit(const ExpertGemmMxArgs& a, c
 // first (layer, us, one part / two: 128 experts of 2880 x 2880, 4096 tokens 967 / 950, 1000 tokens 511 / 501; 16 of
 // 4096 x 6144, 2000 tokens 615 / 600).  With fewer units a part's ends, whose experts two dies share, weigh more (the same
 // 16 experts, 1000 tokens 366 / 374; units of 256 rows: 128 experts, 300 tokens 404 / 410).
-constexpr int kTwoPartUnits = 1536;
 template <int MODE, int NG>
 __global__ __launch_bounds__(64 * kMxWaves, NG == 2 ? 3 : 2) void expert_gemm_mx_kernel(ExpertGemmMxArgs a) {
   extern __shared__ __align__(16) unsigned char smem[];
   const int n_units = *a.n_mtiles * a.n_ntiles;
   const int die = blockIdx.x % kDies, slot = blockIdx.x / kDies;
-  const bool two_parts = NG == kMxNG && n_units >= kTwoPartUnits;
+  const bool two_parts = NG == kMxNG && n_units >= a.two_part_units;
   const int part = two_parts ? (n_units + 2 * kDies - 1) / (2 * kDies) : (n_units + kDies - 1) / kDies;
   const int unit = slot < part ? die * part + slot : (2 * kDies - 2 - die) * part + slot;  // (the part 2 kDies - 1 - die)
   if (slot >= (two_parts ? 2 : 1) * part || unit >= n_units) return;

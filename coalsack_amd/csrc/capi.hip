@@ -878,20 +878,6 @@ int launch_f16_split(const float* x, int64_t rows, int64_t K, const int* gather_
   return check_launch("f16_split_rows_kernel");
 }
 
-// Units of the fp16 down projection: 256 weight rows, or 128 where 256 would leave nearly half of the chip without a unit --
-// then half a unit's time is worth more than the token rows that are read twice as often.  Units are counted as M tiles of
-// 64 tokens that can be expected: one per expert with few tokens, half a tile more than its tokens fill for one with many; no
-// expert holds more than T tokens (a single one is called with T k assignments, most of which are other experts').
-// Measured (us, 256 / 128 rows, by that count): a projection through host buffers with 58 units of 256 rows (200 x 2880 x 4096)
-// 205 / 196, with 125 (300 x 2880 x 6144) 330 / 321, 133 (500 x 2880 x 4096) 398 / 390, 137 (700 x 2880 x 2880) 444 / 435, 158
-// (600 x 2880 x 4096) 464 / 468, 194 (1000 x 2880 x 2880) 599 / 600; layers of 8 experts of 2880 x 2880, top-2, 200 tokens (123)
-// 142 / 135, of 16 of them, 100 tokens (192) 189 / 192.
-bool f16_low_tiles(int64_t E, int64_t T, int64_t P, int64_t N) {
-  const double tokens = (double)std::min(P, E * T), experts = (double)std::min(E, P), per_expert = tokens / (double)E;
-  const double mtiles = tokens / 64.0 + experts * std::max(0.5, 1.0 - per_expert / 64.0);
-  return 2.0 * mtiles * (double)cdiv(N, 256) <= 1.1 * std::max(g_cus, 1);
-}
-
 // y[P, N] <- W_down(expert of the position) x rows + b_down over two-term fp16 rows [P, K]:
 // the down projection of the experts, and any plain linear layer (one descriptor).
 int launch_f16_projection(int64_t E, int64_t T, int64_t P, int64_t K, int64_t N, const uint16_t* rows,
@@ -923,10 +909,11 @@ int launch_f16_projection(int64_t E, int64_t T, int64_t P, int64_t K, int64_t N,
     ga.ntile = (int)f16_tile_count(N);
     ga.out = y;
     const int64_t max_mtiles = P / 64 + std::min<int64_t>(E, P);
-    const bool low = f16_low_tiles(E, T, P, N);
-    ga.n_ntiles = (int)cdiv(N, low ? 128 : 256);
-    const auto kernel = low ? expert_f16_gemm_kernel<1, 1> : expert_f16_gemm_kernel<1, 2>;
-    kernel<<<dim3((unsigned)(cdiv(max_mtiles * ga.n_ntiles, kF16Dies) * kF16Dies)), 256, 0, g_stream>>>(ga);
+    ga.n_ntiles = (int)cdiv(N, 256);
+    ga.low_units = std::max(g_cus, 1);
+    // units of 256 rows, or of 128 as long as there are no more than low_units of them
+    const int64_t units = std::max(max_mtiles * ga.n_ntiles, std::min<int64_t>(max_mtiles * cdiv(N, 128), ga.low_units));
+    expert_f16_gemm_kernel<1><<<dim3((unsigned)(cdiv(units, kF16Dies) * kF16Dies)), 256, 0, g_stream>>>(ga);
   }
   return check_launch("expert_f16_kernel<1>");
 }
@@ -983,7 +970,7 @@ int run_experts_f16(int64_t E, int64_t T, int64_t k, int64_t H, int64_t F, int a
     ga.wscale[0] = a.wscale[0], ga.wscale[1] = a.wscale[1];
     ga.ntile = a.ntile, ga.out = a.out;
     ga.n_ntiles = (int)cdiv(F, 128);
-    expert_f16_gemm_kernel<0, 2><<<gemm_grid(ga.n_ntiles), 256, 0, g_stream>>>(ga);
+    expert_f16_gemm_kernel<0><<<gemm_grid(ga.n_ntiles), 256, 0, g_stream>>>(ga);
   }
   if ((rc = check_launch("expert_f16_kernel<0>")) != CSK_OK) return rc;
   if (timed) mark(CSK_STAGE_DOWN);

@@ -569,9 +569,14 @@ __global__ __launch_bounds__(256) void expert_f16_kernel(ExpertF16Args a) {
 // 2048 1106 / 1060; 8 experts, 300 tokens, top-2 200 / 180; 200 x 2880 x 4096 projection (host
 // buffers) 212 / 202.  Eight waves and 128 tokens per workgroup, which fetch the weights of a
 // full tile once, were slower (1000 tokens: 715), and so were 128 tokens per four waves (690).
-// Where that leaves the chip short of units, the down projection takes units of 128 rows (NS = 1: one group of 32 rows per
-// wave, half the matrix instructions per fragment): the K loop of 45 steps is then the whole launch, and a step as long as its
-// products (200 x 2880 x 4096, host buffers: 64 units of 256 rows 205 us, 128 of 128 196).
+// Where a compute unit gets no more than one of them, the down projection takes units of 128 rows (NS = 1: one group of 32
+// rows per wave, half the matrix instructions per fragment): the K loop is then the whole launch, and a step as long as its
+// products.  With a second one on some compute units the launch is as long as theirs, in which every token row is read
+// twice as often.  Launch (us, 256 / 128 rows, 256 compute units): a projection of 1024 values with 256 units of 128 rows
+// 20.1 / 16.8, with 264 20.4 / 21.9; of 2880 with 253 40.8 / 31.4, 256 40.7 / 32.6, 264 40.8 / 46.1; of 5120 with 256
+// 64.6 / 52.2, 264 64.6 / 78.5; layers of 2, 4, 8 and 32 experts with 230 38.4 / 29.6, 276 38.0 / 42.2, 240 (short
+// tiles) 68.6 / 51.2, 256 53.6 / 43.4.  The kernel chooses, by the M tiles that there are: how many the experts' tokens make is
+// not known where it is launched (4 experts of 2880, 548 tokens: 10.6 expected, 12).
 // Work units (M tile, N tile) are numbered expert by expert and dealt to the eight dies in
 // contiguous eighths.
 struct ExpertF16GemmArgs {
@@ -582,7 +587,8 @@ struct ExpertF16GemmArgs {
   const u32x4* B;       // two-term fp16 activation rows
   const float* rscale;
   float wscale[2];      // as in ExpertF16Args
-  int nkb, N, ntile, n_ntiles, act_type;
+  int nkb, N, ntile, n_ntiles, act_type;  // n_ntiles: N tiles of 256 rows
+  int low_units;        // down: up to this many units of 128 rows, they are taken
   float* out;
 };
 
@@ -781,10 +787,13 @@ __device__ __forceinline__ void expert_f16_gemm_unit(const ExpertF16GemmArgs& a,
   }
 }
 
-template <int MODE, int NS>
+template <int MODE>
 __global__ __launch_bounds__(256, 2) void expert_f16_gemm_kernel(ExpertF16GemmArgs a) {
   __shared__ F16GemmLds lds;
-  const int n_units = *a.n_mtiles * a.n_ntiles;
+  const int n_mtiles = *a.n_mtiles, n_low = (a.N + 127) / 128;
+  const bool low = MODE == 1 && n_mtiles * n_low <= a.low_units;
+  if (low) a.n_ntiles = n_low;
+  const int n_units = n_mtiles * a.n_ntiles;
   const int per_die = (n_units + kF16Dies - 1) / kF16Dies;
   const int slot_i = blockIdx.x / kF16Dies;
   const int unit = (blockIdx.x % kF16Dies) * per_die + slot_i;
@@ -805,10 +814,16 @@ __global__ __launch_bounds__(256, 2) void expert_f16_gemm_kernel(ExpertF16GemmAr
     m0 = (r - nt * tiles_e) * 64;
   }
   const int mcount = min(64, wd->Te - m0);
-  if (mcount <= 32)
-    expert_f16_gemm_unit<MODE, 1, NS>(a, wd, m0, mcount, nt, lds);
-  else
-    expert_f16_gemm_unit<MODE, 2, NS>(a, wd, m0, mcount, nt, lds);
+  if (MODE == 1 && low) {
+    if (mcount <= 32)
+      expert_f16_gemm_unit<1, 1, 1>(a, wd, m0, mcount, nt, lds);
+    else
+      expert_f16_gemm_unit<1, 2, 1>(a, wd, m0, mcount, nt, lds);
+  } else if (mcount <= 32) {
+    expert_f16_gemm_unit<MODE, 1, 2>(a, wd, m0, mcount, nt, lds);
+  } else {
+    expert_f16_gemm_unit<MODE, 2, 2>(a, wd, m0, mcount, nt, lds);
+  }
 }
 
 }  // namespace csk

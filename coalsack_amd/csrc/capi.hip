@@ -296,6 +296,11 @@ struct csk_event {
   hipEvent_t ev;
 };
 
+// both scale planes of a matrix
+static long matrix_scale_bytes(int64_t ntile, int64_t nblk) {
+  return (long)step_scale_plane(ntile, (int)nblk) + (long)ntile * 256 * step_scale_groups((int)nblk);
+}
+
 struct csk_mxfp4 {
   uint4* q = nullptr;
   uint8_t* s = nullptr;
@@ -303,7 +308,7 @@ struct csk_mxfp4 {
   int64_t ntile = 0, nblk = 0;
   bool owned = true;
   long entries() const { return (long)(ntile * nblk * 16); }
-  long scale_bytes() const { return (long)ntile * 256 * scale_slots((int)nblk); }
+  long scale_bytes() const { return matrix_scale_bytes(ntile, nblk); }
 };
 
 struct csk_layer {
@@ -354,8 +359,8 @@ struct csk_layer {
   long ent_gu() const { return (long)(ntF * nblkH * 16); }  // gate or up: [F,H]
   long ent_d() const { return (long)(ntH * nblkF * 16); }   // down: [H,F]
   long ent_expert() const { return 2 * ent_gu() + ent_d(); }
-  long sc_gu() const { return (long)ntF * 256 * scale_slots((int)nblkH); }  // scale bytes of gate or up
-  long sc_d() const { return (long)ntH * 256 * scale_slots((int)nblkF); }
+  long sc_gu() const { return matrix_scale_bytes(ntF, nblkH); }  // scale bytes of gate or up
+  long sc_d() const { return matrix_scale_bytes(ntH, nblkF); }
   long sc_expert() const { return 2 * sc_gu() + sc_d(); }
   csk_mxfp4 view(int64_t e, int which) const {
     csk_mxfp4 m;
@@ -1228,8 +1233,7 @@ static int layer_create(int64_t E, int64_t k, int64_t H, int64_t F, bool f16, cs
   L->ew_host.assign((size_t)E, ExpertW{});
   rc = dev_alloc(&L->gate_w, (size_t)E * H);
   if (rc == CSK_OK) rc = dev_alloc(&L->gate_b, (size_t)E);
-  // kWeightSlack: the grouped GEMM reads up to three blocks (and the scale loads three
-  // bytes) past the end of a plane; behind the last plane that must still be mapped memory
+  // kWeightSlack: the grouped GEMM reads up to three blocks past the end of a plane; behind the last plane that must still be mapped memory
   if (view) {
     // no planes of its own
   } else if (f16) {

@@ -26,7 +26,9 @@ constexpr int kStreamG = 4;      // tokens per pass of the weight-streaming expe
 //   s: scale bytes (E8M0), per tile [4 waves][64 lanes][slots]: the scale of block kb
 //      of row n sits with wave (kb/4)%4, lane (kb%4)*16+n, slot kb/16, so that the
 //      wave that owns K steps w, w+4, ... fetches all its scales of a tile with one
-//      8-byte load per lane (slots = K steps per wave, rounded up to 8).
+//      8-byte load per lane (slots = K steps per wave, rounded up to 2, 4 or a multiple of 8).
+//      Behind it the same bytes once more, [tiles][K steps / 4][64 lanes][4 steps], as the grouped
+//      GEMM reads them, whose workgroups walk all of K.
 // A wave reading entries [kb..kb+3][0..15] of one tile fetches 1 KiB of
 // contiguous nibbles; lane (g = lane/16, n = lane%16) owns block kb+g of row n.
 struct ExpertW {
@@ -79,11 +81,22 @@ __device__ __forceinline__ const CSK_GLOBAL T* as_global(const T* p) {
 // Scale-plane geometry (see ExpertW).
 __host__ __device__ inline int scale_slots(int nblk) {
   const int per_wave = (((nblk + 3) >> 2) + 3) >> 2;
-  return (per_wave + 7) & ~7;
+  return per_wave <= 2 ? 2 : per_wave <= 4 ? 4 : (per_wave + 7) & ~7;
 }
 __host__ __device__ inline size_t scale_index(long tile, int kb, int n, int slots) {
   const int j = kb >> 2;
   return ((size_t)tile * 256 + (size_t)(j & 3) * 64 + (kb & 3) * 16 + n) * slots + (j >> 2);
+}
+
+// The second scale plane of a matrix begins step_scale_plane bytes behind the first: per tile [groups of four K steps][64
+// cells][4 steps], so that the scale bytes of four consecutive steps are one 4-byte load per lane.  (2880 values: 1536 bytes
+// per tile beside the first plane's 2048 and 23040 of codes.  Slots were a multiple of 8 throughout: a row of 768 values
+// had 2048 bytes per tile, a quarter of what its matrix took from memory, and has 512; 64 experts of 2048 x 768, top-8, 50
+// tokens, 8 layers 607 -> 584 us.)
+__host__ __device__ inline int step_scale_groups(int nblk) { return (nblk + 15) >> 4; }
+__host__ __device__ inline size_t step_scale_plane(long ntile, int nblk) { return (size_t)ntile * 256 * scale_slots(nblk); }
+__host__ __device__ inline size_t step_scale_index(long tile, int kb, int n, int groups) {
+  return (((size_t)tile * groups + (kb >> 4)) * 64 + (kb & 3) * 16 + n) * 4 + ((kb >> 2) & 3);
 }
 
 // E8M0 byte -> scale of true E2M1 values, 2^(b-127); exact for b in 1..254.

@@ -29,7 +29,11 @@
 // straight to registers; both are requested one step ahead (two LDS stages and register
 // sets, one barrier per step), the weights of the step's second K half half a step later
 // than the rest, so that no request is waited for sooner than half a step after it was
-// made.
+// made.  Scale bytes come four steps at a time, one 4-byte load per lane, row group and K half, from a plane in that
+// order (common.h).  As one byte per step from the streaming kernel's plane they were two fifths of the kernel's vector
+// memory instructions, and each line of them was fetched again every fourth step (gate/up, 300 tokens on 128 experts:
+// 1.47 GB, now 1.2): us per layer, before / now, 2880 x 2880, top-4: 128 experts 300 tokens 409 / 375, 4096 947 / 884, 32
+// experts 2048 tokens 424 / 406.
 // Where a work unit's time goes (cycle counter per unit, 120b shape, 4096 tokens, two
 // workgroups per compute unit at a shader clock of about 1.6 GHz): 67 us in all -- 10 us
 // until the first step's operands have landed (descriptor chain, token rows, then the
@@ -93,9 +97,9 @@ struct MxGeom {
   static constexpr int kFrags = 6 * MS;                              // activation fragments per step
   // LDS stages and register sets, one more than the steps of lead.  Units of few tokens (and the
   // low tile, whose accumulators leave the registers) wait for memory, not for the matrix cores: they ask
-  // two steps ahead (32 experts of 2880 x 2880, 70 tokens: 125.5 -> 119.5 us per layer; 128 of them, 150
-  // tokens 365 -> 350, 300 tokens 420 -> 416).
-  static constexpr int kStages = NG == 2 && MS == 1 ? 3 : 2;
+  // three steps ahead (with two stages more than one, 32 experts of 2880 x 2880, 70 tokens: 125.5 -> 119.5 us per layer; 128
+  // of them, 150 tokens 365 -> 350).  Two or four stages: the four steps of the loop's body find theirs at compile time.
+  static constexpr int kStages = NG == 2 && MS == 1 ? 4 : 2;
   // Floats per token in a wave's epilogue tile: whole 16-byte chunks, four banks further with every token, so that a lane's
   // blocks are read and written 16 bytes at a time without conflicts.  (The workgroup's stores read a token's chunks across the
   // waves' tiles, which begin at the same bank: two accesses for one, SQ_LDS_BANK_CONFLICT 3.6 % of the LDS cycles and 0.6 %
@@ -144,7 +148,7 @@ __device__ __forceinline__ void expert_gemm_mx_unit(const ExpertGemmMxArgs& a, c
   const int n16 = n32 & 15, th = n32 >> 4;  // row within a packed tile, tile of the pair
   const int nblk = a.nblk;
   const int nsteps = (nblk + 3) >> 2;
-  const int slots = scale_slots(nblk);
+  const int sgroups = step_scale_groups(nblk);
 
   // Group g of this wave is the pair of packed tiles (t0(g), t0(g) + 1).  Every address of
   // the main loop is a wave-uniform base (the group's plane and tile pair, advanced per step
@@ -152,7 +156,7 @@ __device__ __forceinline__ void expert_gemm_mx_unit(const ExpertGemmMxArgs& a, c
   // same for every group, so the loads cost no vector instructions.  Nothing is clamped
   // along K: activation rows are padded with zero blocks to a whole number of steps, so
   // the weight blocks read past K (the next tile's, or the slack behind the last plane)
-  // and the scale bytes read past K (slot padding, 127) are multiplied by exact zeros.
+  // and the scale bytes read past K (padding, 127) are multiplied by exact zeros.
   // Groups past the last tile (ragged last N tile) re-read the last pair; their results
   // are dropped.  A wave none of whose groups exists (the ragged last N tile again: with
   // 2880 features three of its four waves) issues no matrix instructions at all and only
@@ -171,14 +175,15 @@ __device__ __forceinline__ void expert_gemm_mx_unit(const ExpertGemmMxArgs& a, c
   const auto s_rsrc0 = plane_rsrc(MODE == 0 ? w.s_gate : w.s_down);
   const auto s_rsrc1 = plane_rsrc(MODE == 0 ? w.s_up : w.s_down);
   uint32_t goff_q[NG], goff_s[NG];  // byte offset of the group's tile pair in its planes
+  const uint32_t splane = (uint32_t)step_scale_plane(a.ntile, nblk);
 #pragma unroll
   for (int g = 0; g < NG; ++g) {
     const int tc = min(group_tile(g), a.ntile - 2);
     goff_q[g] = (uint32_t)__builtin_amdgcn_readfirstlane(tc * nblk * 256);
-    goff_s[g] = (uint32_t)__builtin_amdgcn_readfirstlane(tc * 256 * slots);
+    goff_s[g] = splane + (uint32_t)__builtin_amdgcn_readfirstlane(tc * 256 * sgroups);
   }
   const uint32_t qoff = (uint32_t)(((th * nblk + kg) * 16 + n16) * 16);  // entry (tile th, block kg, row)
-  const uint32_t soff = (uint32_t)scale_index(th, kg, n16, slots);
+  const uint32_t soff = (uint32_t)step_scale_index(th, kg, n16, sgroups);
   const int rowblk = mx3_row_blocks(nblk);
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem;
 
@@ -215,9 +220,14 @@ __device__ __forceinline__ void expert_gemm_mx_unit(const ExpertGemmMxArgs& a, c
   // LDS destination of copy c of this wave within a stage (wave-uniform)
   const uint32_t lds_wave = lds0 + (uint32_t)(kCopies * wv * 64 * 16);
   struct BSet {
-    u32x4 q[2][NG];     // [64-wide K chunk of the step][row group]
-    uint8_t s[2][NG];   // the block's scale byte (widened where it is used: widening it where it is loaded would wait for the load there)
+    u32x4 q[2][NG];  // [64-wide K chunk of the step][row group]
   };
+  // Scale bytes of four consecutive steps, one register for each: the matrix instruction picks its byte.  While four steps
+  // are worked off those of the next four arrive.
+  struct SSet {
+    uint32_t w[2][NG];  // [64-wide K chunk of a step][row group]
+  };
+  SSet sc, sn;
   // copy c of the activation tile of step j into LDS stage `stage` (inline assembly: nothing
   // of it lives in a register; the explicit wait at the step boundary guarantees its arrival)
   auto issue_copy = [&](int c, int stage, int j) {
@@ -237,11 +247,10 @@ __device__ __forceinline__ void expert_gemm_mx_unit(const ExpertGemmMxArgs& a, c
     const uint32_t so = goff_q[g] + (uint32_t)j * 1024u + (uint32_t)kc * 512u;
     b.q[kc][g] = __builtin_amdgcn_raw_buffer_load_b128(second ? q_rsrc1 : q_rsrc0, qoff, so, 0);
   };
-  auto issue_s = [&](int kc, int g, BSet& b, int j) {
+  auto issue_s = [&](int kc, int g, SSet& b, int grp) {  // steps 4 grp .. 4 grp + 3
     const bool second = MODE == 0 && g >= NG / 2;
-    // the block's scale byte (the matrix instruction reads only byte 0 of its scale operand)
-    const uint32_t so = goff_s[g] + (uint32_t)(((j & 3) * 64 + 32 * kc) * slots + (j >> 2));
-    b.s[kc][g] = __builtin_amdgcn_raw_buffer_load_b8(second ? s_rsrc1 : s_rsrc0, soff, so, 0);
+    const uint32_t so = goff_s[g] + (uint32_t)(grp * 256 + kc * 128);
+    b.w[kc][g] = __builtin_amdgcn_raw_buffer_load_b32(second ? s_rsrc1 : s_rsrc0, soff, so, 0);
   };
   // The loads of step j are issued in two parts, each spread over the fragments of half a
   // step: first the activation tile and the weights of the step's first K half, then the
@@ -254,13 +263,9 @@ __device__ __forceinline__ void expert_gemm_mx_unit(const ExpertGemmMxArgs& a, c
   auto issue_part = [&](int part, int x, int stage, BSet& b, int j) {  // item x of a part
     if (part == 0) {
       if (x < kCopies) issue_copy(x, stage, j);
-      if (x < NG) {
-        issue_q(0, x, b, j);
-        issue_s(0, x, b, j);
-      }
+      if (x < NG) issue_q(0, x, b, j);
     } else if (x < NG) {
       issue_q(1, x, b, j);
-      issue_s(1, x, b, j);
     }
   };
   constexpr int kPart0Items = kCopies > NG ? kCopies : NG;
@@ -330,7 +335,8 @@ __device__ __forceinline__ void expert_gemm_mx_unit(const ExpertGemmMxArgs& a, c
   // instructions rather than in a burst at the step boundary: the texture address unit
   // takes 16 cycles per 64-lane 128-bit load, and a burst per wave would hold every wave at
   // the start of the step.
-  auto compute = [&](const BSet& b, int stage, BSet& bn, int stage_n, int jn, auto prefetch) {
+  auto compute = [&](const BSet& b, int stage, BSet& bn, int stage_n, int jn, int grp_n, auto phase_t, auto prefetch, auto scales) {
+    constexpr int phase = decltype(phase_t)::value;
     u32x4 flo[kFragBufs], fhi[kFragBufs];
     auto read_frag = [&](int i) {
       const int kc = i / (3 * MS), t = (i % (3 * MS)) / MS, ms = i % MS;
@@ -346,10 +352,13 @@ __device__ __forceinline__ void expert_gemm_mx_unit(const ExpertGemmMxArgs& a, c
       const int kc = i / (3 * MS), ms = i % MS;
       if (i + kFragBufs - 1 < kFrags) read_frag(i + kFragBufs - 1);
       if constexpr (!decltype(prefetch)::value) {
-        // the last step of an odd count: nothing left to request
-      } else
+        // nothing left to request
+      } else {
+        if constexpr (decltype(scales)::value && phase < 2)
+          if (i < NG) issue_s(phase, i, sn, grp_n);
 #pragma unroll
-      for (int x = i % kHalf; x < (i < kHalf ? kPart0Items : NG); x += kHalf) issue_part(i / kHalf, x, stage_n, bn, jn);
+        for (int x = i % kHalf; x < (i < kHalf ? kPart0Items : NG); x += kHalf) issue_part(i / kHalf, x, stage_n, bn, jn);
+      }
       __builtin_amdgcn_sched_barrier(0);
       // FP6 reads the first six registers; fhi[2] (register 6) is the term's scale byte
       i32x8 aw = (i32x8)__builtin_shufflevector(flo[i % kFragBufs], fhi[i % kFragBufs], 0, 1, 2, 3, 4, 5, 6, 7);
@@ -362,21 +371,24 @@ __device__ __forceinline__ void expert_gemm_mx_unit(const ExpertGemmMxArgs& a, c
         // FP4 reads four registers
         const i32x8 bw = (i32x8)__builtin_shufflevector(b.q[kc][g], b.q[kc][g], 0, 1, 2, 3, -1, -1, -1, -1);
         acc[ms][g] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(aw, bw, acc[ms][g], 2, 4, 0,
-                                                                     aw[6], 0, (int)b.s[kc][g]);
+                                                                     aw[6], phase, (int)sc.w[kc][g]);
       }
       __builtin_amdgcn_sched_barrier(0);
     }
   };
 
-  // Loads one (or two) steps ahead.  The step boundary is an explicit
+  // Loads one (or three) steps ahead.  The step boundary is an explicit
   // wait + bare barrier: the first part of what this wave requested for step j (during step
-  // j - kLead) has landed once at most the 2 NG loads of the second part and what was
+  // j - kLead) has landed once at most the NG loads of the second part and what was
   // requested for later steps are still in flight,
   // and the barrier extends that to the other waves' parts of the activation tile and tells
-  // that every wave is done reading the stage about to be overwritten.
-  constexpr int kInFlight = 2 * NG + (kLead - 1) * (kCopies + 4 * NG);
-  constexpr int kWaitStep = (kInFlight & 15) | (7 << 4) | (15 << 8) | ((kInFlight >> 4) << 14);
-  constexpr int kWaitLast = 2 * NG | (7 << 4) | (15 << 8);  // nothing was requested for a step after the last one
+  // that every wave is done reading the stage about to be overwritten.  (Scale bytes are not counted: where some of them
+  // are in flight as well the wait is for more than it has to be.)
+  constexpr int kSet = kCopies + 2 * NG;  // loads of a step, apart from scale bytes
+  auto wait_for = [](auto sets) {  // all but the second part of the step's own and what was requested for `sets` later ones
+    constexpr int n = NG + decltype(sets)::value * kSet;
+    __builtin_amdgcn_s_waitcnt((n & 15) | (7 << 4) | (15 << 8) | ((n >> 4) << 14));
+  };
   // First step: the biases (unconditional, the row clamped: what belongs to rows past N is
   // dropped), then the activation tile and the weights in the order of the steady state.  Behind
   // the operands, each under its own branch, the biases were four full waits in a row (20b shape, 2048
@@ -388,6 +400,10 @@ __device__ __forceinline__ void expert_gemm_mx_unit(const ExpertGemmMxArgs& a, c
     bias0[g] = as_global(bias)[min(group_tile(g) * 16 + n32, a.N - 1)];
   }
   BSet bs[kStages];
+#pragma unroll
+  for (int kc = 0; kc < 2; ++kc)
+#pragma unroll
+    for (int g = 0; g < NG; ++g) issue_s(kc, g, sn, 0);
 #pragma unroll
   for (int u = 0; u < kLead; ++u) {
 #pragma unroll
@@ -416,37 +432,51 @@ __device__ __forceinline__ void expert_gemm_mx_unit(const ExpertGemmMxArgs& a, c
     for (int g = 0; g < NG; ++g) asm volatile("" : "+a"(acc[ms][g]));
 
   {
-    auto step = [&](int u, int jj, auto prefetch, auto last) {
-      __builtin_amdgcn_s_waitcnt(decltype(last)::value ? kWaitLast : kWaitStep);
+    // `sets`: steps after this one whose loads may be in flight; `prefetch`, `scales`: whether it requests those of the
+    // step kLead further on, and scale bytes of the next four steps.  Four steps to the loop's body, what is left
+    // of them behind it: one loop body and one back edge (with an exit in the middle the compiler's wait-count pass loses
+    // track and drains the load queue before the first fragment reads of every step), and behind it a pair and a single
+    // step, each under one condition (as a case for each number of steps left the accumulators are spilled).  The last step
+    // requests nothing: weights that nobody reads would be dropped by the compiler, and the waits count them.
+    int j = 0;
+    auto step = [&](auto phase_t, auto sets, auto prefetch, auto scales) {
+      constexpr int phase = decltype(phase_t)::value, u = phase % kStages, un = (u + kLead) % kStages;
+      wait_for(sets);
       __builtin_amdgcn_s_barrier();
       __builtin_amdgcn_sched_barrier(0);
-      const int un = (u + kLead) % kStages;
-      compute(bs[u], u, bs[un], un, min(jj + kLead, nsteps - 1), prefetch);
+      if constexpr (phase == 0) sc = sn;
+      compute(bs[u], u, bs[un], un, min(j + phase + kLead, nsteps - 1), min((j >> 2) + 1, sgroups - 1), phase_t, prefetch, scales);
       __builtin_amdgcn_sched_barrier(0);
     };
-    // Steps in pairs (the two register sets and LDS stages alternate), the last step of an
-    // odd count on its own and without requests for a step after it.  One loop body and one
-    // back edge: with an exit in the middle of the body the compiler's wait-count pass
-    // loses track across the two exits and drains the load queue before the first fragment
-    // reads of every step.
-    // (With three stages: in threes, and one or two last steps.)
-    int j = 0;
-    for (; j + kStages - 1 < nsteps; j += kStages) {
-      step(0, j, std::true_type{}, std::false_type{});
-      step(1, j + 1, std::true_type{}, std::false_type{});
-      if constexpr (kStages == 3) step(2, j + 2, std::true_type{}, std::false_type{});
+    using Yes = std::true_type;
+    using No = std::false_type;
+    using P0 = std::integral_constant<int, 0>;
+    using P1 = std::integral_constant<int, 1>;
+    using P2 = std::integral_constant<int, 2>;
+    using P3 = std::integral_constant<int, 3>;
+    using Ahead = std::integral_constant<int, kLead - 1>;
+    for (; j + 3 < nsteps; j += 4) {
+      step(P0{}, Ahead{}, Yes{}, Yes{});
+      step(P1{}, Ahead{}, Yes{}, Yes{});
+      step(P2{}, Ahead{}, Yes{}, Yes{});
+      step(P3{}, Ahead{}, Yes{}, Yes{});
     }
-    // (none of the steps left over requests anything: weights that nobody reads would be dropped
-    // by the compiler, and the waits count them)
-    if constexpr (kStages == 3) {
-      if (j + 1 < nsteps) {
-        step(0, j, std::false_type{}, std::false_type{});
-        step(1, j + 1, std::false_type{}, std::true_type{});
-      } else if (j < nsteps) {
-        step(0, j, std::false_type{}, std::true_type{});
-      }
-    } else {
-      if (j < nsteps) step(0, j, std::false_type{}, std::true_type{});
+    using More = std::integral_constant<bool, kLead == 1>;  // (with a longer lead all of them have been requested)
+    const bool two = ((nsteps - j) & 2) != 0, one = ((nsteps - j) & 1) != 0;
+    if (two) {
+      step(P0{}, Ahead{}, More{}, No{});
+      step(P1{}, std::integral_constant<int, kLead == 1 ? 0 : 1>{}, More{}, No{});
+    }
+    if constexpr (kStages == 4) {
+      if (two && one) step(P2{}, P0{}, No{}, No{});
+      if (!two && one) step(P0{}, P0{}, No{}, No{});
+    } else if (one) {
+      // the third step of four or the first: one copy of it, its scale bytes in place 0
+#pragma unroll
+      for (int kc = 0; kc < 2; ++kc)
+#pragma unroll
+        for (int g = 0; g < NG; ++g) sn.w[kc][g] = two ? sc.w[kc][g] >> 16 : sn.w[kc][g];
+      step(P0{}, P0{}, No{}, No{});
     }
   }
   // the copies requested past the last step are still in flight: nothing may reuse their LDS before they land

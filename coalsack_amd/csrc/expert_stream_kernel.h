@@ -239,12 +239,13 @@ __global__ __launch_bounds__(256, 2) void expert_stream_kernel(ExpertStreamArgs 
     }
   }
 
-  // a lane's scale bytes of one tile: 8 (up to 8 steps per wave) or 16 (scale_slots)
-  constexpr int kScWords = NS <= 8 ? 2 : 4;
-  typedef uint32_t ScaleCell __attribute__((ext_vector_type(kScWords)));
+  // a lane's scale bytes of one tile: 2, 4, 8 or 16, one per step of the wave rounded up (scale_slots)
+  constexpr int kScWords = NS <= 4 ? 1 : NS <= 8 ? 2 : 4;
+  typedef uint32_t ScaleWords __attribute__((ext_vector_type(kScWords)));
+  using ScaleCell = std::conditional_t<NS == 2, uint16_t, ScaleWords>;
   struct WSet {
     u32x4 q[ND][NT];
-    ScaleCell sc[NT];  // this wave's scale bytes of the tiles, one byte per K step
+    ScaleWords sc[NT];  // this wave's scale bytes of the tiles, one byte per K step
     float b[NT];
   };
 
@@ -298,7 +299,8 @@ __global__ __launch_bounds__(256, 2) void expert_stream_kernel(ExpertStreamArgs 
 #pragma unroll
       for (int m = 0; m < NT; ++m) {
         const int t = tile_of(unit, m);
-        ws.sc[m] = (m < TU ? s0 : s1)[(size_t)t * 256];
+        if constexpr (NS == 2) ws.sc[m][0] = (m < TU ? s0 : s1)[(size_t)t * 256];
+        else ws.sc[m] = (m < TU ? s0 : s1)[(size_t)t * 256];
         ws.b[m] = (m < TU ? bp0 : bp1)[min(t * 16 + n, a.N - 1)];  // bias pointers are never null (absent bias = zero vector)
       }
     };
@@ -406,11 +408,17 @@ __global__ __launch_bounds__(256, 2) void expert_stream_kernel(ExpertStreamArgs 
     auto compute_unit = [&](WSet& ws, int unit, int next) {
       const bool idle = next == unit;
       float bias[NT];
-      ScaleCell scb[NT];
+      uint32_t scb[NT][kScWords];
 #pragma unroll
-      for (int m = 0; m < NT; ++m) bias[m] = ws.b[m], scb[m] = ws.sc[m];
+      for (int m = 0; m < NT; ++m) {
+        bias[m] = ws.b[m];
+        asm volatile("" : "+v"(bias[m]));  // (copied before they are overwritten)
 #pragma unroll
-      for (int m = 0; m < NT; ++m) asm volatile("" : "+v"(bias[m]), "+v"(scb[m]));  // (copied before they are overwritten)
+        for (int w = 0; w < kScWords; ++w) {
+          scb[m][w] = ws.sc[m][w];
+          asm volatile("" : "+v"(scb[m][w]));
+        }
+      }
       // in front of the weights: a unit's first matrix instruction needs its scale bytes, and
       // loads retire in order
       load_unit_scalars(ws, next);

@@ -47,6 +47,12 @@ __device__ __forceinline__ void entry_to_ref_block(uint4 q, uint8_t scale, uint8
   for (int j = 0; j < 16; ++j) blk[1 + j] = (uint8_t)(code[j] | (code[j + 16] << 4));
 }
 
+// A block's scale byte in both scale planes of its matrix (entries = ntile * nblk * 16).
+__device__ __forceinline__ void put_scale_byte(uint8_t* s, long entries, long tile, int kb, int n, int nblk, uint8_t v) {
+  s[scale_index(tile, kb, n, scale_slots(nblk))] = v;
+  s[step_scale_plane(entries / (16 * nblk), nblk) + step_scale_index(tile, kb, n, step_scale_groups(nblk))] = v;
+}
+
 // Every code of the entry is 0 or 0.5 in magnitude (E2M1 codes 0, 1, 8, 9).
 __device__ __forceinline__ bool entry_below_one(const uint4& e) {
   return ((e.x | e.y | e.z | e.w) & 0x66666666u) == 0u;
@@ -75,10 +81,10 @@ __global__ void pack_mxfp4_kernel(const uint8_t* __restrict__ src, uint4* __rest
   const int kb = (int)(tk % nblk);
   const long tile = tk / nblk;
   const long row = tile * 16 + n;
-  const size_t si = scale_index(tile, kb, n, scale_slots(nblk));
+  auto put_scale = [&](uint8_t v) { put_scale_byte(s, entries, tile, kb, n, nblk, v); };
   if (row >= rows) {
     q[i] = make_uint4(0, 0, 0, 0);
-    s[si] = 127;
+    put_scale(127);
     return;
   }
   const uint8_t* blk = src + (row * nblk + kb) * 17;
@@ -93,7 +99,7 @@ __global__ void pack_mxfp4_kernel(const uint8_t* __restrict__ src, uint4* __rest
     }
   }
   q[i] = e;
-  s[si] = sb;
+  put_scale(sb);
 }
 
 __global__ void export_mxfp4_kernel(const uint4* __restrict__ q, const uint8_t* __restrict__ s,
@@ -185,10 +191,10 @@ __global__ void synth_mxfp4_kernel(uint4* __restrict__ q, uint8_t* __restrict__ 
   const int kb = (int)(tk % nblk);
   const long tile = tk / nblk;
   const long row = tile * 16 + n;
-  const size_t si = scale_index(tile, kb, n, scale_slots(nblk));
+  auto put_scale = [&](uint8_t v) { put_scale_byte(s, entries, tile, kb, n, nblk, v); };
   if (row >= rows) {
     q[i] = make_uint4(0, 0, 0, 0);
-    s[si] = 127;
+    put_scale(127);
     return;
   }
   const uint64_t b = (uint64_t)(row * nblk + kb);
@@ -201,7 +207,7 @@ __global__ void synth_mxfp4_kernel(uint4* __restrict__ q, uint8_t* __restrict__ 
     blk[9 + j] = (uint8_t)(h2 >> (8 * j));
   }
   q[i] = ref_block_to_entry(blk);
-  s[si] = blk[0];
+  put_scale(blk[0]);
 }
 
 }  // namespace csk

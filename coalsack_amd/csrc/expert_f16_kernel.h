@@ -600,6 +600,14 @@ struct F16GemmLds {
   float rs[64];
 };
 
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t f16_out_rsrc(float* p, uint32_t bytes) {
+  const uint64_t v = reinterpret_cast<uint64_t>(p);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
+  return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<char*>(((uint64_t)hi << 32) | lo), 0,
+                                           __builtin_amdgcn_readfirstlane((int)bytes), 0x00020000);
+}
+
 // One work unit: MS = 2 for M tiles of more than 32 tokens, MS = 1 for those of at most 32 (the
 // ragged end of an expert's list), which cost half the matrix instructions and half the panel.  NS: groups of 32 weight
 // rows per wave (of gate and of up; one or two of down).
@@ -766,22 +774,30 @@ __device__ __forceinline__ void expert_f16_gemm_unit(const ExpertF16GemmArgs& a,
     rv[s] = rows[s] < a.N;
     bias[s] = rv[s] ? (s == 0 ? b0 : b1)[rows[s]] : 0.0f;
   }
+  // The descriptor spans this unit's rows and no more: what belongs to tokens past the tile is out of its range and dropped,
+  // and so is what belongs to weight rows past N, whose offset is moved there (a comparison, a branch and a 64-bit address
+  // for each value before: 32 experts of 2880 x 2880, top-4, 1000 tokens 604 / now 599 us per layer).
+  const uint32_t pitch = (uint32_t)a.N * 4u;
+  const auto out_rsrc = f16_out_rsrc(a.out + (long)base * a.N, (uint32_t)mcount * pitch);
+  uint32_t at[NS];
+#pragma unroll
+  for (int s = 0; s < NS; ++s) at[s] = rv[s] ? 4u * kg * pitch + 4u * (uint32_t)rows[s] : 0x80000000u;
 #pragma unroll
   for (int ms = 0; ms < MS; ++ms) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      const int tl = ms * 32 + (r & 3) + 8 * (r >> 2) + 4 * kg;
-      if (tl >= mcount) continue;
-      const float sc_t = rs_sh[tl] * a.wscale[0];
-      float* o = a.out + (long)(base + tl) * a.N;
+      const int t = ms * 32 + (r & 3) + 8 * (r >> 2);
+      const uint32_t row_off = (uint32_t)t * pitch;
+      const float rs = rs_sh[t + 4 * kg];
+      const float sc_t = rs * a.wscale[0];
       if (MODE == 0) {
-        const float sc_u = rs_sh[tl] * a.wscale[1];
-        if (rv[0])
-          o[rows[0]] = moe_activation(acc[ms][0][r] * sc_t + bias[0], acc[ms][NS - 1][r] * sc_u + bias[NS - 1], a.act_type);
+        const float sc_u = rs * a.wscale[1];
+        const float v = moe_activation(acc[ms][0][r] * sc_t + bias[0], acc[ms][NS - 1][r] * sc_u + bias[NS - 1], a.act_type);
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), out_rsrc, at[0] + row_off, 0, 0);
       } else {
 #pragma unroll
         for (int s = 0; s < NS; ++s)
-          if (rv[s]) o[rows[s]] = acc[ms][s][r] * sc_t + bias[s];
+          __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc[ms][s][r] * sc_t + bias[s]), out_rsrc, at[s] + row_off, 0, 0);
       }
     }
   }

@@ -532,18 +532,25 @@ __device__ __forceinline__ void expert_gemm_mx_unit(const ExpertGemmMxArgs& a, c
     __syncthreads();
     store_rows();
   } else {
+    // The descriptor spans this unit's rows of y and no more: what belongs to tokens past the tile is out of its range and
+    // dropped, and so is what belongs to rows past N, whose offset is moved there: an addition and a store per value, where a
+    // comparison, a branch and a 64-bit product for each took (us per layer, 2880 x 2880, top-4) 32 experts 2048 tokens 411 /
+    // now 404, 128 experts 300 tokens 365 / 359, 4096 890 / 878.  Stores past the caches (non-temporal, or written through)
+    // change nothing.
+    const uint32_t pitch = (uint32_t)a.N * 4u;
+    const auto y_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<char*>(uniform_ptr(reinterpret_cast<const char*>(a.y_out + (size_t)base * (size_t)a.N))), 0,
+        __builtin_amdgcn_readfirstlane((int)((uint32_t)mcount * pitch)), 0x00020000);
 #pragma unroll
     for (int g = 0; g < NG; ++g) {
       const int row = group_tile(g) * 16 + n32;
-      if (row >= a.N) continue;
+      const uint32_t at = row < a.N ? 4u * kg * pitch + 4u * (uint32_t)row : 0x80000000u;
 #pragma unroll
       for (int ms = 0; ms < MS; ++ms) {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int tl = ms * 32 + (r & 3) + 8 * (r >> 2) + 4 * kg;
-          if (tl >= mcount) continue;
-          a.y_out[(size_t)(base + tl) * (size_t)a.N + row] = acc[ms][g][r];
-        }
+        for (int r = 0; r < 16; ++r)
+          __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc[ms][g][r]), y_rsrc,
+                                                at + (uint32_t)(ms * 32 + (r & 3) + 8 * (r >> 2)) * pitch, 0, 0);
       }
     }
   }

@@ -116,7 +116,7 @@ int fill_words(void* p, size_t bytes, uint32_t v) {
 constexpr uint32_t kScalesOfOne = 0x7f7f7f7f;  // four E8M0 bytes
 
 // Above this many token-expert assignments the token-group list of the
-// weight-streaming kernel is not built.
+// weight-streaming kernels is not built.
 constexpr int64_t kStreamMaxP = 2048;
 constexpr size_t kWeightSlack = 32768;  // bytes of mapped memory kept behind weight planes (the expert kernels read whole K steps: up to three blocks, 768 bytes, past the last tile)
 constexpr int kStreamWgPerCu = 2;  // resident workgroups of the streaming kernel per compute unit ...
@@ -590,49 +590,59 @@ int launch_mx3(const float* x, uint16_t* x3, int64_t rows, int64_t H, const int*
   return check_launch("mx3_rows_kernel");
 }
 
-// Tokens of an expert contracted per pass over its weights by the streaming kernel.  An
-// expert with more tokens than that is streamed once per group, so larger batches take
-// as many as two workgroups per compute unit can hold in LDS at the longer of the two row
-// lengths (seven at K = 2880, measured against six: 20b T = 64 162 -> 151 us, 120b T = 64
-// 245 -> 239 us); up to 16 tokens few experts see more than four, the second pass of those
-// that do is served by the memory-side cache, and the four-token form is marginally the
-// faster one (measured at T = 8, 16, 32).
-inline int stream_group_tokens(int64_t T, int64_t H, int64_t F) {
-  if (T == 1) return 1;
-  if (T <= 16) return kStreamG;
-  const int ns = std::max(stream_steps((int)(H / 32)), stream_steps((int)(F / 32)));
-  return ns <= 3 ? 12 : ns <= 5 ? 8 : ns == 6 ? 7 : ns == 8 ? 5 : kStreamG;
-}
+// The kernels of a batch, one decision per forward: it fixes the activation format of both projections and whether the
+// dispatch lists token groups or M tiles.
+//   kPasses  expert_stream_kernel: groups of up to four tokens, fp32 rows, weights in pieces of 24 to 49 KB
+//   kTiles   expert_stream_kernel_tiles: groups of up to 64 tokens on the grouped GEMM's low tile, rows as FP6 terms
+//   kGemm    expert_gemm_mx_kernel: M tiles of 64 tokens, in the order of the experts' lists
+enum class ExpertPath { kPasses, kTiles, kGemm };
+inline int group_tokens(ExpertPath path, int64_t T) { return path == ExpertPath::kPasses ? (int)std::min<int64_t>(T, kStreamG) : kGemmBM; }
 
-// Small batches stream the weights (HBM-bound, activations quantised in the kernel); larger
-// ones run the grouped GEMM on the block-scaled matrix instruction (three-term FP6
-// activations).  One decision per forward: it fixes the activation format of both GEMMs.
-// The GEMM passes over an expert once per 64 of its tokens but has about 25 us more of
-// latency in front and behind; the streaming kernel passes over it once per token group, so
-// what counts is how many bytes are streamed again by second and further passes.  Both move
-// about 5 TB/s, hence the line at 120 MB of repeated weights.  Measured (layer, us, streaming
-// / GEMM), m assignments per expert: 128 x 2880 x 2880 (1.7 GB) m = 2 308 / 350, 4 400 / 396,
-// 8 505 / 409; 32 experts of it m = 6 124 / 124, 8 141 / 125; 8 experts m = 4 50 / 66, 12 70 / 69,
-// 16 75 / 70; 16 x 4096 x 6144 (0.6 GB, groups of four) m = 4 164 / 164, 6 207 / 165.  Tokens per
-// expert are taken as Poisson distributed about m, except that none can have more than T: up to one
-// pass of tokens the weights are streamed once whatever their size (8 x 4096 x 8192, top-8, one token 90 / 121;
-// 8 x 6144 x 8192, top-8, four tokens 149 / 184).  (The exact distribution beyond that, binomial, moves calls
-// across the line both ways: 64 x 5120 x 6144, top-4, 30 tokens 485 / 656 to the streaming side, but
-// 16 x 2048 x 5120, top-2, 34 tokens 103 / 92 as well.)
-bool stream_path(int64_t T, int64_t H, int64_t F, int64_t E, int64_t k) {
-  if (H / 32 > kStreamMaxBlocks || F / 32 > kStreamMaxBlocks || T * k > kStreamMaxP) return false;
-  const int g = stream_group_tokens(T, H, F);
-  if (T <= g) return true;  // no expert holds more than T tokens: one pass each
-  const double m = std::min((double)(T * k) / (double)E, (double)T);
-  if (T > 64 && m > g) return false;  // two passes and more, however small the matrices
-  double again = 0.0;  // expected passes per expert beyond the first
-  double p = std::exp(-m), above = 1.0 - p;  // P(n), P(more than n); m is at most 64 here
+// Expected passes beyond the first over the weights of an expert, in groups of g of its m tokens (Poisson distributed).
+double passes_again(double m, int g) {
+  double again = 0.0, p = std::exp(-m), above = 1.0 - p;  // P(n), P(more than n)
   for (int n = 1; above > 1e-4; ++n) {
     p *= m / n;
     above -= p;
     if (n % g == 0) again += std::max(above, 0.0);
   }
-  return again * (double)(E * 3 * H * F) * (17.0 / 32.0) <= 120e6;
+  return again;
+}
+
+// Batches whose token groups are listed, as opposed to the M tiles of the experts: as many as repeat at most 120 MB of weights
+// in groups of what two workgroups per compute unit could hold the rows of.  Up to one group of tokens the weights are
+// streamed once whatever their size.  On the far side the GEMM's low tile does the same work from the other list (128
+// experts of 2880 x 2880, 96 tokens, groups / M tiles 317 / 316 us per layer; 32 of them, 48 tokens 108 / 107), and with more tokens
+// its tall tile.
+bool stream_path(int64_t T, int64_t H, int64_t F, int64_t E, int64_t k) {
+  if (H / 32 > kStreamMaxBlocks || F / 32 > kStreamMaxBlocks || T * k > kStreamMaxP) return false;
+  const int ns = std::max(stream_steps((int)(H / 32)), stream_steps((int)(F / 32)));
+  const int g = T <= 16 ? kStreamG : ns <= 3 ? 12 : ns <= 5 ? 8 : ns == 6 ? 7 : ns == 8 ? 5 : kStreamG;
+  if (T <= g) return true;  // no expert holds more than T tokens: one pass each
+  const double m = std::min((double)(T * k) / (double)E, (double)T);
+  if (T > 64 && m > g) return false;  // two passes and more, however small the matrices
+  return passes_again(m, g) * (double)(E * 3 * H * F) * (17.0 / 32.0) <= 120e6;  // m is at most 64 here
+}
+
+// Passes of four tokens against tiles (us per layer, measured both ways), m assignments per expert: 128 experts of 2880 x 2880,
+// top-4, 8 tokens 93 / 98, 16 141 / 148, 32 (m = 1) 230 / 225, 64 309 / 295; 32 of them 8 tokens 75 / 76, 12 83 / 90, 16 (m = 2)
+// 92 / 94, 24 105 / 99, 48 120 / 107; 8 of them 8 tokens (m = 4) 47 / 39; 16 of 4096 x 6144, top-2, 6 tokens 86 / 87, 16 (m = 2)
+// 119 / 115, 24 144 / 126; 64 of 2048 x 768, top-8, 16 tokens (m = 2) 52 / 53, 32 66 / 63, 50 67 / 61; one expert of 2880 x 2880, 8
+// tokens 29 / 33, 12 34 / 34.  A tile's units are 200 to 400 KB, so with few of them per compute unit the last round weighs: 64
+// of 3072 x 1536, top-4, 17 tokens (2.0 per compute unit expected, some get three) 88 / 98; 16 of 4096 x 4096, top-1, 17
+// tokens (1.3) 63 / 67, 32 tokens (1.7) 87 / 81.  Over 220 layers drawn at random, 2 to 160 tokens, these lines lose 1 %
+// against the better of the two, the line at 120 MB alone 3.3.  With the routing weight in front, tiles need a launch more for the
+// gathered rows, about as long as 40 MB of weights (16 of 3328 x 544, top-2, 19 tokens 76 / 83).
+ExpertPath expert_path(int64_t T, int64_t H, int64_t F, int64_t E, int64_t k, bool weight_first) {
+  if (!stream_path(T, H, F, E, k)) return ExpertPath::kGemm;
+  if (T <= kStreamG) return ExpertPath::kPasses;
+  const double m = std::min((double)(T * k) / (double)E, (double)T);
+  const double again = passes_again(m, kStreamG) * (double)(E * 3 * H * F) * (17.0 / 32.0);
+  if (weight_first) return again <= 40e6 ? ExpertPath::kPasses : ExpertPath::kTiles;
+  if (T <= 16) return m < 3.0 || again <= 19e6 ? ExpertPath::kPasses : ExpertPath::kTiles;
+  const double active = (double)E * (1.0 - std::pow(1.0 - std::min(1.0, (double)k / (double)E), (double)T));
+  const double per_cu = active * (double)cdiv(F, 128) / std::max(g_cus, 1);
+  return m < 0.75 || (m < 1.5 && per_cu < 0.8 * std::ceil(per_cu)) ? ExpertPath::kPasses : ExpertPath::kTiles;
 }
 
 // mx3_out: also rewrite the rows x as FP6 terms (the grouped GEMM's operand), riding on the
@@ -689,53 +699,63 @@ int launch_dispatch(const int* ids, const float* pairs, int64_t P, int64_t k, in
   return check_launch("dispatch_scatter_kernel");
 }
 
-// Weight-streaming kernel for small batches (every expert sees few tokens, the
-// layer is HBM-bound); grouped GEMM otherwise.
-template <int MODE, int LG, int NS, bool ROUTE1>
+template <int MODE, int NS, bool ROUTE1>
 int launch_stream_form(ExpertStreamArgs a, int64_t P) {
   // kStreamWgPerCu workgroups per compute unit in steady state (one where the rows of a
   // group take more than half of the LDS); a batch so small that every work unit can have a
   // resident workgroup of its own gets that
   constexpr int TU = MODE == 0 ? stream_tiles(NS) / 2 : stream_tiles(NS);
-  size_t lds = stream_lds_bytes(NS, LG, a.group_tokens);
+  size_t lds = stream_lds_bytes(NS, a.group_tokens);
   if (ROUTE1) lds = std::max(lds, sizeof(CloseCallLds));  // a close call is recomputed where the rows go afterwards
   const int64_t units = cdiv(a.ntile, TU);
   const int64_t places = (lds <= kStreamLdsHalf ? kStreamWgPerCu : 1) * (int64_t)std::max(g_cus, 1);
-  const int64_t nwg = LG == 1 ? std::min(P * units, places) : places;
+  const int64_t nwg = std::min(P * units, places);
   static bool lds_attr_set = false;  // per instantiation: dynamic LDS beyond the default limit is asked for once
   if (!lds_attr_set) {
-    HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(&expert_stream_kernel<MODE, LG, NS, ROUTE1>),
+    HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(&expert_stream_kernel<MODE, NS, ROUTE1>),
                                 hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)std::max(stream_lds_bytes(NS, LG, 4 * LG), sizeof(CloseCallLds))));
+                                (int)std::max(stream_lds_bytes(NS, kStreamG), sizeof(CloseCallLds))));
     lds_attr_set = true;
   }
-  launch_expert_kernel(MODE, expert_stream_kernel<MODE, LG, NS, ROUTE1>, dim3((unsigned)nwg), dim3(256), lds, a);
+  launch_expert_kernel(MODE, expert_stream_kernel<MODE, NS, ROUTE1>, dim3((unsigned)nwg), dim3(256), lds, a);
   return check_launch("expert_stream_kernel");
 }
-template <int MODE, int LG, bool ROUTE1 = false>
+template <int MODE, bool ROUTE1 = false>
 int launch_stream_steps(const ExpertStreamArgs& a, int64_t P) {
   switch (stream_steps(a.nblk)) {
-    case 2: return launch_stream_form<MODE, LG, 2, ROUTE1>(a, P);
-    case 3: return launch_stream_form<MODE, LG, 3, ROUTE1>(a, P);
-    // the longer rows come in smaller groups (stream_group_tokens)
-    case 4: if constexpr (LG <= 2) return launch_stream_form<MODE, LG, 4, ROUTE1>(a, P); break;
-    case 5: if constexpr (LG <= 2) return launch_stream_form<MODE, LG, 5, ROUTE1>(a, P); break;
-    case 6: if constexpr (LG <= 2) return launch_stream_form<MODE, LG, 6, ROUTE1>(a, P); break;
-    case 8: if constexpr (LG <= 2) return launch_stream_form<MODE, LG, 8, ROUTE1>(a, P); break;
-    case 12: if constexpr (LG <= 1) return launch_stream_form<MODE, LG, 12, ROUTE1>(a, P); break;
-    case 16: if constexpr (LG <= 1) return launch_stream_form<MODE, LG, 16, ROUTE1>(a, P); break;
+    case 2: return launch_stream_form<MODE, 2, ROUTE1>(a, P);
+    case 3: return launch_stream_form<MODE, 3, ROUTE1>(a, P);
+    case 4: return launch_stream_form<MODE, 4, ROUTE1>(a, P);
+    case 5: return launch_stream_form<MODE, 5, ROUTE1>(a, P);
+    case 6: return launch_stream_form<MODE, 6, ROUTE1>(a, P);
+    case 8: return launch_stream_form<MODE, 8, ROUTE1>(a, P);
+    case 12: return launch_stream_form<MODE, 12, ROUTE1>(a, P);
+    default: return launch_stream_form<MODE, 16, ROUTE1>(a, P);
   }
-  return fail(CSK_ERR_STATE, "expert_stream_kernel: token groups too large for these rows");
 }
 template <int MODE>
 int launch_stream(ExpertStreamArgs a, int64_t P, Workspace& ws) {
   a.groups = ws.groups;
   a.nv = ws.nv;
   if constexpr (MODE == 0)
-    if (a.rin.logits) return launch_stream_steps<MODE, 1, true>(a, P);  // one token, routed by the kernel itself
-  return a.group_tokens <= 4 ? launch_stream_steps<MODE, 1>(a, P)
-         : a.group_tokens <= 8 ? launch_stream_steps<MODE, 2>(a, P)
-                               : launch_stream_steps<MODE, 3>(a, P);
+    if (a.rin.logits) return launch_stream_steps<MODE, true>(a, P);  // one token, routed by the kernel itself
+  return launch_stream_steps<MODE>(a, P);
+}
+
+template <int MODE>
+int launch_tiles(ExpertGemmMxArgs& ga, int64_t E, int64_t P) {
+  using Geom = MxGeom<2, 2>;
+  ga.n_ntiles = (int)cdiv(ga.ntile, Geom::tiles_per_wg(MODE));
+  static bool lds_attr_set = false;
+  if (!lds_attr_set) {
+    HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(&expert_stream_kernel_tiles<MODE>),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)Geom::kLdsBytes));
+    lds_attr_set = true;
+  }
+  const int64_t max_groups = P / kGemmBM + std::min<int64_t>(E, P);
+  const dim3 grid((unsigned)(cdiv(max_groups * ga.n_ntiles, kDies) * kDies));
+  launch_expert_kernel(MODE, expert_stream_kernel_tiles<MODE>, grid, dim3(64 * kMxWaves), Geom::kLdsBytes, ga);
+  return check_launch("expert_stream_kernel_tiles");
 }
 
 // Weight rows per work unit of the grouped GEMM: 512, or 256 where that many leave the chip
@@ -770,12 +790,14 @@ int launch_gemm_mx(ExpertGemmMxArgs& ga, int64_t E, int64_t P) {
 
 template <int NMAT>
 int launch_experts(ExpertStreamArgs a, const uint16_t* a_mx3, uint16_t* act_mx3, int64_t E, int64_t T, int64_t P,
-                   Workspace& ws, bool stream) {
-  if (stream) return launch_stream<NMAT == 2 ? 0 : 1>(a, P, ws);
+                   Workspace& ws, ExpertPath path) {
+  if (path == ExpertPath::kPasses) return launch_stream<NMAT == 2 ? 0 : 1>(a, P, ws);
   ExpertGemmMxArgs ga{};
   ga.desc = a.desc;
   ga.mtiles = ws.tiles;
   ga.n_mtiles = ws.n_tiles;
+  ga.groups = ws.groups;
+  ga.n_groups = ws.nv;
   ga.list_row = a.list_row;
   ga.A = reinterpret_cast<const uint4*>(a_mx3);
   ga.nblk = a.nblk;
@@ -790,6 +812,7 @@ int launch_experts(ExpertStreamArgs a, const uint16_t* a_mx3, uint16_t* act_mx3,
   if (a_rows * mx3_row_blocks(a.nblk) * 96 >= ((int64_t)1 << 32))
     return fail(CSK_ERR_ARG, "batch too large for the grouped GEMM (activation rows exceed 4 GiB)");
   constexpr int kMode = NMAT == 2 ? 0 : 1;
+  if (path == ExpertPath::kTiles) return launch_tiles<kMode>(ga, E, P);
   return gemm_wide_tiles(E, P, a.ntile) ? launch_gemm_mx<kMode, kMxNG>(ga, E, P) : launch_gemm_mx<kMode, kMxNG / 2>(ga, E, P);
 }
 
@@ -810,19 +833,20 @@ struct ExpertInput {
 
 // Experts' MLPs over the dispatched tokens: ws.y[P,H] <- down(act(gate, up)).
 int run_experts(int64_t E, int64_t T, int64_t k, int64_t H, int64_t F,
-                int act_type, const ExpertInput& in, Workspace& ws, bool stream, bool timed = false) {
+                int act_type, const ExpertInput& in, Workspace& ws, ExpertPath path, bool timed = false) {
   const int64_t P = T * k;
+  const bool passes = path == ExpertPath::kPasses;
   ExpertStreamArgs a{};
   a.desc = ws.desc;
   a.act_type = act_type;
-  a.group_tokens = stream_group_tokens(T, H, F);
+  a.group_tokens = group_tokens(path, T);
   // a single token of a routed layer names k different experts: k token groups, known here
-  a.nv_known = (stream && T == 1 && E > 1) ? (int)k : 0;
+  a.nv_known = (passes && T == 1 && E > 1) ? (int)k : 0;
   // gate/up + activation
-  a.list_row = stream ? in.list_row : in.mx3_list_row;
+  a.list_row = passes ? in.list_row : in.mx3_list_row;
   a.gather_w = in.gather_w;
   a.X = in.x;
-  a.X3 = stream ? reinterpret_cast<const u32x4*>(in.x_mx3_tokens) : nullptr;
+  a.X3 = passes ? reinterpret_cast<const u32x4*>(in.x_mx3_tokens) : nullptr;
   a.zeros = g_zero;
   a.nblk = (int)(H / 32);
   a.N = (int)F;
@@ -831,10 +855,10 @@ int run_experts(int64_t E, int64_t T, int64_t k, int64_t H, int64_t F,
   a.y_out = nullptr;
   if (timed) mark(CSK_STAGE_GATEUP);
   if (in.rin && in.rout) {
-    if (!stream || T != 1) return fail(CSK_ERR_STATE, "in-kernel routing is for one token on the streaming path");
+    if (!passes || T != 1) return fail(CSK_ERR_STATE, "in-kernel routing is for one token on the streaming path");
     a.rin = *in.rin, a.rout = *in.rout;
   }
-  int rc = launch_experts<2>(a, in.x_mx3, ws.act, E, T, P, ws, stream);
+  int rc = launch_experts<2>(a, in.x_mx3, ws.act, E, T, P, ws, path);
   if (rc != CSK_OK) return rc;
   a.rin = RouteIn{}, a.rout = RouteOut{};
   if (timed) mark(CSK_STAGE_DOWN);
@@ -848,7 +872,7 @@ int run_experts(int64_t E, int64_t T, int64_t k, int64_t H, int64_t F,
   a.ntile = (int)cdiv(H, 16);
   a.act_out = nullptr;
   a.y_out = ws.y;
-  return launch_experts<1>(a, ws.act, nullptr, E, T, P, ws, stream);
+  return launch_experts<1>(a, ws.act, nullptr, E, T, P, ws, path);
 }
 
 int launch_combine(const float* y, const float* pairs, const int* pos, const float* residual,
@@ -1180,7 +1204,7 @@ extern "C" int csk_mxfp4_upload(const uint8_t* blocks, int64_t rows, int64_t K, 
   m->ntile = cdiv(rows, 16);
   int rc = dev_alloc(&m->q, (size_t)m->entries() + kWeightSlack / sizeof(uint4));
   if (rc == CSK_OK) rc = dev_alloc(&m->s, (size_t)m->scale_bytes() + kWeightSlack);
-  if (rc == CSK_OK) rc = fill_words(m->s, (size_t)m->scale_bytes(), kScalesOfOne);
+  if (rc == CSK_OK) rc = fill_words(m->s, (size_t)m->scale_bytes() + kWeightSlack, kScalesOfOne);  // padding and slack
   csk_mxfp4* const ms[1] = {m};
   if (rc == CSK_OK) rc = queue_pack(&blocks, ms, 1);
   if (rc == CSK_OK) rc = finish_pack(1);
@@ -1842,7 +1866,8 @@ int forward_pass(csk_layer* L, const float* hidden, int64_t T, float* out, int f
   }
   const int64_t P = T * L->k;
   const bool norm = (flags & CSK_FWD_RMSNORM) != 0;
-  const bool stream = !L->f16 && stream_path(T, L->H, L->F, L->E, L->k);
+  const ExpertPath path = L->f16 ? ExpertPath::kGemm : expert_path(T, L->H, L->F, L->E, L->k, L->wbf != 0);
+  const bool groups = path != ExpertPath::kGemm, passes = path == ExpertPath::kPasses;
   const float* xr = norm ? ws.xn : hidden;
   bool route_in_kernel = false, rows_mx3_ready = false;
   RouteIn rin_kept{};
@@ -1874,15 +1899,15 @@ int forward_pass(csk_layer* L, const float* hidden, int64_t T, float* out, int f
     if ((rc = check_launch("router_prep_logits_kernel")) != CSK_OK) return rc;
     mark(CSK_STAGE_DISPATCH);
     RouteIn rin{ws.logits, xr, L->gate_w, L->has_gate_b ? L->gate_b : nullptr, L->ew_dev,
-                (int)T, (int)L->E, (int)L->k, (int)L->H, L->sigmoid, stream_group_tokens(T, L->H, L->F)};
+                (int)T, (int)L->E, (int)L->k, (int)L->H, L->sigmoid, group_tokens(path, T)};
     RouteOut rout{ws.pairs, ws.ids, ws.pos, ws.counts, ws.offsets, ws.desc, ws.groups, ws.nv,
                   ws.tiles, ws.n_tiles, ws.list_tok, ws.list_w};
-    if (T == 1 && phase == 0 && L->E > 1 && stream) {
+    if (T == 1 && phase == 0 && L->E > 1 && passes) {
       // one token: the gate/up kernel routes it itself (no launch here); phases keep the
       // routing kernel, whose output they hand out before the experts run
       route_in_kernel = true;
       rin_kept = rin, rout_kept = rout;
-    } else if (T <= kRouteTinyTokens && P <= kRouteTinyMaxP && stream) {
+    } else if (T <= kRouteTinyTokens && P <= kRouteTinyMaxP && passes) {
       // a handful of tokens on the streaming kernels: each active expert is one token group
       route_tiny_kernel<<<dim3(1), 256, 0, g_stream>>>(rin, rout);
       if ((rc = check_launch("route_tiny_kernel")) != CSK_OK) return rc;
@@ -1893,7 +1918,7 @@ int forward_pass(csk_layer* L, const float* hidden, int64_t T, float* out, int f
           ws.logits, ws.pairs, ws.ids, (int)T, (int)L->E, (int)L->k, L->sigmoid, xr, L->gate_w,
           L->has_gate_b ? L->gate_b : nullptr, (int)L->H, ws.logits + T * L->E, 0, Mx3Rider{});
       if ((rc = check_launch("router_topk_kernel")) != CSK_OK) return rc;
-      if ((rc = launch_dispatch(ws.ids, ws.pairs, P, L->k, L->E, L->ew_dev, ws, stream_group_tokens(T, L->H, L->F), stream)) != CSK_OK) return rc;
+      if ((rc = launch_dispatch(ws.ids, ws.pairs, P, L->k, L->E, L->ew_dev, ws, group_tokens(path, T), groups)) != CSK_OK) return rc;
     } else {
       route_small_kernel<<<dim3(1), kRouteSmallThreads, 0, g_stream>>>(rin, rout);
       if ((rc = check_launch("route_small_kernel")) != CSK_OK) return rc;
@@ -1906,13 +1931,13 @@ int forward_pass(csk_layer* L, const float* hidden, int64_t T, float* out, int f
     }
     // the rows' FP6 form for the grouped GEMM is written by extra workgroups of the top-k launch
     const bool ride = !L->f16 && !L->wbf;  // (the streaming kernels copy the rows in this form, too)
-    rows_mx3_ready = ride && stream;
+    rows_mx3_ready = ride && passes;
     mark(CSK_STAGE_ROUTER);
     rc = launch_router(xr, L->gate_w, L->has_gate_b ? L->gate_b : nullptr, T, L->E, L->H, L->k,
                        L->sigmoid, ws.logits, ws.pairs, ws.ids, ride ? ws.xs : nullptr);
     if (rc != CSK_OK) return rc;
     mark(CSK_STAGE_DISPATCH);
-    rc = launch_dispatch(ws.ids, ws.pairs, P, L->k, L->E, L->ew_dev, ws, stream_group_tokens(T, L->H, L->F), stream);
+    rc = launch_dispatch(ws.ids, ws.pairs, P, L->k, L->E, L->ew_dev, ws, group_tokens(path, T), groups);
     if (rc != CSK_OK) return rc;
   }
   if (phase == 1) return CSK_OK;
@@ -1932,12 +1957,12 @@ int forward_pass(csk_layer* L, const float* hidden, int64_t T, float* out, int f
   ExpertInput in{xr, ws.list_tok, L->wbf ? ws.list_w : nullptr, ws.xs, ws.list_tok};
   if (route_in_kernel) in.rin = &rin_kept, in.rout = &rout_kept;
   if (rows_mx3_ready) in.x_mx3_tokens = ws.xs;
-  if (L->wbf && !stream) {
+  if (L->wbf && !passes) {
     if ((rc = launch_mx3(xr, ws.xg, P, L->H, ws.list_tok, ws.list_w)) != CSK_OK) return rc;
     in.x_mx3 = ws.xg;
     in.mx3_list_row = nullptr;
   }
-  rc = run_experts(L->E, T, L->k, L->H, L->F, L->act, in, ws, stream, true);
+  rc = run_experts(L->E, T, L->k, L->H, L->F, L->act, in, ws, path, true);
   if (rc != CSK_OK) return rc;
   mark(CSK_STAGE_COMBINE);
   rc = launch_combine(ws.y, ws.pairs, ws.pos, (flags & CSK_FWD_RESIDUAL) ? hidden : nullptr, out, T,
@@ -2323,10 +2348,10 @@ extern "C" int csk_expert_mlp_mxfp4(int expert_id, const float* hidden, int64_t 
     select_expert_ids_kernel<<<dim3((unsigned)cdiv(P, 256)), 256, 0, g_stream>>>(
         up.pairs, ws.ids, (int)P, expert_id, ws.list_tok, ws.list_w);
     if ((rc = check_launch("select_expert_ids_kernel")) != CSK_OK) return rc;
-    const bool stream = stream_path(tn, H, F, 1, k);
-    if ((rc = launch_dispatch(ws.ids, up.pairs, P, k, 1, up.ew, ws, stream_group_tokens(tn, H, F), stream)) != CSK_OK) return rc;
+    const ExpertPath path = expert_path(tn, H, F, 1, k, weight_before_ffn != 0);
+    if ((rc = launch_dispatch(ws.ids, up.pairs, P, k, 1, up.ew, ws, group_tokens(path, tn), path != ExpertPath::kGemm)) != CSK_OK) return rc;
     ExpertInput in{up.x, ws.list_tok, weight_before_ffn ? ws.list_w : nullptr, ws.xs, ws.list_tok};
-    if (!stream) {
+    if (path != ExpertPath::kPasses) {
       if (weight_before_ffn) {
         // The expert's token count is only known on the device, and at most tn
         // tokens can select it: gather tn rows.  Positions past the count read the
@@ -2339,7 +2364,7 @@ extern "C" int csk_expert_mlp_mxfp4(int expert_id, const float* hidden, int64_t 
       }
       if (rc != CSK_OK) return rc;
     }
-    rc = run_experts(1, tn, k, H, F, activation, in, ws, stream);
+    rc = run_experts(1, tn, k, H, F, activation, in, ws, path);
     if (rc != CSK_OK) return rc;
     expand_expert_rows_kernel<<<dim3((unsigned)cdiv(H, 256), (unsigned)tn), 256, 0, g_stream>>>(
         ws.y, ws.ids, ws.pos, dout.as<float>(), (int)k, (int)H, 0);
@@ -2394,7 +2419,7 @@ extern "C" int csk_expert_mlp_f16(int expert_id, const float* hidden, int64_t T,
     select_expert_ids_kernel<<<dim3((unsigned)cdiv(P, 256)), 256, 0, g_stream>>>(
         up.pairs, ws.ids, (int)P, expert_id, ws.list_tok, ws.list_w);
     if ((rc = check_launch("select_expert_ids_kernel")) != CSK_OK) return rc;
-    if ((rc = launch_dispatch(ws.ids, up.pairs, P, k, 1, up.ew, ws, stream_group_tokens(tn, H, F), false)) != CSK_OK) return rc;
+    if ((rc = launch_dispatch(ws.ids, up.pairs, P, k, 1, up.ew, ws, kGemmBM, false)) != CSK_OK) return rc;
     // with weight_before_ffn at most tn tokens can select the expert: tn rows are gathered; the
     // ones past its count read the zeroed tail of the lists and are never consumed
     rc = run_experts_f16(1, tn, k, H, F, activation, up.x, weight_before_ffn != 0, tn, ws);

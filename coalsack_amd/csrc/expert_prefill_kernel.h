@@ -66,6 +66,8 @@ struct ExpertGemmMxArgs {
   const WorkDesc* desc;
   const int* mtiles;     // [2 * n]: (expert slot, first token) of each M tile
   const int* n_mtiles;
+  const StreamGroup* groups;  // expert_stream_kernel_tiles: the M tiles as token groups, in place of the three above
+  const int* n_groups;
   const int* list_row;   // packed position -> row of A; null: row = packed position
   const uint4* A;        // [rows][mx3_row_blocks(nblk)][6] x 16 B (mx3.h); blocks past nblk are zeros
   int nblk;              // K / 32
@@ -130,18 +132,17 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t plane_rsrc(const void* p) {
 
 typedef __attribute__((address_space(3))) const u32x4 lds_u32x4;
 
-// One work unit: M tile (expert `wd`, tokens [m0, m0 + mcount) of its list) x N tile nt.
+// One work unit: M tile (packed positions [base, base + mcount), tokens of the expert with weights `w`) x N tile nt.
 // MS = 2 for M tiles that hold more than 32 tokens, MS = 1 for those that hold at most 32
 // (the ragged end of an expert's token list), so that a tail of a few tokens costs one
 // 32-token sub-tile of matrix work instead of two.
 template <int MODE, int NG, int MS>
-__device__ __forceinline__ void expert_gemm_mx_unit(const ExpertGemmMxArgs& a, const WorkDesc* wd, int m0, int mcount,
+__device__ __forceinline__ void expert_gemm_mx_unit(const ExpertGemmMxArgs& a, const ExpertW& w, int base, int mcount,
                                                     int nt, unsigned char* smem) {
   using G = MxGeom<NG, MS>;
   constexpr int kCopies = G::kCopies, kStages = G::kStages, kLead = kStages - 1;
   static_assert(kStages * G::kStageChunks * 16 <= MxGeom<NG, 2>::kLdsBytes, "the launch asks for the LDS of full tiles");
   constexpr int kStageChunks = G::kStageChunks, kFrags = G::kFrags, kBM = G::kBM;
-  const int base = wd->base + m0;
   const int lane = threadIdx.x & 63;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform, and known to be
   const int n32 = lane & 31, kg = lane >> 5;
@@ -169,7 +170,6 @@ __device__ __forceinline__ void expert_gemm_mx_unit(const ExpertGemmMxArgs& a, c
   const bool idle_wave = __builtin_amdgcn_readfirstlane((int)(group_tile(0) >= a.ntile)) != 0;
   // One buffer descriptor per weight plane; a group's tile pair and the K step go into the
   // scalar offset of the load, the lane's place within the pair into the vector offset.
-  const ExpertW& w = wd->w;
   const auto q_rsrc0 = plane_rsrc(MODE == 0 ? w.q_gate : w.q_down);
   const auto q_rsrc1 = plane_rsrc(MODE == 0 ? w.q_up : w.q_down);
   const auto s_rsrc0 = plane_rsrc(MODE == 0 ? w.s_gate : w.s_down);
@@ -591,9 +591,30 @@ __global__ __launch_bounds__(64 * kMxWaves, NG == 2 ? 3 : 2) void expert_gemm_mx
   }
   const int mcount = min(kGemmBM, wd->Te - m0);
   if (mcount <= 32)
-    expert_gemm_mx_unit<MODE, NG, 1>(a, wd, m0, mcount, nt, smem);
+    expert_gemm_mx_unit<MODE, NG, 1>(a, wd->w, wd->base + m0, mcount, nt, smem);
   else
-    expert_gemm_mx_unit<MODE, NG, 2>(a, wd, m0, mcount, nt, smem);
+    expert_gemm_mx_unit<MODE, NG, 2>(a, wd->w, wd->base + m0, mcount, nt, smem);
+}
+
+// The same units of 256 weight rows over the streaming kernels' token groups of up to 64 tokens (self-contained records: two
+// dependent reads in front of a unit's token rows, where list, descriptor and rows are three).  For batches of a few
+// tokens per expert it waits for memory, and three workgroups per compute unit with three steps requested ahead each keep
+// more of it in flight than the streaming kernel's groups of five to twelve tokens did, whose rows took most of the LDS (64
+// experts of 2048 x 768, top-8, 50 tokens, 8 layers 587 -> 546 us; 32 of 2880 x 2880, top-4, 48 tokens 120 -> 107).
+template <int MODE>
+__global__ __launch_bounds__(64 * kMxWaves, 3) void expert_stream_kernel_tiles(ExpertGemmMxArgs a) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int n_units = *a.n_groups * a.n_ntiles;
+  const int part = (n_units + kDies - 1) / kDies;
+  const int slot = blockIdx.x / kDies, unit = (blockIdx.x % kDies) * part + slot;
+  if (slot >= part || unit >= n_units) return;
+  const int v = unit / a.n_ntiles, nt = unit - v * a.n_ntiles;
+  const StreamGroup* gr = a.groups + v;
+  const int mcount = min(kGemmBM, gr->left);
+  if (mcount <= 32)
+    expert_gemm_mx_unit<MODE, 2, 1>(a, gr->w, gr->base, mcount, nt, smem);
+  else
+    expert_gemm_mx_unit<MODE, 2, 2>(a, gr->w, gr->base, mcount, nt, smem);
 }
 
 }  // namespace csk

@@ -1,7 +1,7 @@
 // Expert MLP for the weight-streaming (decode) regime.
 //
 // Every active expert's matrices are streamed from HBM once per group of up to
-// twelve of its tokens: 64 lanes x 16 bytes = 1 KiB of contiguous nibbles per
+// four of its tokens (batches with more per expert take tiles, expert_prefill_kernel.h): 64 lanes x 16 bytes = 1 KiB of contiguous nibbles per
 // 16-row tile per K step, the four waves of a workgroup taking interleaved K
 // steps (128 elements each).  The MXFP4 entries are the B operand of the block-scaled
 // matrix instruction as they are stored, their E8M0 bytes its scale operand; the group's
@@ -74,8 +74,8 @@ __device__ __forceinline__ float moe_activation(float gate_v, float up_v, int ac
 // unit (stream_tiles: together they set the loads in flight).
 // MODE 0: a work unit is NT/2 gate tiles and the up tiles of the same features, SwiGLU epilogue.
 // MODE 1: a work unit is NT consecutive down tiles.
-// LG = lane groups that hold tokens: up to 4 LG tokens are contracted per pass (rows
-// 0..4 LG - 1 of the instruction's 16 token rows; the launch says how many, a.group_tokens).
+// Up to four tokens are contracted per pass (rows 0..3 of the instruction's 16 token rows; the launch says how many,
+// a.group_tokens).
 //
 // The work is (token group of an expert) x (tile pair): every group costs the
 // same, so teams of gridDim.x / groups workgroups take one group each and
@@ -134,19 +134,19 @@ constexpr int stream_tiles(int ns) {
   return ns <= 3 ? 4 : 2;
 }
 constexpr int stream_depth(int ns) { return ns <= 8 ? ns : ns / 2; }  // divides ns: a step's registers are known at compile time
-constexpr size_t stream_lds_bytes(int ns, int lg, int group_tokens) {
+constexpr size_t stream_lds_bytes(int ns, int group_tokens) {
   // activation rows as three FP6 terms (96 B per block, 16 ns blocks per row: zeros past K) + the reduction buffers
-  return (size_t)group_tokens * ns * 16 * 96 + (size_t)2 * 4 * lg * (4 * stream_tiles(ns)) * 16 * sizeof(float);
+  return (size_t)group_tokens * ns * 16 * 96 + (size_t)2 * 4 * (4 * stream_tiles(ns)) * 16 * sizeof(float);
 }
 
-template <int MODE, int LG, int NS, bool ROUTE1 = false>
+template <int MODE, int NS, bool ROUTE1 = false>
 __global__ __launch_bounds__(256, 2) void expert_stream_kernel(ExpertStreamArgs a) {
   static_assert(!ROUTE1 || MODE == 0, "the gate/up kernel is the one that routes");
   constexpr int NT = stream_tiles(NS);  // weight tiles per unit
   constexpr int TU = MODE == 0 ? NT / 2 : NT; // tiles of one plane per unit
   constexpr int ND = stream_depth(NS);        // K steps whose weights are held or in flight
   constexpr int NV = 4 * NT;                  // accumulator floats per lane per unit
-  constexpr int G = 4 * LG;                   // tokens per pass, at most
+  constexpr int G = kStreamG;                 // tokens per pass, at most
   extern __shared__ __align__(16) unsigned char smem[];
   const int nblk = a.nblk;
   // blocks per activation row in LDS: all the blocks the steps touch, those past K zero, so
@@ -154,7 +154,7 @@ __global__ __launch_bounds__(256, 2) void expert_stream_kernel(ExpertStreamArgs 
   // next tile's, or the slack behind the plane, times exact zeros)
   constexpr int lrb = NS * 16;
   u32x4* As = reinterpret_cast<u32x4*>(smem);  // [group_tokens][lrb][3 terms][2] x 16 B
-  float* red = reinterpret_cast<float*>(smem + (size_t)a.group_tokens * lrb * (kMx3ChunksPerBlock * 16));  // [2][4][LG][NV][16]: live lanes only
+  float* red = reinterpret_cast<float*>(smem + (size_t)a.group_tokens * lrb * (kMx3ChunksPerBlock * 16));  // [2][4][NV][16]: live lanes only
 
   const int npair = (a.ntile + TU - 1) / TU;  // units per token group
   // Teams of W workgroups share one token group and interleave its units
@@ -304,8 +304,7 @@ __global__ __launch_bounds__(256, 2) void expert_stream_kernel(ExpertStreamArgs 
         ws.b[m] = (m < TU ? bp0 : bp1)[min(t * 16 + n, a.N - 1)];  // bias pointers are never null (absent bias = zero vector)
       }
     };
-    static_assert(LG <= 4, "the instruction has sixteen token rows");
-    const bool live = g < LG;  // token t is accumulator row t % 4 of lanes 16 (t / 4) .. 16 (t / 4) + 15
+    const bool live = g == 0;  // token t is accumulator row t of the first sixteen lanes
 
     // A thread's first block of activations is requested first (loads return in order: asked
     // for after the weights it would arrive behind them), then the first unit's weights ...
@@ -460,13 +459,13 @@ __global__ __launch_bounds__(256, 2) void expert_stream_kernel(ExpertStreamArgs 
         if (s + ND < NS) load_step(ws, unit, s + ND, false);
         else load_step(ws, next, s + ND - NS, idle);
       }
-      float* rbuf = red + (size_t)par * 4 * LG * NV * 16;
+      float* rbuf = red + (size_t)par * 4 * NV * 16;
       par ^= 1;
       if (live) {
 #pragma unroll
         for (int m = 0; m < NT; ++m)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) rbuf[((wv * LG + g) * NV + m * 4 + i) * 16 + n] = acc[m][i];
+          for (int i = 0; i < 4; ++i) rbuf[(wv * NV + m * 4 + i) * 16 + n] = acc[m][i];
       }
       __syncthreads();
       if (wv == (unit & 3) && live) {
@@ -476,14 +475,13 @@ __global__ __launch_bounds__(256, 2) void expert_stream_kernel(ExpertStreamArgs 
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
             const int o = m * 4 + i;
-            v2[m][i] = ((rbuf[((0 * LG + g) * NV + o) * 16 + n] + rbuf[((1 * LG + g) * NV + o) * 16 + n]) +
-                        rbuf[((2 * LG + g) * NV + o) * 16 + n]) + rbuf[((3 * LG + g) * NV + o) * 16 + n];
+            v2[m][i] = ((rbuf[(0 * NV + o) * 16 + n] + rbuf[(1 * NV + o) * 16 + n]) + rbuf[(2 * NV + o) * 16 + n]) +
+                       rbuf[(3 * NV + o) * 16 + n];
           }
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const int t = g * 4 + i;  // token slot within the group
-          if (t < gcount) {
-            const size_t p = (size_t)(base + t);
+          if (i < gcount) {
+            const size_t p = (size_t)(base + i);  // token i of the group
 #pragma unroll
             for (int m = 0; m < TU; ++m) {
               const int r = (unit * TU + m) * 16 + n;  // output feature

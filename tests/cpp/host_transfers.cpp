@@ -413,6 +413,43 @@ static int kernels_of_a_batch() {
   return 0;
 }
 
+// Token groups of four in passes, or tiles of up to 64 tokens.
+static int groups_of_a_batch() {
+  struct Call {
+    int64_t E, k, H, F, T;
+    int wbf;
+    bool tiles;
+  };
+  const Call calls[] = {
+      {8, 4, 2880, 2880, 4, 0, false},    {8, 4, 2880, 2880, 8, 0, true},    {32, 4, 2880, 2880, 16, 0, false},
+      {32, 4, 2880, 2880, 24, 0, true},   {128, 4, 2880, 2880, 16, 0, false}, {128, 4, 2880, 2880, 20, 0, false},
+      {128, 4, 2880, 2880, 64, 0, true},  {64, 8, 2048, 768, 50, 0, true},   {1, 1, 2880, 2880, 8, 0, false},
+      {1, 1, 2880, 2880, 17, 0, true},    {16, 2, 3328, 544, 19, 1, false},  {16, 2, 3328, 544, 19, 0, true},
+      {4, 4, 2880, 1536, 33, 1, true},
+  };
+  for (const Call& c : calls) {
+    csk_layer* L;
+    OK(csk_layer_create(c.E, c.k, c.H, c.F, &L));
+    std::vector<float> gate(c.E * c.H), hidden(c.T * c.H), out(c.T * c.H);
+    OK(csk_layer_set_router(L, gate.data(), nullptr));
+    OK(csk_layer_set_options(L, 0, CSK_ACT_MODIFIED_SWIGLU, c.wbf));
+    OK(csk_layer_fill_synthetic(L, 1, 0, 117, 5));
+    fake::launched.clear();
+    OK(csk_moe_forward(L, hidden.data(), c.T, out.data(), 0));
+    int tiles = 0, all = 0;
+    for (const std::string& name : fake::launched) {
+      tiles += name.find("expert_stream_kernel_tiles") != std::string::npos;
+      all += name.find("expert_stream_kernel") != std::string::npos;
+    }
+    if (all != 2 || tiles != (c.tiles ? 2 : 0)) {
+      std::printf("E %ld k %ld H %ld F %ld T %ld: not the kernels expected\n", c.E, c.k, c.H, c.F, c.T);
+      return 1;
+    }
+    csk_layer_destroy(L);
+  }
+  return 0;
+}
+
 // The pinned ring (16 MiB, quarters of 4, pieces of 64 KiB) entered at many offsets and gone round
 // several times within a call, on a stream that reads and writes it as late as it may.
 static int ring_entered_anywhere() {
@@ -492,6 +529,7 @@ int main(int argc, char** argv) {
       {"threads_sleep_while_the_stream_works", threads_sleep_while_the_stream_works},
       {"staging_memory_after_a_large_upload", staging_memory_after_a_large_upload},
       {"kernels_of_a_batch", kernels_of_a_batch},
+      {"groups_of_a_batch", groups_of_a_batch},
       {"ring_entered_anywhere", ring_entered_anywhere},
       {"expert_that_did_not_arrive", expert_that_did_not_arrive},
       {"scales_of_an_uploaded_matrix", scales_of_an_uploaded_matrix},

@@ -25,7 +25,7 @@ def driver(tmp_path_factory):
 
 CHECKS = ["results_of_a_failed_call", "pinned_area_after_a_failed_call", "scales_of_an_uploaded_matrix",
           "no_pinned_memory", "threads_sleep_while_the_stream_works", "staging_memory_after_a_large_upload",
-          "kernels_of_a_batch", "ring_entered_anywhere", "expert_that_did_not_arrive"]
+          "kernels_of_a_batch", "groups_of_a_batch", "ring_entered_anywhere", "expert_that_did_not_arrive"]
 
 
 @pytest.mark.parametrize("check", CHECKS)

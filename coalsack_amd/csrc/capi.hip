@@ -596,7 +596,7 @@ int launch_mx3(const float* x, uint16_t* x3, int64_t rows, int64_t H, const int*
 //   kTiles   expert_stream_kernel_tiles: groups of up to 64 tokens on the grouped GEMM's low tile, rows as FP6 terms
 //   kGemm    expert_gemm_mx_kernel: M tiles of 64 tokens, in the order of the experts' lists
 enum class ExpertPath { kPasses, kTiles, kGemm };
-inline int group_tokens(ExpertPath path, int64_t T) { return path == ExpertPath::kPasses ? (int)std::min<int64_t>(T, kStreamG) : kGemmBM; }
+inline int group_tokens(ExpertPath path, int64_t T) { return path != ExpertPath::kPasses ? kGemmBM : T == 1 ? 1 : kStreamG; }
 
 // Expected passes beyond the first over the weights of an expert, in groups of g of its m tokens (Poisson distributed).
 double passes_again(double m, int g) {
@@ -1848,11 +1848,12 @@ namespace {
 // kernels.
 int64_t g_pass_tokens = 32768;
 
-// Largest batch routed by the single-workgroup kernel.  Its sixteen waves take the tokens four
-// at a time one after the other; beyond 32 tokens, selection spread over T / 4 workgroups
-// followed by the dispatch kernel is faster although it is a launch more (120b shape, routing
-// stage: 17.6 -> 15.7 us at T = 48, 20.8 -> 15.9 at T = 64; no gain at 32, a loss at 24).
-constexpr int64_t kRouteSmallTokens = 32;
+// Largest batch routed by the single-workgroup kernel.  Its sixteen waves take the tokens one
+// after the other; beyond, selection spread over T / 4 workgroups
+// followed by the dispatch kernel is faster although it is a launch more (us, one workgroup / two launches, 8 layers: 64
+// experts of 2048 x 768, top-8, 20 tokens 462 / 473, 32 tokens 511 / 491, 50 tokens 568 / 501; 128 of 2880 x 2880, top-4, 24
+// tokens 985 / 996, 32 tokens 1150 / 1145, 64 tokens 1684 / 1635).
+constexpr int64_t kRouteSmallTokens = 31;
 // phase 0: the whole forward; 1: up to and including the dispatch (router output and lists
 // are in ws); 2: the rest (experts and combine) of a pass whose phase 1 ran in the same ws.
 int forward_pass(csk_layer* L, const float* hidden, int64_t T, float* out, int flags, Workspace& ws = g_ws,
@@ -1899,7 +1900,7 @@ int forward_pass(csk_layer* L, const float* hidden, int64_t T, float* out, int f
     if ((rc = check_launch("router_prep_logits_kernel")) != CSK_OK) return rc;
     mark(CSK_STAGE_DISPATCH);
     RouteIn rin{ws.logits, xr, L->gate_w, L->has_gate_b ? L->gate_b : nullptr, L->ew_dev,
-                (int)T, (int)L->E, (int)L->k, (int)L->H, L->sigmoid, group_tokens(path, T)};
+                (int)T, (int)L->E, (int)L->k, (int)L->H, L->sigmoid, group_tokens(path, T), groups ? kListGroups : kListDesc};
     RouteOut rout{ws.pairs, ws.ids, ws.pos, ws.counts, ws.offsets, ws.desc, ws.groups, ws.nv,
                   ws.tiles, ws.n_tiles, ws.list_tok, ws.list_w};
     if (T == 1 && phase == 0 && L->E > 1 && passes) {

@@ -554,7 +554,7 @@ __global__ void pairs_to_ids_kernel(const float* __restrict__ pairs, int* __rest
 // atomics over all P expert ids (they are L2-resident; every workgroup does this, which
 // saves a launch and any global atomics), how many assignments name each expert in total
 // and how many of them lie before its own chunk; inside the chunk the lanes of a wave
-// that name the same expert find one another by ballots, and a prefix over the sixteen
+// that name the same expert find one another in a word of bits per expert, and a prefix over the sixteen
 // waves completes the rank.  An assignment's place is offset(expert) + before + rank: each
 // expert's list is ascending in token index -- the order the reference's per-expert token
 // loop visits them (expert_mlp_node.h:503-529).  Ids below zero (assignments that do not
@@ -575,10 +575,11 @@ __global__ __launch_bounds__(kDispatchThreads) void dispatch_scatter_kernel(
   const int chunk0 = blockIdx.x * kDispatchThreads;
   __shared__ int cnt[kMaxExperts], before[kMaxExperts], off_sh[kMaxExperts], act_e[kMaxExperts];
   __shared__ int first_sh[kMaxExperts], slot_sh[kMaxExperts];
+  __shared__ unsigned long long named[NW][kMaxExperts];  // per wave: the assignments that name the expert
   __shared__ int wcnt[NW][kMaxExperts];
   __shared__ int na_sh;
   if (tid < kMaxExperts) cnt[tid] = 0, before[tid] = 0;
-  for (int i = tid; i < NW * kMaxExperts; i += kDispatchThreads) (&wcnt[0][0])[i] = 0;
+  for (int i = tid; i < NW * kMaxExperts; i += kDispatchThreads) (&named[0][0])[i] = 0ull;
   __syncthreads();
   for (int p0 = 0; p0 < P; p0 += kDispatchThreads * 4) {  // four loads in flight per thread
     int id[4];
@@ -649,18 +650,10 @@ __global__ __launch_bounds__(kDispatchThreads) void dispatch_scatter_kernel(
       }
     }
   }
-  // this chunk: lanes of a wave that name the same expert, their rank among themselves
+  // this chunk: an expert's word has a bit for every assignment of the wave that names it
   const int my_p = chunk0 + tid;
   const int my_id = my_p < P ? ids[my_p] : -1;
-  unsigned long long same = 0ull, todo = __ballot(my_id >= 0);
-  while (todo != 0ull) {  // the same in every lane
-    const int id0 = __builtin_amdgcn_readlane(my_id, (int)__builtin_ctzll(todo));
-    const unsigned long long m = __ballot(my_id == id0);
-    if (my_id == id0) same = m;
-    todo &= ~m;
-  }
-  const int rank_in_wave = __popcll(same & ((1ull << lane) - 1ull));
-  if (my_id >= 0 && rank_in_wave == 0) wcnt[wv][my_id] = __popcll(same);
+  if (my_id >= 0) atomicOr(&named[wv][my_id], 1ull << lane);
   __syncthreads();
   if (pub) {
     // The list that the expert kernels walk (token groups or M tiles, not both): four threads per
@@ -682,8 +675,8 @@ __global__ __launch_bounds__(kDispatchThreads) void dispatch_scatter_kernel(
       }
     }
   }
-  if (pub && tid < E) {
-    counts[tid] = cnt[tid];
+  if (pub && tid < E) counts[tid] = cnt[tid];
+  if (pub && tid < E && !groups) {  // (the kernels that walk token groups read no descriptors)
     const bool on = tid < na_sh;
     const int e = on ? act_e[tid] : 0;
     write_work_desc(desc + tid, on, e, cnt[e], off_sh[e], ew);
@@ -692,14 +685,13 @@ __global__ __launch_bounds__(kDispatchThreads) void dispatch_scatter_kernel(
     int run = 0;
 #pragma unroll
     for (int w = 0; w < NW; ++w) {
-      const int v = wcnt[w][tid];
       wcnt[w][tid] = run;
-      run += v;
+      run += __popcll(named[w][tid]);
     }
   }
   __syncthreads();
   if (my_id >= 0) {
-    const int pos = off_sh[my_id] + before[my_id] + wcnt[wv][my_id] + rank_in_wave;
+    const int pos = off_sh[my_id] + before[my_id] + wcnt[wv][my_id] + __popcll(named[wv][my_id] & ((1ull << lane) - 1ull));
     list_tok[pos] = my_p / k;
     list_w[pos] = pairs[2 * (size_t)my_p + 1];
     pos_of_slot[my_p] = pos;

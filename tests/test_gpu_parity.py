@@ -616,7 +616,7 @@ def test_layer_few_tokens_long_rows(lib, oracle):
 @pytest.mark.parametrize("H,F", [(8224, 64), (64, 8224)])
 def test_layer_few_tokens_on_the_grouped_gemm(lib, oracle, H, F, opts):
     """Rows one block longer than the streaming kernels take (8192): batches of one to 64 tokens on the
-    grouped GEMM, whose M tiles are listed by the single-workgroup routing kernel up to 32 tokens and by
+    grouped GEMM, whose M tiles are listed by the single-workgroup routing kernel up to 31 tokens and by
     the dispatch kernel beyond, and whose FP6 rows come from the routing prologue -- or, with the weight
     in front of the FFN, from the gathered and scaled rows."""
     opts = dict(opts)
@@ -966,8 +966,8 @@ def test_layer_many_experts_small_batch(lib, oracle, E, T, norm):
 @pytest.mark.parametrize("T", [3, 4, 5, 32, 33, 64, 65, 200])
 def test_layer_maximum_experts_and_top_k(lib, oracle, T):
     """The limits of a layer: 256 experts, top-16 -- four tokens fill the one-wave-per-token
-    router (64 assignments), 32 are the most the single-workgroup one takes (512 assignments),
-    33 to 64 go through the multi-workgroup selection and the dispatch kernel behind the fused
+    router (64 assignments), 31 are the most the single-workgroup one takes (496 assignments),
+    32 to 64 go through the multi-workgroup selection and the dispatch kernel behind the fused
     norm + logits kernel, 65 through the separate kernels, 200 take the grouped GEMM."""
     L = synth.LayerInputs(256, 16, 64, 96, seed=71)
     _check_layer(lib, oracle, L, T)

@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("E,k,H,F,T", [(2, 1, 1024, 1024, 16), (1, 1, 96, 64, 17), (1, 1, 64, 96, 33), (1, 1, 64, 96, 64),
                                        (2, 2, 160, 64, 65), (8, 8, 128, 256, 20), (3, 1, 256, 96, 60), (64, 8, 64, 96, 40),
-                                       (256, 16, 64, 64, 30), (5, 5, 32, 32, 29)])
+                                       (256, 16, 64, 64, 31), (5, 5, 32, 32, 29)])
 @pytest.mark.parametrize("opts", [dict(), dict(weight_before_ffn=True, sigmoid=True), dict(act=1, norm=True)])
 def test_tiles(lib, oracle, E, k, H, F, T, opts):
     opts = dict(opts)

@@ -699,47 +699,51 @@ int launch_dispatch(const int* ids, const float* pairs, int64_t P, int64_t k, in
   return check_launch("dispatch_scatter_kernel");
 }
 
-template <int MODE, int NS, bool ROUTE1>
+template <int MODE, int NS, bool ROUTE1, bool ROWS3>
 int launch_stream_form(ExpertStreamArgs a, int64_t P) {
   // kStreamWgPerCu workgroups per compute unit in steady state (one where the rows of a
   // group take more than half of the LDS); a batch so small that every work unit can have a
   // resident workgroup of its own gets that
   constexpr int TU = MODE == 0 ? stream_tiles(NS) / 2 : stream_tiles(NS);
   size_t lds = stream_lds_bytes(NS, a.group_tokens);
-  if (ROUTE1) lds = std::max(lds, sizeof(CloseCallLds));  // a close call is recomputed where the rows go afterwards
+  if (ROUTE1) lds = std::max(lds, sizeof(RouteOneLds));  // a close call is recomputed where the rows go afterwards
   const int64_t units = cdiv(a.ntile, TU);
-  const int64_t places = (lds <= kStreamLdsHalf ? kStreamWgPerCu : 1) * (int64_t)std::max(g_cus, 1);
+  const int64_t places = (ROUTE1 && ROWS3 ? 3 : lds <= kStreamLdsHalf ? kStreamWgPerCu : 1) * (int64_t)std::max(g_cus, 1);
   const int64_t nwg = std::min(P * units, places);
   static bool lds_attr_set = false;  // per instantiation: dynamic LDS beyond the default limit is asked for once
   if (!lds_attr_set) {
-    HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(&expert_stream_kernel<MODE, NS, ROUTE1>),
+    HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(&expert_stream_kernel<MODE, NS, ROUTE1, ROWS3>),
                                 hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)std::max(stream_lds_bytes(NS, kStreamG), sizeof(CloseCallLds))));
+                                (int)std::max(stream_lds_bytes(NS, kStreamG), sizeof(RouteOneLds))));
     lds_attr_set = true;
   }
-  launch_expert_kernel(MODE, expert_stream_kernel<MODE, NS, ROUTE1>, dim3((unsigned)nwg), dim3(256), lds, a);
+  launch_expert_kernel(MODE, expert_stream_kernel<MODE, NS, ROUTE1, ROWS3>, dim3((unsigned)nwg), dim3(256), lds, a);
   return check_launch("expert_stream_kernel");
 }
-template <int MODE, bool ROUTE1 = false>
+template <int MODE, bool ROUTE1, bool ROWS3>
 int launch_stream_steps(const ExpertStreamArgs& a, int64_t P) {
   switch (stream_steps(a.nblk)) {
-    case 2: return launch_stream_form<MODE, 2, ROUTE1>(a, P);
-    case 3: return launch_stream_form<MODE, 3, ROUTE1>(a, P);
-    case 4: return launch_stream_form<MODE, 4, ROUTE1>(a, P);
-    case 5: return launch_stream_form<MODE, 5, ROUTE1>(a, P);
-    case 6: return launch_stream_form<MODE, 6, ROUTE1>(a, P);
-    case 8: return launch_stream_form<MODE, 8, ROUTE1>(a, P);
-    case 12: return launch_stream_form<MODE, 12, ROUTE1>(a, P);
-    default: return launch_stream_form<MODE, 16, ROUTE1>(a, P);
+    case 2: return launch_stream_form<MODE, 2, ROUTE1, ROWS3>(a, P);
+    case 3: return launch_stream_form<MODE, 3, ROUTE1, ROWS3>(a, P);
+    case 4: return launch_stream_form<MODE, 4, ROUTE1, ROWS3>(a, P);
+    case 5: return launch_stream_form<MODE, 5, ROUTE1, ROWS3>(a, P);
+    case 6: return launch_stream_form<MODE, 6, ROUTE1, ROWS3>(a, P);
+    case 8: return launch_stream_form<MODE, 8, ROUTE1, ROWS3>(a, P);
+    case 12: return launch_stream_form<MODE, 12, ROUTE1, ROWS3>(a, P);
+    default: return launch_stream_form<MODE, 16, ROUTE1, ROWS3>(a, P);
   }
 }
 template <int MODE>
 int launch_stream(ExpertStreamArgs a, int64_t P, Workspace& ws) {
   a.groups = ws.groups;
   a.nv = ws.nv;
-  if constexpr (MODE == 0)
-    if (a.rin.logits) return launch_stream_steps<MODE, true>(a, P);  // one token, routed by the kernel itself
-  return launch_stream_steps<MODE>(a, P);
+  if constexpr (MODE == 0) {
+    const bool rows3 = a.X3 != nullptr && a.gather_w == nullptr;
+    if (a.rin.logits)  // one token, routed by the kernel itself
+      return rows3 ? launch_stream_steps<MODE, true, true>(a, P) : launch_stream_steps<MODE, true, false>(a, P);
+    if (rows3) return launch_stream_steps<MODE, false, true>(a, P);
+  }
+  return launch_stream_steps<MODE, false, false>(a, P);
 }
 
 template <int MODE>

@@ -74,6 +74,10 @@ __device__ __forceinline__ float moe_activation(float gate_v, float up_v, int ac
 // unit (stream_tiles: together they set the loads in flight).
 // MODE 0: a work unit is NT/2 gate tiles and the up tiles of the same features, SwiGLU epilogue.
 // MODE 1: a work unit is NT consecutive down tiles.
+// ROWS3: the rows arrive as FP6 terms and are only copied.  Without the quantiser and its hundred registers the kernel takes
+// 98 to 148 instead of 180 to 220, and the one-token form has three workgroups per compute unit, a place for each of 720
+// units of a 2880 x 2880 layer (8 layers, one token 239 -> 235 us, 16 tokens 785 -> 782; three per compute unit change
+// nothing for more tokens).
 // Up to four tokens are contracted per pass (rows 0..3 of the instruction's 16 token rows; the launch says how many,
 // a.group_tokens).
 //
@@ -96,6 +100,9 @@ __device__ __forceinline__ float moe_activation(float gate_v, float up_v, int ac
 // fixed order w0 + w1 + w2 + w3, and wave t mod 4 finishes unit t.
 typedef int i32x8 __attribute__((ext_vector_type(8)));
 
+// A close call of the one token: four logits side by side, in as much LDS as leaves room for three workgroups per compute unit.
+constexpr int kRouteOneBatch = 4;
+using RouteOneLds = CloseCallLdsT<kRouteOneBatch>;
 // Descriptor of a whole weight plane as a raw buffer (the pointer is the same in every lane).
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t stream_plane_rsrc(const void* p) {
   const uint64_t v = reinterpret_cast<uint64_t>(p);
@@ -139,8 +146,8 @@ constexpr size_t stream_lds_bytes(int ns, int group_tokens) {
   return (size_t)group_tokens * ns * 16 * 96 + (size_t)2 * 4 * (4 * stream_tiles(ns)) * 16 * sizeof(float);
 }
 
-template <int MODE, int NS, bool ROUTE1 = false>
-__global__ __launch_bounds__(256, 2) void expert_stream_kernel(ExpertStreamArgs a) {
+template <int MODE, int NS, bool ROUTE1 = false, bool ROWS3 = false>
+__global__ __launch_bounds__(256, ROUTE1 && ROWS3 ? 3 : 2) void expert_stream_kernel(ExpertStreamArgs a) {
   static_assert(!ROUTE1 || MODE == 0, "the gate/up kernel is the one that routes");
   constexpr int NT = stream_tiles(NS);  // weight tiles per unit
   constexpr int TU = MODE == 0 ? NT / 2 : NT; // tiles of one plane per unit
@@ -180,7 +187,7 @@ __global__ __launch_bounds__(256, 2) void expert_stream_kernel(ExpertStreamArgs 
     const RouteOut& o = a.rout;
     const int E = r.E, k = r.k;
     // the recomputation's staging area lies where the activation rows go afterwards
-    CloseCallLds& cc = *reinterpret_cast<CloseCallLds*>(smem);
+    RouteOneLds& cc = *reinterpret_cast<RouteOneLds*>(smem);
     const float NEG = -__builtin_inff();
     float v[4];
 #pragma unroll
@@ -205,7 +212,7 @@ __global__ __launch_bounds__(256, 2) void expert_stream_kernel(ExpertStreamArgs 
     }
     if (close_call) {  // the same in every wave, and in every workgroup
       const float thr = runner_up - 2.0f * tol * fmaxf(1.0f, fabsf(runner_up));
-      logits_reference_order_wg<256>(r.x, r.g, r.b, r.logits, E, r.H, thr, cc);
+      logits_reference_order_wg<256, kRouteOneBatch>(r.x, r.g, r.b, r.logits, E, r.H, thr, cc);
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const int e = lane + 64 * j;
@@ -311,7 +318,7 @@ __global__ __launch_bounds__(256, 2) void expert_stream_kernel(ExpertStreamArgs 
     const int nfill = gcount * lrb;
     // Rows that arrive as FP6 terms already (written once per token by the routing prologue)
     // are only copied into LDS, behind the first unit's weights (below).
-    const bool copy_rows = MODE == 0 && a.X3 != nullptr && a.gather_w == nullptr;
+    constexpr bool copy_rows = ROWS3;
     int copy_row[G];  // the rows' numbers, read before the weights are requested
     if (copy_rows) {
 #pragma unroll
@@ -321,7 +328,7 @@ __global__ __launch_bounds__(256, 2) void expert_stream_kernel(ExpertStreamArgs 
       }
     }
     float4 pre[8];
-    if (!copy_rows) {
+    if constexpr (!ROWS3) {
       const int rr = threadIdx.x / lrb, kb = threadIdx.x - rr * lrb;
       if ((int)threadIdx.x < nfill && kb < nblk) {
         const int row = ROUTE1 ? 0 : a.list_row ? a.list_row[base + rr] : base + rr;
@@ -339,7 +346,7 @@ __global__ __launch_bounds__(256, 2) void expert_stream_kernel(ExpertStreamArgs 
     // quantised into LDS, one thread per 32-value block (every wave is past its last read
     // of the previous group: it has crossed that unit's barrier).  Rows may be gathered
     // through list_row and scaled by the routing weight (weight_before_ffn).
-    if (MODE == 0 && copy_rows) {
+    if constexpr (ROWS3) {
       // The LDS image of a row is its blocks in order, [lrb][6 chunks of 16 bytes]; the row in
       // memory has mx3_row_blocks(nblk) of them, the rest are zeros (any scale byte will do
       // for a block of zero codes: they come from the library's page of zeros).  Copied by
@@ -369,8 +376,9 @@ __global__ __launch_bounds__(256, 2) void expert_stream_kernel(ExpertStreamArgs 
       }
       __builtin_amdgcn_s_waitcnt((7 << 4) | (15 << 8));  // vmcnt(0): the copies (and the first weights) have landed
     }
+    if constexpr (!ROWS3) {
 #pragma unroll 1
-    for (int idx = threadIdx.x; idx < (copy_rows ? 0 : nfill); idx += 256) {
+    for (int idx = threadIdx.x; idx < nfill; idx += 256) {
       const int rr = idx / lrb, kb = idx - rr * lrb;
       u32x4 out[kMx3ChunksPerBlock];
       if (kb >= nblk) {
@@ -399,6 +407,7 @@ __global__ __launch_bounds__(256, 2) void expert_stream_kernel(ExpertStreamArgs 
       u32x4* dst = As + (size_t)idx * kMx3ChunksPerBlock;
 #pragma unroll
       for (int c = 0; c < kMx3ChunksPerBlock; ++c) dst[c] = out[c];
+    }
     }
     // lanes past the group's tokens re-read its last row; their outputs are unused
     const int frag0 = (min(n, gcount - 1) * lrb + 4 * wv + g) * kMx3ChunksPerBlock;

@@ -689,8 +689,8 @@ def test_layer_120b_shape_skewed_16_tokens(lib, oracle):
 
 @pytest.mark.parametrize("T", [32, 48, 64])
 def test_layer_20b_shape_wide_token_groups(lib, oracle, T):
-    """32 experts of 2880 x 2880 above 16 tokens: 32 and 48 tokens stream in groups of seven, 64 (eight
-    assignments per expert) take the grouped GEMM with tiles of 256 weight rows."""
+    """32 experts of 2880 x 2880 above 16 tokens: 32 and 48 tokens in token groups on the grouped GEMM's low tile, 64
+    (eight assignments per expert) on the same tile from the list of M tiles."""
     L = synth.LayerInputs(32, 4, 2880, 2880, seed=52)
     _check_layer(lib, oracle, L, T, device_weights=True, subset=True)
 
@@ -705,7 +705,7 @@ def test_layer_120b_shape_skewed_1_and_64_tokens(lib, oracle, T):
 @pytest.mark.parametrize("T", [96, 128, 160, 320])
 def test_layer_120b_shape_many_experts_few_tokens_each(lib, oracle, T):
     """More than 64 tokens, but at most ten assignments per expert on average: up to four such a batch
-    still streams (96 and 128 tokens, groups of seven; the hot experts take many), with more
+    still goes by token groups (96 and 128 tokens; the hot experts take more than one), with more
     it takes the grouped GEMM (160 and 320 tokens, most M tiles nearly empty)."""
     L = synth.LayerInputs(128, 4, 2880, 2880, seed=44, hot_experts=8)
     _check_layer(lib, oracle, L, T, device_weights=True, subset=True)

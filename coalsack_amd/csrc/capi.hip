@@ -2302,12 +2302,16 @@ int router_host(const float* hidden, int64_t T, int64_t H, const float* gate_w, 
 }  // namespace
 
 namespace {
+// An expert takes a token once, with the weight of the first slot that names it (expert_mlp_node.h:784-805), whatever the
+// caller's pairs hold: no more than T assignments take part, which is what the gathers of T rows below count on.
 __global__ void select_expert_ids_kernel(const float* __restrict__ pairs, int* __restrict__ ids,
-                                         int P, int expert_id, int* __restrict__ list_tok,
+                                         int P, int k, int expert_id, int* __restrict__ list_tok,
                                          float* __restrict__ list_w) {
   const int p = blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= P) return;
-  ids[p] = ((int)pairs[2 * (size_t)p] == expert_id) ? 0 : -1;
+  bool takes = (int)pairs[2 * (size_t)p] == expert_id;
+  for (int q = p - p % k; takes && q < p; ++q) takes = (int)pairs[2 * (size_t)q] != expert_id;
+  ids[p] = takes ? 0 : -1;
   // positions of the lists that the dispatch leaves unwritten read as token 0, weight 0
   list_tok[p] = 0;
   list_w[p] = 0.0f;
@@ -2351,15 +2355,15 @@ extern "C" int csk_expert_mlp_mxfp4(int expert_id, const float* hidden, int64_t 
     DevBuf dout;
     if ((rc = dout.alloc((size_t)tn * H * 4)) != CSK_OK) return rc;
     select_expert_ids_kernel<<<dim3((unsigned)cdiv(P, 256)), 256, 0, g_stream>>>(
-        up.pairs, ws.ids, (int)P, expert_id, ws.list_tok, ws.list_w);
+        up.pairs, ws.ids, (int)P, (int)k, expert_id, ws.list_tok, ws.list_w);
     if ((rc = check_launch("select_expert_ids_kernel")) != CSK_OK) return rc;
     const ExpertPath path = expert_path(tn, H, F, 1, k, weight_before_ffn != 0);
     if ((rc = launch_dispatch(ws.ids, up.pairs, P, k, 1, up.ew, ws, group_tokens(path, tn), path != ExpertPath::kGemm)) != CSK_OK) return rc;
     ExpertInput in{up.x, ws.list_tok, weight_before_ffn ? ws.list_w : nullptr, ws.xs, ws.list_tok};
     if (path != ExpertPath::kPasses) {
       if (weight_before_ffn) {
-        // The expert's token count is only known on the device, and at most tn
-        // tokens can select it: gather tn rows.  Positions past the count read the
+        // The expert's token count is only known on the device; it is at most tn (select_expert_ids_kernel):
+        // gather tn rows.  Positions past the count read the
         // zeroed tail of the lists (token 0, weight 0) and are never consumed.
         rc = launch_mx3(up.x, ws.xg, tn, H, ws.list_tok, ws.list_w);
         in.x_mx3 = ws.xg;
@@ -2422,11 +2426,11 @@ extern "C" int csk_expert_mlp_f16(int expert_id, const float* hidden, int64_t T,
     DevBuf dout;
     if ((rc = dout.alloc((size_t)tn * H * 4)) != CSK_OK) return rc;
     select_expert_ids_kernel<<<dim3((unsigned)cdiv(P, 256)), 256, 0, g_stream>>>(
-        up.pairs, ws.ids, (int)P, expert_id, ws.list_tok, ws.list_w);
+        up.pairs, ws.ids, (int)P, (int)k, expert_id, ws.list_tok, ws.list_w);
     if ((rc = check_launch("select_expert_ids_kernel")) != CSK_OK) return rc;
     if ((rc = launch_dispatch(ws.ids, up.pairs, P, k, 1, up.ew, ws, kGemmBM, false)) != CSK_OK) return rc;
-    // with weight_before_ffn at most tn tokens can select the expert: tn rows are gathered; the
-    // ones past its count read the zeroed tail of the lists and are never consumed
+    // with weight_before_ffn tn rows are gathered, as many as the expert can have (select_expert_ids_kernel);
+    // the ones past its count read the zeroed tail of the lists and are never consumed
     rc = run_experts_f16(1, tn, k, H, F, activation, up.x, weight_before_ffn != 0, tn, ws);
     if (rc != CSK_OK) return rc;
     expand_expert_rows_kernel<<<dim3((unsigned)cdiv(H, 256), (unsigned)tn), 256, 0, g_stream>>>(

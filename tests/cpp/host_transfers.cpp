@@ -521,7 +521,63 @@ static int scales_of_an_uploaded_matrix() {
   return 0;
 }
 
+// The expert kernels of one batch, by name: a layer's (layer E k H F T weight_before_ffn), or a single expert's (expert k H F T
+// weight_before_ffn, expert_f16 the same).
+static int names_of_a_batch(const std::string& what, const std::vector<int64_t>& v) {
+  const bool layer = what == "layer", f16 = what == "expert_f16";
+  const int64_t E = layer ? v[0] : 1, k = v[layer], H = v[layer + 1], F = v[layer + 2], T = v[layer + 3];
+  const int wbf = (int)v[layer + 4];
+  std::vector<float> hidden(T * H), out(T * H);
+  if (layer) {
+    csk_layer* L;
+    std::vector<float> gate(E * H);
+    OK(csk_layer_create(E, k, H, F, &L));
+    OK(csk_layer_set_router(L, gate.data(), nullptr));
+    OK(csk_layer_set_options(L, 0, CSK_ACT_MODIFIED_SWIGLU, wbf));
+    OK(csk_layer_fill_synthetic(L, 1, 0, 117, 5));
+    fake::launched.clear();
+    OK(csk_moe_forward(L, hidden.data(), T, out.data(), 0));
+    csk_layer_destroy(L);
+  } else {
+    std::vector<float> pairs(T * k * 2);
+    int empty = 0;
+    if (f16) {
+      std::vector<uint16_t> w(H * F);
+      csk_f16 *u, *g, *d;
+      OK(csk_f16_upload(w.data(), F, H, &u));
+      OK(csk_f16_upload(w.data(), F, H, &g));
+      OK(csk_f16_upload(w.data(), H, F, &d));
+      fake::launched.clear();
+      OK(csk_expert_mlp_f16(0, hidden.data(), T, H, F, u, g, d, nullptr, nullptr, nullptr, pairs.data(), k, 0, wbf, out.data(), &empty));
+    } else {
+      std::vector<uint8_t> w(H * F / 32 * 17, 1);
+      csk_mxfp4 *u, *g, *d;
+      OK(csk_mxfp4_upload(w.data(), F, H, &u));
+      OK(csk_mxfp4_upload(w.data(), F, H, &g));
+      OK(csk_mxfp4_upload(w.data(), H, F, &d));
+      fake::launched.clear();
+      OK(csk_expert_mlp_mxfp4(0, hidden.data(), T, H, F, u, g, d, nullptr, nullptr, nullptr, pairs.data(), k, 0, wbf, out.data(), &empty));
+    }
+  }
+  for (const std::string& name : fake::launched)
+    for (const char* kernel : {"expert_stream_kernel_tiles", "expert_stream_kernel", "expert_gemm_mx_kernel", "expert_f16_gemm_kernel", "expert_f16_kernel"})
+      if (name.find(kernel) != std::string::npos) {
+        std::printf("%s\n", kernel);
+        break;
+      }
+  return 0;
+}
+
 int main(int argc, char** argv) {
+  if (argc > 2) {
+    std::vector<int64_t> v;
+    for (int i = 2; i < argc; ++i) v.push_back(std::atoll(argv[i]));
+    const std::string what = argv[1];
+    if (v.size() != (what == "layer" ? 6u : 5u) || csk_init(0) != CSK_OK) return 2;
+    const int rc = names_of_a_batch(what, v);
+    std::fflush(stdout);
+    std::_Exit(rc);
+  }
   const std::map<std::string, int (*)()> checks = {
       {"results_of_a_failed_call", results_of_a_failed_call},
       {"pinned_area_after_a_failed_call", pinned_area_after_a_failed_call},

@@ -6,6 +6,8 @@ import subprocess
 
 import pytest
 
+from tests import test_gpu_expert_slots
+
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 
@@ -32,3 +34,14 @@ CHECKS = ["results_of_a_failed_call", "pinned_area_after_a_failed_call", "scales
 def test_host_side(driver, check):
     p = subprocess.run([driver, check], capture_output=True, text=True, timeout=120)
     assert p.returncode == 0, (p.returncode, p.stdout[-2000:], p.stderr[-2000:])
+
+
+# What the GPU tests of these batches say they run.
+BATCHES = [(kernel, (what, k, H, F, T, wbf)) for what, kernel, k, H, F, T in test_gpu_expert_slots.BATCHES for wbf in (0, 1)]
+
+
+@pytest.mark.parametrize("kernel,batch", BATCHES)
+def test_kernels_of_the_gpu_tests(driver, kernel, batch):
+    p = subprocess.run([driver, *map(str, batch)], capture_output=True, text=True, timeout=120)
+    names = p.stdout.split()
+    assert p.returncode == 0 and len(names) >= 1 and set(names) == {kernel}, (p.returncode, p.stdout[-2000:], p.stderr[-2000:])

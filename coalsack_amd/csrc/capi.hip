@@ -708,7 +708,7 @@ int launch_stream_form(ExpertStreamArgs a, int64_t P) {
   size_t lds = stream_lds_bytes(NS, a.group_tokens);
   if (ROUTE1) lds = std::max(lds, sizeof(RouteOneLds));  // a close call is recomputed where the rows go afterwards
   const int64_t units = cdiv(a.ntile, TU);
-  const int64_t places = (ROUTE1 && ROWS3 ? 3 : lds <= kStreamLdsHalf ? kStreamWgPerCu : 1) * (int64_t)std::max(g_cus, 1);
+  const int64_t places = (ROUTE1 && ROWS3 ? kRouteOneWgPerCu : lds <= kStreamLdsHalf ? kStreamWgPerCu : 1) * (int64_t)std::max(g_cus, 1);
   const int64_t nwg = std::min(P * units, places);
   static bool lds_attr_set = false;  // per instantiation: dynamic LDS beyond the default limit is asked for once
   if (!lds_attr_set) {

@@ -100,9 +100,15 @@ __device__ __forceinline__ float moe_activation(float gate_v, float up_v, int ac
 // fixed order w0 + w1 + w2 + w3, and wave t mod 4 finishes unit t.
 typedef int i32x8 __attribute__((ext_vector_type(8)));
 
-// A close call of the one token: four logits side by side, in as much LDS as leaves room for three workgroups per compute unit.
-constexpr int kRouteOneBatch = 4;
-using RouteOneLds = CloseCallLdsT<kRouteOneBatch>;
+// A close call of the one token: eight logits side by side, their products staged in pieces of half the length, so that the
+// staging area leaves room for three workgroups per compute unit.  (Four of them in whole pieces take as much LDS, but top-4
+// has at least five to recompute, one chain of dependent additions after the other in every workgroup.  8 layers of 2880 x
+// 2880, top-4, with a close call in each: four at a time 455 us, in pieces of 512 357, of 384 353; without any 237, and 239.5 with
+// pieces of 512, whose code is longer.)
+using RouteOneLds = CloseCallLdsT<kCcBatch, kCcChunk / 2>;
+constexpr int kRouteOneWgPerCu = 3;
+static_assert(kRouteOneWgPerCu * (sizeof(RouteOneLds) + kMaxExperts * sizeof(ExpertW) + 1280) <= 160 * 1024,
+              "the staging area beside the pointer table, allocated in units of 1280 bytes");
 // Descriptor of a whole weight plane as a raw buffer (the pointer is the same in every lane).
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t stream_plane_rsrc(const void* p) {
   const uint64_t v = reinterpret_cast<uint64_t>(p);
@@ -147,7 +153,7 @@ constexpr size_t stream_lds_bytes(int ns, int group_tokens) {
 }
 
 template <int MODE, int NS, bool ROUTE1 = false, bool ROWS3 = false>
-__global__ __launch_bounds__(256, ROUTE1 && ROWS3 ? 3 : 2) void expert_stream_kernel(ExpertStreamArgs a) {
+__global__ __launch_bounds__(256, ROUTE1 && ROWS3 ? kRouteOneWgPerCu : 2) void expert_stream_kernel(ExpertStreamArgs a) {
   static_assert(!ROUTE1 || MODE == 0, "the gate/up kernel is the one that routes");
   constexpr int NT = stream_tiles(NS);  // weight tiles per unit
   constexpr int TU = MODE == 0 ? NT / 2 : NT; // tiles of one plane per unit
@@ -212,7 +218,7 @@ __global__ __launch_bounds__(256, ROUTE1 && ROWS3 ? 3 : 2) void expert_stream_ke
     }
     if (close_call) {  // the same in every wave, and in every workgroup
       const float thr = runner_up - 2.0f * tol * fmaxf(1.0f, fabsf(runner_up));
-      logits_reference_order_wg<256, kRouteOneBatch>(r.x, r.g, r.b, r.logits, E, r.H, thr, cc);
+      logits_reference_order_wg<256>(r.x, r.g, r.b, r.logits, E, r.H, thr, cc);
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const int e = lane + 64 * j;

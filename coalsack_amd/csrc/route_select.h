@@ -106,14 +106,14 @@ __device__ __forceinline__ void select_topk(float (&v)[4], int lane, int E, int 
 // add rounded separately (moe_router_node.h:161-167).  The chain of H dependent additions
 // cannot be shortened, everything else can be taken out of its way: the whole workgroup
 // multiplies (coalesced loads, the products do not depend on the running sum) and stages
-// the rounded products of up to kCcBatch logits in LDS, one chunk of K ahead; lane c of
+// the rounded products of up to B logits in LDS, one chunk of K ahead; lane c of
 // wave 0 then only reads row c back and adds, all rows side by side.
 constexpr int kCcBatch = 8;              // logits recomputed side by side
 constexpr int kCcChunk = 768;            // elements of K staged per step
-constexpr int kCcStride = kCcChunk + 4;  // LDS row stride: rows start four banks apart
 
-template <int B>
+template <int B, int CH = kCcChunk>
 struct CloseCallLdsT {
+  static constexpr int kCcStride = CH + 4;  // LDS row stride: rows start four banks apart
   alignas(16) float prod[2][B][kCcStride];
   float fixed[kMaxExperts];  // the token's logits, recomputed ones replaced
   int cand[kMaxExperts];
@@ -126,14 +126,14 @@ using CloseCallLds = CloseCallLdsT<kCcBatch>;
 // margin under the (k+1)-th largest; the others keep their tree-ordered values, which the
 // bound on the difference keeps on their side of thr -- and leaves all E logits of the
 // token in s.fixed.  H must be a multiple of 4.
-template <int NT, int B = kCcBatch>
+template <int NT, int B, int CH>
 __device__ __forceinline__ void logits_reference_order_wg(const float* __restrict__ x,
                                                           const float* __restrict__ g,
                                                           const float* __restrict__ b,
                                                           const float* __restrict__ logit_row, int E,
-                                                          int H, float thr, CloseCallLdsT<B>& s) {
+                                                          int H, float thr, CloseCallLdsT<B, CH>& s) {
 #pragma clang fp contract(off)
-  constexpr int kC4 = kCcChunk / 4;
+  constexpr int kC4 = CH / 4;
   constexpr int kProducers = NT - 64;  // wave 0 only adds
   constexpr int kItems = (B * kC4 + kProducers - 1) / kProducers;
   const int tid = threadIdx.x, ptid = tid - 64;

@@ -611,9 +611,11 @@ double passes_again(double m, int g) {
 
 // Batches whose token groups are listed, as opposed to the M tiles of the experts: as many as repeat at most 120 MB of weights
 // in groups of what two workgroups per compute unit could hold the rows of.  Up to one group of tokens the weights are
-// streamed once whatever their size.  On the far side the GEMM's low tile does the same work from the other list (128
-// experts of 2880 x 2880, 96 tokens, groups / M tiles 317 / 316 us per layer; 32 of them, 48 tokens 108 / 107), and with more tokens
-// its tall tile.
+// streamed once whatever their size.  No kernel holds groups of that size any more: the line says up to where passes of four
+// can be the better choice at all.  Between tiles and the GEMM little hangs on it, their units being the same: tiles take 0.988 of
+// the GEMM's time over the 880 batches of profiles/expert_paths.txt on this side, and 0.993 over the 406 on the far side, where the
+// GEMM gains on them as experts hold several M tiles, which it walks side by side (16 of 5472 x 5856, top-8, 142
+// tokens 427 / 376 us per layer), and with more tokens has its tall tile.
 bool stream_path(int64_t T, int64_t H, int64_t F, int64_t E, int64_t k) {
   if (H / 32 > kStreamMaxBlocks || F / 32 > kStreamMaxBlocks || T * k > kStreamMaxP) return false;
   const int ns = std::max(stream_steps((int)(H / 32)), stream_steps((int)(F / 32)));
@@ -630,18 +632,34 @@ bool stream_path(int64_t T, int64_t H, int64_t F, int64_t E, int64_t k) {
 // 119 / 115, 24 144 / 126; 64 of 2048 x 768, top-8, 16 tokens (m = 2) 52 / 53, 32 66 / 63, 50 67 / 61; one expert of 2880 x 2880, 8
 // tokens 29 / 33, 12 34 / 34.  A tile's units are 200 to 400 KB, so with few of them per compute unit the last round weighs: 64
 // of 3072 x 1536, top-4, 17 tokens (2.0 per compute unit expected, some get three) 88 / 98; 16 of 4096 x 4096, top-1, 17
-// tokens (1.3) 63 / 67, 32 tokens (1.7) 87 / 81.  Over 220 layers drawn at random, 2 to 160 tokens, these lines lose 1 %
-// against the better of the two, the line at 120 MB alone 3.3.  With the routing weight in front, tiles need a launch more for the
-// gathered rows, about as long as 40 MB of weights (16 of 3328 x 544, top-2, 19 tokens 76 / 83).
-ExpertPath expert_path(int64_t T, int64_t H, int64_t F, int64_t E, int64_t k, bool weight_first) {
+// tokens (1.3) 63 / 67, 32 tokens (1.7) 87 / 81.  Over the 505 batches of profiles/expert_paths.txt that
+// come this far these lines lose 1.3 % against the better of the two, and up to 32 (128 experts with eight hot ones, top-1, 94 tokens:
+// what the router makes of a batch is not known here).  Where tiles need a launch of their own for their rows (with the
+// routing weight in front), it takes about as long as 40 MB of weights (16 of 3328 x 544,
+// top-2, 19 tokens 76 / 83).
+//
+// Few experts are another matter: where their tiles have work for less than half of the compute units, a layer takes as long as
+// one tile's walk along both row lengths, half as long again if it holds more than 32 tokens, while passes have four to
+// eight times as many units and read repeated weights from the caches.  One expert of 2880 x 2880, 16 tokens 34.3 / 34.8, 24
+// 42.6 / 35.4, 34 43.0 / 54.9, 64 52.2 / 56.8; of 4096 x 6144 8 tokens 43.7 / 51.9; of 1152 x 7392 24 tokens 41.1 / 40.9, 34 47.4 /
+// 67.3; 2 of 5312 x 5472, top-1, 7 tokens 49.0 / 56.7; 4 of 2400 x 960, 35 tokens 43.6 / 43.8.  The lines are those that lose least
+// over such batches, the length of rows weighing more than in proportion: over the 375 of them in profiles/expert_paths.txt 0.4 %
+// against the better of the two, and up to 17; by the lines above, which they took before, 3.2 and up to 43.
+ExpertPath expert_path(int64_t T, int64_t H, int64_t F, int64_t E, int64_t k, bool rows_launch) {
   if (!stream_path(T, H, F, E, k)) return ExpertPath::kGemm;
   if (T <= kStreamG) return ExpertPath::kPasses;
   const double m = std::min((double)(T * k) / (double)E, (double)T);
   const double again = passes_again(m, kStreamG) * (double)(E * 3 * H * F) * (17.0 / 32.0);
-  if (weight_first) return again <= 40e6 ? ExpertPath::kPasses : ExpertPath::kTiles;
-  if (T <= 16) return m < 3.0 || again <= 19e6 ? ExpertPath::kPasses : ExpertPath::kTiles;
   const double active = (double)E * (1.0 - std::pow(1.0 - std::min(1.0, (double)k / (double)E), (double)T));
-  const double per_cu = active * (double)cdiv(F, 128) / std::max(g_cus, 1);
+  const int cus = std::max(g_cus, 1);
+  if (active * (double)(cdiv(F, 128) + cdiv(H, 256)) / 2.0 < 0.5 * cus) {
+    const double rows = (double)(H + F) / 5760.0;
+    const double limit = (m > 32.0 ? 220e6 : 46e6) * rows * std::sqrt(rows) + (rows_launch ? 40e6 : 0.0);
+    return again <= limit ? ExpertPath::kPasses : ExpertPath::kTiles;
+  }
+  if (rows_launch) return again <= 40e6 ? ExpertPath::kPasses : ExpertPath::kTiles;
+  if (T <= 16) return m < 3.0 || again <= 19e6 ? ExpertPath::kPasses : ExpertPath::kTiles;
+  const double per_cu = active * (double)cdiv(F, 128) / cus;
   return m < 0.75 || (m < 1.5 && per_cu < 0.8 * std::ceil(per_cu)) ? ExpertPath::kPasses : ExpertPath::kTiles;
 }
 

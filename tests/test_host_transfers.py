@@ -6,7 +6,7 @@ import subprocess
 
 import pytest
 
-from tests import test_gpu_expert_slots
+from tests import test_gpu_expert_slots, test_gpu_few_experts
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
@@ -38,6 +38,7 @@ def test_host_side(driver, check):
 
 # What the GPU tests of these batches say they run.
 BATCHES = [(kernel, (what, k, H, F, T, wbf)) for what, kernel, k, H, F, T in test_gpu_expert_slots.BATCHES for wbf in (0, 1)]
+BATCHES += [(kernel, ("layer", *layer)) for kernel, *layer in test_gpu_few_experts.LAYERS]
 
 
 @pytest.mark.parametrize("kernel,batch", BATCHES)

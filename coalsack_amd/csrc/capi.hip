@@ -635,7 +635,7 @@ bool stream_path(int64_t T, int64_t H, int64_t F, int64_t E, int64_t k) {
 // tokens (1.3) 63 / 67, 32 tokens (1.7) 87 / 81.  Over the 505 batches of profiles/expert_paths.txt that
 // come this far these lines lose 1.3 % against the better of the two, and up to 32 (128 experts with eight hot ones, top-1, 94 tokens:
 // what the router makes of a batch is not known here).  Where tiles need a launch of their own for their rows (with the
-// routing weight in front), it takes about as long as 40 MB of weights (16 of 3328 x 544,
+// routing weight in front, and in a call of a single expert), it takes about as long as 40 MB of weights (16 of 3328 x 544,
 // top-2, 19 tokens 76 / 83).
 //
 // Few experts are another matter: where their tiles have work for less than half of the compute units, a layer takes as long as
@@ -645,11 +645,14 @@ bool stream_path(int64_t T, int64_t H, int64_t F, int64_t E, int64_t k) {
 // 67.3; 2 of 5312 x 5472, top-1, 7 tokens 49.0 / 56.7; 4 of 2400 x 960, 35 tokens 43.6 / 43.8.  The lines are those that lose least
 // over such batches, the length of rows weighing more than in proportion: over the 375 of them in profiles/expert_paths.txt 0.4 %
 // against the better of the two, and up to 17; by the lines above, which they took before, 3.2 and up to 43.
-ExpertPath expert_path(int64_t T, int64_t H, int64_t F, int64_t E, int64_t k, bool rows_launch) {
+//
+// taken: how many of the T tokens the expert of a single-expert call takes, where the caller's pairs are at hand (else -1).
+ExpertPath expert_path(int64_t T, int64_t H, int64_t F, int64_t E, int64_t k, bool rows_launch, int64_t taken = -1) {
   if (!stream_path(T, H, F, E, k)) return ExpertPath::kGemm;
   if (T <= kStreamG) return ExpertPath::kPasses;
-  const double m = std::min((double)(T * k) / (double)E, (double)T);
-  const double again = passes_again(m, kStreamG) * (double)(E * 3 * H * F) * (17.0 / 32.0);
+  const double m = taken >= 0 ? (double)taken : std::min((double)(T * k) / (double)E, (double)T);
+  const double times = taken >= 0 ? (double)(cdiv(taken, kStreamG) - 1) : passes_again(m, kStreamG);
+  const double again = times * (double)(E * 3 * H * F) * (17.0 / 32.0);
   const double active = (double)E * (1.0 - std::pow(1.0 - std::min(1.0, (double)k / (double)E), (double)T));
   const int cus = std::max(g_cus, 1);
   if (active * (double)(cdiv(F, 128) + cdiv(H, 256)) / 2.0 < 0.5 * cus) {
@@ -2334,6 +2337,17 @@ __global__ void select_expert_ids_kernel(const float* __restrict__ pairs, int* _
   list_tok[p] = 0;
   list_w[p] = 0.0f;
 }
+
+int64_t tokens_taken(const float* pairs, int64_t T, int64_t k, int expert_id) {
+  int64_t n = 0;
+  for (int64_t t = 0; t < T; ++t)
+    for (int64_t s = 0; s < k; ++s)
+      if ((int)pairs[2 * (t * k + s)] == expert_id) {
+        ++n;
+        break;
+      }
+  return n;
+}
 }  // namespace
 
 extern "C" int csk_expert_mlp_mxfp4(int expert_id, const float* hidden, int64_t T, int64_t H,
@@ -2375,7 +2389,7 @@ extern "C" int csk_expert_mlp_mxfp4(int expert_id, const float* hidden, int64_t 
     select_expert_ids_kernel<<<dim3((unsigned)cdiv(P, 256)), 256, 0, g_stream>>>(
         up.pairs, ws.ids, (int)P, (int)k, expert_id, ws.list_tok, ws.list_w);
     if ((rc = check_launch("select_expert_ids_kernel")) != CSK_OK) return rc;
-    const ExpertPath path = expert_path(tn, H, F, 1, k, weight_before_ffn != 0);
+    const ExpertPath path = expert_path(tn, H, F, 1, k, true, P <= kStreamMaxP ? tokens_taken(pairs + t0 * k * 2, tn, k, expert_id) : -1);
     if ((rc = launch_dispatch(ws.ids, up.pairs, P, k, 1, up.ew, ws, group_tokens(path, tn), path != ExpertPath::kGemm)) != CSK_OK) return rc;
     ExpertInput in{up.x, ws.list_tok, weight_before_ffn ? ws.list_w : nullptr, ws.xs, ws.list_tok};
     if (path != ExpertPath::kPasses) {

@@ -522,7 +522,7 @@ static int scales_of_an_uploaded_matrix() {
 }
 
 // The expert kernels of one batch, by name: a layer's (layer E k H F T weight_before_ffn), or a single expert's (expert k H F T
-// weight_before_ffn, expert_f16 the same).
+// weight_before_ffn, expert_f16 the same, expert_eighth where every eighth token takes the expert).
 static int names_of_a_batch(const std::string& what, const std::vector<int64_t>& v) {
   const bool layer = what == "layer", f16 = what == "expert_f16";
   const int64_t E = layer ? v[0] : 1, k = v[layer], H = v[layer + 1], F = v[layer + 2], T = v[layer + 3];
@@ -540,6 +540,7 @@ static int names_of_a_batch(const std::string& what, const std::vector<int64_t>&
     csk_layer_destroy(L);
   } else {
     std::vector<float> pairs(T * k * 2);
+    for (int64_t i = 0; i < T * k; ++i) pairs[2 * i] = what == "expert_eighth" && i / k % 8 ? 1.0f : 0.0f;
     int empty = 0;
     if (f16) {
       std::vector<uint16_t> w(H * F);

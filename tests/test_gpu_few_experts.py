@@ -25,3 +25,27 @@ def test_few_experts(lib, oracle, kernel, E, k, H, F, T, wbf):
     want, wpairs = oracle_layer(oracle, L, hidden, weight_before_ffn=bool(wbf))
     assert np.array_equal(pairs[..., 0], wpairs[..., 0])
     assert_layer_close(got, want)
+
+
+# calls of a single expert that takes every eighth token: k, H, F, T, weight in front
+CALLS = [(PASSES, 4, 2880, 2880, 20, 0), (PASSES, 4, 2880, 2880, 28, 1), (PASSES, 4, 2048, 768, 60, 0), (PASSES, 2, 1024, 4096, 33, 1)]
+
+
+@pytest.mark.parametrize("kernel,k,H,F,T,wbf", CALLS)
+def test_an_eighth_of_the_tokens(lib, oracle, kernel, k, H, F, T, wbf):
+    rng = np.random.default_rng(T)
+    hidden = rng.normal(0, 1, (T, H)).astype(np.float32)
+    pairs = np.empty((T, k, 2), np.float32)
+    pairs[..., 0], pairs[..., 1] = np.arange(10, 10 + k), rng.uniform(0.1, 0.9, (T, k))
+    pairs[::8, k - 1, 0] = 5
+    b = [rng.normal(0, 0.01, n).astype(np.float32) for n in (F, F, H)]
+    w = [synth.mxfp4_blocks(3, 0, 5, i, F if i < 2 else H, H if i < 2 else F) for i in range(3)]
+    hs = [lib.mxfp4_upload(m, H if i == 2 else F, F if i == 2 else H) for i, m in enumerate(w)]
+    try:
+        got = lib.expert_mlp(5, hidden, F, *hs, *b, pairs, weight_before_ffn=bool(wbf))
+    finally:
+        for h in hs:
+            lib.mxfp4_free(h)
+    want = oracle.expert_mlp(5, hidden, F, *w, *b, pairs, weight_before_ffn=bool(wbf))
+    assert np.all(got[np.arange(T) % 8 != 0] == 0)
+    assert_layer_close(got, want)

@@ -39,6 +39,7 @@ def test_host_side(driver, check):
 # What the GPU tests of these batches say they run.
 BATCHES = [(kernel, (what, k, H, F, T, wbf)) for what, kernel, k, H, F, T in test_gpu_expert_slots.BATCHES for wbf in (0, 1)]
 BATCHES += [(kernel, ("layer", *layer)) for kernel, *layer in test_gpu_few_experts.LAYERS]
+BATCHES += [(kernel, ("expert_eighth", *call)) for kernel, *call in test_gpu_few_experts.CALLS]
 
 
 @pytest.mark.parametrize("kernel,batch", BATCHES)

@@ -21,8 +21,13 @@ def spread_scales(L, n=10):
     return L
 
 
-@pytest.mark.parametrize("nblk", [1, 3, 4, 5, 8, 9, 12, 13, 16, 17, 21, 28, 31, 33])
-@pytest.mark.parametrize("E,T", [(4, 90), (2, 130)])  # about 22 and 65 tokens per expert: short tiles, and full ones with a tail
+BLOCKS, BATCHES = [1, 3, 4, 5, 8, 9, 12, 13, 16, 17, 21, 28, 31, 33], [(4, 90), (2, 130)]
+# all of them on the grouped GEMM (tests/test_host_transfers.py holds them to it): E, k, H, F, T, weight in front
+LAYERS = [(E, 1, *shape, T, 0) for nblk in BLOCKS for E, T in BATCHES for shape in ((32 * nblk, 96), (96, 32 * nblk))]
+
+
+@pytest.mark.parametrize("nblk", BLOCKS)
+@pytest.mark.parametrize("E,T", BATCHES)  # about 22 and 65 tokens per expert: short tiles, and full ones with a tail
 @pytest.mark.parametrize("long_rows", ["gate/up", "down"])
 def test_steps_left_over(lib, oracle, nblk, E, T, long_rows):
     H, F = (32 * nblk, 96) if long_rows == "gate/up" else (96, 32 * nblk)
@@ -30,8 +35,6 @@ def test_steps_left_over(lib, oracle, nblk, E, T, long_rows):
     hidden = synth.hidden_states(T, H, seed=nblk + T)
     with build_layer(lib, L) as layer:
         got, pairs = layer.forward(hidden, want_pairs=True)
-        counts, _ = layer.last_dispatch(T)
-    assert counts.max() > 12  # more than one pass of the weight-streaming kernels holds: the grouped GEMM
     want, wpairs = oracle_layer_subset(oracle, L, hidden, T)
     assert np.array_equal(pairs[..., 0], wpairs[..., 0])
     assert_layer_close(got, want)

@@ -488,13 +488,13 @@ def _check_layer(lib, oracle, L, T, bias=True, norm=False, residual=False, devic
 
 
 def test_layer_config1_20b_8_tokens(lib, oracle):
-    """20b shape, 8 tokens -- the parity configuration."""
+    """The 20b shape with 8 tokens: the parity configuration."""
     L = synth.LayerInputs(32, 4, 2880, 2880, seed=1234)
     _check_layer(lib, oracle, L, 8)
 
 
 def test_layer_config1_dequant_all_planes(lib, oracle):
-    """Dequantised weights bit-exact, config 1 in full: every expert, all three planes."""
+    """Dequantised weights bit-exact, the 20b shape in full: every expert, all three planes."""
     L = synth.LayerInputs(32, 4, 2880, 2880, seed=1234)
     with build_layer(lib, L) as layer:
         for e in range(L.E):
@@ -520,8 +520,8 @@ def test_layer_120b_dequant_sampled_experts(lib, oracle):
 
 @pytest.mark.parametrize("T", [1, 2, 4, 16])
 def test_layer_config2_20b_decode_sweep(lib, oracle, T):
-    """BASELINE config 2 at its real shape: the decode sweep's batch sizes that no other test of
-    the 20b shape meets (8 is config 1, 32 and 64 follow below), against the CPU path."""
+    """The 20b shape: the decode sweep's batch sizes that no other test of
+    the 20b shape meets (8 is the parity configuration, 32 and 64 follow below), against the CPU path."""
     L = synth.LayerInputs(32, 4, 2880, 2880, seed=1234 + T)
     _check_layer(lib, oracle, L, T, device_weights=True, subset=True)
 
@@ -626,22 +626,30 @@ def test_layer_few_tokens_on_the_grouped_gemm(lib, oracle, H, F, opts):
         _check_layer(lib, oracle, L, T, norm=norm, residual=residual, **opts)
 
 
-@pytest.mark.parametrize("H,F", [(3072, 3072), (32, 3072), (3072, 32), (32, 32), (3040, 2976)])
-@pytest.mark.parametrize("T", [3, 23])
+ROW_LENGTHS = [(3072, 3072), (32, 3072), (3072, 32), (32, 32), (3040, 2976)]
+
+
+@pytest.mark.parametrize("H,F", ROW_LENGTHS)
+@pytest.mark.parametrize("T", [3, 8, 23])
 def test_layer_streaming_row_length_limits(lib, oracle, H, F, T):
     """The streaming kernels' form for 3072-long rows at its end (every block of the activation rows
     in LDS holds data, none is a zero tail), rows of one block of 32, and lengths whose last
-    128-wide step is partly past the row."""
+    128-wide step is partly past the row; 3 and 8 tokens in passes of four, 23 as well if one of the rows is short
+    (tests/test_host_transfers.py), else on tiles."""
     L = synth.LayerInputs(5, 2, H, F, seed=11 + H // 32 + F // 64, with_norm=True)
     _check_layer(lib, oracle, L, T, norm=True, residual=True)
 
 
-@pytest.mark.parametrize("D", [1024, 1056, 1568, 2080, 2592, 3104, 4096, 4128, 6176, 8192])
+STEP_COUNTS = [1024, 1056, 1568, 2080, 2592, 3104, 4096, 4128, 6176, 8192]
+
+
+@pytest.mark.parametrize("D", STEP_COUNTS)
 @pytest.mark.parametrize("long_rows", ["gate/up", "down"])
 def test_layer_streaming_step_counts(lib, oracle, D, long_rows):
     """The streaming kernels' forms for row lengths up to 8192 -- two to sixteen K steps per
     wave, four or two tiles per unit -- at the last length of a form and one block past it;
-    one token (routed by the gate/up kernel), one group per expert, several groups."""
+    one token (routed by the gate/up kernel), one group per expert, several groups of four (tests/test_host_transfers.py
+    holds all three to the kernel of passes)."""
     H, F = (D, 96) if long_rows == "gate/up" else (96, D)
     L = synth.LayerInputs(3, 2, H, F, seed=D + len(long_rows))
     for T in (1, 6, 29):
@@ -681,7 +689,7 @@ def test_layer_many_tokens_per_expert(lib, oracle):
 
 
 def test_layer_120b_shape_skewed_16_tokens(lib, oracle):
-    """BASELINE config 4 at T=16: 128 experts, 8 hot experts with +2.0 bias;
+    """128 experts at T=16, 8 hot experts with +2.0 bias;
     weights generated on the device, replayed on the host for the oracle."""
     L = synth.LayerInputs(128, 4, 2880, 2880, seed=42, hot_experts=8)
     _check_layer(lib, oracle, L, 16, device_weights=True)
@@ -697,7 +705,7 @@ def test_layer_20b_shape_wide_token_groups(lib, oracle, T):
 
 @pytest.mark.parametrize("T", [1, 64])
 def test_layer_120b_shape_skewed_1_and_64_tokens(lib, oracle, T):
-    """BASELINE config 4 / 5 shape at the ends of the decode range, with the skewed bias."""
+    """The same layer at the ends of the decode range."""
     L = synth.LayerInputs(128, 4, 2880, 2880, seed=43, hot_experts=8)
     _check_layer(lib, oracle, L, T, device_weights=True, subset=True)
 
@@ -765,14 +773,14 @@ def _prefill_case(lib, oracle, L, T, ntok_oracle):
 
 
 def test_prefill_20b_2048_tokens(lib, oracle):
-    """20b shape, 2048 tokens (about 256 tokens per expert)."""
+    """The 20b shape with 2048 tokens (about 256 tokens per expert)."""
     L = synth.LayerInputs(32, 4, 2880, 2880, seed=77)
     counts = _prefill_case(lib, oracle, L, 2048, 48)
     assert counts.min() > 64  # natural routing: every expert sees several M tiles
 
 
 def test_prefill_120b_skewed_4096_tokens(lib, oracle):
-    """BASELINE config 4 at T=4096: 8 hot experts take about half of the assignments."""
+    """The 120b shape at T=4096: 8 hot experts take about half of the assignments."""
     L = synth.LayerInputs(128, 4, 2880, 2880, seed=78, hot_experts=8)
     counts = _prefill_case(lib, oracle, L, 4096, 48)
     hot = np.sort(counts)[-8:].sum() / counts.sum()
@@ -840,7 +848,7 @@ def test_concurrent_forwards_equal_sequential(lib):
 @pytest.mark.parametrize("E,k,H,F,T,n_layers", [(8, 2, 128, 160, 1, 4), (8, 2, 128, 160, 8, 4), (16, 4, 256, 192, 64, 3),
                                                 (128, 4, 2880, 2880, 1, 2), (128, 4, 2880, 2880, 8, 2)])
 def test_stack_config5(lib, oracle, E, k, H, F, T, n_layers):
-    """BASELINE config 5: h <- h + MoE(RMSNorm(h)) through several layers on the device
+    """h <- h + MoE(RMSNorm(h)) through several layers on the device
     (csk_moe_stack_forward).  The stack equals the same layers called one at a time bit for
     bit, and every layer's output matches the CPU path fed with that layer's actual input
     (so that a routing near-tie in one layer is not carried into the next comparison)."""
@@ -876,7 +884,7 @@ def test_stack_config5(lib, oracle, E, k, H, F, T, n_layers):
 
 
 def test_stack_config5_36_resident_layers(lib, oracle):
-    """BASELINE config 5 as stated: 36 layers of the 120b shape resident at once (61 GB of
+    """36 layers of the 120b shape resident at once (61 GB of
     expert planes, generated on the device), decode batches of 1, 8 and 64 tokens.  The stack
     call equals the layers called one at a time bit for bit; on sampled layers the output of
     the layer matches the CPU path fed with that layer's actual input, on sampled tokens

@@ -6,7 +6,7 @@ import subprocess
 
 import pytest
 
-from tests import test_gpu_expert_slots, test_gpu_few_experts
+from tests import test_gpu_expert_slots, test_gpu_few_experts, test_gpu_gemm_steps, test_gpu_parity, test_gpu_stream_tiles
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
@@ -40,6 +40,12 @@ def test_host_side(driver, check):
 BATCHES = [(kernel, (what, k, H, F, T, wbf)) for what, kernel, k, H, F, T in test_gpu_expert_slots.BATCHES for wbf in (0, 1)]
 BATCHES += [(kernel, ("layer", *layer)) for kernel, *layer in test_gpu_few_experts.LAYERS]
 BATCHES += [(kernel, ("expert_eighth", *call)) for kernel, *call in test_gpu_few_experts.CALLS]
+BATCHES += [(test_gpu_stream_tiles.TILES, ("layer", *layer)) for *layer, _ in test_gpu_stream_tiles.LAYERS + test_gpu_stream_tiles.WEIGHT_FIRST]
+BATCHES += [("expert_gemm_mx_kernel", ("layer", *layer)) for layer in test_gpu_gemm_steps.LAYERS]
+BATCHES += [(test_gpu_few_experts.PASSES, ("layer", 5, 2, H, F, T, 0)) for H, F in test_gpu_parity.ROW_LENGTHS for T in (3, 8, 23)
+            if T < 23 or min(H, F) < 2976]
+BATCHES += [(test_gpu_few_experts.PASSES, ("layer", 3, 2, *shape, T, 0)) for D in test_gpu_parity.STEP_COUNTS for T in (1, 6, 29)
+            for shape in ((D, 96), (96, D))]
 
 
 @pytest.mark.parametrize("kernel,batch", BATCHES)

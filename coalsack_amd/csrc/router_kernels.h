@@ -102,11 +102,14 @@ __global__ __launch_bounds__(256) void router_logits_mfma_kernel(const float* __
     xa[i] = in ? *reinterpret_cast<const floatx4*>(xr + k0) : floatx4{0.f, 0.f, 0.f, 0.f};
     xb[i] = in ? *reinterpret_cast<const floatx4*>(xr + k0 + 4) : floatx4{0.f, 0.f, 0.f, 0.f};
   }
-  // the last chunk this lane may load from the expert rows (clamped loads meet zeros above)
+  // The last chunk this lane may load from the expert rows, and its columns there (clamped loads meet zeros above).  Rows
+  // shorter than a chunk have no columns for some lanes, which read the row's first ones: their own would lie in the
+  // next expert's row, and behind the last one's past the end of the gate.
   const int c_last = max(0, (H - k_lane - 8) / 64);
+  const int g_lane = k_lane + 8 <= H ? k_lane : 0;
   float* out = partial + (size_t)blockIdx.y * T * E;
   for (int e0 = blockIdx.z * 32; e0 < E; e0 += 32 * gridDim.z) {
-    const float* gr = g + (size_t)min(e0 + r32, E - 1) * H + k_lane;
+    const float* gr = g + (size_t)min(e0 + r32, E - 1) * H + g_lane;
     floatx16 acc;
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[r] = 0.0f;

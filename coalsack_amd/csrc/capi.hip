@@ -1879,6 +1879,7 @@ int64_t g_pass_tokens = 32768;
 // experts of 2048 x 768, top-8, 20 tokens 462 / 473, 32 tokens 511 / 491, 50 tokens 568 / 501; 128 of 2880 x 2880, top-4, 24
 // tokens 985 / 996, 32 tokens 1150 / 1145, 64 tokens 1684 / 1635).
 constexpr int64_t kRouteSmallTokens = 31;
+static_assert(kRouteSmallTokens * kMaxTopK <= kRouteSmallMaxP, "what its LDS is laid out for");
 // phase 0: the whole forward; 1: up to and including the dispatch (router output and lists
 // are in ws); 2: the rest (experts and combine) of a pass whose phase 1 ran in the same ws.
 int forward_pass(csk_layer* L, const float* hidden, int64_t T, float* out, int flags, Workspace& ws = g_ws,

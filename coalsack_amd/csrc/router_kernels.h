@@ -705,7 +705,7 @@ __global__ __launch_bounds__(kDispatchThreads) void dispatch_scatter_kernel(
 // A single workgroup of sixteen waves routes the batch (route_workgroup) and writes every
 // output.
 constexpr int kRouteSmallThreads = 1024;
-constexpr int kRouteSmallMaxP = 1024;
+constexpr int kRouteSmallMaxP = 512;  // assignments
 __global__ __launch_bounds__(kRouteSmallThreads) void route_small_kernel(RouteIn in, RouteOut out) {
   __shared__ RouteLds<kCcBatch, kRouteSmallMaxP> lds;
   route_workgroup<kRouteSmallThreads, kCcBatch, kRouteSmallMaxP>(in, out, lds);

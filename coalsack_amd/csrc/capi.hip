@@ -119,7 +119,7 @@ constexpr uint32_t kScalesOfOne = 0x7f7f7f7f;  // four E8M0 bytes
 // weight-streaming kernels is not built.
 constexpr int64_t kStreamMaxP = 2048;
 constexpr size_t kWeightSlack = 32768;  // bytes of mapped memory kept behind weight planes (the expert kernels read whole K steps: up to three blocks, 768 bytes, past the last tile)
-constexpr int kStreamWgPerCu = 2;  // resident workgroups of the streaming kernel per compute unit ...
+constexpr int kStreamWgPerCu = 2;  // resident workgroups of the streaming kernel per compute unit (kRouteOneWgPerCu of one form) ...
 constexpr size_t kStreamLdsHalf = 80 * 1024 - 512;  // ... if each takes no more LDS than this (and its few static words)
 
 // ---- workspace shared by every layer (single stream, one call at a time) --
@@ -723,7 +723,8 @@ int launch_dispatch(const int* ids, const float* pairs, int64_t P, int64_t k, in
 template <int MODE, int NS, bool ROUTE1, bool ROWS3>
 int launch_stream_form(ExpertStreamArgs a, int64_t P) {
   // kStreamWgPerCu workgroups per compute unit in steady state (one where the rows of a
-  // group take more than half of the LDS); a batch so small that every work unit can have a
+  // group take more than half of the LDS, kRouteOneWgPerCu of the form that routes one token and copies its row: its launch
+  // bounds and its LDS are made for that); a batch so small that every work unit can have a
   // resident workgroup of its own gets that
   constexpr int TU = MODE == 0 ? stream_tiles(NS) / 2 : stream_tiles(NS);
   size_t lds = stream_lds_bytes(NS, a.group_tokens);
@@ -1939,8 +1940,7 @@ int forward_pass(csk_layer* L, const float* hidden, int64_t T, float* out, int f
       route_tiny_kernel<<<dim3(1), 256, 0, g_stream>>>(rin, rout);
       if ((rc = check_launch("route_tiny_kernel")) != CSK_OK) return rc;
     } else if (T > kRouteSmallTokens) {
-      // more tokens than the single workgroup has waves: selection spread over T / 4
-      // workgroups, then the dispatch kernel -- a launch more, each much shorter
+      // selection spread over T / 4 workgroups, then the dispatch kernel -- a launch more, each much shorter
       router_topk_kernel<false><<<dim3((unsigned)cdiv(T, 4)), 256, 0, g_stream>>>(
           ws.logits, ws.pairs, ws.ids, (int)T, (int)L->E, (int)L->k, L->sigmoid, xr, L->gate_w,
           L->has_gate_b ? L->gate_b : nullptr, (int)L->H, ws.logits + T * L->E, 0, Mx3Rider{});
@@ -1978,9 +1978,9 @@ int forward_pass(csk_layer* L, const float* hidden, int64_t T, float* out, int f
     g_stage_valid = g_timing;
     return rc;
   }
-  // streaming path: the kernel gathers, scales and quantises the fp32 rows itself;
-  // grouped GEMM: rows written as three FP6 terms beforehand (per token, or gathered and
-  // pre-scaled per dispatch position when the routing weight goes in front of the FFN)
+  // All three paths read the rows as three FP6 terms, which the routing prologue has written per token.  With the routing
+  // weight in front of the FFN they are gathered and scaled per dispatch position: by the passes themselves, which then
+  // quantise fp32 rows, and in a launch in front of tiles and the grouped GEMM.
   ExpertInput in{xr, ws.list_tok, L->wbf ? ws.list_w : nullptr, ws.xs, ws.list_tok};
   if (route_in_kernel) in.rin = &rin_kept, in.rout = &rout_kept;
   if (rows_mx3_ready) in.x_mx3_tokens = ws.xs;

@@ -600,8 +600,8 @@ def test_layer_variants_grouped_gemm(lib, oracle, opts):
 
 
 def test_layer_few_tokens_long_rows(lib, oracle):
-    """A handful of tokens on rows past 3072 (one group of the streaming kernels, with one workgroup
-    per compute unit) and past 4096."""
+    """A handful of tokens on rows past 3072 (passes of four, whose rows take a third of the LDS)
+    and past 4096."""
     L = synth.LayerInputs(4, 2, 3200, 64, seed=23, with_norm=True)
     _check_layer(lib, oracle, L, 6, norm=True, residual=True)
     L = synth.LayerInputs(4, 2, 64, 3200, seed=24)

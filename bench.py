@@ -9,7 +9,7 @@ synthetic tokens with weights, input and output resident in HBM.  `value` is
 tokens/s of the whole layer; `roofline` describes the dominant kernel (gate/up
 projections), timed live by a start and a stop event attached to its dispatch on
 the library's stream (the kernel's own begin-to-end time, as a kernel trace
-reports it); `cpu_baseline` is the CPU checker (a restatement of the
+reports it); `cpu_baseline` is the oracle (a restatement of the
 reference's single-threaded path) timed on this host on a bounded sample.
 
 The default line is the 120b-shaped layer (128 experts, 8 hot) at 16 tokens and
@@ -18,7 +18,7 @@ stack at 1, 8 and 64 tokens, each with its own `roofline` and `cpu_baseline`.
 Decode batches rotate over 8 layer instances x 8 token batches, so that no weight
 byte is touched again before more than the 256 MB last-level cache has streamed by.
 
-Workloads (BASELINE.json configs):
+Workloads:
   c4_120b         128 experts, 8 hot experts (+2.0 router bias), T in {1,16,4096} (default, T=16)
   c2_20b_decode   32 experts, top-4, H = F = 2880, T in {1,2,4,8,16,32,64}
   c3_20b_prefill  same layer, T = 2048
@@ -412,7 +412,7 @@ def host_cpu():
 
 
 def cpu_baseline(insts, gpu_out, budget_s=12.0, stack_layers=0):
-    """Times the CPU checker (single thread, as the reference's layer runs) on the same
+    """Times the oracle (single thread, as the reference's layer runs) on the same
     layers and tokens.  `insts`: (LayerInputs, hidden) pairs -- the layer instances and token
     batches the GPU measurement rotates over; gpu_out is the GPU's output for insts[0].
 
@@ -422,7 +422,7 @@ def cpu_baseline(insts, gpu_out, budget_s=12.0, stack_layers=0):
     host's last-level cache has streamed by, which is how the reference meets them in a
     model of 36 layers.  `warm` is the same work with the sample small enough to be re-read
     from cache (one token repeated), reported beside it.  Only the tokens that are timed
-    are handed to the checker (its router runs over every token it is given).
+    are handed to the oracle (its router runs over every token it is given).
     stack_layers > 0: each instance is a layer of a stack of that many (RMSNorm in front,
     residual add behind); the stack's rate is the layer's divided by the number of layers."""
     from oracle.binding import Oracle
@@ -485,7 +485,7 @@ def cpu_baseline(insts, gpu_out, budget_s=12.0, stack_layers=0):
         m += 1
     warm = m / (time.perf_counter() - t0)
     # not reference behaviour (its layer runs on one thread): the same work farmed over the
-    # host's cores, one token slice per thread (the checker releases the GIL inside the call)
+    # host's cores, one token slice per thread (the oracle releases the GIL inside the call)
     ncores = max(1, min(16, os.cpu_count() or 1))
     all_cores = None
     if Ts >= ncores and ncores > 1:
@@ -523,7 +523,7 @@ def cpu_baseline(insts, gpu_out, budget_s=12.0, stack_layers=0):
 
 
 def cpu_baseline_f16(L, hidden, gpu_out, budget_s=12.0):
-    """The CPU checker's fp16 expert path on the first tokens of the batch (the ones whose
+    """The oracle's fp16 expert path on the first tokens of the batch (the ones whose
     experts' generated weights were read back), one thread."""
     from oracle.binding import Oracle
     orc = Oracle()

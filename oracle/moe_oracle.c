@@ -2,7 +2,7 @@
  * CPU restatement of coalsack's mixture-of-experts path (router -> per-expert
  * MXFP4 MLP -> merge, plus the RMSNorm / residual add that bracket it).
  *
- * THIS FILE IS TEST INFRASTRUCTURE.  It is the checker the HIP path is compared
+ * THIS FILE IS TEST INFRASTRUCTURE.  It is the oracle the HIP path is compared
  * against and the CPU baseline that the benchmark times; nothing the library
  * ships may call it.
  *

@@ -2,7 +2,7 @@
 // the reference's test/test_moe_router.cpp, test/test_expert_mlp.cpp and
 // test/test_frame_sync.cpp, without googletest.
 //   test_nodes --cpu   argument / error-path behaviour (no GPU call is reached)
-//   test_nodes --gpu   numerics on the GPU against the CPU checker (oracle/)
+//   test_nodes --gpu   numerics on the GPU against the oracle (oracle/)
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -22,7 +22,7 @@
 
 using namespace coalsack;
 
-extern "C" {  // the CPU checker, oracle/moe_oracle.c
+extern "C" {  // the oracle, oracle/moe_oracle.c
 int orc_router(const float*, int64_t, int64_t, const float*, int64_t, const float*, int64_t, int, float*);
 int orc_expert_token_mxfp4(const float*, const uint8_t*, const uint8_t*, const uint8_t*, const float*,
                            const float*, const float*, float*, int64_t, int64_t, int);
@@ -424,7 +424,7 @@ static void gpu_router_tests() {
     auto out = node.compute_test(h, g);
     CHECK((int)out.data_ptr<float>()[0] == 5 && (int)out.data_ptr<float>()[2] == 4 && (int)out.data_ptr<float>()[4] == 3);
   }
-  {  // :141-203 gpt-oss scale, and agreement with the CPU checker
+  {  // :141-203 gpt-oss scale, and agreement with the oracle
     moe_router_node node;
     node.set_config(32, 4);
     auto h = random_tensor({2, 8, 128}, gen, -1, 1), g = random_tensor({32, 128}, gen, -0.2f, 0.2f);
@@ -467,7 +467,7 @@ static void gpu_expert_known_answer() {
 }
 
 // The reference's four float16 tests (test/test_expert_mlp.cpp) on the GPU node, each
-// also compared with the CPU checker.
+// also compared with the oracle.
 static void gpu_expert_fp16_tests() {
   std::printf("expert_mlp (float16 weights): Basic, ModifiedSwigluActivation, MultipleExperts, GptOssScale\n");
   std::mt19937 gen(42);
@@ -707,7 +707,7 @@ static void gpu_variant_branches() {
 }
 
 // router -> E expert nodes -> merge, wired with edges and result messages the way
-// llm_engine builds the block (src/llm/llm_engine.cpp:721-753), against the CPU checker.
+// llm_engine builds the block (src/llm/llm_engine.cpp:721-753), against the oracle.
 static void gpu_node_chain() {
   std::printf("router -> experts -> merge through result messages\n");
   std::mt19937 gen(7);

@@ -90,7 +90,7 @@ ROUTING_WEIGHT_TOL = 1e-5
 def oracle_layer_tokens(oracle, L, hidden, idx, threads=16):
     """Oracle output and router pairs for the tokens hidden[idx] (any index set), replaying on
     the host only the experts those tokens select; the tokens are farmed over threads (the
-    checker releases the interpreter lock inside a call and tokens are independent)."""
+    oracle releases the interpreter lock inside a call and tokens are independent)."""
     import threading
     idx = np.asarray(idx, dtype=np.int64)
     sub = np.ascontiguousarray(hidden[idx])

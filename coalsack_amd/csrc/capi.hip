@@ -702,11 +702,11 @@ int launch_router(const float* x, const float* gate_w, const float* gate_b, int6
   Mx3Rider rider{};
   int64_t riders = 0;
   if (mx3_out) {
-    rider = Mx3Rider{x, reinterpret_cast<u32x4*>(mx3_out), (long)T, (int)(H / 32), (int)cdiv(T, 4)};
-    riders = cdiv(T * mx3_row_blocks((int)(H / 32)), 256);
+    rider = Mx3Rider{x, reinterpret_cast<u32x4*>(mx3_out), (long)T, (int)(H / 32), (int)cdiv(T, kTopkTokens)};
+    riders = cdiv(T * mx3_row_blocks((int)(H / 32)), kTopkThreads);
   }
   const auto topk = nsplit > 0 ? router_topk_kernel<true> : router_topk_kernel<false>;
-  topk<<<dim3((unsigned)(cdiv(T, 4) + riders)), 256, 0, g_stream>>>(
+  topk<<<dim3((unsigned)(cdiv(T, kTopkTokens) + riders)), kTopkThreads, 0, g_stream>>>(
       logits, pairs, ids, (int)T, (int)E, (int)k, sigmoid, x, gate_w, gate_b, (int)H, logits + T * E, nsplit, rider);
   return check_launch("router_topk_kernel");
 }
@@ -1940,8 +1940,8 @@ int forward_pass(csk_layer* L, const float* hidden, int64_t T, float* out, int f
       route_tiny_kernel<<<dim3(1), 256, 0, g_stream>>>(rin, rout);
       if ((rc = check_launch("route_tiny_kernel")) != CSK_OK) return rc;
     } else if (T > kRouteSmallTokens) {
-      // selection spread over T / 4 workgroups, then the dispatch kernel -- a launch more, each much shorter
-      router_topk_kernel<false><<<dim3((unsigned)cdiv(T, 4)), 256, 0, g_stream>>>(
+      // selection spread over T / 8 workgroups, then the dispatch kernel -- a launch more, each much shorter
+      router_topk_kernel<false><<<dim3((unsigned)cdiv(T, kTopkTokens)), kTopkThreads, 0, g_stream>>>(
           ws.logits, ws.pairs, ws.ids, (int)T, (int)L->E, (int)L->k, L->sigmoid, xr, L->gate_w,
           L->has_gate_b ? L->gate_b : nullptr, (int)L->H, ws.logits + T * L->E, 0, Mx3Rider{});
       if ((rc = check_launch("router_topk_kernel")) != CSK_OK) return rc;

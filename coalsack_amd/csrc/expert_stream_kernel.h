@@ -105,7 +105,7 @@ typedef int i32x8 __attribute__((ext_vector_type(8)));
 // has at least five to recompute, one chain of dependent additions after the other in every workgroup.  8 layers of 2880 x
 // 2880, top-4, with a close call in each: four at a time 455 us, in pieces of 512 357, of 384 353; without any 237, and 239.5 with
 // pieces of 512, whose code is longer.)
-using RouteOneLds = CloseCallLdsT<kCcBatch, kCcChunk / 2>;
+using RouteOneLds = CloseCallLdsT<256, kCcBatch, kCcChunk / 2>;
 constexpr int kRouteOneWgPerCu = 3;
 static_assert(kRouteOneWgPerCu * (sizeof(RouteOneLds) + kMaxExperts * sizeof(ExpertW) + 1280) <= 160 * 1024,
               "the staging area beside the pointer table, allocated in units of 1280 bytes");
@@ -190,7 +190,6 @@ __global__ __launch_bounds__(256, ROUTE1 && ROWS3 ? kRouteOneWgPerCu : 2) void e
   __shared__ unsigned long long s_ew[ROUTE1 ? kEwWords : 1];  // the experts' weight pointers, staged beside the logits
   if constexpr (ROUTE1) {
     const RouteIn& r = a.rin;
-    const RouteOut& o = a.rout;
     const int E = r.E, k = r.k;
     // the recomputation's staging area lies where the activation rows go afterwards
     RouteOneLds& cc = *reinterpret_cast<RouteOneLds*>(smem);
@@ -207,29 +206,34 @@ __global__ __launch_bounds__(256, ROUTE1 && ROWS3 ? kRouteOneWgPerCu : 2) void e
       const int w = threadIdx.x + i * 256;
       ew_reg[i] = w < E * (int)(sizeof(ExpertW) / 8) ? reinterpret_cast<const unsigned long long*>(r.ew)[w] : 0ull;
     }
-    float my_val, vmax, runner_up;  // lane s keeps slot s
+    float my_val, vmax;  // lane s keeps slot s
     bool close_call;
     const float tol = close_call_tolerance(r.H);
-    select_topk(v, lane, E, k, my_val, r_idx, vmax, close_call, tol, runner_up);
+    select_topk(v, lane, E, k, my_val, r_idx, vmax, close_call, tol);
 #pragma unroll
     for (int i = 0; i < kEwPerThread; ++i) {
       const int w = threadIdx.x + i * 256;
       if (w < kEwWords) s_ew[w] = ew_reg[i];
     }
     if (close_call) {  // the same in every wave, and in every workgroup
-      const float thr = runner_up - 2.0f * tol * fmaxf(1.0f, fabsf(runner_up));
-      logits_reference_order_wg<256>(r.x, r.g, r.b, r.logits, E, r.H, thr, cc);
+      float lo, hi;
+      close_call_range(my_val, lane, E, k, tol, lo, hi);
+      logits_reference_order_wg(r.x, r.g, r.b, r.logits, E, r.H, lo, hi, cc);
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const int e = lane + 64 * j;
         v[j] = e < E ? cc.fixed[e] : NEG;
       }
-      select_topk(v, lane, E, k, my_val, r_idx, vmax, close_call, 0.0f, runner_up);
+      select_topk(v, lane, E, k, my_val, r_idx, vmax, close_call, 0.0f);
     }
     r_wt = routing_weight(my_val, vmax, lane, k, r.sigmoid);
     __syncthreads();  // the pointer table is in LDS; every thread is done with cc before the activation rows overwrite it
     if (blockIdx.x == 0) {
-      // what the routing kernel would have written
+      // what the routing kernel would have written (where to: read from the arguments here -- left to the compiler the addresses
+      // are read in every workgroup and held in scalar registers over all that comes before)
+      auto args = (const __attribute__((address_space(4))) ExpertStreamArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+      asm volatile("" : "+s"(args));
+      const auto& o = args->rout;
       __shared__ int w_ids[kMaxTopK];
       if (wv == 0 && lane < k) w_ids[lane] = r_idx;
       __syncthreads();

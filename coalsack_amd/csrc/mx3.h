@@ -33,11 +33,12 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x32 __attribute__((ext_vector_type(32)));
 typedef uint32_t u32x6 __attribute__((ext_vector_type(6)));
 
-// Quantises one block held in registers; out[2t], out[2t+1] are the chunks of term t.
+// Quantises one block held in registers; put(t, lo, hi) takes the two chunks of term t.
 // v_cvt_scalef32_2xpk16_fp6_f32 divides by the scale, rounds to nearest even, saturates
 // at +-7.5 and packs value i of its first operand at position 2i, of its second at
 // 2i+1; v_cvt_scalef32_pk32_f32_fp6 is its inverse in position order (both probed).
-__device__ __forceinline__ void mx3_quantize_block(float (&r)[32], u32x4 (&out)[kMx3ChunksPerBlock]) {
+template <class Put>
+__device__ __forceinline__ void mx3_quantize_terms(float (&r)[32], Put put) {
 #pragma unroll
   for (int t = 0; t < kMx3Terms; ++t) {
     uint32_t eb;
@@ -79,9 +80,12 @@ __device__ __forceinline__ void mx3_quantize_block(float (&r)[32], u32x4 (&out)[
 #pragma unroll
       for (int j = 0; j < 32; ++j) r[j] = r[j] - d[j];  // exact: d is r rounded to 4 bits
     }
-    out[2 * t] = u32x4{q[0], q[1], q[2], q[3]};
-    out[2 * t + 1] = u32x4{q[4], q[5], s, 0u};
+    put(t, u32x4{q[0], q[1], q[2], q[3]}, u32x4{q[4], q[5], s, 0u});
   }
+}
+// out[2t], out[2t+1] are the chunks of term t.
+__device__ __forceinline__ void mx3_quantize_block(float (&r)[32], u32x4 (&out)[kMx3ChunksPerBlock]) {
+  mx3_quantize_terms(r, [&](int t, const u32x4& lo, const u32x4& hi) { out[2 * t] = lo, out[2 * t + 1] = hi; });
 }
 
 // rows of fp32 -> three-term FP6 blocks, one thread per block (padding blocks included):
@@ -135,12 +139,12 @@ __device__ __forceinline__ void mx3_rows_wave(long b0, const float* __restrict__
     r[4 * i] = v.x, r[4 * i + 1] = v.y, r[4 * i + 2] = v.z, r[4 * i + 3] = v.w;
   }
   // (a padding block is 32 zeros: codes 0 and scale byte 127 on every term)
-  u32x4 out[kMx3ChunksPerBlock];
-  mx3_quantize_block(r, out);
   __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
   u32x4* o4 = reinterpret_cast<u32x4*>(lds);
-#pragma unroll
-  for (int c = 0; c < kMx3ChunksPerBlock; ++c) o4[lane * kMx3ChunksPerBlock + c] = out[c];
+  mx3_quantize_terms(r, [&](int t, const u32x4& lo, const u32x4& hi) {
+    o4[lane * kMx3ChunksPerBlock + 2 * t] = lo;
+    o4[lane * kMx3ChunksPerBlock + 2 * t + 1] = hi;
+  });
   __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
   const long n_out = min((total - b0), 64L) * kMx3ChunksPerBlock;
   u32x4* dst = x3 + b0 * kMx3ChunksPerBlock;

@@ -29,6 +29,30 @@ __device__ __forceinline__ float wave_max_all(float v) {
   return fmaxf(fmaxf(r0, r1), fmaxf(r2, r3));
 }
 
+// Lanes 0..k hold the k+1 largest logits in descending order (fewer when E == k): the lanes whose logit and the next one are
+// closer than tol.
+__device__ __forceinline__ unsigned long long close_pairs(float my_val, int lane, int E, int k, float tol) {
+  // the value one lane up (wave_shl:1, a vector-ALU operation): no trip through the LDS crossbar
+  const int mv = __float_as_int(my_val);
+  const float below = __int_as_float(__builtin_amdgcn_update_dpp(mv, mv, 0x130, 0xf, 0xf, false));
+  return __ballot(lane < k && lane + 1 < E && (my_val - below) <= tol * fmaxf(1.0f, fabsf(my_val)));
+}
+
+// The logits that a close call puts in question are those in [lo, hi]: from the first member of a close pair to the last; where the
+// last pair's lower member is the runner-up, a safe margin below it too, since what is there might outrank it.  All others
+// keep their tree-ordered values, which differ from their neighbours' by more than both can move.  (A function of its own, for the
+// callers that have a close call: inside select_topk it took 0.4 us of the one-token kernel, which then held more values than
+// it has scalar registers.)
+__device__ __forceinline__ void close_call_range(float my_val, int lane, int E, int k, float tol, float& lo, float& hi) {
+  const unsigned long long pairs = close_pairs(my_val, lane, E, k, tol);  // not empty
+  const int mv = __float_as_int(my_val);
+  const int first = (int)__builtin_ctzll(pairs), last = 64 - (int)__builtin_clzll(pairs);
+  hi = __int_as_float(__builtin_amdgcn_readlane(mv, first));
+  lo = __int_as_float(__builtin_amdgcn_readlane(mv, last));
+  if (last == k) lo = lo - 2.0f * tol * fmaxf(1.0f, fabsf(lo));
+  asm volatile("" : "+v"(lo), "+v"(hi));  // kept in vector registers: the one-token kernel has no scalar ones to spare
+}
+
 // One wave selects one token's top k.  Lane l holds the logits of experts l, l+64,
 // l+128, l+192; each round finds the wave-wide maximum, locates its owner with ballots
 // (ties -> lowest expert index) and retires it.  One round more than k records
@@ -50,8 +74,7 @@ __device__ __forceinline__ float wave_max_all(float v) {
 // its partial sort then returns is unspecified.  Here such a token gets NaN in every slot's value, hence NaN
 // weights, k distinct experts, and no close-call recomputation.
 __device__ __forceinline__ void select_topk(float (&v)[4], int lane, int E, int k, float& my_val,
-                                            int& my_idx, float& vmax, bool& close_call, float tol,
-                                            float& runner_up) {
+                                            int& my_idx, float& vmax, bool& close_call, float tol) {
   const float NEG = -__builtin_inff();
   constexpr float kLowest = -3.402823466e+38f;
   bool bad = false, finite = false;
@@ -88,14 +111,7 @@ __device__ __forceinline__ void select_topk(float (&v)[4], int lane, int E, int 
         if ((bi >> 6) == j) v[j] = NEG;
     }
   }
-  // lanes 0..k hold the k+1 largest in descending order (fewer when E == k)
-  // the value one lane up (wave_shl:1, a vector-ALU operation) and slot min(k, E - 1) through
-  // a scalar register: no trip through the LDS crossbar
-  const int mv = __float_as_int(my_val);
-  const float below = __int_as_float(__builtin_amdgcn_update_dpp(mv, mv, 0x130, 0xf, 0xf, false));
-  const bool close = lane < k && lane + 1 < E && (my_val - below) <= tol * fmaxf(1.0f, fabsf(my_val));
-  close_call = __any(close) && !poisoned;
-  runner_up = __int_as_float(__builtin_amdgcn_readlane(mv, min(k, E - 1)));
+  close_call = close_pairs(my_val, lane, E, k, tol) != 0ull && !poisoned;
   if (poisoned) {
     my_val = __builtin_nanf("");
     vmax = my_val;
@@ -104,34 +120,140 @@ __device__ __forceinline__ void select_topk(float (&v)[4], int lane, int E, int 
 
 // Logits in the reference's order: a strictly sequential fp32 sum per logit, multiply and
 // add rounded separately (moe_router_node.h:161-167).  The chain of H dependent additions
-// cannot be shortened, everything else can be taken out of its way: the whole workgroup
+// cannot be reordered, but everything else can be taken out of its way: the whole workgroup
 // multiplies (coalesced loads, the products do not depend on the running sum) and stages
-// the rounded products of up to B logits in LDS, one chunk of K ahead; lane c of
-// wave 0 then only reads row c back and adds, all rows side by side.
+// the rounded products in LDS, the waves then only read back and add.
+//
+// A few logits (as a rule two: a close pair): the chain is cut into segments that run side by side, a wave each.  A segment
+// needs the exact sum in front of it, which is not known yet -- but it is known to a few units in the last place, from a sum in
+// any order, and a wave has 64 lanes: each lane adds the segment's products to a sum of its own, the approximate one and
+// the 63 floating-point numbers around it.  When the segment before is done its end is looked up among them, bit for
+// bit, and the segment's end is that lane's.  Where no lane began there (7 to 12 % of the segments of 2880 normally
+// distributed products in four) the segment is added again from its true beginning.  The result is the chain's either way.
+// Many logits: a row per lane of wave 0, all rows side by side, products one chunk of K ahead.
+// A dependent addition takes 8 cycles, 2880 of them 15 us at the 1.5 GHz that a long prompt's GEMMs leave the part at.  The launch
+// with a close call in it: 2048 tokens on 32 experts 31.0 -> 21 us, 4096 on 128 38 -> 27 (8 waves, two rows in four segments);
+// 50 tokens of eight layers, top-8, whose nine largest logits were recomputed in two rounds whichever were close, 515 -> 506 us
+// on average over inputs.
 constexpr int kCcBatch = 8;              // logits recomputed side by side
 constexpr int kCcChunk = 768;            // elements of K staged per step
+constexpr int kCcSplitFloats = 6144;     // products staged at once where chains are cut
 
-template <int B, int CH = kCcChunk>
+template <int NT, int B, int CH = kCcChunk>
 struct CloseCallLdsT {
   static constexpr int kCcStride = CH + 4;  // LDS row stride: rows start four banks apart
   alignas(16) float prod[2][B][kCcStride];
+  static constexpr bool kCut = CH == kCcChunk;  // (the smaller area is that of the one-token kernel, which has none to spare)
+  static_assert(!kCut || 2 * B * kCcStride >= kCcSplitFloats + 64, "reads run up to 64 products past the last row's end");
+  float ends[kCut ? NT / 64 : 1][kCut ? 64 : 1];  // per segment: the lanes' sums ...
+  int around[kCut ? NT / 64 : 1];                 // ... and the bits of the number that lane 32 began with
+  float carry[B];                                 // per row: the sum so far
   float fixed[kMaxExperts];  // the token's logits, recomputed ones replaced
   int cand[kMaxExperts];
   int ncand;
 };
-using CloseCallLds = CloseCallLdsT<kCcBatch>;
+
+// sum + the products of n4 (a multiple of 8) quads in LDS, one after the other, in every lane; quads up to 4 past them are read
+__device__ __forceinline__ float add_in_order(const floatx4* q, int n4, float sum) {
+#pragma clang fp contract(off)
+  floatx4 qa[4], qb[4];
+  auto rd = [&](floatx4(&r)[4], int i0) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r[i] = q[i0 + i];
+  };
+  auto add = [&](const floatx4(&r)[4]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      sum = sum + r[i][0];
+      sum = sum + r[i][1];
+      sum = sum + r[i][2];
+      sum = sum + r[i][3];
+    }
+  };
+  rd(qa, 0);
+  for (int i0 = 0; i0 < n4; i0 += 8) {
+    rd(qb, i0 + 4);
+    add(qa);
+    rd(qa, i0 + 8);
+    add(qb);
+  }
+  return sum;
+}
+
+// The m logits of s.cand (at least two, at most NT / 128 and kCcBatch), chains cut into segments.
+template <int NT, int B, int CH>
+__device__ __forceinline__ void logits_reference_order_cut(const float* __restrict__ x, const float* __restrict__ g,
+                                                           const float* __restrict__ b, int H4, int m,
+                                                           CloseCallLdsT<NT, B, CH>& s) {
+#pragma clang fp contract(off)
+  constexpr int NW = NT / 64, kQuads = kCcSplitFloats / 4;
+  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const CSK_GLOBAL floatx4* x4 = as_global(reinterpret_cast<const floatx4*>(x));
+  const CSK_GLOBAL floatx4* g4 = as_global(reinterpret_cast<const floatx4*>(g));
+  const int R = m <= 2 ? 2 : m <= 4 ? 4 : 8, S = NW / R;  // rows, segments of a row: powers of two
+  const int row4 = kQuads / R;                            // quads of a row that are staged at once
+  const int nb = (H4 + row4 - 1) / row4, per = (H4 + nb - 1) / nb;
+  const int seg4 = ((per + S - 1) / S + 7) & ~7;          // S * seg4 <= row4: row4 / S is a multiple of 8
+  floatx4* const prod = reinterpret_cast<floatx4*>(&s.prod[0][0][0]);
+  const int c = wv / S, j = wv - c * S;
+  const floatx4* const row = prod + c * row4;
+  float sum = 0.0f;
+  for (int h0 = 0; h0 < H4; h0 += per) {
+    const int n4 = min(per, H4 - h0);
+    constexpr int kItems = (kQuads + NT - 1) / NT;
+    floatx4 xq[kItems], gq[kItems];
+#pragma unroll
+    for (int it = 0; it < kItems; ++it) {
+      const int idx = tid + it * NT, r = idx * R / kQuads, i4 = idx - r * row4;
+      xq[it] = gq[it] = floatx4{0.f, 0.f, 0.f, 0.f};  // behind the row's end: adding a zero changes no sum
+      if (r < m && i4 < n4) {
+        xq[it] = x4[h0 + i4];
+        gq[it] = g4[(size_t)s.cand[r] * H4 + h0 + i4];
+      }
+    }
+#pragma unroll
+    for (int it = 0; it < kItems; ++it)
+      if (tid + it * NT < kQuads) prod[tid + it * NT] = xq[it] * gq[it];
+    __syncthreads();
+    if (c < m) {
+      if (j > 0) {
+        float a = 0.0f;
+        for (int i = lane; i < j * seg4; i += 64) a += (row[i][0] + row[i][1]) + (row[i][2] + row[i][3]);
+        const int around = __float_as_int(sum + wave_sum(a));
+        const float end = add_in_order(row + j * seg4, seg4, __int_as_float(around + lane - 32));
+        s.ends[wv][lane] = end;
+        if (lane == 0) s.around[wv] = around;
+      } else {
+        sum = add_in_order(row, seg4, sum);
+      }
+    }
+    __syncthreads();
+    if (c < m && j == 0) {
+      for (int i = 1; i < S; ++i) {
+        const unsigned at = (unsigned)(__float_as_int(sum) - s.around[wv + i] + 32);
+        sum = at < 64u ? s.ends[wv + i][at] : add_in_order(row + i * seg4, seg4, sum);
+      }
+      s.carry[c] = sum;
+    }
+    __syncthreads();
+    if (c < m) sum = s.carry[c];
+  }
+  if (c < m && j == 0 && lane == 0) {
+    const int e = s.cand[c];
+    s.fixed[e] = sum + (b ? b[e] : 0.0f);
+  }
+  __syncthreads();
+}
 
 // Called by all NT threads of the workgroup with the same arguments.  Recomputes the
-// logits that can take part in a close call -- those not below thr, which is set a safe
-// margin under the (k+1)-th largest; the others keep their tree-ordered values, which the
-// bound on the difference keeps on their side of thr -- and leaves all E logits of the
+// logits in [lo, hi] (select_topk) and leaves all E logits of the
 // token in s.fixed.  H must be a multiple of 4.
 template <int NT, int B, int CH>
 __device__ __forceinline__ void logits_reference_order_wg(const float* __restrict__ x,
                                                           const float* __restrict__ g,
                                                           const float* __restrict__ b,
                                                           const float* __restrict__ logit_row, int E,
-                                                          int H, float thr, CloseCallLdsT<B, CH>& s) {
+                                                          int H, float lo, float hi, CloseCallLdsT<NT, B, CH>& s) {
 #pragma clang fp contract(off)
   constexpr int kC4 = CH / 4;
   constexpr int kProducers = NT - 64;  // wave 0 only adds
@@ -142,13 +264,19 @@ __device__ __forceinline__ void logits_reference_order_wg(const float* __restric
   for (int e = tid; e < E; e += NT) {
     const float v = logit_row[e];
     s.fixed[e] = v;
-    if (v >= thr) s.cand[atomicAdd(&s.ncand, 1)] = e;
+    if (v >= lo && v <= hi) s.cand[atomicAdd(&s.ncand, 1)] = e;
   }
   __syncthreads();
   const int m = s.ncand;
   const CSK_GLOBAL floatx4* x4 = as_global(reinterpret_cast<const floatx4*>(x));
   const CSK_GLOBAL floatx4* g4 = as_global(reinterpret_cast<const floatx4*>(g));
   const int H4 = H >> 2;
+  if constexpr (CloseCallLdsT<NT, B, CH>::kCut) {
+    if (m <= min(NT / 128, B)) {
+      logits_reference_order_cut<NT>(x, g, b, H4, m, s);
+      return;
+    }
+  }
   const int nchunk = (H4 + kC4 - 1) / kC4;
   for (int c0 = 0; c0 < m; c0 += B) {
     const int mb = min(B, m - c0);
@@ -159,16 +287,18 @@ __device__ __forceinline__ void logits_reference_order_wg(const float* __restric
 #pragma unroll
       for (int it = 0; it < kItems; ++it) {
         const int idx = ptid + it * kProducers, c = idx / kC4, i4 = idx - c * kC4;
-        if (c < mb && i4 < len4) {
-          xq[it] = x4[h4 + i4];
-          gq[it] = g4[(size_t)s.cand[c0 + c] * H4 + h4 + i4];
+        if (c < mb) {
+          const int i = h4 + min(i4, len4 - 1);
+          xq[it] = x4[i];
+          gq[it] = g4[(size_t)s.cand[c0 + c] * H4 + i];
         }
       }
 #pragma unroll
       for (int it = 0; it < kItems; ++it) {
         const int idx = ptid + it * kProducers, c = idx / kC4, i4 = idx - c * kC4;
-        if (c < mb && i4 < len4)
-          *reinterpret_cast<floatx4*>(&s.prod[ci & 1][c][4 * i4]) = xq[it] * gq[it];
+        const floatx4 p = xq[it] * gq[it];
+        // behind the row's end: adding a zero changes no sum
+        if (c < mb) *reinterpret_cast<floatx4*>(&s.prod[ci & 1][c][4 * i4]) = i4 < len4 ? p : floatx4{0.f, 0.f, 0.f, 0.f};
       }
     };
     if (ptid >= 0) produce(0);
@@ -179,51 +309,8 @@ __device__ __forceinline__ void logits_reference_order_wg(const float* __restric
         if (ci + 1 < nchunk) produce(ci + 1);  // while wave 0 adds chunk ci
       } else if (tid < mb) {
         const int len4 = min(kC4, H4 - ci * kC4);
-        const floatx4* row = reinterpret_cast<const floatx4*>(&s.prod[ci & 1][tid][0]);
-        floatx4 qa[8], qb[8];
-        // reads run up to 15 entries past the chunk (into the next row: never added)
-        auto rd = [&](floatx4(&q)[8], int i0) {
-#pragma unroll
-          for (int i = 0; i < 8; ++i) q[i] = row[i0 + i];
-        };
-        auto add = [&](const floatx4(&q)[8]) {
-#pragma unroll
-          for (int i = 0; i < 8; ++i) {
-            sum = sum + q[i][0];
-            sum = sum + q[i][1];
-            sum = sum + q[i][2];
-            sum = sum + q[i][3];
-          }
-        };
-        auto add_tail = [&](const floatx4(&q)[8], int n) {
-#pragma unroll
-          for (int i = 0; i < 8; ++i) {
-            if (i < n) {
-              sum = sum + q[i][0];
-              sum = sum + q[i][1];
-              sum = sum + q[i][2];
-              sum = sum + q[i][3];
-            }
-          }
-        };
-        // two register sets of eight float4 in rotation: the reads of one are in flight
-        // while the other is added; whole groups carry no guards
-        const int full = len4 & ~7;
-        int i0 = 0;
-        rd(qa, 0);
-        for (; i0 + 16 <= full; i0 += 16) {
-          rd(qb, i0 + 8);
-          add(qa);
-          rd(qa, i0 + 16);
-          add(qb);
-        }
-        if (i0 + 8 <= full) {
-          rd(qb, i0 + 8);
-          add(qa);
-          add_tail(qb, len4 - i0 - 8);
-        } else {
-          add_tail(qa, len4 - i0);
-        }
+        // (reads run into the next row or what lies behind the last one: never added)
+        sum = add_in_order(reinterpret_cast<const floatx4*>(&s.prod[ci & 1][tid][0]), (len4 + 7) & ~7, sum);
       }
       __syncthreads();
     }
@@ -329,7 +416,7 @@ __device__ __forceinline__ int wave_scan_inclusive(int v, int lane) {
 // ceil(c / g) for the group sizes in use (64, 4 and 1) without a run-time integer division
 __device__ __forceinline__ int group_count(int c, int g) { return g == 64 ? (c + 63) >> 6 : g == 4 ? (c + 3) >> 2 : c; }
 
-template <int CCB, int MAXP>
+template <int NT, int CCB, int MAXP>
 struct RouteLds {
   int ids[MAXP];       // expert of assignment p = t * k + slot
   float wts[MAXP];     // its routing weight
@@ -339,13 +426,13 @@ struct RouteLds {
   unsigned long long named[MAXP / 64][kMaxExperts];  // per 64-assignment chunk: the assignments that name the expert
   short before[MAXP / 64][kMaxExperts];              // how many in the chunks before
   unsigned long long ew[kMaxExperts * (sizeof(ExpertW) / 8)];  // the experts' weight pointers, staged early
-  CloseCallLdsT<CCB> cc;
+  CloseCallLdsT<NT, CCB> cc;
   int cc_tok[64], cc_n;
-  float cc_thr[64];
+  float cc_lo[64], cc_hi[64];
 };
 
 template <int NT, int CCB, int MAXP>
-__device__ __forceinline__ void route_workgroup(const RouteIn& r, const RouteOut& o, RouteLds<CCB, MAXP>& s) {
+__device__ __forceinline__ void route_workgroup(const RouteIn& r, const RouteOut& o, RouteLds<NT, CCB, MAXP>& s) {
   constexpr int NW = NT / 64;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int T = r.T, E = r.E, k = r.k;
@@ -394,15 +481,17 @@ __device__ __forceinline__ void route_workgroup(const RouteIn& r, const RouteOut
     for (int q = 0; q < 4; ++q) {
       const int t = t0 + q * NW;
       if (t < T) {
-        float my_val, vmax, runner_up;
+        float my_val, vmax;
         int my_idx;
         bool close_call;
-        select_topk(v[0], lane, E, k, my_val, my_idx, vmax, close_call, tol, runner_up);
+        select_topk(v[0], lane, E, k, my_val, my_idx, vmax, close_call, tol);
         if (close_call) {
+          float lo, hi;
+          close_call_range(my_val, lane, E, k, tol, lo, hi);
           if (lane == 0) {
             const int n = atomicAdd(&s.cc_n, 1);
             s.cc_tok[n] = t;
-            s.cc_thr[n] = runner_up - 2.0f * tol * fmaxf(1.0f, fabsf(runner_up));
+            s.cc_lo[n] = lo, s.cc_hi[n] = hi;
           }
         } else {
           publish_token(t, my_val, my_idx, vmax);
@@ -422,8 +511,8 @@ __device__ __forceinline__ void route_workgroup(const RouteIn& r, const RouteOut
   // reference's order by the whole workgroup, one after the other; wave 0 selects again
   for (int n = 0; n < s.cc_n; ++n) {
     const int t = s.cc_tok[n];
-    logits_reference_order_wg<NT, CCB>(r.x + (size_t)t * r.H, r.g, r.b, r.logits + (size_t)t * E, E, r.H,
-                                       s.cc_thr[n], s.cc);
+    logits_reference_order_wg(r.x + (size_t)t * r.H, r.g, r.b, r.logits + (size_t)t * E, E, r.H, s.cc_lo[n], s.cc_hi[n],
+                              s.cc);
     if (wv == 0) {
       float v[4];
 #pragma unroll
@@ -431,10 +520,10 @@ __device__ __forceinline__ void route_workgroup(const RouteIn& r, const RouteOut
         const int e = lane + 64 * j;
         v[j] = e < E ? s.cc.fixed[e] : NEG;
       }
-      float my_val, vmax, runner_up;
+      float my_val, vmax;
       int my_idx;
       bool close_call;
-      select_topk(v, lane, E, k, my_val, my_idx, vmax, close_call, 0.0f, runner_up);
+      select_topk(v, lane, E, k, my_val, my_idx, vmax, close_call, 0.0f);
       publish_token(t, my_val, my_idx, vmax);
     }
     __syncthreads();

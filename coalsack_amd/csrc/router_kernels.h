@@ -435,12 +435,13 @@ __global__ __launch_bounds__(256) void router_prep_logits_kernel(
 }
 
 // ------------------------------------------------------------------- top-k
-// One wave per token (select_topk).  Weights
+// One wave per token (select_topk), eight tokens to a workgroup: their waves recompute a close call together.  Weights
 // follow moe_router_node.h:180-202: sigmoid of the raw logit, or softmax over
 // the selected k with max subtraction, sum in slot order, multiply by 1/sum.
 // PARTIAL: the logits come as partial sums per split of H.
+constexpr int kTopkThreads = 512, kTopkTokens = kTopkThreads / 64;
 template <bool PARTIAL>
-__global__ __launch_bounds__(256) void router_topk_kernel(float* __restrict__ logits,
+__global__ __launch_bounds__(kTopkThreads, 4) void router_topk_kernel(float* __restrict__ logits,
                                                           float* __restrict__ pairs,
                                                           int* __restrict__ ids, int T, int E,
                                                           int k, int sigmoid,
@@ -450,25 +451,25 @@ __global__ __launch_bounds__(256) void router_topk_kernel(float* __restrict__ lo
                                                           const float* __restrict__ partial,
                                                           int nsplit, Mx3Rider rider) {
   union Lds {
-    CloseCallLds cc;
-    float rows[4 * kMx3LdsWave];
+    CloseCallLdsT<kTopkThreads, kCcBatch> cc;
+    float rows[kTopkTokens * kMx3LdsWave];
   };
   __shared__ __align__(16) Lds lds;
-  CloseCallLds& cc = lds.cc;
-  __shared__ float cc_thr[4];
-  __shared__ int cc_flag[4];
+  auto& cc = lds.cc;
+  __shared__ float cc_lo[kTopkTokens], cc_hi[kTopkTokens];
+  __shared__ int cc_flag[kTopkTokens];
   // Riders: workgroups past the tokens' rewrite the activation rows as FP6 terms for the
   // grouped GEMM.  The two jobs share only their input; a token with a close call keeps
   // one workgroup of this kernel busy for a chain of H dependent additions, during which
   // the rest of the chip would have nothing to do.
   if (rider.x3 && (int)blockIdx.x >= rider.first_wg) {
     const int w = threadIdx.x >> 6;
-    mx3_rows_wave((long)(blockIdx.x - rider.first_wg) * 256 + w * 64, rider.x, rider.x3, rider.rows, rider.nblk,
+    mx3_rows_wave((long)(blockIdx.x - rider.first_wg) * kTopkThreads + w * 64, rider.x, rider.x3, rider.rows, rider.nblk,
                   nullptr, nullptr, lds.rows + w * kMx3LdsWave);
     return;
   }
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int t = blockIdx.x * 4 + wv;
+  const int t = blockIdx.x * kTopkTokens + wv;
   const bool live = t < T;  // waves past the end stay for the barriers below
   const float NEG = -__builtin_inff();
   float v[4];
@@ -507,31 +508,32 @@ __global__ __launch_bounds__(256) void router_topk_kernel(float* __restrict__ lo
     for (int j = 0; j < 4; ++j)
       if (lane + 64 * j < E) v[j] = logits[(size_t)t * E + lane + 64 * j];
   }
-  float my_val, vmax, runner_up;  // lane s keeps slot s
+  float my_val, vmax;  // lane s keeps slot s
   int my_idx;
   bool close_call;
   const float tol = close_call_tolerance(H);
-  select_topk(v, lane, E, k, my_val, my_idx, vmax, close_call, tol, runner_up);
+  select_topk(v, lane, E, k, my_val, my_idx, vmax, close_call, tol);
   close_call = close_call && live;
-  if (lane == 0) {
-    cc_flag[wv] = close_call;
-    cc_thr[wv] = runner_up - 2.0f * tol * fmaxf(1.0f, fabsf(runner_up));
+  if (lane == 0) cc_flag[wv] = close_call;
+  if (close_call) {
+    float lo, hi;
+    close_call_range(my_val, lane, E, k, tol, lo, hi);
+    if (lane == 0) cc_lo[wv] = lo, cc_hi[wv] = hi;
   }
   if (__syncthreads_or(close_call)) {
     // rare: some token of this workgroup has a close call among its k+1 largest logits;
-    // the four waves recompute it together, its own wave selects again
-    for (int w = 0; w < 4; ++w) {
+    // the waves recompute it together, its own wave selects again
+    for (int w = 0; w < kTopkTokens; ++w) {
       if (!cc_flag[w]) continue;
-      const int tw = blockIdx.x * 4 + w;
-      logits_reference_order_wg<256>(x + (size_t)tw * H, g, b, logits + (size_t)tw * E, E, H,
-                                     cc_thr[w], cc);
+      const int tw = blockIdx.x * kTopkTokens + w;
+      logits_reference_order_wg(x + (size_t)tw * H, g, b, logits + (size_t)tw * E, E, H, cc_lo[w], cc_hi[w], cc);
       if (wv == w) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           const int e = lane + 64 * j;
           v[j] = e < E ? cc.fixed[e] : NEG;
         }
-        select_topk(v, lane, E, k, my_val, my_idx, vmax, close_call, 0.0f, runner_up);
+        select_topk(v, lane, E, k, my_val, my_idx, vmax, close_call, 0.0f);
       }
       __syncthreads();
     }
@@ -707,7 +709,7 @@ __global__ __launch_bounds__(kDispatchThreads) void dispatch_scatter_kernel(
 constexpr int kRouteSmallThreads = 1024;
 constexpr int kRouteSmallMaxP = 512;  // assignments
 __global__ __launch_bounds__(kRouteSmallThreads) void route_small_kernel(RouteIn in, RouteOut out) {
-  __shared__ RouteLds<kCcBatch, kRouteSmallMaxP> lds;
+  __shared__ RouteLds<kRouteSmallThreads, kCcBatch, kRouteSmallMaxP> lds;
   route_workgroup<kRouteSmallThreads, kCcBatch, kRouteSmallMaxP>(in, out, lds);
 }
 
@@ -725,8 +727,8 @@ __global__ __launch_bounds__(kRouteSmallThreads) void route_small_kernel(RouteIn
 constexpr int kRouteTinyTokens = 4;
 constexpr int kRouteTinyMaxP = 64;
 __global__ __launch_bounds__(256) void route_tiny_kernel(RouteIn r, RouteOut o) {
-  __shared__ CloseCallLds cc;
-  __shared__ float cc_thr[4];
+  __shared__ CloseCallLdsT<256, kCcBatch> cc;
+  __shared__ float cc_lo[4], cc_hi[4];
   __shared__ int cc_flag[4];
   __shared__ int s_ids[kRouteTinyMaxP];
   __shared__ float s_w[kRouteTinyMaxP];
@@ -750,15 +752,17 @@ __global__ __launch_bounds__(256) void route_tiny_kernel(RouteIn r, RouteOut o) 
     const int e = lane + 64 * j;
     v[j] = (live && e < E) ? r.logits[(size_t)t * E + e] : NEG;
   }
-  float my_val, vmax, runner_up;  // lane s keeps slot s
+  float my_val, vmax;  // lane s keeps slot s
   int my_idx;
   bool close_call;
   const float tol = close_call_tolerance(r.H);
-  select_topk(v, lane, E, k, my_val, my_idx, vmax, close_call, tol, runner_up);
+  select_topk(v, lane, E, k, my_val, my_idx, vmax, close_call, tol);
   close_call = close_call && live;
-  if (lane == 0) {
-    cc_flag[wv] = close_call;
-    cc_thr[wv] = runner_up - 2.0f * tol * fmaxf(1.0f, fabsf(runner_up));
+  if (lane == 0) cc_flag[wv] = close_call;
+  if (close_call) {
+    float lo, hi;
+    close_call_range(my_val, lane, E, k, tol, lo, hi);
+    if (lane == 0) cc_lo[wv] = lo, cc_hi[wv] = hi;
   }
 #pragma unroll
   for (int i = 0; i < kEwPerThread; ++i) {
@@ -768,15 +772,14 @@ __global__ __launch_bounds__(256) void route_tiny_kernel(RouteIn r, RouteOut o) 
   if (__syncthreads_or(close_call)) {
     for (int w = 0; w < 4; ++w) {
       if (!cc_flag[w]) continue;
-      logits_reference_order_wg<256>(r.x + (size_t)w * r.H, r.g, r.b, r.logits + (size_t)w * E, E, r.H,
-                                     cc_thr[w], cc);
+      logits_reference_order_wg(r.x + (size_t)w * r.H, r.g, r.b, r.logits + (size_t)w * E, E, r.H, cc_lo[w], cc_hi[w], cc);
       if (wv == w) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           const int e = lane + 64 * j;
           v[j] = e < E ? cc.fixed[e] : NEG;
         }
-        select_topk(v, lane, E, k, my_val, my_idx, vmax, close_call, 0.0f, runner_up);
+        select_topk(v, lane, E, k, my_val, my_idx, vmax, close_call, 0.0f);
       }
       __syncthreads();
     }

@@ -902,10 +902,10 @@ int run_experts(int64_t E, int64_t T, int64_t k, int64_t H, int64_t F,
 }
 
 int launch_combine(const float* y, const float* pairs, const int* pos, const float* residual,
-                   float* out, int64_t T, int64_t k, int64_t H, int pre_weighted) {
+                   float* out, int64_t T, int64_t k, int64_t H, int pre_weighted, float* pairs_out = nullptr) {
   if (T == 0) return CSK_OK;
   combine_kernel<<<dim3((unsigned)cdiv(H, 1024), (unsigned)T), 256, 0, g_stream>>>(
-      y, pairs, pos, residual, out, (int)T, (int)k, (int)H, pre_weighted);
+      y, pairs, pos, residual, out, (int)T, (int)k, (int)H, pre_weighted, reinterpret_cast<float2*>(pairs_out));
   return check_launch("combine_kernel");
 }
 
@@ -1883,8 +1883,9 @@ constexpr int64_t kRouteSmallTokens = 31;
 static_assert(kRouteSmallTokens * kMaxTopK <= kRouteSmallMaxP, "what its LDS is laid out for");
 // phase 0: the whole forward; 1: up to and including the dispatch (router output and lists
 // are in ws); 2: the rest (experts and combine) of a pass whose phase 1 ran in the same ws.
+// pairs_out: takes a copy of the router output, if given.
 int forward_pass(csk_layer* L, const float* hidden, int64_t T, float* out, int flags, Workspace& ws = g_ws,
-                 int phase = 0) {
+                 int phase = 0, float* pairs_out = nullptr) {
   int rc = CSK_OK;
   if (phase != 2) {
     rc = ws.ensure(T, L->E, L->k, L->H, L->F, L->wbf);
@@ -1973,7 +1974,7 @@ int forward_pass(csk_layer* L, const float* hidden, int64_t T, float* out, int f
     if (rc != CSK_OK) return rc;
     mark(CSK_STAGE_COMBINE);
     rc = launch_combine(ws.y, ws.pairs, ws.pos, (flags & CSK_FWD_RESIDUAL) ? hidden : nullptr, out,
-                        T, L->k, L->H, L->wbf);
+                        T, L->k, L->H, L->wbf, pairs_out);
     mark(CSK_N_STAGES);
     g_stage_valid = g_timing;
     return rc;
@@ -1993,7 +1994,7 @@ int forward_pass(csk_layer* L, const float* hidden, int64_t T, float* out, int f
   if (rc != CSK_OK) return rc;
   mark(CSK_STAGE_COMBINE);
   rc = launch_combine(ws.y, ws.pairs, ws.pos, (flags & CSK_FWD_RESIDUAL) ? hidden : nullptr, out, T,
-                      L->k, L->H, L->wbf);
+                      L->k, L->H, L->wbf, pairs_out);
   mark(CSK_N_STAGES);
   g_stage_valid = g_timing;
   return rc;
@@ -2074,10 +2075,15 @@ extern "C" int csk_moe_forward_host(csk_layer* L, const float* hidden, int64_t T
     int64_t np, each;
     pass_plan(T, np, each);
     L->last_T = np == 1 ? T : -1;
+    // a router output that fits the pinned area is written there by the last kernel, too
+    const size_t pair_bytes = (size_t)T * L->k * 2 * sizeof(float);
+    float* const pinned_pairs = rc == CSK_OK && np == 1 ? static_cast<float*>(g_pinned.take(pair_bytes)) : nullptr;
     for (int64_t t0 = 0; t0 < T && rc == CSK_OK; t0 += each) {
       const int64_t tn = std::min(each, T - t0);
-      rc = forward_pass(L, dh + t0 * L->H, tn, dout + t0 * L->H, flags);
-      if (rc == CSK_OK)
+      rc = forward_pass(L, dh + t0 * L->H, tn, dout + t0 * L->H, flags, g_ws, 0, pinned_pairs);
+      if (rc == CSK_OK && pinned_pairs)
+        g_fetches.push_back(PendingFetch{pairs_out, pinned_pairs, nullptr, pair_bytes});
+      else if (rc == CSK_OK)
         // (before the next pass overwrites them)
         rc = fetch(pairs_out + t0 * L->k * 2, g_ws.pairs, (size_t)tn * L->k * 2 * sizeof(float), /*now=*/np > 1);
     }

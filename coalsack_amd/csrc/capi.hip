@@ -481,13 +481,14 @@ int finish_fetches() {
 
 // Upload `rows x K` reference blocks and repack into (q, s).  The staging buffer is kept
 // between calls (a checkpoint is hundreds of matrices of one size; the stream orders one
-// matrix behind the other) up to the size of a large expert matrix; the scale bytes are
+// call behind the other) up to the size of a large expert's matrices; the scale bytes are
 // checked by the pack kernel as it reads them, so the host touches the blocks only to hand
 // them to the link.  After a refused block the planes of m hold partial data.
 uint8_t* g_stage = nullptr;
 size_t g_stage_cap = 0;
 constexpr size_t kStageKept = (size_t)256 << 20;  // (8192 x 8192 halves are 128 MiB)
 unsigned long long* g_bad = nullptr;  // first refused block of up to three matrices
+bool g_bad_dirty = true;              // it may hold something else than ~0
 
 // The end of an entry point.  A call that came to its end has finished its transfers, so only one
 // that failed in between leaves any: its results go nowhere -- the caller's memory may be gone
@@ -505,7 +506,11 @@ void end_call() {
   }
 }
 
-int stage_bytes(size_t bytes) {
+int stage_bytes(size_t bytes) {  // on return g_bad holds ~0: set once, and again after a refused block
+  const auto clear_bad = [] {
+    fill_cells_kernel<<<1, 64, 0, g_stream>>>(g_bad, 3, ~0ull);
+    return check_launch("fill_cells_kernel");
+  };
   if (bytes > g_stage_cap) {
     HIP_TRY(hipStreamSynchronize(g_stream));
     if (g_stage) (void)hipFree(g_stage);
@@ -514,30 +519,59 @@ int stage_bytes(size_t bytes) {
     g_stage_cap = bytes;
   }
   if (!g_bad) HIP_TRY(counted_malloc((void**)&g_bad, 3 * sizeof(unsigned long long)));
+  if (g_bad_dirty) CSK_TRY(clear_bad());
+  g_bad_dirty = false;
   return CSK_OK;
+}
+
+// Up to three matrices of host memory into the staging buffer, side by side, as one transfer; pack(i, staged) queues what turns
+// matrix i into its resident form behind its last bytes.
+template <class Pack>
+int stage_matrices(const void* const* host, const size_t* bytes, int n, Pack pack) {
+  size_t at[CopyCrew::kParts], total = 0, most = 0;
+  bool small = false;
+  for (int i = 0; i < n; ++i) {
+    at[i] = total;
+    total += (bytes[i] + 255) & ~(size_t)255;
+    most = std::max(most, bytes[i]);
+    small = small || bytes[i] <= PinnedArena::kMaxTransfer;
+  }
+  // each on its own, in one place: those that go through the pinned area, and those that would not be kept room for together
+  if (small || total > kStageKept) {
+    CSK_TRY(stage_bytes(most));
+    for (int i = 0; i < n; ++i) {
+      CSK_TRY(upload(g_stage, host[i], bytes[i]));
+      CSK_TRY(pack(i, g_stage));
+    }
+    return CSK_OK;
+  }
+  CSK_TRY(stage_bytes(total));
+  HostLink::Part parts[CopyCrew::kParts];
+  for (int i = 0; i < n; ++i) parts[i] = HostLink::Part{g_stage + at[i], host[i], bytes[i]};
+  int rc = CSK_OK;
+  HIP_TRY(g_link.to_device(parts, n, g_stream, [&](int i) { return (rc = pack(i, g_stage + at[i])) == CSK_OK; }));
+  return rc;
 }
 
 // n <= 3 matrices, queued one behind the other; finish_pack waits for them
 int queue_pack(const uint8_t* const* host, csk_mxfp4* const* ms, int n) {
-  size_t most = 0;
-  for (int i = 0; i < n; ++i) most = std::max(most, (size_t)(ms[i]->rows * ms[i]->nblk) * 17);
-  CSK_TRY(stage_bytes(most));
-  fill_cells_kernel<<<1, 64, 0, g_stream>>>(g_bad, n, ~0ull);
-  CSK_TRY(check_launch("fill_cells_kernel"));
-  for (int i = 0; i < n; ++i) {
+  const void* src[CopyCrew::kParts];
+  size_t bytes[CopyCrew::kParts];
+  for (int i = 0; i < n; ++i) src[i] = host[i], bytes[i] = (size_t)(ms[i]->rows * ms[i]->nblk) * 17;
+  return stage_matrices(src, bytes, n, [&](int i, const uint8_t* staged) {
     csk_mxfp4& m = *ms[i];
-    CSK_TRY(upload(g_stage, host[i], (size_t)(m.rows * m.nblk) * 17));
     const long ent = m.entries();
+    g_bad_dirty = true;  // until finish_pack has seen what it holds
     pack_mxfp4_kernel<<<dim3((unsigned)cdiv(ent, 256)), 256, 0, g_stream>>>(
-        g_stage, m.q, m.s, (int)m.rows, (int)m.nblk, ent, g_bad + i);
-    CSK_TRY(check_launch("pack_mxfp4_kernel"));
-  }
-  return CSK_OK;
+        staged, m.q, m.s, (int)m.rows, (int)m.nblk, ent, g_bad + i);
+    return check_launch("pack_mxfp4_kernel");
+  });
 }
 int finish_pack(int n) {
   unsigned long long bad[3] = {~0ull, ~0ull, ~0ull};
   CSK_TRY(fetch(bad, g_bad, n * sizeof bad[0]));
   CSK_TRY(finish_fetches());
+  g_bad_dirty = bad[0] != ~0ull || bad[1] != ~0ull || bad[2] != ~0ull;
   for (int i = 0; i < n; ++i)
     if (bad[i] != ~0ull)
       return fail(CSK_ERR_SCALE, "MXFP4 scale byte 255 on block " + std::to_string(bad[i]) +
@@ -1518,25 +1552,37 @@ size_t ggml_matrix_bytes(int type, int64_t rows, int64_t K) {
   if (type == kGgmlQ6K) return n % 256 ? 0 : n / 256 * 210;
   return 0;
 }
-// row-major matrix on the host (halves, or a Q4_K / Q6_K stream) -> fp16 tiles at dst, queued on the stream
-int queue_f16_pack(const void* data, int type, int64_t rows, int64_t K, u32x4* dst) {
-  const size_t bytes = ggml_matrix_bytes(type, rows, K);
-  if (!bytes)
-    return fail(CSK_ERR_ARG, "fp16 experts take ggml types F16 (1), Q4_K (12) and Q6_K (14), K-quants with rows * K a multiple of 256");
-  CSK_TRY(stage_bytes(bytes));
-  CSK_TRY(upload(g_stage, data, bytes));
-  const long ent = f16_entries(rows, K);
-  const dim3 grid((unsigned)cdiv(ent, 256));
-  if (type == kGgmlF16Type)
-    f16_pack_kernel<<<grid, 256, 0, g_stream>>>(reinterpret_cast<const uint16_t*>(g_stage), dst, rows, K, ent);
-  else if (type == kGgmlQ4K)
-    kquant_pack_kernel<kGgmlQ4K><<<grid, 256, 0, g_stream>>>(g_stage, dst, rows, K, ent);
-  else
-    kquant_pack_kernel<kGgmlQ6K><<<grid, 256, 0, g_stream>>>(g_stage, dst, rows, K, ent);
-  return check_launch("f16_pack_kernel");
+// row-major matrices on the host (halves, or a Q4_K / Q6_K stream) -> fp16 tiles at dst, queued on the stream
+struct F16Pack {
+  const void* data;
+  int type;
+  int64_t rows, K;
+  u32x4* dst;
+};
+int queue_f16_pack(const F16Pack* ms, int n) {
+  const void* src[CopyCrew::kParts];
+  size_t bytes[CopyCrew::kParts];
+  for (int i = 0; i < n; ++i) {
+    src[i] = ms[i].data, bytes[i] = ggml_matrix_bytes(ms[i].type, ms[i].rows, ms[i].K);
+    if (!bytes[i])
+      return fail(CSK_ERR_ARG, "fp16 experts take ggml types F16 (1), Q4_K (12) and Q6_K (14), K-quants with rows * K a multiple of 256");
+  }
+  return stage_matrices(src, bytes, n, [&](int i, const uint8_t* staged) {
+    const F16Pack& m = ms[i];
+    const long ent = f16_entries(m.rows, m.K);
+    const dim3 grid((unsigned)cdiv(ent, 256));
+    if (m.type == kGgmlF16Type)
+      f16_pack_kernel<<<grid, 256, 0, g_stream>>>(reinterpret_cast<const uint16_t*>(staged), m.dst, m.rows, m.K, ent);
+    else if (m.type == kGgmlQ4K)
+      kquant_pack_kernel<kGgmlQ4K><<<grid, 256, 0, g_stream>>>(staged, m.dst, m.rows, m.K, ent);
+    else
+      kquant_pack_kernel<kGgmlQ6K><<<grid, 256, 0, g_stream>>>(staged, m.dst, m.rows, m.K, ent);
+    return check_launch("f16_pack_kernel");
+  });
 }
 int f16_pack_into(const void* data, int type, int64_t rows, int64_t K, u32x4* dst) {
-  CSK_TRY(queue_f16_pack(data, type, rows, K, dst));
+  const F16Pack m{data, type, rows, K, dst};
+  CSK_TRY(queue_f16_pack(&m, 1));
   return finish_fetches();
 }
 int f16_export_from(const u32x4* src, int64_t rows, int64_t K, uint16_t* halves) {
@@ -1774,6 +1820,7 @@ extern "C" int csk_f16_upload_f32(const float* w_host, int64_t rows, int64_t K, 
     // largest magnitude first (g_bad's eight bytes serve as the 32-bit cell), then the split of w / wscale
     const long n = (long)rows * K;
     unsigned int top = 0u;
+    g_bad_dirty = true;
     fill_cells_kernel<<<1, 64, 0, g_stream>>>(g_bad, 1, 0ull);
     f32_absmax_bits_kernel<<<dim3((unsigned)std::min<long>(cdiv(n, 256), 8L * std::max(g_cus, 1))), 256, 0, g_stream>>>(
         stage.as<float>(), n, reinterpret_cast<unsigned int*>(g_bad));
@@ -1827,9 +1874,10 @@ extern "C" int csk_layer_set_expert_f16(csk_layer* L, int64_t e, const uint16_t*
   CSK_TRY(check_biases(b_up, b_gate, b_down));
   if (w_up) {
     L->matrix_set[(size_t)e] = L->expert_set[(size_t)e] = 0;  // until all of it has arrived
-    CSK_TRY(queue_f16_pack(w_up, kGgmlF16Type, L->F, L->H, L->view16(e, CSK_W_UP)));
-    CSK_TRY(queue_f16_pack(w_gate, kGgmlF16Type, L->F, L->H, L->view16(e, CSK_W_GATE)));
-    CSK_TRY(queue_f16_pack(w_down, kGgmlF16Type, L->H, L->F, L->view16(e, CSK_W_DOWN)));
+    const F16Pack ms[3] = {{w_up, kGgmlF16Type, L->F, L->H, L->view16(e, CSK_W_UP)},
+                           {w_gate, kGgmlF16Type, L->F, L->H, L->view16(e, CSK_W_GATE)},
+                           {w_down, kGgmlF16Type, L->H, L->F, L->view16(e, CSK_W_DOWN)}};
+    CSK_TRY(queue_f16_pack(ms, 3));
   }
   CSK_TRY(upload_biases(L, e, b_up, b_gate, b_down));
   CSK_TRY(finish_fetches());

@@ -12,7 +12,9 @@
 //  * the host side is memcpy, 28 GB/s on one core for memory that no cache holds, so a large
 //    transfer is copied by the calling thread and a few helpers together.
 // Measured: experts of 13.2 MB from host memory into HBM 20 -> 42 GB/s (3 matrices each, a wait per
-// expert); 3.3 MB of results down 255 -> 95 us; a two-token frame through host buffers 79 -> 59 us.
+// expert); 3.3 MB of results down 255 -> 95 us; a two-token frame through host buffers 79 -> 59 us.  With an expert's
+// matrices in one transfer, chunks as long as the host's lead allows and events only where the ring comes round: eight such
+// experts and a token 2870 -> 2600 us (of 1024 x 512 780 -> 645); 1024 x 4096 x 8192 through host buffers 1340 -> 1230.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -89,13 +91,33 @@ class CopyCrew {
     for (std::thread& t : threads_) t.join();
   }
 
-  // byte o of the transfer lies at ring[(at + o) % ring_bytes]; `at` is a multiple of a piece
+  // A transfer of up to kParts arrays, one behind the other, each from the beginning of a piece on.  Piece i lies at
+  // ring[(at + i * kLinkPiece) % ring_bytes]; `at` is a multiple of a piece.
+  static constexpr int kParts = 3;
   struct Job {
-    char* host;
+    char* host[kParts];
+    size_t bytes[kParts];
+    long first[kParts + 1];  // piece that a part begins with
+    int parts;
     char* ring;
-    size_t bytes, at, ring_bytes;
+    size_t at, ring_bytes;
     bool up;
-    long pieces() const { return (long)((bytes + kLinkPiece - 1) / kLinkPiece); }
+    Job(char* ring_, size_t at_, size_t ring_bytes_, bool up_) : parts(0), ring(ring_), at(at_), ring_bytes(ring_bytes_), up(up_) {
+      first[0] = 0;
+    }
+    Job(char* host_, char* ring_, size_t bytes_, size_t at_, size_t ring_bytes_, bool up_) : Job(ring_, at_, ring_bytes_, up_) { add(host_, bytes_); }
+    Job() : Job(nullptr, 0, 1, true) {}
+    void add(void* h, size_t n) {
+      host[parts] = static_cast<char*>(h), bytes[parts] = n;
+      first[parts + 1] = first[parts] + (long)((n + kLinkPiece - 1) / kLinkPiece);
+      ++parts;
+    }
+    long pieces() const { return first[parts]; }
+    int part_of(long piece) const {
+      int p = 0;
+      while (piece >= first[p + 1]) ++p;
+      return p;
+    }
   };
 
   // false: no memory for the list of pieces.  Helpers that cannot be started are done
@@ -136,12 +158,13 @@ class CopyCrew {
     do {
       if (i >= open_.load(std::memory_order_acquire)) return false;
     } while (!next_.compare_exchange_weak(i, i + 1, std::memory_order_acq_rel));
-    const size_t off = (size_t)i * kLinkPiece, len = std::min(kLinkPiece, job_.bytes - off);
-    char* const r = job_.ring + (job_.at + off) % job_.ring_bytes;
+    const int p = job_.part_of(i);
+    const size_t off = (size_t)(i - job_.first[p]) * kLinkPiece, len = std::min(kLinkPiece, job_.bytes[p] - off);
+    char* const r = job_.ring + (job_.at + (size_t)i * kLinkPiece) % job_.ring_bytes;
     if (job_.up)
-      std::memcpy(r, job_.host + off, len);
+      std::memcpy(r, job_.host[p] + off, len);
     else
-      std::memcpy(job_.host + off, r, len);
+      std::memcpy(job_.host[p] + off, r, len);
     done_[(size_t)i].store(true, std::memory_order_release);
     return true;
   }
@@ -254,21 +277,53 @@ class HostLink {
   // dst (device) <- host memory, queued on the stream.  The host memory may be reused on return.
   hipError_t to_device(void* dst, const void* host, size_t bytes, hipStream_t st) {
     if (bytes == 0) return hipSuccess;
-    if (!ready()) return by_runtime(dst, host, bytes, hipMemcpyHostToDevice, st);
+    const Part part{dst, host, bytes};
+    return to_device(&part, 1, st, [](int) { return true; });
+  }
+
+  // The same for up to CopyCrew::kParts arrays, none of them empty.  queued(p) is called when the last of part p has been
+  // queued, and queues what is to be done with it; false: no more of the transfer.  As a transfer of its own each array
+  // began with an empty ring, 20 us in which the device had nothing to do.
+  struct Part {
+    void* dst;
+    const void* host;
+    size_t bytes;
+  };
+  template <class Queued>
+  hipError_t to_device(const Part* parts, int n_parts, hipStream_t st, Queued queued) {
+    CopyCrew::Job job(ring_, at_, kLinkRing, true);
+    for (int p = 0; p < n_parts; ++p) job.add(const_cast<void*>(parts[p].host), parts[p].bytes);
+    if (!ready() || (job.ring = ring_, !crew_->begin(job))) {
+      for (int p = 0; p < n_parts; ++p) {
+        const hipError_t rc = by_runtime(parts[p].dst, parts[p].host, parts[p].bytes, hipMemcpyHostToDevice, st);
+        if (rc != hipSuccess || !queued(p)) return rc;
+      }
+      return hipSuccess;
+    }
     hipError_t err = hipSuccess;
-    CopyCrew::Job job{static_cast<char*>(const_cast<void*>(host)), ring_, bytes, at_, kLinkRing, true};
     const long n = job.pieces();
-    // A copy kernel costs about 3.5 us of its own.  Onto an idle stream the first ones are
-    // short, so that the device starts early; they grow as the host gets ahead.
     const long first = (long)(at_ / kLinkPiece);
+    // Only a transfer that comes round to where it or one before it began has its quarters marked by events: each costs
+    // the device 5 us between two copies.  The others leave that to whoever needs their quarters next.
+    const bool round = first + n > kPieces;
     long ready_to = 0, sent = 0, opened = 0, want = first == 0 ? 3 : 16;
-    if (!crew_->begin(job)) return by_runtime(dst, host, bytes, hipMemcpyHostToDevice, st);
+    int part = 0;
+    // A copy kernel costs about 3.5 us of its own.  Onto an idle stream the first ones are short, so that the device starts
+    // early; they grow to 1 MiB, and beyond where the host gets ahead: pieces are sent only when the device is about to
+    // run out of work, together with all that has been copied by then (chunks of 1 MiB cross the link at 49 GB/s, of 4 at 55).
+    using Clock = std::chrono::steady_clock;
+    constexpr double kLaunchNs = 15000.0;  // from here to a copy kernel's first bytes, a piece copied in between included
+    constexpr double kKernelNs = 3500.0;   // of a copy kernel's own ...
+    constexpr double kNsPerByte = 1.0 / 55.0;  // ... and the link's rate
+    const auto t0 = Clock::now();
+    auto now = [&] { return (double)std::chrono::duration_cast<std::chrono::nanoseconds>(Clock::now() - t0).count(); };
+    double busy_until = 0.0;
     DeviceWait wait;
     while (sent < n && err == hipSuccess) {
       while (opened < n) {  // pieces whose place in the ring is free, up to the end of their quarter
         const long end = quarter_end(first + opened);
         // what lay there a round before has been sent, and the device has read it
-        if (first + sent < end - kPieces || !free_quarter((int)((end - 1) % kPieces / kPerQuarter), err)) break;
+        if (first + sent < end - kPieces || !free_quarter((int)((end - 1) % kPieces / kPerQuarter), st, err)) break;
         opened = std::min(n, end - first);
         crew_->open_to(opened);
       }
@@ -276,18 +331,23 @@ class HostLink {
       const bool worked = crew_->work_one();
       while (ready_to < n && ready_to < opened && crew_->done(ready_to)) ++ready_to;
       // up to the end of a quarter of the ring: its event says when it may be filled again
-      const long q_end = quarter_end(first + sent) - first;
-      const long to = std::min(ready_to, q_end);
-      if (to > sent && (to - sent >= want || to == n || to == q_end)) {
-        const size_t a = (size_t)sent * kLinkPiece, len = std::min(bytes, (size_t)to * kLinkPiece) - a;
-        err = launch(static_cast<char*>(dst) + a, ring_ + (at_ + a) % kLinkRing, len, st);
-        if (err == hipSuccess && to == q_end) {
+      const long q_end = (round ? quarter_end(first + sent) : kPieces) - first, p_end = job.first[part + 1];
+      const long to = std::min(ready_to, std::min(q_end, p_end));
+      double t = 0.0;
+      if (to > sent && (to == p_end || to == q_end || (to - sent >= want && (t = now()) >= busy_until - kLaunchNs))) {
+        const size_t a = (size_t)(sent - job.first[part]) * kLinkPiece;
+        const size_t len = std::min(parts[part].bytes, (size_t)(to - job.first[part]) * kLinkPiece) - a;
+        err = launch(static_cast<char*>(parts[part].dst) + a, ring_ + (at_ + (size_t)sent * kLinkPiece) % kLinkRing, len, st);
+        for (long q = (first + sent) / kPerQuarter; q * kPerQuarter < first + to; ++q) in_use_[q % kQuarters] = true, marked_[q % kQuarters] = false;
+        if (err == hipSuccess && round && to == q_end) {
           const int q = (int)((first + sent) % kPieces / kPerQuarter);
           err = hipEventRecord(quarter_[q], st);
-          in_use_[q] = true;
+          marked_[q] = true;
         }
+        busy_until = std::max(t != 0.0 ? t : now(), busy_until) + kKernelNs + (double)len * kNsPerByte;
         sent = to;
-        want = std::min(2 * want, 16L);  // (longer ones would leave the device waiting for the host)
+        want = std::min(2 * want, 16L);
+        if (sent == p_end && err == hipSuccess && !queued(part++)) break;
         wait.progress();
       } else if (worked) {
         wait.progress();
@@ -308,7 +368,7 @@ class HostLink {
     if (!ready()) return by_runtime(host, src, bytes, hipMemcpyDeviceToHost, st);
     hipError_t err = hipSuccess;
     // (places in the ring that an earlier transfer up still reads are written after it, in stream order)
-    CopyCrew::Job job{static_cast<char*>(host), ring_, bytes, 0, kLinkRing, false};
+    CopyCrew::Job job(static_cast<char*>(host), ring_, bytes, 0, kLinkRing, false);
     const long n = job.pieces();
     long queued = 0, landed = 0, freed = 0;  // pieces requested, in pinned memory, copied out
     long ends[kDown];
@@ -316,10 +376,10 @@ class HostLink {
     if (!crew_->begin(job)) return by_runtime(host, src, bytes, hipMemcpyDeviceToHost, st);
     DeviceWait wait;
     while (freed < n && err == hipSuccess) {
-      // Half of what is left per chunk, at most 1 MiB: few chunks (each costs about 6 us for
-      // its kernel and event), and little left to copy once the last has landed.
+      // Half of what is left per chunk, at most 4 MiB and at least 512 KiB: few chunks (each costs about 9 us for
+      // its kernel and event, half of what a MiB takes), and little left to copy once the last has landed.
       while (queued < n && put - got < kDown && err == hipSuccess) {
-        long len = std::max(4L, std::min(16L, (n - queued + 1) / 2));
+        long len = std::max(8L, std::min(64L, (n - queued + 1) / 2));
         len = std::min(len, n - queued);
         const long to_wrap = kPieces - queued % kPieces;
         len = std::min(len, to_wrap);
@@ -368,6 +428,7 @@ class HostLink {
   size_t at_ = 0;  // where the next transfer up starts
   hipEvent_t quarter_[kQuarters] = {}, down_[kDown] = {};
   bool in_use_[kQuarters] = {};  // the device may still be reading that quarter
+  bool marked_[kQuarters] = {};  // and its event comes behind the last copy that does
   CrewOwner crew_;
   bool refused_ = false;
 
@@ -400,8 +461,13 @@ class HostLink {
     link_copy_kernel<<<dim3(blocks), kLinkThreads, 0, st>>>(static_cast<const unsigned char*>(src), static_cast<unsigned char*>(dst), bytes);
     return hipGetLastError();
   }
-  bool free_quarter(int q, hipError_t& err) {
+  bool free_quarter(int q, hipStream_t st, hipError_t& err) {
     if (!in_use_[q]) return true;
+    if (!marked_[q]) {
+      err = hipEventRecord(quarter_[q], st);
+      if (err != hipSuccess) return false;
+      marked_[q] = true;
+    }
     const hipError_t rc = hipEventQuery(quarter_[q]);
     if (rc == hipErrorNotReady) {
       (void)hipGetLastError();

@@ -843,7 +843,10 @@ int launch_gemm_mx(ExpertGemmMxArgs& ga, int64_t E, int64_t P) {
     lds_attr_set = true;
   }
   const int64_t max_mtiles = P / kGemmBM + std::min<int64_t>(E, P);
-  const dim3 grid((unsigned)(cdiv(max_mtiles * ga.n_ntiles, 2 * kDies) * 2 * kDies));  // (one or two parts per die)
+  ga.cus_per_die = std::max(g_cus / kDies, 1);
+  // one or two parts per die, and a second half for as many units as a die may take in halves
+  const int64_t halves = NG == kMxNG ? kDies * (ga.cus_per_die / 2) : 0;
+  const dim3 grid((unsigned)(cdiv(max_mtiles * ga.n_ntiles, 2 * kDies) * 2 * kDies + halves));
   launch_expert_kernel(MODE, expert_gemm_mx_kernel<MODE, NG>, grid, dim3(64 * kMxWaves), Geom::kLdsBytes, ga);
   return check_launch("expert_gemm_mx_kernel");
 }

@@ -78,6 +78,15 @@ __device__ __forceinline__ const CSK_GLOBAL T* as_global(const T* p) {
   return (const CSK_GLOBAL T*)p;
 }
 
+// How many of a die's work units (n of them, each as long as a compute unit of the die needs for one) the grouped GEMMs of
+// 64-token tiles take in halves of 32 tokens, at the end of its sequence.  Where the last round of units would occupy at most
+// half of the compute units, its halves occupy twice as many and the round is about half as long.  An unbroken
+// last round of more than half of them is no longer than two rounds of halves, which read its weights twice.
+__device__ __forceinline__ int halved_units(int n, int cus_per_die) {
+  const int last = n % cus_per_die;
+  return 2 * last <= cus_per_die ? last : 0;
+}
+
 // Scale-plane geometry (see ExpertW).
 __host__ __device__ inline int scale_slots(int nblk) {
   const int per_wave = (((nblk + 3) >> 2) + 3) >> 2;

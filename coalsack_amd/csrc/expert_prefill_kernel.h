@@ -76,6 +76,7 @@ struct ExpertGemmMxArgs {
   int N;
   int act_type;
   int two_part_units;    // from this many work units on, a die takes two parts of their sequence
+  int cus_per_die;
   u32x4* act_out;        // MODE 0: [P][mx3_row_blocks(N / 32)][6] x 16 B
   float* y_out;          // MODE 1: [P][N]
 };
@@ -566,15 +567,30 @@ __device__ __forceinline__ void expert_gemm_mx_unit(const ExpertGemmMxArgs& a, c
 // first (layer, us, one part / two: 128 experts of 2880 x 2880, 4096 tokens 967 / 950, 1000 tokens 511 / 501; 16 of
 // 4096 x 6144, 2000 tokens 615 / 600).  With fewer units a part's ends, whose experts two dies share, weigh more (the same
 // 16 experts, 1000 tokens 366 / 374; units of 256 rows: 128 experts, 300 tokens 404 / 410).
+// The last of a die's units of 512 rows may be halves (halved_units): layer, us, whole units / so, 32 experts of 2880 x 2880, top-4,
+// 512 tokens 188.6 / 184.6, 700 195.6 / 191.3, 1500 310 / 304, 2048 400 / 394; 16 of 4096 x 6144, top-2, 1000 tokens 334 / 319; 8 of
+// 2880 x 2880, 1000 tokens 199.5 / 193.6; none of 26 such layers more than a per cent slower.  Halves of 256 rows in place
+// of tokens gain as much, but with their code in the kernel the tall units hold 10 registers in memory and lose it again; always
+// halving the last round, or half of it, is 1.7 and 0.9 % slower over the same layers.
 template <int MODE, int NG>
 __global__ __launch_bounds__(64 * kMxWaves, NG == 2 ? 3 : 2) void expert_gemm_mx_kernel(ExpertGemmMxArgs a) {
   extern __shared__ __align__(16) unsigned char smem[];
   const int n_units = *a.n_mtiles * a.n_ntiles;
-  const int die = blockIdx.x % kDies, slot = blockIdx.x / kDies;
+  const int die = blockIdx.x % kDies;
+  int slot = blockIdx.x / kDies;
   const bool two_parts = NG == kMxNG && n_units >= a.two_part_units;
   const int part = two_parts ? (n_units + 2 * kDies - 1) / (2 * kDies) : (n_units + kDies - 1) / kDies;
+  const int n_slots = two_parts ? 2 * part : part;
+  int half = -1;  // of the unit's 64 tokens: both, the first, the second
+  if (NG == kMxNG) {
+    const int whole = n_slots - halved_units(n_slots, a.cus_per_die);
+    if (slot >= whole) {
+      half = (slot - whole) & 1;
+      slot = whole + (slot - whole) / 2;
+    }
+  }
   const int unit = slot < part ? die * part + slot : (2 * kDies - 2 - die) * part + slot;  // (the part 2 kDies - 1 - die)
-  if (slot >= (two_parts ? 2 : 1) * part || unit >= n_units) return;
+  if (slot >= n_slots || unit >= n_units) return;
   const int mt = unit / a.n_ntiles;
   int nt = unit - mt * a.n_ntiles;
   const WorkDesc* wd = a.desc + a.mtiles[2 * mt];
@@ -589,7 +605,10 @@ __global__ __launch_bounds__(64 * kMxWaves, NG == 2 ? 3 : 2) void expert_gemm_mx
     nt = r / tiles_e;
     m0 = (r - nt * tiles_e) * kGemmBM;
   }
-  const int mcount = min(kGemmBM, wd->Te - m0);
+  int mcount = min(kGemmBM, wd->Te - m0);
+  if (half == 1) m0 += 32, mcount -= 32;
+  if (half >= 0) mcount = min(mcount, 32);
+  if (mcount <= 0) return;
   if (mcount <= 32)
     expert_gemm_mx_unit<MODE, NG, 1>(a, wd->w, wd->base + m0, mcount, nt, smem);
   else

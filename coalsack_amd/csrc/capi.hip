@@ -754,7 +754,7 @@ int launch_dispatch(const int* ids, const float* pairs, int64_t P, int64_t k, in
   return check_launch("dispatch_scatter_kernel");
 }
 
-template <int MODE, int NS, bool ROUTE1, bool ROWS3>
+template <int MODE, int NS, int ROUTE, bool ROWS3>
 int launch_stream_form(ExpertStreamArgs a, int64_t P) {
   // kStreamWgPerCu workgroups per compute unit in steady state (one where the rows of a
   // group take more than half of the LDS, kRouteOneWgPerCu of the form that routes one token and copies its row: its launch
@@ -762,31 +762,32 @@ int launch_stream_form(ExpertStreamArgs a, int64_t P) {
   // resident workgroup of its own gets that
   constexpr int TU = MODE == 0 ? stream_tiles(NS) / 2 : stream_tiles(NS);
   size_t lds = stream_lds_bytes(NS, a.group_tokens);
-  if (ROUTE1) lds = std::max(lds, sizeof(RouteOneLds));  // a close call is recomputed where the rows go afterwards
+  if (ROUTE) lds = std::max(lds, sizeof(RouteOneLds));  // a close call is recomputed where the rows go afterwards
   const int64_t units = cdiv(a.ntile, TU);
-  const int64_t places = (ROUTE1 && ROWS3 ? kRouteOneWgPerCu : lds <= kStreamLdsHalf ? kStreamWgPerCu : 1) * (int64_t)std::max(g_cus, 1);
+  const size_t table = ROUTE > 1 ? kMaxExperts * sizeof(ExpertW) + 1024 : 0;  // its static LDS
+  const int64_t places = (ROUTE == 1 && ROWS3 ? kRouteOneWgPerCu : lds + table <= kStreamLdsHalf ? kStreamWgPerCu : 1) * (int64_t)std::max(g_cus, 1);
   const int64_t nwg = std::min(P * units, places);
   static bool lds_attr_set = false;  // per instantiation: dynamic LDS beyond the default limit is asked for once
   if (!lds_attr_set) {
-    HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(&expert_stream_kernel<MODE, NS, ROUTE1, ROWS3>),
+    HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(&expert_stream_kernel<MODE, NS, ROUTE, ROWS3>),
                                 hipFuncAttributeMaxDynamicSharedMemorySize,
                                 (int)std::max(stream_lds_bytes(NS, kStreamG), sizeof(RouteOneLds))));
     lds_attr_set = true;
   }
-  launch_expert_kernel(MODE, expert_stream_kernel<MODE, NS, ROUTE1, ROWS3>, dim3((unsigned)nwg), dim3(256), lds, a);
+  launch_expert_kernel(MODE, expert_stream_kernel<MODE, NS, ROUTE, ROWS3>, dim3((unsigned)nwg), dim3(256), lds, a);
   return check_launch("expert_stream_kernel");
 }
-template <int MODE, bool ROUTE1, bool ROWS3>
+template <int MODE, int ROUTE, bool ROWS3>
 int launch_stream_steps(const ExpertStreamArgs& a, int64_t P) {
   switch (stream_steps(a.nblk)) {
-    case 2: return launch_stream_form<MODE, 2, ROUTE1, ROWS3>(a, P);
-    case 3: return launch_stream_form<MODE, 3, ROUTE1, ROWS3>(a, P);
-    case 4: return launch_stream_form<MODE, 4, ROUTE1, ROWS3>(a, P);
-    case 5: return launch_stream_form<MODE, 5, ROUTE1, ROWS3>(a, P);
-    case 6: return launch_stream_form<MODE, 6, ROUTE1, ROWS3>(a, P);
-    case 8: return launch_stream_form<MODE, 8, ROUTE1, ROWS3>(a, P);
-    case 12: return launch_stream_form<MODE, 12, ROUTE1, ROWS3>(a, P);
-    default: return launch_stream_form<MODE, 16, ROUTE1, ROWS3>(a, P);
+    case 2: return launch_stream_form<MODE, 2, ROUTE, ROWS3>(a, P);
+    case 3: return launch_stream_form<MODE, 3, ROUTE, ROWS3>(a, P);
+    case 4: return launch_stream_form<MODE, 4, ROUTE, ROWS3>(a, P);
+    case 5: return launch_stream_form<MODE, 5, ROUTE, ROWS3>(a, P);
+    case 6: return launch_stream_form<MODE, 6, ROUTE, ROWS3>(a, P);
+    case 8: return launch_stream_form<MODE, 8, ROUTE, ROWS3>(a, P);
+    case 12: return launch_stream_form<MODE, 12, ROUTE, ROWS3>(a, P);
+    default: return launch_stream_form<MODE, 16, ROUTE, ROWS3>(a, P);
   }
 }
 template <int MODE>
@@ -795,11 +796,14 @@ int launch_stream(ExpertStreamArgs a, int64_t P, Workspace& ws) {
   a.nv = ws.nv;
   if constexpr (MODE == 0) {
     const bool rows3 = a.X3 != nullptr && a.gather_w == nullptr;
-    if (a.rin.logits)  // one token, routed by the kernel itself
-      return rows3 ? launch_stream_steps<MODE, true, true>(a, P) : launch_stream_steps<MODE, true, false>(a, P);
-    if (rows3) return launch_stream_steps<MODE, false, true>(a, P);
+    if (a.rin.logits && a.rin.T > 1)  // a few tokens, routed by the kernel itself
+      return rows3 ? launch_stream_steps<MODE, kRouteFewTokens, true>(a, P)
+                   : fail(CSK_ERR_STATE, "in-kernel routing of several tokens is for rows as FP6 terms");
+    if (a.rin.logits)  // one token
+      return rows3 ? launch_stream_steps<MODE, 1, true>(a, P) : launch_stream_steps<MODE, 1, false>(a, P);
+    if (rows3) return launch_stream_steps<MODE, 0, true>(a, P);
   }
-  return launch_stream_steps<MODE, false, false>(a, P);
+  return launch_stream_steps<MODE, 0, false>(a, P);
 }
 
 template <int MODE>
@@ -918,7 +922,7 @@ int run_experts(int64_t E, int64_t T, int64_t k, int64_t H, int64_t F,
   a.y_out = nullptr;
   if (timed) mark(CSK_STAGE_GATEUP);
   if (in.rin && in.rout) {
-    if (!passes || T != 1) return fail(CSK_ERR_STATE, "in-kernel routing is for one token on the streaming path");
+    if (!passes || T > kRouteFewTokens) return fail(CSK_ERR_STATE, "in-kernel routing is for up to eight tokens on the streaming path");
     a.rin = *in.rin, a.rout = *in.rout;
   }
   int rc = launch_experts<2>(a, in.x_mx3, ws.act, E, T, P, ws, path);
@@ -1932,6 +1936,15 @@ int64_t g_pass_tokens = 32768;
 // tokens 985 / 996, 32 tokens 1150 / 1145, 64 tokens 1684 / 1635).
 constexpr int64_t kRouteSmallTokens = 31;
 static_assert(kRouteSmallTokens * kMaxTopK <= kRouteSmallMaxP, "what its LDS is laid out for");
+// Batches of several tokens that the gate/up kernel routes itself.  Up to four tokens its waves select for one each, beside one
+// another, and a launch of 6 us goes (8 layers, us, with that launch / without: 32 experts of 2880 x 2880, top-4, 2 tokens 317 /
+// 290, 4 tokens 424 / 400; 64 of 2048 x 768, top-8, 4 tokens 321 / 294).  Beyond, a second selection per wave and the
+// walk over all assignments weigh against a routing kernel of sixteen waves: top-4 5 tokens 462 / 454, 6 tokens 507 / 502, 8 tokens
+// 566 / 566, 10 tokens 621 / 634, 16 774 / 810; top-8 6 tokens 345 / 363; 64 experts, top-1, 8 tokens 201 / 192; 16 of 1024 x
+// 512, top-2, 6 tokens 191 / 189, 12 tokens 209 / 216.
+bool routed_by_experts(int64_t T, int64_t P) {
+  return T <= kRouteTinyTokens ? P <= kRouteTinyMaxP : T <= kRouteFewTokens && P <= 24;
+}
 // phase 0: the whole forward; 1: up to and including the dispatch (router output and lists
 // are in ws); 2: the rest (experts and combine) of a pass whose phase 1 ran in the same ws.
 // pairs_out: takes a copy of the router output, if given.
@@ -1982,9 +1995,9 @@ int forward_pass(csk_layer* L, const float* hidden, int64_t T, float* out, int f
                 (int)T, (int)L->E, (int)L->k, (int)L->H, L->sigmoid, group_tokens(path, T), groups ? kListGroups : kListDesc};
     RouteOut rout{ws.pairs, ws.ids, ws.pos, ws.counts, ws.offsets, ws.desc, ws.groups, ws.nv,
                   ws.tiles, ws.n_tiles, ws.list_tok, ws.list_w};
-    if (T == 1 && phase == 0 && L->E > 1 && passes) {
-      // one token: the gate/up kernel routes it itself (no launch here); phases keep the
-      // routing kernel, whose output they hand out before the experts run
+    if (phase == 0 && passes && (T == 1 ? L->E > 1 : rows_mx3 && routed_by_experts(T, P))) {
+      // a token or a few: the gate/up kernel routes them itself (no launch here); phases keep the
+      // routing kernel, whose output they hand out before the experts run, and so do rows that the routing weight multiplies
       route_in_kernel = true;
       rin_kept = rin, rout_kept = rout;
     } else if (T <= kRouteTinyTokens && P <= kRouteTinyMaxP && passes) {

@@ -118,7 +118,7 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t stream_plane_rsrc(const void* 
 }
 
 //
-// ROUTE1 (gate/up of a one-token batch): there is no routing kernel in front.  Every
+// ROUTE = 1 (gate/up of a one-token batch): there is no routing kernel in front.  Every
 // workgroup selects the token's k experts itself from the logits -- select_topk in each of
 // its four waves, so that nothing passes from wave to wave; a close call recomputed by the
 // whole workgroup, exactly as route_tiny_kernel does; all workgroups compute the same thing
@@ -129,6 +129,12 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t stream_plane_rsrc(const void* 
 // positions, lists, counts, token groups) for the down kernel, the combine and
 // csk_layer_last_dispatch.  A 5.4 us launch with its dependent reads is replaced by 3 us in
 // front of this kernel's first weight loads (120b shape: 32.6 -> 30.0 us per layer).
+//
+// ROUTE = kRouteFewTokens (gate/up of up to eight tokens with at most 64 assignments): the same for a few tokens.  Wave w
+// selects for tokens w and w + 4, the selections meet in LDS, and from there each wave places all of them, an assignment
+// per lane, as route_tiny_kernel does; the workgroup's token group, its place and its tokens then come out of ballots, and
+// how many groups there are, which the teams go by, is known only here (8 layers of 2880 x 2880, 2 tokens 317 -> 290 us, of which a
+// launch and its dependent reads are 27; a two-token host frame 54.6 -> 51.5).
 //
 // Shape of a work unit.  Twelve or more 1 KiB weight loads in flight per wave keep the memory
 // system busy; a K of 2880 gives that from two tiles of six steps, a shorter one walks fewer
@@ -152,9 +158,11 @@ constexpr size_t stream_lds_bytes(int ns, int group_tokens) {
   return (size_t)group_tokens * ns * 16 * 96 + (size_t)2 * 4 * (4 * stream_tiles(ns)) * 16 * sizeof(float);
 }
 
-template <int MODE, int NS, bool ROUTE1 = false, bool ROWS3 = false>
-__global__ __launch_bounds__(256, ROUTE1 && ROWS3 ? kRouteOneWgPerCu : 2) void expert_stream_kernel(ExpertStreamArgs a) {
-  static_assert(!ROUTE1 || MODE == 0, "the gate/up kernel is the one that routes");
+template <int MODE, int NS, int ROUTE = 0, bool ROWS3 = false>
+__global__ __launch_bounds__(256, ROUTE == 1 && ROWS3 ? kRouteOneWgPerCu : 2) void expert_stream_kernel(ExpertStreamArgs a) {
+  static_assert(ROUTE == 0 || MODE == 0, "the gate/up kernel is the one that routes");
+  static_assert(ROUTE <= 1 || (ROUTE == kRouteFewTokens && ROWS3), "several tokens: rows that are only copied");
+  constexpr bool ROUTE1 = ROUTE == 1;
   constexpr int NT = stream_tiles(NS);  // weight tiles per unit
   constexpr int TU = MODE == 0 ? NT / 2 : NT; // tiles of one plane per unit
   constexpr int ND = stream_depth(NS);        // K steps whose weights are held or in flight
@@ -173,11 +181,17 @@ __global__ __launch_bounds__(256, ROUTE1 && ROWS3 ? kRouteOneWgPerCu : 2) void e
   // Teams of W workgroups share one token group and interleave its units
   // (workgroup j takes units j, j + W, ...), so that at any moment a team reads one
   // contiguous window of the expert's planes.
-  const int nvv = a.nv_known > 0 ? a.nv_known : *a.nv;  // one dependent read fewer in front of the first weights
-  const int W = max(1, (int)gridDim.x / max(nvv, 1));
-  const int teams = gridDim.x / W;
-  const int team = blockIdx.x / W, tj = blockIdx.x % W;
-  if (team >= teams || tj >= npair) return;
+  int nvv = 0, W = 1, teams = 1, team = 0, tj = 0;
+  auto take_place = [&](int groups) {  // false: no work for this workgroup
+    nvv = groups;
+    W = max(1, (int)gridDim.x / max(nvv, 1));
+    teams = gridDim.x / W;
+    team = blockIdx.x / W, tj = blockIdx.x % W;
+    return team < teams && tj < npair;
+  };
+  if constexpr (ROUTE <= 1) {
+    if (!take_place(a.nv_known > 0 ? a.nv_known : *a.nv)) return;  // (known: one dependent read fewer in front of the first weights)
+  }
   const int lane = threadIdx.x & 63;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform, and known to be: it is part of the weight loads' scalar offsets
   const int n = lane & 15, g = lane >> 4;
@@ -187,7 +201,7 @@ __global__ __launch_bounds__(256, ROUTE1 && ROWS3 ? kRouteOneWgPerCu : 2) void e
   int r_idx = 0;
   float r_wt = 0.0f;
   constexpr int kEwWords = kMaxExperts * (int)(sizeof(ExpertW) / 8), kEwPerThread = (kEwWords + 255) / 256;
-  __shared__ unsigned long long s_ew[ROUTE1 ? kEwWords : 1];  // the experts' weight pointers, staged beside the logits
+  __shared__ unsigned long long s_ew[ROUTE ? kEwWords : 1];  // the experts' weight pointers, staged beside the logits
   if constexpr (ROUTE1) {
     const RouteIn& r = a.rin;
     const int E = r.E, k = r.k;
@@ -256,6 +270,122 @@ __global__ __launch_bounds__(256, ROUTE1 && ROWS3 ? kRouteOneWgPerCu : 2) void e
     }
   }
 
+  // ROUTE > 1: assignment p = token * k + slot in lane p of every wave
+  int r_lower = 0, r_same = 0, r_before = 0;  // assignments of lower experts, of its own, and of its own from earlier tokens
+  int r_group = 0;                            // token groups in front of the one that it begins ...
+  bool r_first = false;                       // ... if it begins one
+  if constexpr (ROUTE > 1) {
+    const RouteIn& r = a.rin;
+    const int E = r.E, k = r.k, T = r.T, P = T * k;
+    RouteOneLds& cc = *reinterpret_cast<RouteOneLds*>(smem);
+    __shared__ int s_ids[kRouteTinyMaxP], s_cc[kRouteFewTokens];
+    __shared__ float s_wt[kRouteTinyMaxP], s_lo[kRouteFewTokens], s_hi[kRouteFewTokens];
+    const float NEG = -__builtin_inff();
+    constexpr int kTurns = kRouteFewTokens / 4;  // wave w selects for tokens w, w + 4, ...
+    float v[kTurns][4];
+#pragma unroll
+    for (int q = 0; q < kTurns; ++q) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int t = wv + 4 * q, e = lane + 64 * j;
+        v[q][j] = t < T && e < E ? r.logits[(size_t)t * E + e] : NEG;
+      }
+    }
+    unsigned long long ew_reg[kEwPerThread];
+#pragma unroll
+    for (int i = 0; i < kEwPerThread; ++i) {
+      const int w = threadIdx.x + i * 256;
+      ew_reg[i] = w < E * (int)(sizeof(ExpertW) / 8) ? reinterpret_cast<const unsigned long long*>(r.ew)[w] : 0ull;
+    }
+    const float tol = close_call_tolerance(r.H);
+    auto publish = [&](int t, float my_val, int my_idx, float vmax) {
+      const float w = routing_weight(my_val, vmax, lane, k, r.sigmoid);
+      if (lane < k) s_ids[t * k + lane] = my_idx, s_wt[t * k + lane] = w;
+    };
+    bool close_any = false;
+#pragma unroll 1  // one copy of the selection code: the token in turn sits in v[0], the others move up
+    for (int t = wv; t < T; t += 4) {
+      float my_val, vmax;
+      int my_idx;
+      bool close_call;
+      select_topk(v[0], lane, E, k, my_val, my_idx, vmax, close_call, tol);
+      if (lane == 0) s_cc[t] = close_call;
+      if (close_call) {
+        float lo, hi;
+        close_call_range(my_val, lane, E, k, tol, lo, hi);
+        if (lane == 0) s_lo[t] = lo, s_hi[t] = hi;
+        close_any = true;
+      } else {
+        publish(t, my_val, my_idx, vmax);
+      }
+#pragma unroll
+      for (int q = 0; q + 1 < kTurns; ++q)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[q][j] = v[q + 1][j];
+    }
+#pragma unroll
+    for (int i = 0; i < kEwPerThread; ++i) {
+      const int w = threadIdx.x + i * 256;
+      if (w < kEwWords) s_ew[w] = ew_reg[i];
+    }
+    if (__syncthreads_or(close_any)) {
+      for (int t = 0; t < T; ++t) {
+        if (!s_cc[t]) continue;
+        logits_reference_order_wg(r.x + (size_t)t * r.H, r.g, r.b, r.logits + (size_t)t * E, E, r.H, s_lo[t], s_hi[t], cc);
+        if (wv == 0) {
+          float vt[4], my_val, vmax;
+          int my_idx;
+          bool close_call;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const int e = lane + 64 * j;
+            vt[j] = e < E ? cc.fixed[e] : NEG;
+          }
+          select_topk(vt, lane, E, k, my_val, my_idx, vmax, close_call, 0.0f);
+          publish(t, my_val, my_idx, vmax);
+        }
+        __syncthreads();
+      }
+    }
+    const bool lp = lane < P;
+    r_idx = lp ? s_ids[lane] : 0x7fffffff;
+    for (int q = 0; q < P; ++q) {  // q is the same in every lane
+      const int idq = __builtin_amdgcn_readlane(r_idx, q);
+      r_lower += idq < r_idx;
+      r_same += idq == r_idx;
+      r_before += idq == r_idx && q < lane;
+    }
+    r_first = lp && r_before % G == 0;
+    const unsigned long long firsts = __ballot(r_first);
+    for (unsigned long long m = firsts; m != 0ull; m &= m - 1ull) {
+      const int q = (int)__builtin_ctzll(m), idq = __builtin_amdgcn_readlane(r_idx, q);
+      r_group += idq < r_idx || (idq == r_idx && q < lane);
+    }
+    if (blockIdx.x == 0) {
+      // what the routing kernel would have written (see the one-token form for where to)
+      auto args = (const __attribute__((address_space(4))) ExpertStreamArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+      asm volatile("" : "+s"(args));
+      const auto& o = args->rout;
+      for (int e = threadIdx.x; e < E; e += 256) {
+        int c = 0;
+        for (int q = 0; q < P; ++q) c += s_ids[q] == e;
+        o.counts[e] = c;
+      }
+      if (wv == 0 && lp) {
+        const int pos = r_lower + r_before;
+        const unsigned inv_k = (65536u + (unsigned)k - 1u) / (unsigned)k;  // p / k == p * inv_k >> 16 for p < 64, k <= 16
+        reinterpret_cast<float2*>(o.pairs)[lane] = make_float2((float)r_idx, s_wt[lane]);
+        o.ids[lane] = r_idx;
+        o.list_tok[pos] = (int)(((unsigned)lane * inv_k) >> 16);
+        o.list_w[pos] = s_wt[lane];
+        o.pos_of_slot[lane] = pos;
+        if (r_first) write_stream_group(o.groups + r_group, reinterpret_cast<const ExpertW*>(s_ew) + r_idx, r_idx, r_same - r_before, pos);
+        if (lane == 0) *o.nv = __popcll(firsts);
+      }
+    }
+    if (!take_place(__popcll(firsts))) return;
+  }
+
   // a lane's scale bytes of one tile: 2, 4, 8 or 16, one per step of the wave rounded up (scale_slots)
   constexpr int kScWords = NS <= 4 ? 1 : NS <= 8 ? 2 : 4;
   typedef uint32_t ScaleWords __attribute__((ext_vector_type(kScWords)));
@@ -281,9 +411,25 @@ __global__ __launch_bounds__(256, ROUTE1 && ROWS3 ? kRouteOneWgPerCu : 2) void e
       r_e = __builtin_amdgcn_readlane(r_idx, sl);
       r_gw = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(r_wt), sl));
     }
-    const ExpertW* gw_ptr = ROUTE1 ? reinterpret_cast<const ExpertW*>(s_ew) + r_e : &gr->w;
-    const int gcount = ROUTE1 ? 1 : min(a.group_tokens, gr->left);
-    const int base = ROUTE1 ? v : gr->base;
+    int r_base = 0, r_count = 0;
+    int r_tok[G] = {};
+    if constexpr (ROUTE > 1) {  // the group with v groups before it, and its tokens: the assignments that name its expert
+      const int sl = (int)__builtin_ctzll(__ballot(r_first && r_group == v) | (1ull << 63));
+      const int skip = __builtin_amdgcn_readlane(r_before, sl);
+      r_e = __builtin_amdgcn_readlane(r_idx, sl);
+      r_base = __builtin_amdgcn_readlane(r_lower, sl) + skip;
+      r_count = min(G, __builtin_amdgcn_readlane(r_same, sl) - skip);
+      const unsigned inv_k = (65536u + (unsigned)a.rin.k - 1u) / (unsigned)a.rin.k;
+      unsigned long long named = __ballot(r_idx == r_e && r_before >= skip);
+#pragma unroll
+      for (int i = 0; i < G; ++i) {
+        r_tok[i] = named != 0ull ? (int)(((unsigned)__builtin_ctzll(named) * inv_k) >> 16) : r_tok[i > 0 ? i - 1 : 0];
+        named &= named - 1ull;
+      }
+    }
+    const ExpertW* gw_ptr = ROUTE ? reinterpret_cast<const ExpertW*>(s_ew) + r_e : &gr->w;
+    const int gcount = ROUTE1 ? 1 : ROUTE ? r_count : min(a.group_tokens, gr->left);
+    const int base = ROUTE1 ? v : ROUTE ? r_base : gr->base;
     // One buffer descriptor per weight plane: the unit's tile and the K step go into the
     // scalar offset of a load, the lane's place within the step (block g, row n) into its
     // vector offset, which never changes.
@@ -334,7 +480,7 @@ __global__ __launch_bounds__(256, ROUTE1 && ROWS3 ? kRouteOneWgPerCu : 2) void e
 #pragma unroll
       for (int rr = 0; rr < G; ++rr) {
         const int p = base + min(rr, gcount - 1);
-        copy_row[rr] = ROUTE1 ? 0 : a.list_row ? a.list_row[p] : p;
+        copy_row[rr] = ROUTE1 ? 0 : ROUTE ? r_tok[rr] : a.list_row ? a.list_row[p] : p;
       }
     }
     float4 pre[8];

@@ -363,6 +363,10 @@ __device__ __forceinline__ void write_work_desc(WorkDesc* d, bool on, int e, int
 }
 
 
+constexpr int kRouteTinyTokens = 4;  // a wave of a workgroup of four selects for each
+constexpr int kRouteTinyMaxP = 64;   // their assignments: one per lane
+constexpr int kRouteFewTokens = 8;   // tokens that the gate/up kernel may route itself
+
 // ------------------------------------- small batches: top-k + dispatch, fused
 // One workgroup does, for P = T * k <= MAXP assignments, what router_topk_kernel and
 // dispatch_scatter_kernel do in two launches: top-k and weights per token (one wave per

@@ -724,8 +724,6 @@ __global__ __launch_bounds__(kRouteSmallThreads) void route_small_kernel(RouteIn
 // token group of the weight-streaming kernels.  Writes what those kernels, the combine and
 // csk_layer_last_dispatch read: pairs, ids, positions, the lists, counts, the token groups
 // and their number; the grouped GEMM's descriptors and tiles are not written.
-constexpr int kRouteTinyTokens = 4;
-constexpr int kRouteTinyMaxP = 64;
 __global__ __launch_bounds__(256) void route_tiny_kernel(RouteIn r, RouteOut o) {
   __shared__ CloseCallLdsT<256, kCcBatch> cc;
   __shared__ float cc_lo[4], cc_hi[4];

@@ -120,6 +120,7 @@ constexpr uint32_t kScalesOfOne = 0x7f7f7f7f;  // four E8M0 bytes
 constexpr int64_t kStreamMaxP = 2048;
 constexpr size_t kWeightSlack = 32768;  // bytes of mapped memory kept behind weight planes (the expert kernels read whole K steps: up to three blocks, 768 bytes, past the last tile)
 constexpr int kStreamWgPerCu = 2;  // resident workgroups of the streaming kernel per compute unit (kRouteOneWgPerCu of one form) ...
+constexpr size_t kMergeLdsMost = 160 * 1024;  // one workgroup per compute unit
 constexpr size_t kStreamLdsHalf = 80 * 1024 - 512;  // ... if each takes no more LDS than this (and its few static words)
 
 // ---- workspace shared by every layer (single stream, one call at a time) --
@@ -806,6 +807,43 @@ int launch_stream(ExpertStreamArgs a, int64_t P, Workspace& ws) {
   return launch_stream_steps<MODE, 0, false>(a, P);
 }
 
+// The down projection and the merge of a few tokens in one launch (expert_stream_kernel_merge).
+template <int NT>
+int launch_merge_steps(const ExpertMergeArgs& a) {
+  auto launch = [&](auto ns) {
+    constexpr int NS = decltype(ns)::value;
+    const size_t lds = merge_lds_bytes(NS, NT, a.T * a.k);
+    static bool lds_attr_set = false;
+    if (!lds_attr_set) {
+      HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(&expert_stream_kernel_merge<NS, NT>),
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMergeLdsMost));
+      lds_attr_set = true;
+    }
+    launch_expert_kernel(1, expert_stream_kernel_merge<NS, NT>, dim3((unsigned)cdiv(a.ntile, NT)), dim3(256 * merge_teams(NS, NT)), lds, a);
+    return check_launch("expert_stream_kernel_merge");
+  };
+  switch (stream_steps(a.nblk)) {
+    case 2: return launch(std::integral_constant<int, 2>{});
+    case 3: return launch(std::integral_constant<int, 3>{});
+    case 4: return launch(std::integral_constant<int, 4>{});
+    case 5: return launch(std::integral_constant<int, 5>{});
+    case 6: return launch(std::integral_constant<int, 6>{});
+    case 8: return launch(std::integral_constant<int, 8>{});
+    case 12: return launch(std::integral_constant<int, 12>{});
+    default: return launch(std::integral_constant<int, 16>{});
+  }
+}
+// Its tiles per workgroup, or 0: two launches.  The assignments are those up to which one launch is the faster: more mean a
+// second round of groups and longer waits for the rows' quantisation, the sooner the longer the rows are (8 layers, us, two
+// launches / one: rows of 768, 64 experts, top-8 190 / 175, sixteen assignments 236 / 247; 2048, top-5 203 / 191, eight 226 /
+// 230; 2880, top-4 232 / 220, top-5 257 / 254, eight 296 / 308; one layer: 6144, two 26.9 / 25.4, four 37.9 / 37.7; 8192, one
+// 27.1 / 26.2, two 39.8 / 39.8, four 67 / 71).
+int merge_tiles(int64_t P, int64_t H, int64_t F) {
+  const int ns = stream_steps((int)(F / 32)), nt = cdiv(H, 16) <= std::max(g_cus, 1) ? 1 : 2;
+  if (P > (ns <= 3 ? (nt == 1 ? 8 : 6) : ns <= 8 ? 4 : 2) || cdiv(H, 16 * nt) > std::max(g_cus, 1)) return 0;
+  return merge_lds_bytes(ns, nt, (int)P) <= kMergeLdsMost ? nt : 0;
+}
+
 template <int MODE>
 int launch_tiles(ExpertGemmMxArgs& ga, int64_t E, int64_t P) {
   using Geom = MxGeom<2, 2>;
@@ -894,8 +932,10 @@ struct ExpertInput {
   const uint16_t* x_mx3;
   const int* mx3_list_row;
   const uint16_t* x_mx3_tokens = nullptr;  // streaming path: the token rows already as FP6 terms (written by the routing prologue)
-  const RouteIn* rin = nullptr;    // both set: a one-token batch that the gate/up kernel routes itself
+  const RouteIn* rin = nullptr;    // both set: a batch that the gate/up kernel routes itself
   const RouteOut* rout = nullptr;
+  const ExpertMergeArgs* merge = nullptr;  // set: where the merged rows go (the output and what the merge needs), merge_tiles of them
+  int merge_tiles = 0;                     // per workgroup
 };
 
 // Experts' MLPs over the dispatched tokens: ws.y[P,H] <- down(act(gate, up)).
@@ -929,6 +969,13 @@ int run_experts(int64_t E, int64_t T, int64_t k, int64_t H, int64_t F,
   if (rc != CSK_OK) return rc;
   a.rin = RouteIn{}, a.rout = RouteOut{};
   if (timed) mark(CSK_STAGE_DOWN);
+  if (in.merge) {
+    ExpertMergeArgs m = *in.merge;
+    m.act = reinterpret_cast<const float*>(ws.act);
+    m.groups = ws.groups, m.nv = ws.nv, m.nv_known = a.nv_known;
+    m.T = (int)T, m.k = (int)k, m.nblk = (int)(F / 32), m.N = (int)H, m.ntile = (int)cdiv(H, 16);
+    return in.merge_tiles == 1 ? launch_merge_steps<1>(m) : launch_merge_steps<2>(m);
+  }
   // down
   a.list_row = nullptr;
   a.gather_w = nullptr;
@@ -2054,11 +2101,20 @@ int forward_pass(csk_layer* L, const float* hidden, int64_t T, float* out, int f
     in.x_mx3 = ws.xg;
     in.mx3_list_row = nullptr;
   }
+  ExpertMergeArgs merge{};
+  if (const int nt = passes && phase == 0 ? merge_tiles(P, L->H, L->F) : 0) {
+    merge.pairs = ws.pairs, merge.pos_of_slot = ws.pos;
+    merge.residual = (flags & CSK_FWD_RESIDUAL) ? hidden : nullptr;
+    merge.out = out;
+    merge.pairs_out = reinterpret_cast<float2*>(pairs_out);
+    merge.pre_weighted = L->wbf;
+    in.merge = &merge, in.merge_tiles = nt;
+  }
   rc = run_experts(L->E, T, L->k, L->H, L->F, L->act, in, ws, path, true);
   if (rc != CSK_OK) return rc;
   mark(CSK_STAGE_COMBINE);
-  rc = launch_combine(ws.y, ws.pairs, ws.pos, (flags & CSK_FWD_RESIDUAL) ? hidden : nullptr, out, T,
-                      L->k, L->H, L->wbf, pairs_out);
+  if (!in.merge)
+    rc = launch_combine(ws.y, ws.pairs, ws.pos, (flags & CSK_FWD_RESIDUAL) ? hidden : nullptr, out, T, L->k, L->H, L->wbf, pairs_out);
   mark(CSK_N_STAGES);
   g_stage_valid = g_timing;
   return rc;

@@ -672,4 +672,219 @@ __global__ __launch_bounds__(256, ROUTE == 1 && ROWS3 ? kRouteOneWgPerCu : 2) vo
   }
 }
 
+// ---------------------------------------------------------------------------
+// Down projection and merge of a few tokens in one launch: a workgroup owns NT tiles of 16 output features for all token groups
+// of the batch, so that the weighted sum over a token's experts (combine_kernel) needs nothing from another workgroup.
+// Its waves are teams of four; a team takes every second or fourth group, its waves split K as those of expert_stream_kernel
+// do, and the same partial sums are added in the same order, then weighted and added slot by slot as combine_kernel does: the
+// same bits.  The rows of all assignments are quantised into LDS once, beside the first groups' weights on their way:
+// those of four groups are requested at the start, by four teams, or by two with two register sets where a row's steps
+// take more registers than sixteen waves can have.  A workgroup streams the tiles of all active experts, with one
+// workgroup on two compute units of three, so this is for batches whose weights are on their way in one or two
+// rounds of latency, of which the launch that the merge needs costs another (8 layers, us, two launches / one: 32
+// experts of 2880 x 2880, one token, top-4 230.4 / 218.9, top-2 177 / 163; 64 of 2048 x 768, top-1 141 / 119, top-4 156 / 143; two tokens,
+// top-4, eight assignments of 2880 x 2880 290 / 308).
+struct ExpertMergeArgs {
+  const float* act;  // [P][32 nblk] fp32, by packed position
+  const StreamGroup* groups;
+  const int* nv;
+  int nv_known;      // > 0: the number of groups
+  int T, k, nblk, N, ntile;
+  const float* pairs;      // [T, k, 2]
+  const int* pos_of_slot;  // [T * k]
+  const float* residual;   // null: none
+  float* out;              // [T, N]
+  float2* pairs_out;       // takes a copy of the router output, if given
+  int pre_weighted;
+};
+constexpr int merge_teams(int ns, int nt) { return ns <= 3 && nt == 1 ? 4 : 2; }
+constexpr size_t merge_lds_bytes(int ns, int nt, int P) {
+  return (size_t)P * ns * 16 * 96 + (size_t)2 * merge_teams(ns, nt) * 4 * 4 * nt * 16 * 4 + (size_t)P * nt * 16 * 4 + (size_t)P * 8;
+}
+
+template <int NS, int NT>
+__global__ __launch_bounds__(256 * merge_teams(NS, NT)) void expert_stream_kernel_merge(ExpertMergeArgs a) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  constexpr int kMergeTeams = merge_teams(NS, NT), kMergeThreads = 256 * kMergeTeams, kSets = 4 / kMergeTeams;
+  constexpr int ND = stream_depth(NS), lrb = NS * 16, NV = 4 * NT;
+  const int P = a.T * a.k, nblk = a.nblk;
+  u32x4* const As = reinterpret_cast<u32x4*>(smem);                                               // [P][lrb][3 terms][2]
+  float* const red = reinterpret_cast<float*>(smem + (size_t)P * lrb * kMx3ChunksPerBlock * 16);  // [2][teams][4][NV][16]
+  float* const ys = red + 2 * kMergeTeams * 4 * NV * 16;                                          // [P][NT * 16]
+  int* const s_pos = reinterpret_cast<int*>(ys + P * NT * 16);
+  float* const s_wt = reinterpret_cast<float*>(s_pos + P);
+  const int lane = threadIdx.x & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), team = wid >> 2, wv = wid & 3;
+  const int n = lane & 15, g = lane >> 4;
+  const int nvv = a.nv_known > 0 ? a.nv_known : *a.nv;
+  const int tile0 = blockIdx.x * NT;
+
+  // the first block of activations is requested first (loads return in order), then weights
+  const int nfill = P * lrb;
+  float4 pre[8];
+  auto fetch_block = [&](int idx) {
+    const int rr = idx / lrb, kb = idx - rr * lrb;
+    if (idx < nfill && kb < nblk) {
+      const float4* src = reinterpret_cast<const float4*>(a.act + ((size_t)rr * nblk + kb) * 32);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) pre[i] = src[i];
+    }
+  };
+  fetch_block(threadIdx.x);
+  if ((int)threadIdx.x < P) {
+    s_pos[threadIdx.x] = a.pos_of_slot[threadIdx.x];
+    s_wt[threadIdx.x] = a.pre_weighted ? 1.0f : a.pairs[2 * threadIdx.x + 1];
+  }
+  if (a.pairs_out && blockIdx.x == 0 && (int)threadIdx.x < P)
+    a.pairs_out[threadIdx.x] = reinterpret_cast<const float2*>(a.pairs)[threadIdx.x];
+
+  constexpr int kScWords = NS <= 4 ? 1 : NS <= 8 ? 2 : 4;
+  typedef uint32_t ScaleWords __attribute__((ext_vector_type(kScWords)));
+  using ScaleCell = std::conditional_t<NS == 2, uint16_t, ScaleWords>;
+  struct WSet {
+    u32x4 q[ND][NT];
+    ScaleWords sc[NT];
+    float b[NT];
+    int base, count;
+  };
+  const uint32_t qoff = (uint32_t)((g * 16 + n) * 16);
+  auto tile_of = [&](int m) { return min(tile0 + m, a.ntile - 1); };
+  auto load_step = [&](WSet& ws, __amdgpu_buffer_rsrc_t rsrc, int s) {
+    const uint32_t step = 4 * (wv + 4 * s) >= nblk ? 0u : (uint32_t)(wv + 4 * s) * 1024u;  // (wholly past K: zeros are contracted)
+#pragma unroll
+    for (int m = 0; m < NT; ++m)
+      ws.q[s % ND][m] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, qoff, (uint32_t)tile_of(m) * (uint32_t)nblk * 256u + step, 0);
+  };
+  auto plane = [&](int v) { return stream_plane_rsrc(a.groups[v].w.q_down); };
+  auto load_group = [&](WSet& ws, int v) {
+    const StreamGroup* gr = a.groups + v;
+    const CSK_GLOBAL ScaleCell* sp = as_global(reinterpret_cast<const ScaleCell*>(gr->w.s_down)) + wv * 64 + lane;
+    const CSK_GLOBAL float* bp = as_global(gr->w.b_down);
+    ws.base = gr->base, ws.count = min(kStreamG, gr->left);
+#pragma unroll
+    for (int m = 0; m < NT; ++m) {
+      const int t = tile_of(m);
+      if constexpr (NS == 2) ws.sc[m][0] = sp[(size_t)t * 256];
+      else ws.sc[m] = sp[(size_t)t * 256];
+      ws.b[m] = bp[min(t * 16 + n, a.N - 1)];
+    }
+    const auto rsrc = plane(v);
+#pragma unroll
+    for (int s = 0; s < ND; ++s) load_step(ws, rsrc, s);
+  };
+  WSet ws[kSets];
+#pragma unroll
+  for (int i = 0; i < kSets; ++i)
+    if (team + i * kMergeTeams < nvv) load_group(ws[i], team + i * kMergeTeams);
+
+#pragma unroll 1
+  for (int idx = threadIdx.x; idx < nfill; idx += kMergeThreads) {
+    const int kb = idx % lrb;
+    u32x4* dst = As + (size_t)idx * kMx3ChunksPerBlock;
+    if (idx != (int)threadIdx.x) fetch_block(idx);
+    if (kb >= nblk) {
+#pragma unroll
+      for (int t = 0; t < kMx3Terms; ++t) {
+        dst[2 * t] = u32x4{0u, 0u, 0u, 0u};
+        dst[2 * t + 1] = u32x4{0u, 0u, 127u, 0u};
+      }
+    } else {
+      float r[32];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) r[4 * i] = pre[i].x, r[4 * i + 1] = pre[i].y, r[4 * i + 2] = pre[i].z, r[4 * i + 3] = pre[i].w;
+      mx3_quantize_terms(r, [&](int t, const u32x4& lo, const u32x4& hi) { dst[2 * t] = lo, dst[2 * t + 1] = hi; });
+    }
+  }
+  __syncthreads();  // the rows are in LDS
+
+  // Group v of this team out of ws, which is loaded again with group `next` (if there is one); every thread passes the barrier.
+  auto group = [&](WSet& ws, int v, int next, int par) {
+    float* const rbuf = red + (size_t)(par * kMergeTeams + team) * 4 * NV * 16;
+    int base = 0, count = 0;
+    float bias[NT];
+    if (v < nvv) {
+      base = ws.base, count = ws.count;
+#pragma unroll
+      for (int m = 0; m < NT; ++m) bias[m] = ws.b[m];
+      floatx4 acc[NT];
+#pragma unroll
+      for (int m = 0; m < NT; ++m) acc[m] = floatx4{0.f, 0.f, 0.f, 0.f};
+      int frag = ((base + min(n, count - 1)) * lrb + 4 * wv + g) * kMx3ChunksPerBlock;
+      asm volatile("" : "+v"(frag));  // (fragments are read one ahead of their use, as in expert_stream_kernel)
+      u32x4 flo[2], fhi[2];
+      auto read_frag = [&](int i) {
+        const int s = i / kMx3Terms, t = i - s * kMx3Terms;
+        const u32x4* f = As + frag + (16 * s * kMx3Terms + t) * 2;
+        flo[i & 1] = f[0];
+        fhi[i & 1] = f[1];
+      };
+      read_frag(0);
+      const auto rsrc = plane(v);
+#pragma unroll
+      for (int s = 0; s < NS; ++s) {
+#pragma unroll
+        for (int t = 0; t < kMx3Terms; ++t) {
+          const int i = s * kMx3Terms + t;
+          if (i + 1 < NS * kMx3Terms) read_frag(i + 1);
+          const i32x8 aw = (i32x8)__builtin_shufflevector(flo[i & 1], fhi[i & 1], 0, 1, 2, 3, 4, 5, 6, 7);
+#pragma unroll
+          for (int m = 0; m < NT; ++m) {
+            const int byte = (int)((ws.sc[m][s >> 2] >> (8 * (s & 3))) & 0xFFu);
+            const i32x8 bw = (i32x8)__builtin_shufflevector(ws.q[s % ND][m], ws.q[s % ND][m], 0, 1, 2, 3, -1, -1, -1, -1);
+            acc[m] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(aw, bw, acc[m], 2, 4, 0, aw[6], 0, byte);
+          }
+          // The matrix instructions stay here, where all lanes take part: the results are used by sixteen of them, and moved
+          // behind that condition the instructions would read operands that only those lanes have completed, and
+          // overwrite what the others still hold in the registers.
+#pragma unroll
+          for (int m = 0; m < NT; ++m) asm volatile("" : "+v"(acc[m]));
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        if (s + ND < NS) load_step(ws, rsrc, s + ND);
+      }
+      if (g == 0) {
+#pragma unroll
+        for (int m = 0; m < NT; ++m)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) rbuf[(wv * NV + m * 4 + i) * 16 + n] = acc[m][i];
+      }
+      if (next < nvv) load_group(ws, next);
+    }
+    __syncthreads();
+    if (v < nvv && wv == 0 && g == 0) {
+#pragma unroll
+      for (int m = 0; m < NT; ++m) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int o = m * 4 + i;
+          const float sum = ((rbuf[(0 * NV + o) * 16 + n] + rbuf[(1 * NV + o) * 16 + n]) + rbuf[(2 * NV + o) * 16 + n]) +
+                            rbuf[(3 * NV + o) * 16 + n];
+          if (i < count) ys[(base + i) * (NT * 16) + m * 16 + n] = sum + bias[m];
+        }
+      }
+    }
+  };
+  for (int v = 0; v < nvv; v += 2 * kMergeTeams) {  // v: the first team's; the same count of barriers in every wave
+    group(ws[0], v + team, v + team + kSets * kMergeTeams, 0);
+    group(ws[kSets - 1], v + team + kMergeTeams, v + team + (1 + kSets) * kMergeTeams, 1);
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < a.T * NT * 16; i += kMergeThreads) {
+#pragma clang fp contract(off)  // w * y and the add round separately, as in the reference
+    const int t = i / (NT * 16), c = i - t * (NT * 16), d = tile0 * 16 + c;
+    if (d >= a.N) continue;
+    float acc = 0.0f;
+    for (int s = 0; s < a.k; ++s) {
+      const int pos = s_pos[t * a.k + s];
+      if (pos < 0) continue;  // no expert: skipped, as there
+      const float y = ys[pos * (NT * 16) + c];
+      if (a.pre_weighted) acc = acc + y;
+      else acc = acc + s_wt[t * a.k + s] * y;
+    }
+    const size_t at = (size_t)t * a.N + d;
+    if (a.residual) acc = a.residual[at] + acc;
+    a.out[at] = acc;
+  }
+}
+
 }  // namespace csk

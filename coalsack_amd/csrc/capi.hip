@@ -2605,7 +2605,7 @@ namespace {
 // One work descriptor holding every token (position p = token p) and its 64-token tiles.
 __global__ void dense_desc_kernel(WorkDesc* desc, const ExpertW* ew, int T, int* mtiles, int* n_mtiles) {
   if (threadIdx.x == 0) {
-    write_work_desc(desc, true, 0, T, 0, ew);
+    write_work_desc(desc, true, 0, T, 0, *ew);
     *n_mtiles = (T + 63) / 64;
   }
   for (int i = threadIdx.x; i < (T + 63) / 64; i += blockDim.x) {

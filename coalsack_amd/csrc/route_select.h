@@ -345,21 +345,20 @@ __device__ __forceinline__ float routing_weight(float my_val, float vmax, int la
 // Work descriptor of one active-expert slot (all zero when the slot is unused), written
 // field by field: a local copy of the structure would live in scratch memory.
 __device__ __forceinline__ void write_work_desc(WorkDesc* d, bool on, int e, int Te, int base,
-                                                const ExpertW* __restrict__ ew) {
-  const ExpertW* src = ew + e;
+                                                const ExpertW& w) {
   d->e = e;
   d->Te = on ? Te : 0;
   d->base = on ? base : 0;
   d->pad = 0;
-  d->w.q_gate = on ? src->q_gate : nullptr;
-  d->w.s_gate = on ? src->s_gate : nullptr;
-  d->w.q_up = on ? src->q_up : nullptr;
-  d->w.s_up = on ? src->s_up : nullptr;
-  d->w.q_down = on ? src->q_down : nullptr;
-  d->w.s_down = on ? src->s_down : nullptr;
-  d->w.b_gate = on ? src->b_gate : nullptr;
-  d->w.b_up = on ? src->b_up : nullptr;
-  d->w.b_down = on ? src->b_down : nullptr;
+  d->w.q_gate = on ? w.q_gate : nullptr;
+  d->w.s_gate = on ? w.s_gate : nullptr;
+  d->w.q_up = on ? w.q_up : nullptr;
+  d->w.s_up = on ? w.s_up : nullptr;
+  d->w.q_down = on ? w.q_down : nullptr;
+  d->w.s_down = on ? w.s_down : nullptr;
+  d->w.b_gate = on ? w.b_gate : nullptr;
+  d->w.b_up = on ? w.b_up : nullptr;
+  d->w.b_down = on ? w.b_down : nullptr;
 }
 
 
@@ -614,7 +613,7 @@ __device__ __forceinline__ void route_workgroup(const RouteIn& r, const RouteOut
     for (int i = threadIdx.x; i < E; i += NT) {
       const bool on = i < s.na;
       const int e = on ? s.act_e[i] : 0;
-      write_work_desc(o.desc + i, on, e, s.cnt[e], s.off[e], reinterpret_cast<const ExpertW*>(s.ew));
+      write_work_desc(o.desc + i, on, e, s.cnt[e], s.off[e], reinterpret_cast<const ExpertW*>(s.ew)[e]);
     }
   }
 }

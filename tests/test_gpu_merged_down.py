@@ -13,13 +13,13 @@ pytestmark = pytest.mark.gpu
 
 
 # rows of the down projection of every count of steps per wave; one and two tiles of outputs per workgroup, a last tile that
-# is half empty; fewer groups than teams, more than one round of them, one group for all tokens
+# is half empty; fewer groups than teams, more than one round of them, one group for all tokens, one expert
 @pytest.mark.parametrize("E,H,F,hot,batches", [
     (8, 96, 32, 0, [(1, 1), (1, 8), (2, 4), (8, 1), (3, 2)]), (16, 1056, 1536, 0, [(1, 2), (1, 8), (4, 2)]),
     (9, 8192, 256, 0, [(1, 1), (1, 6), (3, 2)]), (4, 4128, 1504, 2, [(1, 4), (5, 1)]),
     (8, 2880, 2048, 0, [(1, 3), (4, 1)]), (8, 96, 2496, 1, [(1, 4), (2, 2)]), (8, 2080, 2880, 0, [(1, 4), (3, 1)]),
     (6, 4160, 2912, 0, [(2, 2)]), (4, 64, 3584, 0, [(1, 4)]), (4, 4352, 4096, 0, [(1, 4)]), (4, 1024, 6144, 0, [(1, 2), (2, 1)]),
-    (4, 96, 8192, 0, [(1, 1), (1, 2)]), (4, 4128, 8160, 0, [(2, 1)])])
+    (4, 96, 8192, 0, [(1, 1), (1, 2)]), (4, 4128, 8160, 0, [(2, 1)]), (1, 2080, 96, 0, [(1, 1), (3, 1), (8, 1)])])
 @pytest.mark.parametrize("wbf", [False, True])
 def test_one_launch(lib, oracle, E, H, F, hot, batches, wbf):
     for T, k in batches:
